@@ -579,7 +579,7 @@ def bench_pressure_guess(a):
            "unit": "ms", "n_gpus": 1, "higher_is_better": False, "vs_baseline": None, "dtype": "f64",
            "data": "synthetic", "scaling": "weak", "steps": 5, "warmup": 1,
            "config": {"workload": "pressure_guess_box", "grid": main_row["grid"],
-                      "solver": "Jacobi BiCGStab, rtol 1e-10, five kernels per iteration"},
+                      "solver": "BiCGStab preconditioned by a multigrid V-cycle, rtol 1e-10"},
            "grids": rows,
            # one iteration streams 37 FP64 values per node through its five kernels
            # (p: r, p, v, Dinv -> p, y; v: y, 5 coefficients, rhat -> v; s: r, v, y, x,

@@ -28,6 +28,8 @@ struct fvm_ctx {
   fvm_buf popc, popc2;  // population control: per-quarter plan and out list; added markers
   fvm_buf payload;     // bucket-ordered copies of the marker columns a projection reads
   fvm_buf payload_xy;  // bucket-ordered X, Y, Mat: valid while xy_serial == sort_serial
+  fvm_buf mg;          // levels of the nodal solves' preconditioner
+  struct fvm_precond *precond = nullptr;
   fvm_buf reord;       // fvm_markers_reorder: flags, prefix, scan state, order, column staging
   uint64_t sort_serial = 0, xy_serial = 0;
   // columns held in `payload` (slot k = payload + k * stride doubles) for sort
@@ -64,6 +66,16 @@ struct fvm_ctx {
 
 int fvm_set_err(fvm_ctx *ctx, int code, const char *fmt, ...);
 int fvm_ws(fvm_ctx *ctx, fvm_buf &b, size_t bytes);  // ensure workspace capacity
+
+// Preconditioner of a 5-point system on NX x NY nodes (mg.hip): y = M b stands for
+// the system with every row divided by its diagonal d.  scale: the couplings are
+// not divided by d yet.  *out is null where no preconditioner is offered.  It
+// belongs to the context and lasts until the next build.
+struct fvm_precond;
+int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const double *e, const double *w, const double *s,
+                      const double *n, bool scale, fvm_precond **out);
+int fvm_precond_apply(fvm_ctx *ctx, const fvm_precond *m, const double *b, double *y);
+void fvm_precond_free(fvm_precond *m);
 
 #define FVM_HIP(ctx, call)                                                               \
   do {                                                                                   \
@@ -484,7 +496,7 @@ int fvm_advect_with_subgrid_t2(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays 
                                const BoundaryValues *bv, double dt, const double *deltaT, const double *dTsub,
                                double dt_thermal);
 
-// Jacobi BiCGStab (pressure_guess.hip) on a 5-point system over the NX*NY
+// BiCGStab (pressure_guess.hip, preconditioned by mg.hip) on a 5-point system over the NX*NY
 // nodes in node order: diagonal d, east (i+1), west (i-1), south (i+NX) and
 // north (i-NX) coefficients, 0 where a row has no such neighbour; x0 = 0.
 // Writes x, synchronises; FVM_ERR_NOT_CONVERGED when rtol is not reached.

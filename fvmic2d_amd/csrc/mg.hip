@@ -1,0 +1,591 @@
+// Preconditioners of the nodal solves' BiCGStab (pressure_guess.hip): y = M b for
+// a 5-point system whose rows are divided by their diagonal (unit diagonal,
+// couplings e, w, s, n; a row without couplings is solved by its right-hand side).
+//
+// Jacobi alone needs hundreds to thousands of iterations on the Poisson problem
+// of the pressure guess (1304 at 257x257), each five short kernels bound by launch
+// and reduction latency.  Two preconditioners replace it:
+//
+// * a multigrid V-cycle: FV_NU Chebyshev-Jacobi sweeps before and after the coarse
+//   correction, cells aggregated in pairs along each axis (along one axis only
+//   while its couplings are much the stronger), the coarse couplings rediscretised
+//   from the aggregated ones (divided by the grown distance), restriction by sums,
+//   prolongation bilinear.  6 iterations at 257x257 (solve 31.7 -> 1.10 ms).
+// * where every row is dominated by its diagonal (an energy equation with a
+//   moderate time step) the same polynomial at degree FV_POLY on the finest
+//   level alone, over the interval the row sums give: 5 iterations instead of 40
+//   at 801x401 (assembly and solve 1.67 -> 0.47 ms).
+//
+// What bounds them is latency, so a kernel does as much as its tile allows: a
+// tile and a halo as wide as the number of sweeps are read once, all sweeps run in
+// LDS (the halo is swept redundantly: 2.3 times the tile's points), and everything
+// below FV_COARSE_MAX points is one workgroup's kernel.
+#include <new>
+#include <vector>
+
+#include "fvm_internal.h"
+
+namespace {
+
+constexpr int FV_NU = 4;        // sweeps on each side of the coarse correction
+constexpr int FV_POLY = 8;      // degree of the one-level preconditioner
+constexpr int FV_T = 16;        // tile of the level kernels
+constexpr int FV_R = FV_T + 2 * FV_NU;
+constexpr int FV_PT = 32;       // tile of the one-level kernel
+constexpr int FV_PR = FV_PT + 2 * (FV_POLY - 1);
+constexpr int FV_COARSE_MAX = 4400;
+constexpr int FV_CT = 1024;     // threads of the coarse kernel
+constexpr int FV_CLEVELS = 16;
+constexpr int FV_LAST = 12;     // sweeps on the last level
+
+struct Coefs {
+  const double *e, *w, *s, *n;
+};
+
+// Chebyshev steps d = c1 d + c2 r, x += d for the spectrum [a, b]
+struct Cheb {
+  double c1[16], c2[16];
+};
+
+struct Pt {
+  double e, w, s, n;
+  __device__ __forceinline__ bool live() const { return e != 0.0 || w != 0.0 || s != 0.0 || n != 0.0; }
+};
+__device__ __forceinline__ Pt load_pt(const Coefs &c, bool in, int64_t i) {
+  Pt p = {0.0, 0.0, 0.0, 0.0};
+  if (in) p = Pt{c.e[i], c.w[i], c.s[i], c.n[i]};
+  return p;
+}
+
+// ---- one level: x = p(A) b ----------------------------------------------------------
+// 1024 threads sweep a 46x46 region for a 32x32 tile.
+__global__ void __launch_bounds__(1024) k_poly(int NX, int NY, Coefs c, Cheb ch, const double *__restrict__ b,
+                                               double *__restrict__ x) {
+  constexpr int RW = FV_PR + 2, NP = FV_PR * FV_PR, PTS = (NP + 1023) / 1024;
+  __shared__ double sh[2][RW * RW];
+  for (int k = threadIdx.x; k < 2 * RW * RW; k += 1024) (&sh[0][0])[k] = 0.0;
+  const int x0 = blockIdx.x * FV_PT - (FV_POLY - 1), y0 = blockIdx.y * FV_PT - (FV_POLY - 1);
+  Pt p[PTS];
+  double bb[PTS], d[PTS], xv[PTS];
+  int at[PTS];
+  bool live[PTS];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PTS; k++) {
+    const int q = threadIdx.x + 1024 * k, ry = q / FV_PR, rx = q - ry * FV_PR;
+    const int ix = x0 + rx, iy = y0 + ry;
+    const bool in = q < NP && ix >= 0 && ix < NX && iy >= 0 && iy < NY;
+    const int64_t i = (int64_t)iy * NX + ix;
+    p[k] = load_pt(c, in, i);
+    bb[k] = in ? b[i] : 0.0;
+    live[k] = p[k].live();
+    d[k] = live[k] ? bb[k] * ch.c2[0] : 0.0;
+    xv[k] = live[k] ? d[k] : bb[k];
+    at[k] = q < NP ? (ry + 1) * RW + rx + 1 : -1;
+    if (at[k] >= 0) sh[0][at[k]] = xv[k];
+  }
+  __syncthreads();
+#pragma unroll 1
+  for (int t = 1; t < FV_POLY; t++) {
+    const double *xs = sh[(t - 1) & 1];
+    double *xn = sh[t & 1];
+#pragma unroll
+    for (int k = 0; k < PTS; k++) {
+      if (at[k] < 0) continue;
+      const int a = at[k];
+      const double r = bb[k] - (xv[k] + p[k].e * xs[a + 1] + p[k].w * xs[a - 1] + p[k].s * xs[a + RW] + p[k].n * xs[a - RW]);
+      if (live[k]) {
+        d[k] = ch.c1[t] * d[k] + ch.c2[t] * r;
+        xv[k] += d[k];
+      }
+      xn[a] = xv[k];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int k = 0; k < PTS; k++) {
+    const int q = threadIdx.x + 1024 * k, ry = q / FV_PR, rx = q - ry * FV_PR;
+    const int ix = x0 + rx, iy = y0 + ry;
+    if (q < NP && rx >= FV_POLY - 1 && rx < FV_PT + FV_POLY - 1 && ry >= FV_POLY - 1 && ry < FV_PT + FV_POLY - 1 && ix < NX && iy < NY)
+      x[(int64_t)iy * NX + ix] = xv[k];
+  }
+}
+
+// ---- multigrid ------------------------------------------------------------------------
+struct Lv {
+  int NX, NY;
+  int fx, fy;       // aggregation to the next level: 2 pairs (2I-1, 2I), 1 none
+  int NXc, NYc;
+  Coefs c;
+  const double *idc;  // 1 / diagonal of the next level's rows before their scaling
+};
+
+__device__ __forceinline__ int agg(int i, int f) { return f == 2 ? (i + 1) >> 1 : i; }
+// fine indices in aggregate I of an axis with N indices
+__device__ __forceinline__ int agg_count(int I, int f, int N) {
+  return f == 2 && I > 0 && 2 * I < N ? 2 : 1;
+}
+
+__device__ __forceinline__ double row_residual(const Pt &p, double b, const double *xs, int a, int w) {
+  return b - (xs[a] + p.e * xs[a + 1] + p.w * xs[a - 1] + p.s * xs[a + w] + p.n * xs[a - w]);
+}
+
+// x = FV_NU sweeps from 0, then the residual summed over the aggregates
+__global__ void __launch_bounds__(FV_R *FV_R) k_down(Lv L, Cheb ch, const double *__restrict__ b, double *__restrict__ x,
+                                                     double *__restrict__ bc) {
+  constexpr int RW = FV_R + 2;
+  __shared__ double sh[2][RW * RW];
+  const int t = threadIdx.x, ry = t / FV_R, rx = t - ry * FV_R;
+  for (int k = t; k < 2 * RW * RW; k += FV_R * FV_R) (&sh[0][0])[k] = 0.0;
+  // tiles start on an aggregate's first index
+  const int fx0 = blockIdx.x * FV_T - (L.fx == 2 ? 1 : 0), fy0 = blockIdx.y * FV_T - (L.fy == 2 ? 1 : 0);
+  const int ix = fx0 - FV_NU + rx, iy = fy0 - FV_NU + ry;
+  const bool in = ix >= 0 && ix < L.NX && iy >= 0 && iy < L.NY;
+  const int64_t i = (int64_t)iy * L.NX + ix;
+  const Pt p = load_pt(L.c, in, i);
+  const double bb = in ? b[i] : 0.0;
+  const bool live = p.live();
+  double d = live ? bb * ch.c2[0] : 0.0, xv = live ? d : bb;
+  const int a = (ry + 1) * RW + rx + 1;
+  __syncthreads();
+  sh[0][a] = xv;
+  __syncthreads();
+#pragma unroll
+  for (int s = 1; s < FV_NU; s++) {
+    const double r = row_residual(p, bb, sh[(s - 1) & 1], a, RW);
+    if (live) {
+      d = ch.c1[s] * d + ch.c2[s] * r;
+      xv += d;
+    }
+    sh[s & 1][a] = xv;
+    __syncthreads();
+  }
+  const double r = live ? row_residual(p, bb, sh[(FV_NU - 1) & 1], a, RW) : 0.0;
+  const bool own = in && rx >= FV_NU && rx < FV_NU + FV_T && ry >= FV_NU && ry < FV_NU + FV_T;
+  if (own) x[i] = xv;
+  sh[FV_NU & 1][a] = own ? r : 0.0;
+  __syncthreads();
+  const int cw = FV_T / L.fx, chh = FV_T / L.fy;
+  if (t < cw * chh) {
+    const int cy = t / cw, cx = t - cy * cw;
+    const int I = blockIdx.x * cw + cx, J = blockIdx.y * chh + cy;
+    if (I < L.NXc && J < L.NYc) {
+      const double *rs = sh[FV_NU & 1] + (cy * L.fy + FV_NU + 1) * RW + cx * L.fx + FV_NU + 1;
+      double v = rs[0];
+      if (L.fx == 2) v += rs[1];
+      if (L.fy == 2) v += L.fx == 2 ? rs[RW] + rs[RW + 1] : rs[RW];
+      const int64_t k = (int64_t)J * L.NXc + I;
+      bc[k] = v * L.idc[k];
+    }
+  }
+}
+
+// value of the coarse correction ec at fine index (ix, iy): bilinear, an axis
+// without a coupling towards the neighbouring aggregate takes its own value
+template <class Get>
+__device__ __forceinline__ double prolong(const Lv &L, const Pt &p, int ix, int iy, Get ec) {
+  const int I = agg(ix, L.fx), J = agg(iy, L.fy);
+  int In = I, Jn = J;
+  double wx = 0.0, wy = 0.0;
+  if (L.fx == 2) {
+    const bool lo = ix & 1;
+    if ((lo ? p.w : p.e) != 0.0) In = lo ? I - 1 : I + 1, wx = 0.25;
+    if (In < 0 || In >= L.NXc) In = I;
+  }
+  if (L.fy == 2) {
+    const bool lo = iy & 1;
+    if ((lo ? p.n : p.s) != 0.0) Jn = lo ? J - 1 : J + 1, wy = 0.25;
+    if (Jn < 0 || Jn >= L.NYc) Jn = J;
+  }
+  const double top = (1.0 - wx) * ec(I, J) + wx * ec(In, J);
+  const double bot = (1.0 - wx) * ec(I, Jn) + wx * ec(In, Jn);
+  return (1.0 - wy) * top + wy * bot;
+}
+
+// out = FV_NU sweeps from x + P ec
+__global__ void __launch_bounds__(FV_R *FV_R) k_up(Lv L, Cheb ch, const double *__restrict__ b, const double *__restrict__ x,
+                                                   const double *__restrict__ ec, double *__restrict__ out) {
+  constexpr int RW = FV_R + 2;
+  __shared__ double sh[2][RW * RW];
+  const int t = threadIdx.x, ry = t / FV_R, rx = t - ry * FV_R;
+  for (int k = t; k < 2 * RW * RW; k += FV_R * FV_R) (&sh[0][0])[k] = 0.0;
+  const int ix = (int)blockIdx.x * FV_T - FV_NU + rx, iy = (int)blockIdx.y * FV_T - FV_NU + ry;
+  const bool in = ix >= 0 && ix < L.NX && iy >= 0 && iy < L.NY;
+  const int64_t i = (int64_t)iy * L.NX + ix;
+  const Pt p = load_pt(L.c, in, i);
+  const double bb = in ? b[i] : 0.0;
+  const bool live = p.live();
+  double xv = in ? x[i] : 0.0, d = 0.0;
+  if (live) xv += prolong(L, p, ix, iy, [&](int I, int J) { return ec[(int64_t)J * L.NXc + I]; });
+  const int a = (ry + 1) * RW + rx + 1;
+  __syncthreads();
+  sh[0][a] = xv;
+  __syncthreads();
+#pragma unroll
+  for (int s = 0; s < FV_NU; s++) {
+    const double r = row_residual(p, bb, sh[s & 1], a, RW);
+    if (live) {
+      d = ch.c1[s] * d + ch.c2[s] * r;
+      xv += d;
+    }
+    sh[(s + 1) & 1][a] = xv;
+    __syncthreads();
+  }
+  if (in && rx >= FV_NU && rx < FV_NU + FV_T && ry >= FV_NU && ry < FV_NU + FV_T) out[i] = xv;
+}
+
+// Every level of at most FV_COARSE_MAX points in one workgroup: x and b of each
+// level lie in LDS between zeros wide enough for the stencil's reach (a missing
+// neighbour's coefficient is 0), a thread's rows in registers during a smoothing.
+struct CoarseArgs {
+  int n;
+  Lv lv[FV_CLEVELS];
+  int off[FV_CLEVELS];  // of point 0 in the LDS arrays
+  int total;            // doubles per LDS array
+};
+constexpr int FV_LDS = 6400;  // doubles per array (x, b)
+
+template <int PTS>
+__device__ __forceinline__ void smooth(const Lv &L, const Cheb &ch, int steps, bool zero, double *x, const double *b) {
+  const int np = L.NX * L.NY;
+  Pt p[PTS];
+  double d[PTS], xv[PTS];
+#pragma unroll
+  for (int k = 0; k < PTS; k++) {
+    const int q = threadIdx.x + FV_CT * k;
+    p[k] = load_pt(L.c, q < np, q);
+    d[k] = 0.0;
+    xv[k] = q < np && !zero ? x[q] : 0.0;
+    if (zero && q < np) {
+      d[k] = p[k].live() ? b[q] * ch.c2[0] : 0.0;
+      xv[k] = p[k].live() ? d[k] : b[q];
+      x[q] = xv[k];
+    }
+  }
+  __syncthreads();
+  for (int s = zero ? 1 : 0; s < steps; s++) {
+#pragma unroll
+    for (int k = 0; k < PTS; k++) {
+      const int q = threadIdx.x + FV_CT * k;
+      if (q < np && p[k].live()) {
+        d[k] = ch.c1[s] * d[k] + ch.c2[s] * row_residual(p[k], b[q], x, q, L.NX);
+        xv[k] += d[k];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PTS; k++) {
+      const int q = threadIdx.x + FV_CT * k;
+      if (q < np) x[q] = xv[k];
+    }
+    __syncthreads();
+  }
+}
+__device__ __forceinline__ void smooth_any(const Lv &L, const Cheb &ch, int steps, bool zero, double *x, const double *b) {
+  const int np = L.NX * L.NY;
+  if (np > 2 * FV_CT) smooth<(FV_COARSE_MAX + FV_CT - 1) / FV_CT>(L, ch, steps, zero, x, b);
+  else if (np > FV_CT) smooth<2>(L, ch, steps, zero, x, b);
+  else smooth<1>(L, ch, steps, zero, x, b);
+}
+
+__global__ void __launch_bounds__(FV_CT) k_coarse(CoarseArgs A, Cheb ch, Cheb last, int last_steps,
+                                                  const double *__restrict__ bin, double *__restrict__ xout) {
+  __shared__ double X[FV_LDS], B[FV_LDS];
+  for (int k = threadIdx.x; k < A.total; k += FV_CT) X[k] = 0.0, B[k] = 0.0;
+  __syncthreads();
+  const int np0 = A.lv[0].NX * A.lv[0].NY;
+  for (int q = threadIdx.x; q < np0; q += FV_CT) B[A.off[0] + q] = bin[q];
+  __syncthreads();
+#pragma unroll 1
+  for (int l = 0; l + 1 < A.n; l++) {
+    const Lv &L = A.lv[l];
+    double *x = X + A.off[l], *b = B + A.off[l], *bc = B + A.off[l + 1];
+    smooth_any(L, ch, FV_NU, true, x, b);
+    for (int q = threadIdx.x; q < L.NXc * L.NYc; q += FV_CT) {
+      const int J = q / L.NXc, I = q - J * L.NXc;
+      const int i0 = L.fx == 2 ? (I ? 2 * I - 1 : 0) : I, j0 = L.fy == 2 ? (J ? 2 * J - 1 : 0) : J;
+      const int ni = agg_count(I, L.fx, L.NX), nj = agg_count(J, L.fy, L.NY);
+      double v = 0.0;
+      for (int j = j0; j < j0 + nj; j++)
+        for (int i = i0; i < i0 + ni; i++) {
+          const int f = j * L.NX + i;
+          const Pt p = load_pt(L.c, true, f);
+          if (p.live()) v += row_residual(p, b[f], x, f, L.NX);
+        }
+      bc[q] = v * L.idc[q];
+    }
+    __syncthreads();
+  }
+  smooth_any(A.lv[A.n - 1], last, last_steps, true, X + A.off[A.n - 1], B + A.off[A.n - 1]);
+#pragma unroll 1
+  for (int l = A.n - 2; l >= 0; l--) {
+    const Lv &L = A.lv[l];
+    double *x = X + A.off[l];
+    const double *ec = X + A.off[l + 1];
+    for (int f = threadIdx.x; f < L.NX * L.NY; f += FV_CT) {
+      const Pt p = load_pt(L.c, true, f);
+      const int iy = f / L.NX, ix = f - iy * L.NX;
+      if (p.live()) x[f] += prolong(L, p, ix, iy, [&](int I, int J) { return ec[J * L.NXc + I]; });
+    }
+    __syncthreads();
+    smooth_any(L, ch, FV_NU, false, x, B + A.off[l]);
+  }
+  for (int q = threadIdx.x; q < np0; q += FV_CT) xout[q] = X[A.off[0] + q];
+}
+
+// The next level's rows.  A coupling between aggregates is the sum of the fine
+// ones over the grown distance between their centres (2 fine steps instead of 1
+// between two pairs); one to a row without couplings of its own (a boundary value,
+// the pinned cell) stays on the diagonal; the row sums (a time derivative) add up.
+__global__ void __launch_bounds__(256) k_coarsen(Lv L, double *__restrict__ ce, double *__restrict__ cw,
+                                                 double *__restrict__ cs, double *__restrict__ cn,
+                                                 double *__restrict__ idc) {
+  const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (q >= (int64_t)L.NXc * L.NYc) return;
+  const int J = (int)(q / L.NXc), I = (int)(q - (int64_t)J * L.NXc);
+  const int i0 = L.fx == 2 ? (I ? 2 * I - 1 : 0) : I, j0 = L.fy == 2 ? (J ? 2 * J - 1 : 0) : J;
+  const int ni = agg_count(I, L.fx, L.NX), nj = agg_count(J, L.fy, L.NY);
+  double off[4] = {0.0, 0.0, 0.0, 0.0}, rho = 0.0, delta = 0.0;
+  int nlive = 0;
+  for (int j = j0; j < j0 + nj; j++)
+    for (int i = i0; i < i0 + ni; i++) {
+      const Pt p = load_pt(L.c, true, (int64_t)j * L.NX + i);
+      if (!p.live()) continue;
+      nlive++;
+      rho += 1.0 + p.e + p.w + p.s + p.n;
+      const double co[4] = {p.e, p.w, p.s, p.n};
+#pragma unroll
+      for (int k = 0; k < 4; k++) {
+        const int jx = i + (k == 0) - (k == 1), jy = j + (k == 2) - (k == 3);
+        if (co[k] == 0.0 || jx < 0 || jx >= L.NX || jy < 0 || jy >= L.NY) continue;
+        const bool alongx = k < 2;
+        const int f = alongx ? L.fx : L.fy, mine = alongx ? ni : nj;
+        const Pt o = load_pt(L.c, true, (int64_t)jy * L.NX + jx);
+        if (!o.live()) {
+          delta -= co[k] * (f == 2 ? 2.0 / (mine + 1) : 1.0);
+        } else if (agg(jx, L.fx) != I || agg(jy, L.fy) != J) {
+          const int his = alongx ? agg_count(agg(jx, L.fx), L.fx, L.NX) : agg_count(agg(jy, L.fy), L.fy, L.NY);
+          off[k] += co[k] * (f == 2 ? 2.0 / (mine + his) : 1.0);
+        }
+      }
+    }
+  const double diag = rho - (((off[0] + off[1]) + off[2]) + off[3]) + delta;
+  const double id = nlive ? 1.0 / diag : 0.0;
+  ce[q] = off[0] * id;
+  cw[q] = off[1] * id;
+  cs[q] = off[2] * id;
+  cn[q] = off[3] * id;
+  idc[q] = id;
+}
+
+// rows divided by their diagonal, and per block what the choice of a
+// preconditioner needs: the sums of |e| + |w| and |s| + |n|, the least row sum
+__global__ void __launch_bounds__(256) k_rows(int64_t n, const double *__restrict__ d, Coefs c, double *__restrict__ e,
+                                              double *__restrict__ w, double *__restrict__ s, double *__restrict__ nn,
+                                              double *__restrict__ part) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  double sx = 0.0, sy = 0.0, lo = 1.0;
+  if (i < n) {
+    const double di = d[i];
+    const Pt p = {c.e[i] / di, c.w[i] / di, c.s[i] / di, c.n[i] / di};
+    if (e) e[i] = p.e, w[i] = p.w, s[i] = p.s, nn[i] = p.n;
+    sx = fabs(p.e) + fabs(p.w);
+    sy = fabs(p.s) + fabs(p.n);
+    lo = 1.0 - sx - sy;
+    if (!(lo == lo)) lo = -1.0;  // NaN rows: no bound
+  }
+  __shared__ double sh[3][4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sx += __shfl_xor(sx, o);
+    sy += __shfl_xor(sy, o);
+    lo = fmin(lo, __shfl_xor(lo, o));
+  }
+  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = sx, sh[1][threadIdx.x >> 6] = sy, sh[2][threadIdx.x >> 6] = lo;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+    part[gridDim.x + blockIdx.x] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+    part[2 * gridDim.x + blockIdx.x] = fmin(fmin(sh[2][0], sh[2][1]), fmin(sh[2][2], sh[2][3]));
+  }
+}
+__global__ void __launch_bounds__(256) k_rows_total(int nb, const double *__restrict__ part, double *__restrict__ out) {
+  double sx = 0.0, sy = 0.0, lo = 1.0;
+  for (int k = threadIdx.x; k < nb; k += 256) {
+    sx += part[k];
+    sy += part[nb + k];
+    lo = fmin(lo, part[2 * nb + k]);
+  }
+  __shared__ double sh[3][4];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sx += __shfl_xor(sx, o);
+    sy += __shfl_xor(sy, o);
+    lo = fmin(lo, __shfl_xor(lo, o));
+  }
+  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = sx, sh[1][threadIdx.x >> 6] = sy, sh[2][threadIdx.x >> 6] = lo;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    out[0] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+    out[1] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+    out[2] = fmin(fmin(sh[2][0], sh[2][1]), fmin(sh[2][2], sh[2][3]));
+  }
+}
+
+Cheb cheb(double a, double b, int steps) {
+  Cheb c;
+  const double th = (b + a) / 2.0, de = (b - a) / 2.0, sg = th / de;
+  double ro = 1.0 / sg;
+  c.c1[0] = 0.0;
+  c.c2[0] = 1.0 / th;
+  for (int k = 1; k < steps; k++) {
+    const double rn = 1.0 / (2.0 * sg - ro);
+    c.c1[k] = rn * ro;
+    c.c2[k] = 2.0 * rn / de;
+    ro = rn;
+  }
+  return c;
+}
+
+int64_t padded(int64_t n) { return (n + 31) / 32 * 32; }
+
+}  // namespace
+
+// A system's preconditioner; its arrays lie in ctx->mg.
+struct fvm_precond {
+  double lo = 0.0;             // least row sum
+  bool one_level = false;      // the polynomial on the finest level
+  std::vector<Lv> lv;          // finest first
+  // per level: right-hand side (not the finest's), the sweeps before its
+  // correction, the result (not the finest's)
+  std::vector<double *> b, x, y;
+  int first_coarse = 0;        // level at which the one-workgroup kernel takes over
+  CoarseArgs coarse;
+  Cheb smooth, last, poly;
+};
+void fvm_precond_free(fvm_precond *m) { delete m; }
+
+int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const double *e, const double *w, const double *s,
+                      const double *n, bool scale, fvm_precond **out) {
+  // how much stronger an axis' couplings are before it alone is coarsened
+  constexpr double SEMI = 2.5;
+  // least row sum from which the finest level alone is preconditioned: degree
+  // FV_POLY then contracts every component about as well as a V-cycle does
+  constexpr double DOMINANT = 0.05;
+  *out = nullptr;
+  const int64_t nn = (int64_t)NX * NY;
+  const unsigned nb = fvm_blocks(nn, 256);
+  // the finest level's rows and sweeps, the levels below (at most half the
+  // points each, and a column and row more)
+  const size_t words = (size_t)(5 * padded(nn) + padded(3 * (int64_t)nb) + 64) +
+                       8 * (size_t)(nn + 24 * ((int64_t)NX + NY) + 4096);
+  FVM_TRY(fvm_ws(ctx, ctx->mg, words * sizeof(double)));
+  double *p = (double *)ctx->mg.ptr, *end = p + words;
+  auto take = [&](int64_t k) {
+    double *r = p;
+    p += padded(k);
+    return r;
+  };
+  if (!ctx->precond) ctx->precond = new (std::nothrow) fvm_precond();
+  fvm_precond *m = ctx->precond;
+  if (!m) return fvm_set_err(ctx, FVM_ERR_NOMEM, "preconditioner");
+  m->lv.clear(), m->b.clear(), m->x.clear(), m->y.clear();
+  m->first_coarse = 0;
+  double *part = take(3 * (int64_t)nb), *tot = take(4);
+  double *rows[4] = {nullptr, nullptr, nullptr, nullptr};
+  Coefs c = {e, w, s, n};
+  if (scale)
+    for (int k = 0; k < 4; k++) rows[k] = take(nn);
+  k_rows<<<nb, 256, 0, ctx->stream>>>(nn, d, c, rows[0], rows[1], rows[2], rows[3], part);
+  k_rows_total<<<1, 256, 0, ctx->stream>>>((int)nb, part, tot);
+  FVM_LAUNCH_CHECK(ctx);
+  double *host = (double *)ctx->pinned.ptr;
+  FVM_HIP(ctx, hipMemcpyAsync(host, tot, 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  double sx = host[0], sy = host[1];
+  m->lo = host[2];
+  if (scale) c = Coefs{rows[0], rows[1], rows[2], rows[3]};
+  auto push = [&](int nx, int ny, const Coefs &co, double *b, double *x, double *y) {
+    Lv L{};
+    L.NX = nx, L.NY = ny, L.c = co, L.fx = L.fy = 1;
+    m->lv.push_back(L);
+    m->b.push_back(b);
+    m->x.push_back(x);
+    m->y.push_back(y);
+  };
+  m->one_level = m->lo >= DOMINANT;
+  if (m->one_level) {
+    push(NX, NY, c, nullptr, nullptr, nullptr);
+    m->poly = cheb(m->lo, 2.0 - m->lo, FV_POLY);
+    *out = m;
+    return FVM_OK;
+  }
+  push(NX, NY, c, nullptr, take(nn), nullptr);
+  m->smooth = cheb(0.1, 2.0, FV_NU);
+  m->last = cheb(0.1, 2.0, FV_LAST);
+  for (;;) {
+    Lv &f = m->lv.back();
+    if ((int64_t)f.NX * f.NY <= 20 || (f.NX <= 3 && f.NY <= 3)) break;
+    f.fx = f.NX > 3 ? 2 : 1, f.fy = f.NY > 3 ? 2 : 1;
+    if (f.fx == 2 && f.fy == 2) {
+      if (sx > SEMI * sy) f.fy = 1, sx /= 4.0;
+      else if (sy > SEMI * sx) f.fx = 1, sy /= 4.0;
+    }
+    f.NXc = f.fx == 2 ? f.NX / 2 + 1 : f.NX;
+    f.NYc = f.fy == 2 ? f.NY / 2 + 1 : f.NY;
+    const int64_t nc = (int64_t)f.NXc * f.NYc;
+    if (p + 8 * padded(nc) > end) return FVM_OK;  // no preconditioner for such a shape
+    double *ce = take(nc), *cw = take(nc), *cs = take(nc), *cn = take(nc), *id = take(nc);
+    f.idc = id;
+    k_coarsen<<<fvm_blocks(nc, 256), 256, 0, ctx->stream>>>(f, ce, cw, cs, cn, id);
+    FVM_LAUNCH_CHECK(ctx);
+    const int nx = f.NXc, ny = f.NYc;  // f dies with the push
+    double *b = take(nc), *x = take(nc), *y = take(nc);
+    push(nx, ny, Coefs{ce, cw, cs, cn}, b, x, y);
+  }
+  // the one-workgroup kernel takes the levels that fit its LDS and threads
+  const int n_lv = (int)m->lv.size();
+  for (int l = 0; l < n_lv; l++) {
+    if ((int64_t)m->lv[l].NX * m->lv[l].NY > FV_COARSE_MAX || n_lv - l > FV_CLEVELS) continue;
+    CoarseArgs &A = m->coarse;
+    int at = 0;
+    for (int k = l; k < n_lv; k++) {
+      const Lv &L = m->lv[k];
+      A.lv[k - l] = L;
+      A.off[k - l] = at + L.NX + 1;
+      at += 2 * (L.NX + 1) + L.NX * L.NY;
+    }
+    A.n = n_lv - l;
+    A.total = at;
+    if (at > FV_LDS) continue;
+    m->first_coarse = l;
+    *out = m;
+    return FVM_OK;
+  }
+  return FVM_OK;  // no level fits: no preconditioner
+}
+
+int fvm_precond_apply(fvm_ctx *ctx, const fvm_precond *m, const double *b, double *x) {
+  const Lv &F = m->lv[0];
+  if (m->one_level) {
+    k_poly<<<dim3(fvm_blocks(F.NX, FV_PT), fvm_blocks(F.NY, FV_PT)), 1024, 0, ctx->stream>>>(F.NX, F.NY, F.c, m->poly, b, x);
+    FVM_LAUNCH_CHECK(ctx);
+    return FVM_OK;
+  }
+  const int fc = m->first_coarse;
+  auto rhs = [&](int l) { return l ? m->b[l] : b; };
+  auto res = [&](int l) { return l ? m->y[l] : x; };
+  for (int l = 0; l < fc; l++) {
+    const Lv &L = m->lv[l];
+    k_down<<<dim3(fvm_blocks(L.NXc, FV_T / L.fx), fvm_blocks(L.NYc, FV_T / L.fy)), FV_R * FV_R, 0, ctx->stream>>>(
+        L, m->smooth, rhs(l), m->x[l], m->b[l + 1]);
+  }
+  k_coarse<<<1, FV_CT, 0, ctx->stream>>>(m->coarse, m->smooth, m->last, FV_LAST, rhs(fc), res(fc));
+  for (int l = fc - 1; l >= 0; l--) {
+    const Lv &L = m->lv[l];
+    k_up<<<dim3(fvm_blocks(L.NX, FV_T), fvm_blocks(L.NY, FV_T)), FV_R * FV_R, 0, ctx->stream>>>(
+        L, m->smooth, rhs(l), m->x[l], res(l + 1), res(l));
+  }
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}

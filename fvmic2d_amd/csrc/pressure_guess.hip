@@ -4,9 +4,10 @@
 // cell-centre pressure, div grad p = g . grad rho, and hands it to the
 // "energy_" KSP.  Here the operator is applied matrix-free, row for row as
 // assembled there (dummy rows for ix == 0 or jy == 0, the pinned cell (3, 3),
-// zero-flux sides, dp/dy = rho g on top and bottom), and solved with
-// Jacobi-preconditioned BiCGStab in five kernels per iteration whose scalars
-// stay on the device.  Dot products reduce in a fixed order (per-block trees,
+// zero-flux sides, dp/dy = rho g on top and bottom), and solved with BiCGStab,
+// preconditioned by mg.hip, in five kernels per iteration (and the two
+// applications of the preconditioner) whose scalars stay on the device.  Where
+// that does not converge, the solve starts again with Jacobi alone.  Dot products reduce in a fixed order (per-block trees,
 // then the same ordered sum in every block of the next kernel), so the
 // iteration is bitwise reproducible.
 #include "fvm_internal.h"
@@ -97,7 +98,7 @@ __global__ void __launch_bounds__(256) k_pg_apply(PGrid g, const double *__restr
   y[i] = s;
 }
 
-// ---- BiCGStab, five kernels per iteration -----------------------------------------
+// ---- BiCGStab, five kernels per iteration and the preconditioner -----------------------------------------
 // Every vector kernel runs one thread per row in blocks of 256 (block k holds
 // rows 256k ..).  Dot products are per-block partial sums (fixed trees) that
 // the next kernel reduces: every block of it sums the same partials in the same
@@ -105,13 +106,14 @@ __global__ void __launch_bounds__(256) k_pg_apply(PGrid g, const double *__restr
 // reproducible.  The stencil coefficients are tabulated once.
 #define BCG_BS 256
 
-enum { S_RHO = 0, S_RHO_OLD, S_ALPHA, S_OMEGA, S_NSC };
+enum { S_RHO = 0, S_RHO_OLD, S_ALPHA, S_OMEGA, S_RR };
 
 struct Coef {
   const double *d, *r, *l, *dn, *up;
 };
 struct BcgVecs {
   double *b, *dinv, *x, *r, *rh, *p, *v, *s, *t, *y, *z;
+  double *q;                                 // what the preconditioner is applied to
   double *cd, *cr, *cl, *cdn, *cup;          // stencil coefficients
   double *prv, *pts, *ptt, *prho, *prr;      // per-block partial sums
   double *sc;                                // scalars (S_*)
@@ -298,6 +300,11 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_x(int64_t n, int nblk, BcgVecs V
   }
 }
 
+__global__ void __launch_bounds__(BCG_BS) k_bcg_norm(int nblk, BcgVecs V) {
+  const double rr = partial_total(V.prr, nblk);
+  if (threadIdx.x == 0) V.sc[S_RR] = rr;
+}
+
 __global__ void __launch_bounds__(256) k_store_p(int64_t n, const double *__restrict__ p, double *__restrict__ S,
                                                  double *__restrict__ pout) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -327,66 +334,79 @@ extern "C" int fvm_pressure_guess_apply(fvm_ctx *ctx, const fvm_grid *g, const d
   return FVM_OK;
 }
 
-// workspace: 11 vectors, 5 coefficient arrays, 5 partial arrays, scalars
+// workspace: 12 vectors, 5 coefficient arrays, 5 partial arrays, scalars
 static int bcg_vecs(fvm_ctx *ctx, int64_t n, BcgVecs *V, int *nblk_out) {
   const int64_t np = (n + 63) / 64 * 64;
   const int nblk = (int)((n + BCG_BS - 1) / BCG_BS);
   const int64_t npart = ((int64_t)nblk + 63) / 64 * 64;
-  FVM_TRY(fvm_ws(ctx, ctx->scratch, (16 * np + 5 * npart + 64) * sizeof(double)));
+  FVM_TRY(fvm_ws(ctx, ctx->scratch, (17 * np + 5 * npart + 64) * sizeof(double)));
   double *w = (double *)ctx->scratch.ptr;
   double **vecs[] = {&V->b, &V->dinv, &V->x, &V->r, &V->rh, &V->p, &V->v, &V->s, &V->t, &V->y, &V->z,
-                     &V->cd, &V->cr, &V->cl, &V->cdn, &V->cup};
-  for (int k = 0; k < 16; k++) *vecs[k] = w + (int64_t)k * np;
-  double *pw = w + 16 * np;
+                     &V->cd, &V->cr, &V->cl, &V->cdn, &V->cup, &V->q};
+  for (int k = 0; k < 17; k++) *vecs[k] = w + (int64_t)k * np;
+  double *pw = w + 17 * np;
   V->prv = pw, V->pts = pw + npart, V->ptt = pw + 2 * npart, V->prho = pw + 3 * npart, V->prr = pw + 4 * npart;
   V->sc = pw + 5 * npart;
   *nblk_out = nblk;
   return FVM_OK;
 }
 
-// BiCGStab iterations after a setup kernel: the host reads ||r|| from the (r, r)
-// partials (summed in block order) every eight iterations
+// BiCGStab from the state that `start` sets up (x = 0).  With a preconditioner
+// the host reads ||r|| after every iteration (5 to 30 are needed); without one,
+// or where that has not converged after PRECOND_MAXIT iterations, Jacobi's
+// (hundreds) are checked every eight.  it_out: of the run that gave x.
+#define PRECOND_MAXIT 60
+template <class Start>
 static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs &V, int64_t n, int nblk,
-                    double rtol, int32_t maxit, int32_t *it_out, double *rel_out) {
+                    const fvm_precond *m, double rtol, int32_t maxit, int32_t *it_out, double *rel_out, Start start) {
   const unsigned nb = (unsigned)nblk;
-  std::vector<double> hp((size_t)nblk);
+  double *host = (double *)ctx->pinned.ptr;
   auto rnorm = [&](double *out) -> int {
-    FVM_HIP(ctx, hipMemcpyAsync(hp.data(), V.prr, sizeof(double) * nblk, hipMemcpyDeviceToHost, ctx->stream));
-    FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    double t = 0.0;
-    for (int k = 0; k < nblk; k++) t += hp[(size_t)k];
-    *out = sqrt(t);
-    return FVM_OK;
-  };
-  double bnorm = 0.0;
-  FVM_TRY(rnorm(&bnorm));
-  auto iteration = [&](int first) -> int {
-    k_bcg_p<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, first, V);
-    k_bcg_v<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
-    k_bcg_s<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, V);
-    k_bcg_t<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
-    k_bcg_x<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, V);
+    k_bcg_norm<<<1, BCG_BS, 0, ctx->stream>>>(nblk, V);
     FVM_LAUNCH_CHECK(ctx);
+    FVM_HIP(ctx, hipMemcpyAsync(host, V.sc + S_RR, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+    FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    *out = sqrt(*host);
     return FVM_OK;
   };
-  int it = 0;
-  double rel = 0.0;
-  if (bnorm > 0.0) {
-    rel = 1.0;
+  auto run = [&](const fvm_precond *pre, int32_t most, int every) -> int {
+    FVM_TRY(start());
+    double bnorm = 0.0;
+    FVM_TRY(rnorm(&bnorm));
+    *it_out = 0;
+    *rel_out = 0.0;
+    if (!(bnorm > 0.0)) return FVM_OK;
+    BcgVecs Vp = V, Vs = V;  // where the scaled p and s go
+    if (pre) Vp.y = V.q, Vs.z = V.q;
+    double rel = 1.0;
+    int it = 0;
     for (;;) {
-      if (it % 8 == 0 || it == maxit) {
+      if (it && (it % every == 0 || it == most)) {
         double rn = 0.0;
         FVM_TRY(rnorm(&rn));
         rel = rn / bnorm;
-        if (!(rel > rtol) || it == maxit) break;  // also stops on NaN
       }
-      FVM_TRY(iteration(it == 0 ? 1 : 0));
+      if (it % every == 0 || it == most)
+        if (!(rel > rtol) || it == most) break;  // also stops on NaN
+      k_bcg_p<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, it == 0 ? 1 : 0, Vp);
+      if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.y));
+      k_bcg_v<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
+      k_bcg_s<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, Vs);
+      if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.z));
+      k_bcg_t<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
+      k_bcg_x<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, V);
+      FVM_LAUNCH_CHECK(ctx);
       it++;
     }
+    *it_out = it;
+    *rel_out = rel;
+    return FVM_OK;
+  };
+  if (m) {
+    FVM_TRY(run(m, maxit < PRECOND_MAXIT ? maxit : PRECOND_MAXIT, 1));
+    if (*rel_out <= rtol) return FVM_OK;
   }
-  *it_out = it;
-  *rel_out = rel;
-  return FVM_OK;
+  return run(nullptr, maxit, 8);
 }
 
 extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const double *rho, double gy, double gx,
@@ -404,11 +424,17 @@ extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const
   const unsigned nb = (unsigned)nblk;
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
   k_pg_rhs<<<nb, BCG_BS, 0, ctx->stream>>>(pg, rho, gy, gx, V.b, V.dinv);
-  k_bcg_setup<<<nb, BCG_BS, 0, ctx->stream>>>(pg, rho, gy, gx, V);
-  FVM_LAUNCH_CHECK(ctx);
+  auto start = [&]() -> int {
+    k_bcg_setup<<<nb, BCG_BS, 0, ctx->stream>>>(pg, rho, gy, gx, V);
+    FVM_LAUNCH_CHECK(ctx);
+    return FVM_OK;
+  };
+  FVM_TRY(start());  // the rows
+  fvm_precond *m = nullptr;
+  FVM_TRY(fvm_precond_build(ctx, g->NX, g->NY, V.cd, V.cr, V.cl, V.cdn, V.cup, true, &m));
   int32_t it = 0;
   double rel = 0.0;
-  FVM_TRY(bcg_loop(ctx, pg, c, V, n, nblk, rtol, maxit, &it, &rel));
+  FVM_TRY(bcg_loop(ctx, pg, c, V, n, nblk, m, rtol, maxit, &it, &rel, start));
   k_store_p<<<nb, BCG_BS, 0, ctx->stream>>>(n, V.x, S, p_out);
   FVM_LAUNCH_CHECK(ctx);
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -418,7 +444,8 @@ extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const
   return FVM_OK;
 }
 
-// Jacobi BiCGStab on a 5-point system over the NX*NY nodes (fvm_internal.h)
+// BiCGStab on a 5-point system with a unit diagonal over the NX*NY nodes
+// (fvm_internal.h)
 int fvm_bicgstab_5pt(fvm_ctx *ctx, int NX, int NY, const double *d, const double *e, const double *w,
                      const double *sth, const double *nth, const double *b, double *x, double rtol, int32_t maxit,
                      int32_t *iters, double *relres) {
@@ -429,11 +456,16 @@ int fvm_bicgstab_5pt(fvm_ctx *ctx, int NX, int NY, const double *d, const double
   const Coef c = {d, e, w, sth, nth};
   const PGrid pg = PGrid{NX, NY, nullptr, nullptr, nullptr, nullptr};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  k_bcg_setup_sys<<<(unsigned)nblk, BCG_BS, 0, ctx->stream>>>(n, b, c, V);
-  FVM_LAUNCH_CHECK(ctx);
+  auto start = [&]() -> int {
+    k_bcg_setup_sys<<<(unsigned)nblk, BCG_BS, 0, ctx->stream>>>(n, b, c, V);
+    FVM_LAUNCH_CHECK(ctx);
+    return FVM_OK;
+  };
+  fvm_precond *m = nullptr;
+  FVM_TRY(fvm_precond_build(ctx, NX, NY, d, e, w, sth, nth, false, &m));
   int32_t it = 0;
   double rel = 0.0;
-  FVM_TRY(bcg_loop(ctx, pg, c, V, n, nblk, rtol, maxit, &it, &rel));
+  FVM_TRY(bcg_loop(ctx, pg, c, V, n, nblk, m, rtol, maxit, &it, &rel, start));
   FVM_HIP(ctx, hipMemcpyAsync(x, V.x, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (iters) *iters = it;
