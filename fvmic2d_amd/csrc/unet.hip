@@ -150,88 +150,209 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
 }
 
 // ---- weight gradient --------------------------------------------------------------
-// dW[tap][co][ci] = sum_p dY[p][co] * X[p + off(tap)][ci]: per tap a GEMM with
-// M = Cout, N = Cin and the pixels as K, split into chunks of KCH pixels whose
-// fp32 partials are summed in chunk order by k_wgrad_reduce.
+// dW[tap][co][ci] = sum_p dY[p][co] * X[p + off(tap)][ci]: a GEMM with M = Cout,
+// N = Cin per tap and the pixels as K.  Both operands have K strided in memory
+// (NHWC), so they are staged in LDS as they lie, [pixel][32 channels], and the
+// fragments are read with the transposing LDS load (ds_read_b64_tr_b16: 16 lanes
+// read four 32-byte rows, lane i gets column i of them); a tap is then only
+// another row address.
+//
+// Block: 4 wavefronts, 32 co x 32 ci, all taps (36 accumulator tiles); patches of
+// 16 x 16 pixels one after the other, wavefront w taking its rows 4w..4w+3 as two
+// K steps of rows (r, r + 2): the rows a tap needs, shifted by dy, are then another
+// step's, and each is read once per dx.  56 LDS reads serve 72 matrix
+// instructions.  Blocks split the patches (`nchunk`) to fill the chip; their fp32
+// partials, and those of the bias, are added in chunk order by k_wgrad_reduce.
+// Before, every bf16 was gathered from global memory by itself and one thread
+// summed a weight's partials over all chunks: one optimiser step's 15 gradients at
+// batch 8, 128 x 128 took 3.29 ms of the step's 4.59; they now take 0.79.
 #define KCH 256
+#define WG_P 16              // patch edge
+#define WG_HW (WG_P + 2)     // with the taps' halo
 struct WgradArgs {
   const uint16_t *X, *dY;
-  float *part;  // [chunk][tap][Cout][Cin]
-  int B, H, Wd, Cin, Cout, K;
-  int64_t nchunk;
+  float *part;  // [chunk][taps * Cout * Cin, then Cout (bias)]
+  int B, H, Wd, Cin, Cout;
+  int npx, npy, npatch, per_chunk;
+  int want_bias;
+  int aligned;  // X and dY on 16-byte boundaries
 };
 
+__device__ __forceinline__ uint4 ld16(const uint16_t *p, int aligned) {
+  if (aligned) return *(const uint4 *)p;
+  uint32_t w[4];
+  for (int i = 0; i < 4; i++) w[i] = (uint32_t)p[2 * i] | ((uint32_t)p[2 * i + 1] << 16);
+  return make_uint4(w[0], w[1], w[2], w[3]);
+}
+
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4 lds_s4;
+
+// K = 32 fragment (8 bf16 per lane): rows k = 8 (lane / 16) .. + 7 of the lane's
+// column lane % 16; p0, p1: this lane's 8-byte address among the first and the
+// last four of its group's rows (row (lane % 16) / 4, channels 4 (lane % 4))
+__device__ __forceinline__ bf8 ld_tr(const uint16_t *p0, const uint16_t *p1) {
+  union {
+    s4 h[2];
+    bf8 v;
+  } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p0);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p1);
+  return u.v;
+}
+
+// four floats at a 4-byte boundary (one 16-byte access where the address allows)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void st4(float *p, f4 v) { *(f4u *)p = v; }
+__device__ __forceinline__ f4 ld4(const float *p) { return *(const f4u *)p; }
+
+template <int K>
 __global__ void __launch_bounds__(256) k_wgrad(WgradArgs a) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int tap = blockIdx.y;
-  const int64_t chunk = blockIdx.x;
-  const int ntn = (a.Cin + 31) / 32;  // 32-wide ci tiles per wavefront
-  const int ntm = (a.Cout + 31) / 32;
-  const int half = a.K / 2;
-  const int dy = tap / a.K - half, dx = tap % a.K - half;
-  const int64_t npix = (int64_t)a.B * a.H * a.Wd;
-  const int ml = lane % 16, kg = lane / 16;
-  for (int tile = blockIdx.z * 4 + wv; tile < ntm * ntn; tile += gridDim.z * 4) {
-    const int co0 = (tile / ntn) * 32, ci0 = (tile % ntn) * 32;
-    f4 acc[2][2];
-    for (int i = 0; i < 2; i++)
-      for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < KCH; k0 += 32) {
-      Bf8Builder fa[2], fb[2];
-      for (int i = 0; i < 8; i++) {
-        const int64_t p = chunk * KCH + k0 + 8 * kg + i;
-        bool ok = p < npix;
-        const int64_t q = ok ? p : 0;
-        const int w = (int)(q % a.Wd), h = (int)((q / a.Wd) % a.H);
-        const int64_t bq = q / ((int64_t)a.Wd * a.H);
-        const int hh = h + dy, ww = w + dx;
-        const bool xok = ok && hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd;
-        const int64_t qx = ((bq * a.H + (xok ? hh : 0)) * a.Wd + (xok ? ww : 0));
-        for (int t = 0; t < 2; t++) {
-          const int co = co0 + t * 16 + ml;
-          fa[t].h[i] = (ok && co < a.Cout) ? a.dY[q * a.Cout + co] : (uint16_t)0;
-        }
-        for (int u = 0; u < 2; u++) {
-          const int ci = ci0 + u * 16 + ml;
-          fb[u].h[i] = (xok && ci < a.Cin) ? a.X[qx * a.Cin + ci] : (uint16_t)0;
+  constexpr int H2 = K / 2, HW = WG_P + 2 * H2, T = K * K;
+  __shared__ union {
+    struct {
+      uint16_t x[HW * HW * 32], y[WG_P * WG_P * 32];
+    } t;
+    float red[T * 32 * 32];
+    float bias[64 * 33];
+  } sh;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int co0 = blockIdx.y * 32, ci0 = blockIdx.z * 32;
+  f4 acc[T][2][2];
+#pragma unroll
+  for (int t = 0; t < T; t++)
+#pragma unroll
+    for (int m = 0; m < 2; m++)
+#pragma unroll
+      for (int n = 0; n < 2; n++) acc[t][m][n] = (f4){0.f, 0.f, 0.f, 0.f};
+  float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  const int q8 = (tid & 3) * 8;  // this thread's channels in the staging loads
+  const bool bias = a.want_bias && blockIdx.z == 0;
+  // fragment addresses: group g holds k = 8g.., i.e. row r + 2 (g / 2), columns 8 (g % 2)..
+  const int g = lane >> 4, li = lane & 15;
+  const int frow = 2 * (g >> 1), fcol = 8 * (g & 1) + (li >> 2), fch = 4 * (li & 3);
+  const int p_end = min(a.npatch, ((int)blockIdx.x + 1) * a.per_chunk);
+  for (int pt = blockIdx.x * a.per_chunk; pt < p_end; pt++) {
+    const int px = pt % a.npx, py = (pt / a.npx) % a.npy, b = pt / (a.npx * a.npy);
+    const int x0 = px * WG_P, y0 = py * WG_P;
+    const int64_t img = (int64_t)b * a.H * a.Wd;
+    __syncthreads();  // the tiles of the patch before are done with
+    for (int k = tid >> 2; k < HW * HW; k += 64) {
+      const int r = k / HW, c = k - r * HW, hh = y0 + r - H2, ww = x0 + c - H2;
+      const bool ok = hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd && ci0 + q8 < a.Cin;
+      *(uint4 *)&sh.t.x[k * 32 + q8] =
+          ok ? ld16(a.X + (img + (int64_t)hh * a.Wd + ww) * a.Cin + ci0 + q8, a.aligned) : make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int k = tid >> 2; k < WG_P * WG_P; k += 64) {
+      const int hh = y0 + k / WG_P, ww = x0 + k % WG_P;
+      const bool ok = hh < a.H && ww < a.Wd && co0 + q8 < a.Cout;
+      const uint4 u =
+          ok ? ld16(a.dY + (img + (int64_t)hh * a.Wd + ww) * a.Cout + co0 + q8, a.aligned) : make_uint4(0u, 0u, 0u, 0u);
+      *(uint4 *)&sh.t.y[k * 32 + q8] = u;
+      if (bias) {
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          bsum[2 * i] += __uint_as_float(w[i] << 16);
+          bsum[2 * i + 1] += __uint_as_float(w[i] & 0xffff0000u);
         }
       }
-      for (int t = 0; t < 2; t++)
-        for (int u = 0; u < 2; u++) acc[t][u] = mfma32(fa[t].get(), fb[u].get(), acc[t][u]);
     }
-    float *out = a.part + ((chunk * (a.K * a.K) + tap) * a.Cout) * (int64_t)a.Cin;
-    for (int t = 0; t < 2; t++)
-      for (int u = 0; u < 2; u++) {
-        const int ci = ci0 + u * 16 + ml;
-        if (ci >= a.Cin) continue;
-        for (int i = 0; i < 4; i++) {
-          const int co = co0 + t * 16 + 4 * kg + i;
-          if (co < a.Cout) out[(int64_t)co * a.Cin + ci] = acc[t][u][i];
+    __syncthreads();
+    // dY of the two K steps
+    bf8 fy[2][2];
+#pragma unroll
+    for (int r = 0; r < 2; r++)
+#pragma unroll
+      for (int m = 0; m < 2; m++) {
+        const uint16_t *p = &sh.t.y[((4 * wv + r + frow) * WG_P + fcol) * 32 + 16 * m + fch];
+        fy[r][m] = ld_tr(p, p + 4 * 32);
+      }
+#pragma unroll
+    for (int j = -H2; j < 2 + H2; j++)
+#pragma unroll
+      for (int dx = 0; dx < K; dx++) {
+        bf8 fx[2];
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+          const uint16_t *p = &sh.t.x[((4 * wv + j + H2 + frow) * HW + fcol + dx) * 32 + 16 * n + fch];
+          fx[n] = ld_tr(p, p + 4 * 32);
+        }
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+          const int dy = j - r + H2;  // 0 .. K - 1
+          if (dy < 0 || dy >= K) continue;
+#pragma unroll
+          for (int m = 0; m < 2; m++)
+#pragma unroll
+            for (int n = 0; n < 2; n++) acc[dy * K + dx][m][n] = mfma32(fy[r][m], fx[n], acc[dy * K + dx][m][n]);
         }
       }
   }
-}
-
-__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, int64_t nchunk, int64_t nw,
-                                                      float *__restrict__ dW) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nw) return;
-  float s = 0.f;
-  for (int64_t c = 0; c < nchunk; c++) s += part[c * nw + i];
-  dW[i] = s;
-}
-
-// db[co] = sum_p dY[p][co], per block partial sums then a chunk-ordered pass
-__global__ void __launch_bounds__(256) k_bias_grad(const uint16_t *__restrict__ dY, int64_t npix, int C,
-                                                   float *__restrict__ part) {
-  // block b sums pixels [b*KCH, (b+1)*KCH) for every channel (thread per channel)
-  for (int c = threadIdx.x; c < C; c += blockDim.x) {
-    float s = 0.f;
-    for (int k = 0; k < KCH; k++) {
-      const int64_t p = (int64_t)blockIdx.x * KCH + k;
-      if (p < npix) s += bf2f(dY[p * C + c]);
+  // the wavefronts' sums, in their order
+  const int cl = lane & 15, rg = lane >> 4;
+#pragma unroll 1
+  for (int w = 0; w < 4; w++) {
+    __syncthreads();
+    if (wv == w) {
+#pragma unroll
+      for (int t = 0; t < T; t++)
+#pragma unroll
+        for (int m = 0; m < 2; m++)
+#pragma unroll
+          for (int n = 0; n < 2; n++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+              float *o = &sh.red[(t * 32 + 16 * m + 4 * rg + i) * 32 + 16 * n + cl];
+              *o = w ? *o + acc[t][m][n][i] : acc[t][m][n][i];
+            }
     }
-    part[(int64_t)blockIdx.x * C + c] = s;
+  }
+  __syncthreads();
+  const int64_t nw = (int64_t)T * a.Cout * a.Cin;
+  float *out = a.part + (int64_t)blockIdx.x * (nw + a.Cout);
+  const int c4 = (tid & 7) * 4;
+  for (int k = tid >> 3; k < T * 32; k += 32) {
+    const int t = k >> 5, co = co0 + (k & 31);
+    if (co < a.Cout && ci0 + c4 < a.Cin)
+      st4(&out[((int64_t)t * a.Cout + co) * a.Cin + ci0 + c4], *(const f4 *)&sh.red[k * 32 + c4]);
+  }
+  if (bias) {
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 8; i++) sh.bias[(tid >> 2) * 33 + q8 + i] = bsum[i];
+    __syncthreads();
+    if (tid < 32 && co0 + tid < a.Cout) {
+      float s = 0.f;
+      for (int k = 0; k < 64; k++) s += sh.bias[k * 33 + tid];
+      out[nw + co0 + tid] = s;
+    }
+  }
+}
+
+// dW and db from the chunks' partials: G groups of threads take every G-th chunk
+// of 4 values, their sums are added in the groups' order
+template <int G>
+__global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ part, int nchunk, int64_t nw, int nb,
+                                                      float *__restrict__ dW, float *__restrict__ db) {
+  constexpr int Q = 256 / G;
+  __shared__ f4 sh[256];
+  const int64_t n = nw + nb;
+  const int64_t q = ((int64_t)blockIdx.x * Q + threadIdx.x % Q) * 4;
+  const int grp = threadIdx.x / Q;
+  f4 s = {0.f, 0.f, 0.f, 0.f};
+  if (q < n) {
+#pragma unroll 4
+    for (int c = grp; c < nchunk; c += G) s += ld4(&part[c * n + q]);
+  }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (grp == 0 && q < n) {
+#pragma unroll
+    for (int k = 1; k < G; k++) s += sh[k * Q + threadIdx.x];
+    if (q < nw) st4(&dW[q], s);
+    else if (db) st4(&db[q - nw], s);
   }
 }
 
@@ -455,22 +576,34 @@ extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t
   if (!ctx || !X || !dY || !work || !dW) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
   const int64_t npix = (int64_t)B * H * Wd;
-  const int64_t nchunk = (npix + KCH - 1) / KCH;
   const int64_t nw = (int64_t)K * K * Cout * Cin;
-  WgradArgs a{X, dY, work, B, H, Wd, Cin, Cout, K, nchunk};
-  const int tiles = ((Cout + 31) / 32) * ((Cin + 31) / 32);
-  const int gz = (tiles + 3) / 4;
+  WgradArgs a{X, dY, work, B, H, Wd, Cin, Cout};
+  a.npx = (Wd + WG_P - 1) / WG_P;
+  a.npy = (H + WG_P - 1) / WG_P;
+  if ((int64_t)B * a.npx * a.npy > INT32_MAX) return fvm_set_err(ctx, FVM_ERR_ARG, "conv: too many pixels");
+  a.npatch = B * a.npx * a.npy;
+  a.want_bias = db != nullptr;
+  a.aligned = (((uintptr_t)X | (uintptr_t)dY) & 15) == 0;
+  // enough blocks to give every CU two, within the workspace (one chunk per 256
+  // pixels) and with at least one patch each; more only grows the partials
+  const int tm = (Cout + 31) / 32, tn = (Cin + 31) / 32;
+  int64_t nchunk = (512 + tm * tn - 1) / (tm * tn);
+  const int64_t most = (npix + KCH - 1) / KCH;
+  if (nchunk > most) nchunk = most;
+  if (nchunk > a.npatch) nchunk = a.npatch;
+  a.per_chunk = (int)((a.npatch + nchunk - 1) / nchunk);
+  nchunk = (a.npatch + a.per_chunk - 1) / a.per_chunk;
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  k_wgrad<<<dim3((unsigned)nchunk, K * K, gz), 256, 0, ctx->stream>>>(a);
+  const dim3 grid((unsigned)nchunk, tm, tn);
+  if (K == 3) k_wgrad<3><<<grid, 256, 0, ctx->stream>>>(a);
+  else k_wgrad<1><<<grid, 256, 0, ctx->stream>>>(a);
   FVM_LAUNCH_CHECK(ctx);
-  k_wgrad_reduce<<<nblk(nw), 256, 0, ctx->stream>>>(work, nchunk, nw, dW);
+  const int64_t quads = (nw + Cout) / 4;  // channel counts are multiples of 16
+  if (nchunk >= 32)
+    k_wgrad_reduce<16><<<(unsigned)((quads + 15) / 16), 256, 0, ctx->stream>>>(work, (int)nchunk, nw, Cout, dW, db);
+  else
+    k_wgrad_reduce<4><<<(unsigned)((quads + 63) / 64), 256, 0, ctx->stream>>>(work, (int)nchunk, nw, Cout, dW, db);
   FVM_LAUNCH_CHECK(ctx);
-  if (db) {
-    float *bp = work + nchunk * nw;
-    k_bias_grad<<<(unsigned)nchunk, 256, 0, ctx->stream>>>(dY, npix, Cout, bp);
-    k_wgrad_reduce<<<nblk(Cout), 256, 0, ctx->stream>>>(bp, nchunk, Cout, db);
-    FVM_LAUNCH_CHECK(ctx);
-  }
   return FVM_OK;
 }
 

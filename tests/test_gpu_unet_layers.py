@@ -1,0 +1,129 @@
+"""The network's convolution kernels at the edges of their tiles (image sides and
+channel counts that leave remainders, one pixel, one and several patches per
+block), each against a plain float64 product of the same bf16 operands.
+Tolerances are the rounding bound of an fp32 sum of n products in any order,
+n 2^-23 sum |a b|, and half a bf16 step for bf16 results."""
+import numpy as np
+import pytest
+
+from oracle.unet_ref import bf16
+from fvmic2d_amd.lib import Context
+from fvmic2d_amd.unet import Buf, bind, from_bf16_bits, to_bf16_bits
+
+pytestmark = pytest.mark.gpu
+
+
+def _dev(ctx, a, dtype):
+    b = Buf(ctx, a.shape, dtype)
+    b.set(to_bf16_bits(a) if dtype == np.uint16 else a)
+    return b
+
+
+def _taps(x, K):
+    """x (B, H, W, C) -> list over taps of x shifted by the tap's offset, zero outside."""
+    h = K // 2
+    p = np.pad(x, ((0, 0), (h, h), (h, h), (0, 0)))
+    H, W = x.shape[1:3]
+    return [p[:, t // K:t // K + H, t % K:t % K + W] for t in range(K * K)]
+
+
+SHAPES = [(1, 1, 1, 16, 16, 3), (1, 5, 16, 16, 32, 3), (2, 16, 16, 32, 16, 1), (1, 17, 33, 48, 48, 3),
+          (3, 15, 9, 32, 64, 3), (1, 16, 20, 96, 32, 3), (2, 40, 35, 16, 16, 3), (1, 8, 8, 256, 128, 3),
+          (5, 33, 18, 64, 16, 1)]
+
+
+def _operands(shape, seed=0):
+    B, H, W, ci, co, K = shape
+    r = np.random.default_rng(seed)
+    X = bf16(r.standard_normal((B, H, W, ci)).astype(np.float32))
+    Wt = bf16((r.standard_normal((K * K, co, ci)) / np.sqrt(K * K * ci)).astype(np.float32))
+    dY = bf16(r.standard_normal((B, H, W, co)).astype(np.float32))
+    return X, Wt, dY
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_weight_gradient(shape):
+    print("CASE wgrad", shape, flush=True)
+    B, H, W, ci, co, K = shape
+    X, _, dY = _operands(shape)
+    ctx, lib = Context(), bind()
+    dX, ddY = _dev(ctx, X, np.uint16), _dev(ctx, dY, np.uint16)
+    dW, db = Buf(ctx, (K * K, co, ci), np.float32), Buf(ctx, (co,), np.float32)
+    ws = Buf(ctx, (lib.fvm_nn_wgrad_workspace(B, H, W, ci, co, K) // 4,), np.float32)
+    assert lib.fvm_nn_conv_wgrad(ctx.h, dX.ptr, ddY.ptr, B, H, W, ci, co, K, ws.ptr, dW.ptr, db.ptr) == 0
+    flat = dY.reshape(-1, co).astype(np.float64)
+    n = flat.shape[0]
+    got = dW.get()
+    for t, x in enumerate(_taps(X, K)):
+        x = x.reshape(-1, ci).astype(np.float64)
+        assert np.all(np.abs(got[t] - flat.T @ x) <= n * 2.0 ** -23 * (np.abs(flat).T @ np.abs(x)) + 1e-30), t
+    assert np.all(np.abs(db.get() - flat.sum(0)) <= n * 2.0 ** -23 * np.abs(flat).sum(0) + 1e-30)
+
+
+def test_weight_gradient_takes_any_even_address():
+    """Operands that start between 16-byte boundaries, as views of a larger array may."""
+    print("CASE wgrad unaligned", flush=True)
+    B, H, W, ci, co, K = shape = (1, 9, 10, 16, 16, 3)
+    X, _, dY = _operands(shape, 3)
+    ctx, lib = Context(), bind()
+    outs = []
+    for off in (0, 1):
+        dX, ddY = Buf(ctx, (X.size + 8,), np.uint16), Buf(ctx, (dY.size + 8,), np.uint16)
+        for buf, a in ((dX, X), (ddY, dY)):
+            full = np.zeros(a.size + 8, np.uint16)
+            full[off:off + a.size] = to_bf16_bits(a).ravel()
+            buf.set(full)
+        n = K * K * co * ci
+        dW, db = Buf(ctx, (n + 4,), np.float32), Buf(ctx, (co + 4,), np.float32)
+        ws = Buf(ctx, (lib.fvm_nn_wgrad_workspace(B, H, W, ci, co, K) // 4 + 4,), np.float32)
+        assert lib.fvm_nn_conv_wgrad(ctx.h, dX.ptr + 2 * off, ddY.ptr + 2 * off, B, H, W, ci, co, K, ws.ptr + 4 * off,
+                                     dW.ptr + 4 * off, db.ptr + 4 * off) == 0
+        outs.append((dW.get()[off:off + n], db.get()[off:off + co]))
+    assert np.array_equal(outs[0][0], outs[1][0]) and np.array_equal(outs[0][1], outs[1][1])
+
+
+def _check_bf16(got, ref, bound):
+    assert np.all(np.abs(got - ref) <= bound + 2.0 ** -8 * (np.abs(ref) + bound)), np.abs(got - ref).max()
+
+
+@pytest.mark.parametrize("relu", [0, 1])
+@pytest.mark.parametrize("shape", SHAPES)
+def test_forward(shape, relu):
+    print("CASE conv", shape, relu, flush=True)
+    B, H, W, ci, co, K = shape
+    X, Wt, _ = _operands(shape, 1)
+    b = np.random.default_rng(2).standard_normal(co).astype(np.float32)
+    ctx, lib = Context(), bind()
+    dX, dW, dB = _dev(ctx, X, np.uint16), _dev(ctx, Wt, np.uint16), _dev(ctx, b, np.float32)
+    Y, Yf = Buf(ctx, (B, H, W, co), np.uint16), Buf(ctx, (B, H, W, co), np.float32)
+    real = co - 5
+    assert lib.fvm_nn_conv_fwd(ctx.h, dX.ptr, dW.ptr, dB.ptr, B, H, W, ci, co, K, relu, real, Y.ptr, Yf.ptr) == 0
+    ref, mag = np.zeros((B, H, W, co)), np.zeros((B, H, W, co))
+    for t, x in enumerate(_taps(X, K)):
+        w = Wt[t].astype(np.float64).T
+        ref += x.astype(np.float64) @ w
+        mag += np.abs(x) @ np.abs(w)
+    ref, mag = ref + b, mag + np.abs(b)
+    if relu:
+        ref = np.maximum(ref, 0.0)
+    ref[..., real:], mag[..., real:] = 0.0, 0.0
+    bound = (K * K * ci + 1) * 2.0 ** -23 * mag
+    assert np.all(np.abs(Yf.get() - ref) <= bound)
+    _check_bf16(from_bf16_bits(Y.get()), ref, bound)
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_data_gradient(shape):
+    print("CASE dgrad", shape, flush=True)
+    B, H, W, ci, co, K = shape
+    _, Wt, dY = _operands(shape, 4)
+    ctx, lib = Context(), bind()
+    ddY, dW = _dev(ctx, dY, np.uint16), _dev(ctx, Wt, np.uint16)
+    scratch, dX = Buf(ctx, (K * K * co * ci,), np.uint16), Buf(ctx, (B, H, W, ci), np.uint16)
+    assert lib.fvm_nn_conv_dgrad(ctx.h, ddY.ptr, dW.ptr, scratch.ptr, B, H, W, ci, co, K, dX.ptr) == 0
+    ref, mag = np.zeros((B, H, W, ci)), np.zeros((B, H, W, ci))
+    for t, y in enumerate(_taps(dY, K)):
+        w = Wt[K * K - 1 - t].astype(np.float64)
+        ref += y.astype(np.float64) @ w
+        mag += np.abs(y) @ np.abs(w)
+    _check_bf16(from_bf16_bits(dX.get()), ref, K * K * co * 2.0 ** -23 * mag)
