@@ -34,13 +34,7 @@ __device__ __forceinline__ f4 mfma32(bf8 a, bf8 b, f4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-// 8 consecutive bf16 from a 16-byte aligned address, or zeros
-__device__ __forceinline__ bf8 ld8(const uint16_t *p, bool ok) {
-  const uint4 u = ok ? *(const uint4 *)p : make_uint4(0u, 0u, 0u, 0u);
-  return __builtin_bit_cast(bf8, u);
-}
-
-// eight bf16 gathered one by one (the weight gradient's pixel-strided operands)
+// eight bf16 one by one (the self-test's operands)
 struct Bf8Builder {
   uint16_t h[8];
   __device__ __forceinline__ bf8 get() const {
@@ -68,85 +62,304 @@ __global__ void __launch_bounds__(64) k_mfma_selftest(const uint16_t *__restrict
   for (int i = 0; i < 4; i++) D[(4 * kg + i) * 16 + m] = c[i];
 }
 
+// transposed fragments from LDS (the weights of the data gradient, both operands
+// of the weight gradient)
+typedef short s4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s4 lds_s4;
+
+// K = 32 fragment (8 bf16 per lane): rows k = 8 (lane / 16) .. + 7 of the lane's
+// column lane % 16; p0, p1: this lane's 8-byte address among the first and the
+// last four of its group's rows (row (lane % 16) / 4, channels 4 (lane % 4))
+__device__ __forceinline__ bf8 ld_tr(const uint16_t *p0, const uint16_t *p1) {
+  union {
+    s4 h[2];
+    bf8 v;
+  } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p0);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p1);
+  return u.v;
+}
+
+// vectors at their elements' alignment (one access where the address allows)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint16_t h4u __attribute__((ext_vector_type(4), aligned(2)));
+__device__ __forceinline__ void st4(float *p, f4 v) { *(f4u *)p = v; }
+__device__ __forceinline__ f4 ld4(const float *p) { return *(const f4u *)p; }
+
 // ---- convolution (implicit GEMM) ------------------------------------------------
 // Y[p][co] = act(bias[co] + sum_{tap, ci} X[p + off(tap)][ci] * W[tap][co][ci])
-// off(tap) = (ky - K/2, kx - K/2); X outside the image reads 0.
-// Block: 256 threads = 4 wavefronts in a 2x2 arrangement, tile 64 pixels x 64
-// output channels; each wavefront 32 x 32 = 2 x 2 MFMA tiles.
+// off(tap) = (ky - K/2, kx - K/2); X outside the image reads 0.  TR: the data
+// gradient, whose weights are W[taps - 1 - tap][ci][co], read as they lie and
+// transposed on the way out of LDS.
+//
+// Block: 4 WN wavefronts, a patch of 16 x 4R pixels and 16 NT WN output channels;
+// a wavefront has R rows of 16 pixels and NT channel tiles.  The patch and its halo
+// are staged in LDS with all their channels, as slabs of 32 ([slab][pixel][32]: a
+// row's 16 pixels are one conflict-free 1 KB fragment); the weights follow in
+// groups of taps, the next group's loads in flight while one is used.  Every
+// output is summed tap by tap, within a tap by channel: the order is the same for
+// every tile shape, so a network's activations do not depend on which one a size
+// takes (a changed order flips bf16 roundings, and each layer multiplies them).
+// The weights are the A operand, so a lane ends with four consecutive channels of
+// one pixel.  The shapes are picked by conv_launch.
 struct ConvArgs {
   const uint16_t *X;
   const uint16_t *W;
   const float *bias;  // may be null
   uint16_t *Y;        // bf16 output (or null)
   float *Yf;          // fp32 output (or null)
-  int B, H, Wd, Cin, Cout, K, relu;
+  int B, H, Wd, Cin, Cout, relu;
   int cout_real;  // channels >= cout_real are written as 0 (padding)
+  int npx, npy;   // patches per image
+  int slabs;      // of 32 input channels
+  int group;      // taps whose weights are staged together
 };
 
-__global__ void __launch_bounds__(256) k_conv(ConvArgs a) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+#define CONV_WPIECES 6  // 16-byte pieces of a weight group per thread
+
+template <int K, int R, int NT, int WN, bool TR>
+__global__ void __launch_bounds__(256 * WN) k_conv(ConvArgs a) {
+  constexpr int H2 = K / 2, T = K * K, PW = 16 + 2 * H2, PH = 4 * R + 2 * H2, NP = PH * PW;
+  constexpr int TH = 256 * WN, CO = 16 * NT * WN;
+  extern __shared__ uint4 lds[];
+  uint16_t *sx = (uint16_t *)lds, *sw = sx + a.slabs * NP * 32;
+  const int tid = threadIdx.x, lane = tid & 63, wv = (tid >> 6) & 3, wn = tid >> 8;
+  const int px = blockIdx.x % a.npx, py = (blockIdx.x / a.npx) % a.npy, b = blockIdx.x / (a.npx * a.npy);
+  const int x0 = px * 16, y0 = py * 4 * R, c0 = blockIdx.y * CO;
+  const int64_t img = (int64_t)b * a.H * a.Wd;
+  uint4 rw[CONV_WPIECES];
+  // weights of taps t0 .. t0 + group - 1, zeros past Cin and Cout:
+  // [tap][slab][co][32 ci], TR: [tap][slab][32 k][co]
+  auto load_w = [&](int t0) {
+    const int n = min(a.group, T - t0) * a.slabs * CO * 4;
+#pragma unroll
+    for (int i = 0; i < CONV_WPIECES; i++) {
+      const int q = tid + TH * i;
+      rw[i] = make_uint4(0u, 0u, 0u, 0u);
+      if (q >= n) continue;
+      const int ts = q / (CO * 4), r = q - ts * (CO * 4);
+      const int t = t0 + ts / a.slabs, k0 = (ts % a.slabs) * 32;
+      if (!TR) {
+        const int co = c0 + (r >> 2), ch = k0 + (r & 3) * 8;
+        if (co < a.Cout && ch < a.Cin) rw[i] = *(const uint4 *)(a.W + ((int64_t)t * a.Cout + co) * a.Cin + ch);
+      } else {
+        const int k = k0 + r / (CO / 8), co = c0 + r % (CO / 8) * 8;
+        if (co < a.Cout && k < a.Cin) rw[i] = *(const uint4 *)(a.W + ((int64_t)(T - 1 - t) * a.Cin + k) * a.Cout + co);
+      }
+    }
+  };
+  load_w(0);
+  // the patch: 4 pieces a pixel and slab, SB slabs' loads in flight together
+  constexpr int XC = (NP * 4 + TH - 1) / TH, SB = XC >= 12 ? 1 : 12 / XC;
+#pragma unroll 1
+  for (int s0 = 0; s0 < a.slabs; s0 += SB) {
+    uint4 rx[SB][XC];
+#pragma unroll
+    for (int s = 0; s < SB; s++)
+#pragma unroll
+      for (int i = 0; i < XC; i++) {
+        const int q = tid + TH * i, pix = q >> 2, c = (s0 + s) * 32 + (q & 3) * 8;
+        const int hh = y0 + pix / PW - H2, ww = x0 + pix % PW - H2;
+        const bool ok = q < NP * 4 && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd;
+        rx[s][i] = ok ? *(const uint4 *)(a.X + (img + (int64_t)hh * a.Wd + ww) * a.Cin + c) : make_uint4(0u, 0u, 0u, 0u);
+      }
+#pragma unroll
+    for (int s = 0; s < SB; s++)
+#pragma unroll
+      for (int i = 0; i < XC; i++)
+        if (tid + TH * i < NP * 4 && s0 + s < a.slabs) *(uint4 *)&sx[(s0 + s) * NP * 32 + (tid + TH * i) * 8] = rx[s][i];
+  }
+  f4 acc[R][NT];
+#pragma unroll
+  for (int r = 0; r < R; r++)
+#pragma unroll
+    for (int n = 0; n < NT; n++) acc[r][n] = (f4){0.f, 0.f, 0.f, 0.f};
+  const int li = lane & 15, g = lane >> 4;
+#pragma unroll 1
+  for (int t0 = 0; t0 < T; t0 += a.group) {
+    const int tn = min(a.group, T - t0), n16 = tn * a.slabs * CO * 4;
+    if (t0) __syncthreads();
+#pragma unroll
+    for (int i = 0; i < CONV_WPIECES; i++)
+      if (tid + TH * i < n16) *(uint4 *)&sw[(tid + TH * i) * 8] = rw[i];
+    __syncthreads();
+    if (t0 + a.group < T) load_w(t0 + a.group);
+    // (tap, slab) steps, the next step's fragments read while one is multiplied
+    const uint16_t *wr = sw + (TR ? (8 * g + (li >> 2)) * CO + wn * 16 * NT + 4 * (li & 3) : (wn * 16 * NT + li) * 32 + 8 * g);
+    int sl = 0, dy = t0 / K, dx = t0 - dy * K;
+    bf8 fx[2][R], fw[2][NT];
+    auto frag = [&](int f) {
+      const uint16_t *xr = sx + sl * NP * 32 + (dy * PW + dx) * 32 + (R * wv * PW + li) * 32 + 8 * g;
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+        fw[f][n] = TR ? ld_tr(wr + 16 * n, wr + 16 * n + 4 * CO) : __builtin_bit_cast(bf8, *(const uint4 *)(wr + n * 16 * 32));
+#pragma unroll
+      for (int r = 0; r < R; r++) fx[f][r] = __builtin_bit_cast(bf8, *(const uint4 *)(xr + r * PW * 32));
+      wr += CO * 32;
+      if (++sl == a.slabs) {
+        sl = 0;
+        if (++dx == K) dx = 0, dy++;
+      }
+    };
+    auto mul = [&](int f) {
+#pragma unroll
+      for (int n = 0; n < NT; n++)
+#pragma unroll
+        for (int r = 0; r < R; r++) acc[r][n] = mfma32(fw[f][n], fx[f][r], acc[r][n]);
+    };
+    const int steps = tn * a.slabs;
+    frag(0);
+    int it = 1;
+#pragma unroll 1
+    for (; it + 1 < steps; it += 2) {
+      frag(1);
+      mul(0);
+      frag(0);
+      mul(1);
+    }
+    if (it < steps) {
+      frag(1);
+      mul(0);
+      mul(1);
+    } else {
+      mul(0);
+    }
+  }
+  // D[m = 4 g + i][n = li]: channel 4 g + i of pixel li of the row
+  const int ww = x0 + li;
+#pragma unroll
+  for (int n = 0; n < NT; n++) {
+    const int co = c0 + 16 * (wn * NT + n) + 4 * g;
+    if (co >= a.Cout) continue;  // Cout is a multiple of 16
+    const f4 bv = a.bias ? ld4(a.bias + co) : (f4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+      const int hh = y0 + R * wv + r;
+      if (hh >= a.H || ww >= a.Wd) continue;
+      f4 v = acc[r][n] + bv;
+      h4u h;
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        if (a.relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
+        if (co + i >= a.cout_real) v[i] = 0.f;
+        h[i] = f2bf(v[i]);
+      }
+      const int64_t o = (img + (int64_t)hh * a.Wd + ww) * a.Cout + co;
+      if (a.Y) *(h4u *)(a.Y + o) = h;
+      if (a.Yf) st4(a.Yf + o, v);
+    }
+  }
+}
+
+// Layers whose patch does not fit LDS with all channels (above 600 or so): the
+// fragments come from global memory, 2 x 2 tiles per wavefront.
+template <int K, bool TR>
+__global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
+  constexpr int T = K * K;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
   const int64_t npix = (int64_t)a.B * a.H * a.Wd;
   const int64_t p0 = (int64_t)blockIdx.x * 64 + (wv & 1) * 32;
   const int c0 = blockIdx.y * 64 + (wv >> 1) * 32;
-  const int ml = lane % 16, kg = lane / 16;
-  // the two pixels (one per M tile) this lane loads A rows for
   int64_t pp[2];
-  int pb[2], ph[2], pw[2];
-  bool pv[2];
-  for (int t = 0; t < 2; t++) {
-    const int64_t p = p0 + t * 16 + ml;
-    pv[t] = p < npix;
-    const int64_t q = pv[t] ? p : 0;
-    pw[t] = (int)(q % a.Wd);
-    ph[t] = (int)((q / a.Wd) % a.H);
-    pb[t] = (int)(q / ((int64_t)a.Wd * a.H));
-    pp[t] = q;
+  int ph[2], pw[2];
+#pragma unroll
+  for (int r = 0; r < 2; r++) {
+    const int64_t p = p0 + r * 16 + li, q = p < npix ? p : 0;
+    pp[r] = p < npix ? q : -1;
+    pw[r] = (int)(q % a.Wd);
+    ph[r] = (int)((q / a.Wd) % a.H);
   }
-  f4 acc[2][2];
-  for (int i = 0; i < 2; i++)
-    for (int j = 0; j < 2; j++) acc[i][j] = (f4){0.f, 0.f, 0.f, 0.f};
-  const int half = a.K / 2;
-  for (int tap = 0; tap < a.K * a.K; tap++) {
-    const int dy = tap / a.K - half, dx = tap % a.K - half;
-    const uint16_t *xs[2];
-    bool xv[2];
-    for (int t = 0; t < 2; t++) {
-      const int hh = ph[t] + dy, ww = pw[t] + dx;
-      xv[t] = pv[t] && hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd;
-      xs[t] = a.X + ((((int64_t)pb[t] * a.H + (xv[t] ? hh : 0)) * a.Wd + (xv[t] ? ww : 0)) * a.Cin);
-    }
-    const uint16_t *wt = a.W + (int64_t)tap * a.Cout * a.Cin;
-    // Cin is a multiple of 16: a lane's eight channels lie wholly inside or
-    // wholly past it (a 16-channel layer leaves half of K at zero)
-    for (int ci0 = 0; ci0 < a.Cin; ci0 += 32) {
-      const int ck = ci0 + 8 * kg;
-      const bool kin = ck < a.Cin;
-      bf8 fa[2], fb[2];
-      for (int t = 0; t < 2; t++) fa[t] = ld8(xs[t] + ck, xv[t] && kin);
-      for (int u = 0; u < 2; u++) {
-        const int co = c0 + u * 16 + ml;
-        fb[u] = ld8(wt + (int64_t)co * a.Cin + ck, co < a.Cout && kin);
+  const bf8 zero = __builtin_bit_cast(bf8, make_uint4(0u, 0u, 0u, 0u));
+  f4 acc[2][2] = {};
+#pragma unroll 1
+  for (int t = 0; t < T; t++) {
+    const int dy = t / K - K / 2, dx = t % K - K / 2;
+    for (int k0 = 0; k0 < a.Cin; k0 += 32) {
+      const int k = k0 + 8 * g;
+      bf8 fx[2], fw[2];
+#pragma unroll
+      for (int r = 0; r < 2; r++) {
+        const bool ok = pp[r] >= 0 && k < a.Cin && ph[r] + dy >= 0 && ph[r] + dy < a.H && pw[r] + dx >= 0 && pw[r] + dx < a.Wd;
+        fx[r] = ok ? __builtin_bit_cast(bf8, *(const uint4 *)(a.X + (pp[r] + (int64_t)dy * a.Wd + dx) * a.Cin + k)) : zero;
       }
-      for (int t = 0; t < 2; t++)
-        for (int u = 0; u < 2; u++) acc[t][u] = mfma32(fa[t], fb[u], acc[t][u]);
+#pragma unroll
+      for (int n = 0; n < 2; n++) {
+        const int co = c0 + 16 * n + li;
+        fw[n] = zero;
+        if (co >= a.Cout || k >= a.Cin) continue;
+        if (!TR) {
+          fw[n] = __builtin_bit_cast(bf8, *(const uint4 *)(a.W + ((int64_t)t * a.Cout + co) * a.Cin + k));
+        } else {
+          Bf8Builder w;
+          for (int i = 0; i < 8; i++) w.h[i] = a.W[((int64_t)(T - 1 - t) * a.Cin + k + i) * a.Cout + co];
+          fw[n] = w.get();
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < 2; n++)
+#pragma unroll
+        for (int r = 0; r < 2; r++) acc[r][n] = mfma32(fw[n], fx[r], acc[r][n]);
     }
   }
-  // epilogue: D[m = 4*kg + i][n = ml] of tile (t, u)
-  for (int t = 0; t < 2; t++)
-    for (int u = 0; u < 2; u++) {
-      const int co = c0 + u * 16 + ml;
-      if (co >= a.Cout) continue;
-      const float bv = a.bias ? a.bias[co] : 0.f;
+#pragma unroll
+  for (int n = 0; n < 2; n++) {
+    const int co = c0 + 16 * n + 4 * g;
+    if (co >= a.Cout) continue;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      if (pp[r] < 0) continue;
       for (int i = 0; i < 4; i++) {
-        const int64_t p = p0 + t * 16 + 4 * kg + i;
-        if (p >= npix) continue;
-        float v = acc[t][u][i] + bv;
+        float v = acc[r][n][i] + (a.bias ? a.bias[co + i] : 0.f);
         if (a.relu) v = v > 0.f ? v : 0.f;
-        if (co >= a.cout_real) v = 0.f;
-        if (a.Y) a.Y[p * a.Cout + co] = f2bf(v);
-        if (a.Yf) a.Yf[p * a.Cout + co] = v;
+        if (co + i >= a.cout_real) v = 0.f;
+        if (a.Y) a.Y[pp[r] * a.Cout + co + i] = f2bf(v);
+        if (a.Yf) a.Yf[pp[r] * a.Cout + co + i] = v;
       }
     }
+  }
+}
+
+// taps whose weights fit a stage's registers and 48 KB; 0: not one tap does
+int conv_group(int T, int slabs, int CO, int threads) {
+  const int per_tap = slabs * CO * 64;  // bytes
+  int g = threads * CONV_WPIECES * 16 / per_tap;
+  return g > T ? T : g;
+}
+
+template <int K, int R, int NT, int WN, bool TR>
+bool conv_try(fvm_ctx *ctx, ConvArgs a, int64_t want, size_t most_lds) {
+  constexpr int H2 = K / 2, NP = (4 * R + 2 * H2) * (16 + 2 * H2), CO = 16 * NT * WN;
+  a.npx = (a.Wd + 15) / 16;
+  a.npy = (a.H + 4 * R - 1) / (4 * R);
+  a.slabs = (a.Cin + 31) / 32;
+  a.group = conv_group(K * K, a.slabs, CO, 256 * WN);
+  const int64_t nx = (int64_t)a.B * a.npx * a.npy, ny = (a.Cout + CO - 1) / CO;
+  const size_t lds = (size_t)a.slabs * (NP + a.group * CO) * 64;
+  if (a.group < 1 || nx * ny < want || lds > most_lds) return false;
+  k_conv<K, R, NT, WN, TR><<<dim3((unsigned)nx, (unsigned)ny), 256 * WN, lds, ctx->stream>>>(a);
+  return true;
+}
+
+// The largest tile that still gives every CU a block and leaves LDS for two of
+// them (CU: 160 KB), then smaller tiles, then the smallest in any case.  A large
+// tile reads its operands least often (R + NT fragments for R NT matrix
+// instructions), but the deep levels have few pixels: 2048 at 16 x 16 and batch 8,
+// 1024 when one 256 x 256 state is predicted.
+template <int K, bool TR>
+void conv_launch(fvm_ctx *ctx, const ConvArgs &a) {
+  constexpr size_t HALF = 80 << 10, ALL = 160 << 10;
+  if (a.Cout >= 64) {
+    if (conv_try<K, 4, 2, 2, TR>(ctx, a, 256, HALF) || conv_try<K, 2, 2, 2, TR>(ctx, a, 256, HALF) ||
+        conv_try<K, 1, 2, 2, TR>(ctx, a, 256, ALL))
+      return;
+  } else if (a.Cout >= 32) {
+    if (conv_try<K, 4, 2, 1, TR>(ctx, a, 512, HALF) || conv_try<K, 2, 2, 1, TR>(ctx, a, 512, HALF)) return;
+  } else if (conv_try<K, 4, 1, 1, TR>(ctx, a, 512, HALF)) {
+    return;
+  }
+  if (conv_try<K, 1, 2, 1, TR>(ctx, a, 512, ALL) || conv_try<K, 1, 1, 1, TR>(ctx, a, 0, ALL)) return;
+  const int64_t npix = (int64_t)a.B * a.H * a.Wd;
+  k_conv_wide<K, TR><<<dim3((unsigned)((npix + 63) / 64), (unsigned)((a.Cout + 63) / 64)), 256, 0, ctx->stream>>>(a);
 }
 
 // ---- weight gradient --------------------------------------------------------------
@@ -184,27 +397,6 @@ __device__ __forceinline__ uint4 ld16(const uint16_t *p, int aligned) {
   for (int i = 0; i < 4; i++) w[i] = (uint32_t)p[2 * i] | ((uint32_t)p[2 * i + 1] << 16);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
-
-typedef short s4 __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) s4 lds_s4;
-
-// K = 32 fragment (8 bf16 per lane): rows k = 8 (lane / 16) .. + 7 of the lane's
-// column lane % 16; p0, p1: this lane's 8-byte address among the first and the
-// last four of its group's rows (row (lane % 16) / 4, channels 4 (lane % 4))
-__device__ __forceinline__ bf8 ld_tr(const uint16_t *p0, const uint16_t *p1) {
-  union {
-    s4 h[2];
-    bf8 v;
-  } u;
-  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p0);
-  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4 *)p1);
-  return u.v;
-}
-
-// four floats at a 4-byte boundary (one 16-byte access where the address allows)
-typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
-__device__ __forceinline__ void st4(float *p, f4 v) { *(f4u *)p = v; }
-__device__ __forceinline__ f4 ld4(const float *p) { return *(const f4u *)p; }
 
 template <int K>
 __global__ void __launch_bounds__(256) k_wgrad(WgradArgs a) {
@@ -354,18 +546,6 @@ __global__ void __launch_bounds__(256) k_wgrad_reduce(const float *__restrict__ 
     if (q < nw) st4(&dW[q], s);
     else if (db) st4(&db[q - nw], s);
   }
-}
-
-// dWd[tap'][ci][co] = W[K*K-1-tap'][co][ci]: weights of the data-gradient conv
-__global__ void __launch_bounds__(256) k_flip_weights(const uint16_t *__restrict__ W, int K, int Cout, int Cin,
-                                                      uint16_t *__restrict__ Wd) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t n = (int64_t)K * K * Cout * Cin;
-  if (i >= n) return;
-  const int ci = (int)(i % Cin);
-  const int co = (int)((i / Cin) % Cout);
-  const int tap = (int)(i / ((int64_t)Cin * Cout));
-  Wd[((int64_t)(K * K - 1 - tap) * Cin + ci) * Cout + co] = W[i];
 }
 
 // ---- elementwise layers ------------------------------------------------------------
@@ -534,33 +714,34 @@ static int conv_check(fvm_ctx *ctx, int B, int H, int W, int Cin, int Cout, int 
   return FVM_OK;
 }
 
+static int conv_run(fvm_ctx *ctx, const ConvArgs &a, int K, bool tr) {
+  if ((int64_t)a.B * ((a.Wd + 15) / 16) * ((a.H + 3) / 4) > INT32_MAX)
+    return fvm_set_err(ctx, FVM_ERR_ARG, "conv: too many pixels");
+  if (K == 3) tr ? conv_launch<3, true>(ctx, a) : conv_launch<3, false>(ctx, a);
+  else tr ? conv_launch<1, true>(ctx, a) : conv_launch<1, false>(ctx, a);
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
 extern "C" int fvm_nn_conv_fwd(fvm_ctx *ctx, const uint16_t *X, const uint16_t *W, const float *bias, int32_t B,
                                int32_t H, int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, int32_t relu,
                                int32_t cout_real, uint16_t *Y, float *Yf) {
   if (!ctx || !X || !W || (!Y && !Yf)) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
-  ConvArgs a{X, W, bias, Y, Yf, B, H, Wd, Cin, Cout, K, relu, cout_real > 0 ? cout_real : Cout};
-  const int64_t npix = (int64_t)B * H * Wd;
+  ConvArgs a{X, W, bias, Y, Yf, B, H, Wd, Cin, Cout, relu, cout_real > 0 ? cout_real : Cout};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  k_conv<<<dim3((unsigned)((npix + 63) / 64), (unsigned)((Cout + 63) / 64)), 256, 0, ctx->stream>>>(a);
-  FVM_LAUNCH_CHECK(ctx);
-  return FVM_OK;
+  return conv_run(ctx, a, K, false);
 }
 
-// dX = conv(dY, flipped transposed W); Wd_scratch: K*K*Cout*Cin bf16
+// dX = conv(dY, flipped transposed W), the flip and the transposition made while
+// the weights are read (Wd_scratch, K*K*Cout*Cin bf16, is no longer written)
 extern "C" int fvm_nn_conv_dgrad(fvm_ctx *ctx, const uint16_t *dY, const uint16_t *W, uint16_t *Wd_scratch, int32_t B,
                                  int32_t H, int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, uint16_t *dX) {
   if (!ctx || !dY || !W || !Wd_scratch || !dX) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
-  const int64_t nw = (int64_t)K * K * Cout * Cin;
+  ConvArgs a{dY, W, nullptr, dX, nullptr, B, H, Wd, Cout, Cin, 0, Cin};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  k_flip_weights<<<nblk(nw), 256, 0, ctx->stream>>>(W, K, Cout, Cin, Wd_scratch);
-  FVM_LAUNCH_CHECK(ctx);
-  ConvArgs a{dY, Wd_scratch, nullptr, dX, nullptr, B, H, Wd, Cout, Cin, K, 0, Cin};
-  const int64_t npix = (int64_t)B * H * Wd;
-  k_conv<<<dim3((unsigned)((npix + 63) / 64), (unsigned)((Cin + 63) / 64)), 256, 0, ctx->stream>>>(a);
-  FVM_LAUNCH_CHECK(ctx);
-  return FVM_OK;
+  return conv_run(ctx, a, K, true);
 }
 
 // bytes of fp32 workspace fvm_nn_conv_wgrad needs
