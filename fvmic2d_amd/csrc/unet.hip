@@ -370,15 +370,18 @@ void conv_launch(fvm_ctx *ctx, const ConvArgs &a) {
 // read four 32-byte rows, lane i gets column i of them); a tap is then only
 // another row address.
 //
-// Block: 4 wavefronts, 32 co x 32 ci, all taps (36 accumulator tiles); patches of
-// 16 x 16 pixels one after the other, wavefront w taking its rows 4w..4w+3 as two
-// K steps of rows (r, r + 2): the rows a tap needs, shifted by dy, are then another
-// step's, and each is read once per dx.  56 LDS reads serve 72 matrix
-// instructions.  Blocks split the patches (`nchunk`) to fill the chip; their fp32
-// partials, and those of the bias, are added in chunk order by k_wgrad_reduce.
+// A wavefront has 32 co x 32 ci and all taps (36 accumulator tiles) and takes
+// patches of 16 x 16 pixels in K steps of two rows, half its rows apart: the rows a
+// tap needs, shifted by dy, are then another step's, and each is read once per dx.
+// SPLIT (few channels): the block's 4 wavefronts share 32 co x 32 ci and split the
+// patch's rows, their sums added in LDS at the end; otherwise they share a patch
+// and have 64 co x 64 ci between them.  Blocks split the patches (`nchunk`) to fill
+// the chip; their fp32 partials, and those of the bias, are added in chunk order
+// by k_wgrad_reduce.  What bounds it is getting the patches in: all loads of a
+// patch are issued together, and two blocks of a CU overlap.
 // Before, every bf16 was gathered from global memory by itself and one thread
 // summed a weight's partials over all chunks: one optimiser step's 15 gradients at
-// batch 8, 128 x 128 took 3.29 ms of the step's 4.59; they now take 0.79.
+// batch 8, 128 x 128 took 3.29 ms; now 0.43.
 #define KCH 256
 #define WG_P 16              // patch edge
 #define WG_HW (WG_P + 2)     // with the taps' halo
@@ -398,18 +401,41 @@ __device__ __forceinline__ uint4 ld16(const uint16_t *p, int aligned) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
-template <int K>
-__global__ void __launch_bounds__(256) k_wgrad(WgradArgs a) {
-  constexpr int H2 = K / 2, HW = WG_P + 2 * H2, T = K * K;
-  __shared__ union {
-    struct {
-      uint16_t x[HW * HW * 32], y[WG_P * WG_P * 32];
-    } t;
-    float red[T * 32 * 32];
-    float bias[64 * 33];
-  } sh;
+// N 16-byte pieces per thread of a patch of PW x PH pixels at (x0, y0), slabs of 32
+// channels from c0 (SL of them), into LDS as [slab][pixel][32]; zeros outside
+template <int SL, int PW, int PH>
+struct Patch {
+  static constexpr int NP = PW * PH, N = (NP * 4 * SL + 255) / 256;
+  uint4 r[N];
+  __device__ __forceinline__ void load(const uint16_t *X, int64_t img, int H, int W, int C, int x0, int y0, int c0, int aligned) {
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+      const int q = threadIdx.x + 256 * i, sl = q / (NP * 4), pix = (q - sl * NP * 4) >> 2, c = c0 + 32 * sl + (q & 3) * 8;
+      const int hh = y0 + pix / PW, ww = x0 + pix % PW;
+      const bool ok = q < NP * 4 * SL && hh >= 0 && hh < H && ww >= 0 && ww < W && c < C;
+      r[i] = ok ? ld16(X + (img + (int64_t)hh * W + ww) * C + c, aligned) : make_uint4(0u, 0u, 0u, 0u);
+    }
+  }
+  __device__ __forceinline__ void store(uint16_t *sh) const {
+#pragma unroll
+    for (int i = 0; i < N; i++)
+      if (threadIdx.x + 256 * i < NP * 4 * SL) *(uint4 *)&sh[(threadIdx.x + 256 * i) * 8] = r[i];
+  }
+};
+
+template <int K, bool SPLIT>
+__global__ void __launch_bounds__(256, 2) k_wgrad(WgradArgs a) {
+  constexpr int H2 = K / 2, HW = WG_P + 2 * H2, T = K * K, SL = SPLIT ? 1 : 2;
+  constexpr int ROWS = SPLIT ? 4 : 16, STEPS = ROWS / 2;  // of a wavefront
+  typedef Patch<SL, HW, HW> PX;
+  typedef Patch<SL, WG_P, WG_P> PY;
+  constexpr int TILES = SL * (HW * HW + WG_P * WG_P) * 64, RED = SPLIT ? 2 * T * 4 * 64 * 16 : 0;
+  __shared__ uint4 lds[(TILES > RED ? TILES : RED) / 16];
+  uint16_t *sx = (uint16_t *)lds, *sy = sx + SL * HW * HW * 32;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int co0 = blockIdx.y * 32, ci0 = blockIdx.z * 32;
+  const int co0 = blockIdx.y * 32 * SL, ci0 = blockIdx.z * 32 * SL;  // the block's
+  const int row0 = SPLIT ? ROWS * wv : 0;
+  const uint16_t *wx = SPLIT ? sx : sx + (wv & 1) * HW * HW * 32, *wy = SPLIT ? sy : sy + (wv >> 1) * WG_P * WG_P * 32;
   f4 acc[T][2][2];
 #pragma unroll
   for (int t = 0; t < T; t++)
@@ -417,107 +443,120 @@ __global__ void __launch_bounds__(256) k_wgrad(WgradArgs a) {
     for (int m = 0; m < 2; m++)
 #pragma unroll
       for (int n = 0; n < 2; n++) acc[t][m][n] = (f4){0.f, 0.f, 0.f, 0.f};
-  float bsum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  const int q8 = (tid & 3) * 8;  // this thread's channels in the staging loads
+  float bsum[SL][8] = {};
   const bool bias = a.want_bias && blockIdx.z == 0;
-  // fragment addresses: group g holds k = 8g.., i.e. row r + 2 (g / 2), columns 8 (g % 2)..
+  // fragment addresses: group g holds k = 8g.., i.e. row r + STEPS (g / 2), columns 8 (g % 2)..
   const int g = lane >> 4, li = lane & 15;
-  const int frow = 2 * (g >> 1), fcol = 8 * (g & 1) + (li >> 2), fch = 4 * (li & 3);
+  const int frow = STEPS * (g >> 1), fcol = 8 * (g & 1) + (li >> 2), fch = 4 * (li & 3);
   const int p_end = min(a.npatch, ((int)blockIdx.x + 1) * a.per_chunk);
+#pragma unroll 1
   for (int pt = blockIdx.x * a.per_chunk; pt < p_end; pt++) {
     const int px = pt % a.npx, py = (pt / a.npx) % a.npy, b = pt / (a.npx * a.npy);
     const int x0 = px * WG_P, y0 = py * WG_P;
     const int64_t img = (int64_t)b * a.H * a.Wd;
-    __syncthreads();  // the tiles of the patch before are done with
-    for (int k = tid >> 2; k < HW * HW; k += 64) {
-      const int r = k / HW, c = k - r * HW, hh = y0 + r - H2, ww = x0 + c - H2;
-      const bool ok = hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd && ci0 + q8 < a.Cin;
-      *(uint4 *)&sh.t.x[k * 32 + q8] =
-          ok ? ld16(a.X + (img + (int64_t)hh * a.Wd + ww) * a.Cin + ci0 + q8, a.aligned) : make_uint4(0u, 0u, 0u, 0u);
-    }
+    {
+      PX tx;
+      PY ty;
+      tx.load(a.X, img, a.H, a.Wd, a.Cin, x0 - H2, y0 - H2, ci0, a.aligned);
+      ty.load(a.dY, img, a.H, a.Wd, a.Cout, x0, y0, co0, a.aligned);
+      __syncthreads();  // the tiles of the patch before are done with
+      tx.store(sx);
+      ty.store(sy);
+      if (bias) {  // a thread's pieces of a slab are of the same 8 channels
 #pragma unroll
-    for (int k = tid >> 2; k < WG_P * WG_P; k += 64) {
-      const int hh = y0 + k / WG_P, ww = x0 + k % WG_P;
-      const bool ok = hh < a.H && ww < a.Wd && co0 + q8 < a.Cout;
-      const uint4 u =
-          ok ? ld16(a.dY + (img + (int64_t)hh * a.Wd + ww) * a.Cout + co0 + q8, a.aligned) : make_uint4(0u, 0u, 0u, 0u);
-      *(uint4 *)&sh.t.y[k * 32 + q8] = u;
-      if (bias) {
-        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+        for (int i = 0; i < PY::N; i++) {
+          const uint32_t w[4] = {ty.r[i].x, ty.r[i].y, ty.r[i].z, ty.r[i].w};
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          bsum[2 * i] += __uint_as_float(w[i] << 16);
-          bsum[2 * i + 1] += __uint_as_float(w[i] & 0xffff0000u);
+          for (int k = 0; k < 4; k++) {
+            bsum[i / 4][2 * k] += __uint_as_float(w[k] << 16);
+            bsum[i / 4][2 * k + 1] += __uint_as_float(w[k] & 0xffff0000u);
+          }
         }
       }
     }
     __syncthreads();
-    // dY of the two K steps
-    bf8 fy[2][2];
+    // row pairs (j, j + STEPS) of X meet the dY of steps j - dy
+    bf8 fy[3][2];
 #pragma unroll
-    for (int r = 0; r < 2; r++)
+    for (int j = -H2; j < STEPS + H2; j++) {
+      const int ry = j + H2;  // the step that comes into reach
+      if (ry < STEPS) {
 #pragma unroll
-      for (int m = 0; m < 2; m++) {
-        const uint16_t *p = &sh.t.y[((4 * wv + r + frow) * WG_P + fcol) * 32 + 16 * m + fch];
-        fy[r][m] = ld_tr(p, p + 4 * 32);
+        for (int m = 0; m < 2; m++) {
+          const uint16_t *p = &wy[((row0 + ry + frow) * WG_P + fcol) * 32 + 16 * m + fch];
+          fy[ry % 3][m] = ld_tr(p, p + 4 * 32);
+        }
       }
-#pragma unroll
-    for (int j = -H2; j < 2 + H2; j++)
 #pragma unroll
       for (int dx = 0; dx < K; dx++) {
         bf8 fx[2];
 #pragma unroll
         for (int n = 0; n < 2; n++) {
-          const uint16_t *p = &sh.t.x[((4 * wv + j + H2 + frow) * HW + fcol + dx) * 32 + 16 * n + fch];
+          const uint16_t *p = &wx[((row0 + j + H2 + frow) * HW + fcol + dx) * 32 + 16 * n + fch];
           fx[n] = ld_tr(p, p + 4 * 32);
         }
 #pragma unroll
-        for (int r = 0; r < 2; r++) {
-          const int dy = j - r + H2;  // 0 .. K - 1
-          if (dy < 0 || dy >= K) continue;
+        for (int dy = 0; dy < K; dy++) {
+          const int r = j - dy + H2;
+          if (r < 0 || r >= STEPS) continue;
 #pragma unroll
           for (int m = 0; m < 2; m++)
 #pragma unroll
-            for (int n = 0; n < 2; n++) acc[dy * K + dx][m][n] = mfma32(fy[r][m], fx[n], acc[dy * K + dx][m][n]);
+            for (int n = 0; n < 2; n++) acc[dy * K + dx][m][n] = mfma32(fy[r % 3][m], fx[n], acc[dy * K + dx][m][n]);
         }
       }
-  }
-  // the wavefronts' sums, in their order
-  const int cl = lane & 15, rg = lane >> 4;
-#pragma unroll 1
-  for (int w = 0; w < 4; w++) {
-    __syncthreads();
-    if (wv == w) {
-#pragma unroll
-      for (int t = 0; t < T; t++)
-#pragma unroll
-        for (int m = 0; m < 2; m++)
-#pragma unroll
-          for (int n = 0; n < 2; n++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              float *o = &sh.red[(t * 32 + 16 * m + 4 * rg + i) * 32 + 16 * n + cl];
-              *o = w ? *o + acc[t][m][n][i] : acc[t][m][n][i];
-            }
     }
   }
-  __syncthreads();
   const int64_t nw = (int64_t)T * a.Cout * a.Cin;
   float *out = a.part + (int64_t)blockIdx.x * (nw + a.Cout);
-  const int c4 = (tid & 7) * 4;
-  for (int k = tid >> 3; k < T * 32; k += 32) {
-    const int t = k >> 5, co = co0 + (k & 31);
-    if (co < a.Cout && ci0 + c4 < a.Cin)
-      st4(&out[((int64_t)t * a.Cout + co) * a.Cin + ci0 + c4], *(const f4 *)&sh.red[k * 32 + c4]);
-  }
-  if (bias) {
+  if (SPLIT) {  // (w0 + w1) + (w2 + w3)
+    f4 *red = (f4 *)lds;
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < 8; i++) sh.bias[(tid >> 2) * 33 + q8 + i] = bsum[i];
+    for (int step = 0; step < 2; step++) {
+      const bool give = step == 0 ? (wv & 1) : wv == 2, get = step == 0 ? !(wv & 1) : wv == 0;
+      f4 *o = red + (step == 0 ? (wv >> 1) : 0) * T * 4 * 64 + lane;
+      if (give) {
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) o[(t * 4 + q) * 64] = acc[t][q >> 1][q & 1];
+      }
+      __syncthreads();
+      if (get) {
+#pragma unroll
+        for (int t = 0; t < T; t++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) acc[t][q >> 1][q & 1] += o[(t * 4 + q) * 64];
+      }
+      __syncthreads();
+    }
+  }
+  if (!SPLIT || wv == 0) {
+    const int cb = co0 + (SPLIT ? 0 : 32 * (wv >> 1)), ib = ci0 + (SPLIT ? 0 : 32 * (wv & 1)) + li;
+#pragma unroll
+    for (int t = 0; t < T; t++)
+#pragma unroll
+      for (int m = 0; m < 2; m++)
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int co = cb + 16 * m + 4 * g + i, ci = ib + 16 * n;
+            if (co < a.Cout && ci < a.Cin) out[((int64_t)t * a.Cout + co) * a.Cin + ci] = acc[t][m][n][i];
+          }
+  }
+  if (bias) {  // uniform over the block
+    float *sb = (float *)lds;
     __syncthreads();
-    if (tid < 32 && co0 + tid < a.Cout) {
+#pragma unroll
+    for (int sl = 0; sl < SL; sl++)
+#pragma unroll
+      for (int i = 0; i < 8; i++) sb[(tid >> 2) * 33 * SL + 33 * sl + (tid & 3) * 8 + i] = bsum[sl][i];
+    __syncthreads();
+    if (tid < 32 * SL && co0 + tid < a.Cout) {
       float s = 0.f;
-      for (int k = 0; k < 64; k++) s += sh.bias[k * 33 + tid];
+      for (int k = 0; k < 64; k++) s += sb[k * 33 * SL + 33 * (tid >> 5) + (tid & 31)];
       out[nw + co0 + tid] = s;
     }
   }
@@ -765,9 +804,11 @@ extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t
   a.npatch = B * a.npx * a.npy;
   a.want_bias = db != nullptr;
   a.aligned = (((uintptr_t)X | (uintptr_t)dY) & 15) == 0;
-  // enough blocks to give every CU two, within the workspace (one chunk per 256
-  // pixels) and with at least one patch each; more only grows the partials
-  const int tm = (Cout + 31) / 32, tn = (Cin + 31) / 32;
+  // wavefronts side by side in co and ci where both have 64 channels, else along
+  // the pixels; two blocks a CU, within the workspace (one chunk per 256 pixels) and
+  // with at least one patch each: more only grows the partials
+  const bool split = Cout < 64 || Cin < 64;
+  const int cw = split ? 32 : 64, tm = (Cout + cw - 1) / cw, tn = (Cin + cw - 1) / cw;
   int64_t nchunk = (512 + tm * tn - 1) / (tm * tn);
   const int64_t most = (npix + KCH - 1) / KCH;
   if (nchunk > most) nchunk = most;
@@ -776,8 +817,8 @@ extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t
   nchunk = (a.npatch + a.per_chunk - 1) / a.per_chunk;
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
   const dim3 grid((unsigned)nchunk, tm, tn);
-  if (K == 3) k_wgrad<3><<<grid, 256, 0, ctx->stream>>>(a);
-  else k_wgrad<1><<<grid, 256, 0, ctx->stream>>>(a);
+  if (K == 3) split ? k_wgrad<3, true><<<grid, 256, 0, ctx->stream>>>(a) : k_wgrad<3, false><<<grid, 256, 0, ctx->stream>>>(a);
+  else split ? k_wgrad<1, true><<<grid, 256, 0, ctx->stream>>>(a) : k_wgrad<1, false><<<grid, 256, 0, ctx->stream>>>(a);
   FVM_LAUNCH_CHECK(ctx);
   const int64_t quads = (nw + Cout) / 4;  // channel counts are multiples of 16
   if (nchunk >= 32)
