@@ -86,6 +86,18 @@ typedef uint16_t h4u __attribute__((ext_vector_type(4), aligned(2)));
 __device__ __forceinline__ void st4(float *p, f4 v) { *(f4u *)p = v; }
 __device__ __forceinline__ f4 ld4(const float *p) { return *(const f4u *)p; }
 
+// The input of a layer: C0 channels from X, the rest from X2 (null when C0 is all).
+// up = 1: X is at half the resolution and read upsampled (nearest): a decoder
+// layer reads its two parents instead of a concatenated copy of them.
+struct Input {
+  const uint16_t *X, *X2;
+  int C0, up;
+};
+__device__ __forceinline__ const uint16_t *input_at(const Input &in, int C, int b, int H, int W, int h, int w, int c) {
+  if (c < in.C0) return in.X + (((int64_t)b * (H >> in.up) + (h >> in.up)) * (W >> in.up) + (w >> in.up)) * in.C0 + c;
+  return in.X2 + (((int64_t)b * H + h) * W + w) * (C - in.C0) + c - in.C0;
+}
+
 // ---- convolution (implicit GEMM) ------------------------------------------------
 // Y[p][co] = act(bias[co] + sum_{tap, ci} X[p + off(tap)][ci] * W[tap][co][ci])
 // off(tap) = (ky - K/2, kx - K/2); X outside the image reads 0.  TR: the data
@@ -103,9 +115,10 @@ __device__ __forceinline__ f4 ld4(const float *p) { return *(const f4u *)p; }
 // The weights are the A operand, so a lane ends with four consecutive channels of
 // one pixel.  The shapes are picked by conv_launch.
 struct ConvArgs {
-  const uint16_t *X;
+  Input in;
   const uint16_t *W;
-  const float *bias;  // may be null
+  const float *bias;     // may be null
+  const uint16_t *mask;  // the layer's own activations (a data gradient leaves through their ReLU), or null
   uint16_t *Y;        // bf16 output (or null)
   float *Yf;          // fp32 output (or null)
   int B, H, Wd, Cin, Cout, relu;
@@ -161,7 +174,7 @@ __global__ void __launch_bounds__(256 * WN) k_conv(ConvArgs a) {
         const int q = tid + TH * i, pix = q >> 2, c = (s0 + s) * 32 + (q & 3) * 8;
         const int hh = y0 + pix / PW - H2, ww = x0 + pix % PW - H2;
         const bool ok = q < NP * 4 && c < a.Cin && hh >= 0 && hh < a.H && ww >= 0 && ww < a.Wd;
-        rx[s][i] = ok ? *(const uint4 *)(a.X + (img + (int64_t)hh * a.Wd + ww) * a.Cin + c) : make_uint4(0u, 0u, 0u, 0u);
+        rx[s][i] = ok ? *(const uint4 *)input_at(a.in, a.Cin, b, a.H, a.Wd, hh, ww, c) : make_uint4(0u, 0u, 0u, 0u);
       }
 #pragma unroll
     for (int s = 0; s < SB; s++)
@@ -245,6 +258,12 @@ __global__ void __launch_bounds__(256 * WN) k_conv(ConvArgs a) {
         h[i] = f2bf(v[i]);
       }
       const int64_t o = (img + (int64_t)hh * a.Wd + ww) * a.Cout + co;
+      if (a.mask) {
+        const h4u y = *(const h4u *)(a.mask + o);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (!(bf2f(y[i]) > 0.f)) h[i] = 0;
+      }
       if (a.Y) *(h4u *)(a.Y + o) = h;
       if (a.Yf) st4(a.Yf + o, v);
     }
@@ -261,13 +280,14 @@ __global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
   const int64_t p0 = (int64_t)blockIdx.x * 64 + (wv & 1) * 32;
   const int c0 = blockIdx.y * 64 + (wv >> 1) * 32;
   int64_t pp[2];
-  int ph[2], pw[2];
+  int pb[2], ph[2], pw[2];
 #pragma unroll
   for (int r = 0; r < 2; r++) {
     const int64_t p = p0 + r * 16 + li, q = p < npix ? p : 0;
     pp[r] = p < npix ? q : -1;
     pw[r] = (int)(q % a.Wd);
     ph[r] = (int)((q / a.Wd) % a.H);
+    pb[r] = (int)(q / ((int64_t)a.Wd * a.H));
   }
   const bf8 zero = __builtin_bit_cast(bf8, make_uint4(0u, 0u, 0u, 0u));
   f4 acc[2][2] = {};
@@ -280,7 +300,8 @@ __global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
 #pragma unroll
       for (int r = 0; r < 2; r++) {
         const bool ok = pp[r] >= 0 && k < a.Cin && ph[r] + dy >= 0 && ph[r] + dy < a.H && pw[r] + dx >= 0 && pw[r] + dx < a.Wd;
-        fx[r] = ok ? __builtin_bit_cast(bf8, *(const uint4 *)(a.X + (pp[r] + (int64_t)dy * a.Wd + dx) * a.Cin + k)) : zero;
+        fx[r] = ok ? __builtin_bit_cast(bf8, *(const uint4 *)input_at(a.in, a.Cin, pb[r], a.H, a.Wd, ph[r] + dy, pw[r] + dx, k))
+                   : zero;
       }
 #pragma unroll
       for (int n = 0; n < 2; n++) {
@@ -312,8 +333,9 @@ __global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
         float v = acc[r][n][i] + (a.bias ? a.bias[co + i] : 0.f);
         if (a.relu) v = v > 0.f ? v : 0.f;
         if (co + i >= a.cout_real) v = 0.f;
-        if (a.Y) a.Y[pp[r] * a.Cout + co + i] = f2bf(v);
-        if (a.Yf) a.Yf[pp[r] * a.Cout + co + i] = v;
+        const int64_t o = pp[r] * a.Cout + co + i;
+        if (a.Y) a.Y[o] = a.mask && !(bf2f(a.mask[o]) > 0.f) ? (uint16_t)0 : f2bf(v);
+        if (a.Yf) a.Yf[o] = v;
       }
     }
   }
@@ -357,7 +379,8 @@ void conv_launch(fvm_ctx *ctx, const ConvArgs &a) {
   } else if (conv_try<K, 4, 1, 1, TR>(ctx, a, 512, HALF)) {
     return;
   }
-  if (conv_try<K, 1, 2, 1, TR>(ctx, a, 512, ALL) || conv_try<K, 1, 1, 1, TR>(ctx, a, 0, ALL)) return;
+  if (a.Cout >= 32 && conv_try<K, 1, 1, 2, TR>(ctx, a, 128, ALL)) return;
+  if (conv_try<K, 1, 1, 1, TR>(ctx, a, 0, ALL)) return;
   const int64_t npix = (int64_t)a.B * a.H * a.Wd;
   k_conv_wide<K, TR><<<dim3((unsigned)((npix + 63) / 64), (unsigned)((a.Cout + 63) / 64)), 256, 0, ctx->stream>>>(a);
 }
@@ -386,12 +409,13 @@ void conv_launch(fvm_ctx *ctx, const ConvArgs &a) {
 #define WG_P 16              // patch edge
 #define WG_HW (WG_P + 2)     // with the taps' halo
 struct WgradArgs {
-  const uint16_t *X, *dY;
+  Input in;
+  const uint16_t *dY;
   float *part;  // [chunk][taps * Cout * Cin, then Cout (bias)]
   int B, H, Wd, Cin, Cout;
   int npx, npy, npatch, per_chunk;
   int want_bias;
-  int aligned;  // X and dY on 16-byte boundaries
+  int aligned;  // the input and dY on 16-byte boundaries
 };
 
 __device__ __forceinline__ uint4 ld16(const uint16_t *p, int aligned) {
@@ -407,13 +431,13 @@ template <int SL, int PW, int PH>
 struct Patch {
   static constexpr int NP = PW * PH, N = (NP * 4 * SL + 255) / 256;
   uint4 r[N];
-  __device__ __forceinline__ void load(const uint16_t *X, int64_t img, int H, int W, int C, int x0, int y0, int c0, int aligned) {
+  __device__ __forceinline__ void load(const Input &in, int b, int H, int W, int C, int x0, int y0, int c0, int aligned) {
 #pragma unroll
     for (int i = 0; i < N; i++) {
       const int q = threadIdx.x + 256 * i, sl = q / (NP * 4), pix = (q - sl * NP * 4) >> 2, c = c0 + 32 * sl + (q & 3) * 8;
       const int hh = y0 + pix / PW, ww = x0 + pix % PW;
       const bool ok = q < NP * 4 * SL && hh >= 0 && hh < H && ww >= 0 && ww < W && c < C;
-      r[i] = ok ? ld16(X + (img + (int64_t)hh * W + ww) * C + c, aligned) : make_uint4(0u, 0u, 0u, 0u);
+      r[i] = ok ? ld16(input_at(in, C, b, H, W, hh, ww, c), aligned) : make_uint4(0u, 0u, 0u, 0u);
     }
   }
   __device__ __forceinline__ void store(uint16_t *sh) const {
@@ -453,12 +477,11 @@ __global__ void __launch_bounds__(256, 2) k_wgrad(WgradArgs a) {
   for (int pt = blockIdx.x * a.per_chunk; pt < p_end; pt++) {
     const int px = pt % a.npx, py = (pt / a.npx) % a.npy, b = pt / (a.npx * a.npy);
     const int x0 = px * WG_P, y0 = py * WG_P;
-    const int64_t img = (int64_t)b * a.H * a.Wd;
     {
       PX tx;
       PY ty;
-      tx.load(a.X, img, a.H, a.Wd, a.Cin, x0 - H2, y0 - H2, ci0, a.aligned);
-      ty.load(a.dY, img, a.H, a.Wd, a.Cout, x0, y0, co0, a.aligned);
+      tx.load(a.in, b, a.H, a.Wd, a.Cin, x0 - H2, y0 - H2, ci0, a.aligned);
+      ty.load(Input{a.dY, nullptr, a.Cout, 0}, b, a.H, a.Wd, a.Cout, x0, y0, co0, a.aligned);
       __syncthreads();  // the tiles of the patch before are done with
       tx.store(sx);
       ty.store(sy);
@@ -672,22 +695,98 @@ __global__ void __launch_bounds__(256) k_add_channels(const uint16_t *__restrict
   Y[i] = f2bf(bf2f(Y[i]) + bf2f(X[p * Cx + xc0 + c]));
 }
 
+// ---- the same layers eight channels a thread, as the whole passes use them ------------
+struct H8 {
+  uint16_t v[8];
+};
+__device__ __forceinline__ H8 ld_h8(const uint16_t *p) { return __builtin_bit_cast(H8, *(const uint4 *)p); }
+__device__ __forceinline__ void st_h8(uint16_t *p, const H8 &h) { *(uint4 *)p = __builtin_bit_cast(uint4, h); }
+
+__global__ void __launch_bounds__(256) k_copy8(int64_t n8, const uint16_t *__restrict__ X, uint16_t *__restrict__ Y) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < n8) ((uint4 *)Y)[i] = ((const uint4 *)X)[i];
+}
+
+__global__ void __launch_bounds__(256) k_pool8(const uint16_t *__restrict__ X, int B, int H, int W, int C,
+                                               uint16_t *__restrict__ Y) {
+  const int C8 = C / 8, Ho = H / 2, Wo = W / 2;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)B * Ho * Wo * C8) return;
+  const int c = (int)(i % C8) * 8;
+  const int64_t q = i / C8;
+  const int w = (int)(q % Wo), h = (int)((q / Wo) % Ho);
+  const int64_t b = q / ((int64_t)Wo * Ho);
+  const uint16_t *r0 = X + ((b * H + 2 * h) * W + 2 * w) * C + c, *r1 = r0 + (int64_t)W * C;
+  const H8 a0 = ld_h8(r0), a1 = ld_h8(r0 + C), b0 = ld_h8(r1), b1 = ld_h8(r1 + C);
+  H8 y;
+#pragma unroll
+  for (int k = 0; k < 8; k++) y.v[k] = f2bf(0.25f * ((bf2f(a0.v[k]) + bf2f(a1.v[k])) + (bf2f(b0.v[k]) + bf2f(b1.v[k]))));
+  st_h8(Y + q * C + c, y);
+}
+
+// gradient of the upsampled part (channels [0, C) of dcat's Ctot), through the ReLU of
+// the activations y it was upsampled from
+__global__ void __launch_bounds__(256) k_up_bwd8(const uint16_t *__restrict__ dcat, int B, int H, int W, int C, int Ctot,
+                                                 const uint16_t *__restrict__ y, uint16_t *__restrict__ dz) {
+  const int C8 = C / 8;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)B * H * W * C8) return;
+  const int c = (int)(i % C8) * 8;
+  const int64_t q = i / C8;
+  const int w = (int)(q % W), h = (int)((q / W) % H);
+  const int64_t b = q / ((int64_t)W * H);
+  const uint16_t *r0 = dcat + ((b * 2 * H + 2 * h) * 2 * W + 2 * w) * Ctot + c, *r1 = r0 + (int64_t)2 * W * Ctot;
+  const H8 a0 = ld_h8(r0), a1 = ld_h8(r0 + Ctot), b0 = ld_h8(r1), b1 = ld_h8(r1 + Ctot), m = ld_h8(y + q * C + c);
+  H8 z;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const uint16_t s = f2bf((bf2f(a0.v[k]) + bf2f(a1.v[k])) + (bf2f(b0.v[k]) + bf2f(b1.v[k])));
+    z.v[k] = bf2f(m.v[k]) > 0.f ? s : (uint16_t)0;
+  }
+  st_h8(dz + q * C + c, z);
+}
+
+// gradient of encoder activations y: the skip part (channels [c0, c0 + C) of dcat's
+// Ctot) plus a quarter of the pooled gradient, through y's ReLU
+__global__ void __launch_bounds__(256) k_skip_bwd8(const uint16_t *__restrict__ dcat, int Ctot, int c0,
+                                                   const uint16_t *__restrict__ dpool, int B, int H, int W, int C,
+                                                   const uint16_t *__restrict__ y, uint16_t *__restrict__ dz) {
+  const int C8 = C / 8, Ho = H / 2, Wo = W / 2;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= (int64_t)B * H * W * C8) return;
+  const int c = (int)(i % C8) * 8;
+  const int64_t q = i / C8;
+  const int w = (int)(q % W), h = (int)((q / W) % H);
+  const int64_t b = q / ((int64_t)W * H);
+  const H8 s = ld_h8(dcat + q * Ctot + c0 + c), p = ld_h8(dpool + ((b * Ho + h / 2) * Wo + w / 2) * C + c), m = ld_h8(y + q * C + c);
+  H8 z;
+#pragma unroll
+  for (int k = 0; k < 8; k++) {
+    const uint16_t v = f2bf(bf2f(s.v[k]) + bf2f(f2bf(0.25f * bf2f(p.v[k]))));
+    z.v[k] = bf2f(m.v[k]) > 0.f ? v : (uint16_t)0;
+  }
+  st_h8(dz + q * C + c, z);
+}
+
 // masked mean squared error over the first Creal of C fp32 output channels:
 // loss partials per block; dOut (bf16, C channels) = 2 (out - tgt) mask / count
+#define MSE_PER 8  // values per thread, 256 apart: fewer partials for k_sum_f
 __global__ void __launch_bounds__(256) k_mse(const float *__restrict__ out, const float *__restrict__ tgt,
                                              const float *__restrict__ mask, int64_t npix, int C, int Creal,
                                              float inv_count, uint16_t *__restrict__ dOut, float *__restrict__ part) {
   __shared__ float sh[256];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   float l = 0.f;
-  if (i < npix * C) {
+#pragma unroll
+  for (int k = 0; k < MSE_PER; k++) {
+    const int64_t i = ((int64_t)blockIdx.x * MSE_PER + k) * 256 + threadIdx.x;
+    if (i >= npix * C) continue;
     const int c = (int)(i % C);
     const int64_t p = i / C;
     float g = 0.f;
     if (c < Creal) {
       const float m = mask ? mask[p * Creal + c] : 1.f;
       const float d = (out[i] - tgt[p * Creal + c]) * m;
-      l = d * d * inv_count;
+      l += d * d * inv_count;
       g = 2.f * d * inv_count;
     }
     dOut[i] = f2bf(g);
@@ -715,19 +814,44 @@ __global__ void __launch_bounds__(256) k_sum_f(const float *__restrict__ part, i
 }
 
 // Adam on fp32 master weights; the bf16 working copy is refreshed
-__global__ void __launch_bounds__(256) k_adam(int64_t n, float *__restrict__ w, const float *__restrict__ g,
-                                              float *__restrict__ m, float *__restrict__ v, uint16_t *__restrict__ wb,
-                                              float lr, float b1, float b2, float eps, float c1, float c2, float wd) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i] + wd * w[i];
-  const float mi = b1 * m[i] + (1.f - b1) * gi;
-  const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-  w[i] = wi;
-  if (wb) wb[i] = f2bf(wi);
+struct AdamArgs {
+  float *w;
+  const float *g;
+  float *m, *v;
+  uint16_t *wb;  // or null
+  int64_t n;
+  float wd;
+};
+struct AdamRates {
+  float lr, b1, b2, eps, c1, c2;
+};
+__device__ __forceinline__ void adam_at(const AdamArgs &a, const AdamRates &r, int64_t i) {
+  const float gi = a.g[i] + a.wd * a.w[i];
+  const float mi = r.b1 * a.m[i] + (1.f - r.b1) * gi;
+  const float vi = r.b2 * a.v[i] + (1.f - r.b2) * gi * gi;
+  a.m[i] = mi;
+  a.v[i] = vi;
+  const float wi = a.w[i] - r.lr * (mi / r.c1) / (sqrtf(vi / r.c2) + r.eps);
+  a.w[i] = wi;
+  if (a.wb) a.wb[i] = f2bf(wi);
+}
+__global__ void __launch_bounds__(256) k_adam(AdamArgs a, AdamRates r) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i < a.n) adam_at(a, r, i);
+}
+// every tensor of a network in one launch (30 of them took 85 us one by one): block
+// b works on the tensor k with first[k] <= b < first[k + 1]
+#define ADAM_MAX 40
+struct AdamAll {
+  AdamArgs t[ADAM_MAX];
+  int first[ADAM_MAX + 1];
+  int n;
+};
+__global__ void __launch_bounds__(256) k_adam_all(AdamAll A, AdamRates r) {
+  int k = 0;
+  while (k + 1 < A.n && (int)blockIdx.x >= A.first[k + 1]) k++;
+  const int64_t i = (int64_t)((int)blockIdx.x - A.first[k]) * 256 + threadIdx.x;
+  if (i < A.t[k].n) adam_at(A.t[k], r, i);
 }
 
 __global__ void __launch_bounds__(256) k_f2bf(int64_t n, const float *__restrict__ x, uint16_t *__restrict__ y) {
@@ -767,7 +891,7 @@ extern "C" int fvm_nn_conv_fwd(fvm_ctx *ctx, const uint16_t *X, const uint16_t *
                                int32_t cout_real, uint16_t *Y, float *Yf) {
   if (!ctx || !X || !W || (!Y && !Yf)) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
-  ConvArgs a{X, W, bias, Y, Yf, B, H, Wd, Cin, Cout, relu, cout_real > 0 ? cout_real : Cout};
+  ConvArgs a{Input{X, nullptr, Cin, 0}, W, bias, nullptr, Y, Yf, B, H, Wd, Cin, Cout, relu, cout_real > 0 ? cout_real : Cout};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
   return conv_run(ctx, a, K, false);
 }
@@ -778,7 +902,7 @@ extern "C" int fvm_nn_conv_dgrad(fvm_ctx *ctx, const uint16_t *dY, const uint16_
                                  int32_t H, int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, uint16_t *dX) {
   if (!ctx || !dY || !W || !Wd_scratch || !dX) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
-  ConvArgs a{dY, W, nullptr, dX, nullptr, B, H, Wd, Cout, Cin, 0, Cin};
+  ConvArgs a{Input{dY, nullptr, Cout, 0}, W, nullptr, nullptr, dX, nullptr, B, H, Wd, Cout, Cin, 0, Cin};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
   return conv_run(ctx, a, K, true);
 }
@@ -790,20 +914,17 @@ extern "C" size_t fvm_nn_wgrad_workspace(int32_t B, int32_t H, int32_t Wd, int32
   return (size_t)nchunk * ((size_t)K * K * Cout * Cin + (size_t)Cout) * sizeof(float);
 }
 
-// dW (fp32 [tap][Cout][Cin]) and db (fp32 [Cout], may be null)
-extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t *dY, int32_t B, int32_t H,
-                                 int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, float *work, float *dW, float *db) {
-  if (!ctx || !X || !dY || !work || !dW) return FVM_ERR_ARG;
-  FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
+static int wgrad_run(fvm_ctx *ctx, const Input &in, const uint16_t *dY, int B, int H, int Wd, int Cin, int Cout, int K,
+                     float *work, float *dW, float *db) {
   const int64_t npix = (int64_t)B * H * Wd;
   const int64_t nw = (int64_t)K * K * Cout * Cin;
-  WgradArgs a{X, dY, work, B, H, Wd, Cin, Cout};
+  WgradArgs a{in, dY, work, B, H, Wd, Cin, Cout};
   a.npx = (Wd + WG_P - 1) / WG_P;
   a.npy = (H + WG_P - 1) / WG_P;
   if ((int64_t)B * a.npx * a.npy > INT32_MAX) return fvm_set_err(ctx, FVM_ERR_ARG, "conv: too many pixels");
   a.npatch = B * a.npx * a.npy;
   a.want_bias = db != nullptr;
-  a.aligned = (((uintptr_t)X | (uintptr_t)dY) & 15) == 0;
+  a.aligned = (((uintptr_t)in.X | (uintptr_t)in.X2 | (uintptr_t)dY) & 15) == 0;
   // wavefronts side by side in co and ci where both have 64 channels, else along
   // the pixels; two blocks a CU, within the workspace (one chunk per 256 pixels) and
   // with at least one patch each: more only grows the partials
@@ -815,7 +936,6 @@ extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t
   if (nchunk > a.npatch) nchunk = a.npatch;
   a.per_chunk = (int)((a.npatch + nchunk - 1) / nchunk);
   nchunk = (a.npatch + a.per_chunk - 1) / a.per_chunk;
-  FVM_PHASE(ctx, FVM_PHASE_OTHER);
   const dim3 grid((unsigned)nchunk, tm, tn);
   if (K == 3) split ? k_wgrad<3, true><<<grid, 256, 0, ctx->stream>>>(a) : k_wgrad<3, false><<<grid, 256, 0, ctx->stream>>>(a);
   else split ? k_wgrad<1, true><<<grid, 256, 0, ctx->stream>>>(a) : k_wgrad<1, false><<<grid, 256, 0, ctx->stream>>>(a);
@@ -827,6 +947,15 @@ extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t
     k_wgrad_reduce<4><<<(unsigned)((quads + 63) / 64), 256, 0, ctx->stream>>>(work, (int)nchunk, nw, Cout, dW, db);
   FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;
+}
+
+// dW (fp32 [tap][Cout][Cin]) and db (fp32 [Cout], may be null)
+extern "C" int fvm_nn_conv_wgrad(fvm_ctx *ctx, const uint16_t *X, const uint16_t *dY, int32_t B, int32_t H,
+                                 int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, float *work, float *dW, float *db) {
+  if (!ctx || !X || !dY || !work || !dW) return FVM_ERR_ARG;
+  FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
+  FVM_PHASE(ctx, FVM_PHASE_OTHER);
+  return wgrad_run(ctx, Input{X, nullptr, Cin, 0}, dY, B, H, Wd, Cin, Cout, K, work, dW, db);
 }
 
 extern "C" int fvm_nn_relu_bwd(fvm_ctx *ctx, int64_t n, const uint16_t *y, const uint16_t *dy, uint16_t *dz) {
@@ -889,7 +1018,7 @@ extern "C" int fvm_nn_mse(fvm_ctx *ctx, const float *out, const float *tgt, cons
                           int32_t Creal, float inv_count, uint16_t *dOut, float *work, float *loss) {
   if (!ctx || !out || !tgt || !dOut || !work || !loss || Creal > C) return FVM_ERR_ARG;
   const int64_t n = npix * C;
-  const unsigned nb = nblk(n);
+  const unsigned nb = (unsigned)((n + 256 * MSE_PER - 1) / (256 * MSE_PER));
   k_mse<<<nb, 256, 0, ctx->stream>>>(out, tgt, mask, npix, C, Creal, inv_count, dOut, work);
   k_sum_f<<<1, 256, 0, ctx->stream>>>(work, nb, loss);
   FVM_LAUNCH_CHECK(ctx);
@@ -900,7 +1029,7 @@ extern "C" int fvm_nn_adam(fvm_ctx *ctx, int64_t n, float *w, const float *g, fl
                            float lr, float b1, float b2, float eps, int32_t step, float wd) {
   if (!ctx || !w || !g || !m || !v || step < 1) return FVM_ERR_ARG;
   const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
-  k_adam<<<nblk(n), 256, 0, ctx->stream>>>(n, w, g, m, v, wb, lr, b1, b2, eps, c1, c2, wd);
+  k_adam<<<nblk(n), 256, 0, ctx->stream>>>(AdamArgs{w, g, m, v, wb, n, wd}, AdamRates{lr, b1, b2, eps, c1, c2});
   FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;
 }
@@ -908,6 +1037,158 @@ extern "C" int fvm_nn_adam(fvm_ctx *ctx, int64_t n, float *w, const float *g, fl
 extern "C" int fvm_nn_f32_to_bf16(fvm_ctx *ctx, int64_t n, const float *x, uint16_t *y) {
   if (!ctx || !x || !y) return FVM_ERR_ARG;
   k_f2bf<<<nblk(n), 256, 0, ctx->stream>>>(n, x, y);
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
+// ---- the whole network -----------------------------------------------------------------
+// One call per pass, instead of one per layer: the host's part of a pass shrinks to its
+// launches, and the layers' copies, concatenations and ReLU passes go into the
+// kernels beside them.  Tensors are NHWC bf16 unless noted, level i at H >> i, W >> i.
+#define NN_LEVELS 8
+typedef struct {
+  int32_t levels, B, H, W, cin, cout, cout_real;
+  int32_t ch[NN_LEVELS];
+  // layers e0_1, e0_2, e1_1, ..., d(L-2)_1, d(L-2)_2, ..., d0_2, out
+  const uint16_t *wb[4 * NN_LEVELS];
+  const float *b[4 * NN_LEVELS];
+  float *gw[4 * NN_LEVELS], *gb[4 * NN_LEVELS];
+  uint16_t *x[NN_LEVELS], *h[NN_LEVELS], *e[NN_LEVELS];  // encoder: input, first and second activations
+  uint16_t *dh[NN_LEVELS], *d[NN_LEVELS];                // decoder: first and second activations
+  float *out;                                            // fp32
+  // backward: gradients of x, of the pre-activations of h, e (g1, g2), dh, d, of the
+  // decoder's input (concatenated), of out (bf16)
+  uint16_t *dx[NN_LEVELS], *g1[NN_LEVELS], *g2[NN_LEVELS], *gdh[NN_LEVELS], *gd[NN_LEVELS], *dcat[NN_LEVELS], *dout;
+  float *work;  // fvm_nn_wgrad_workspace of the largest layer
+} fvm_unet;
+
+namespace {
+struct Layer {
+  int at, K, ci, co, lvl;
+};
+Layer enc(const fvm_unet &u, int i, int j) {
+  return Layer{2 * i + j, 3, j ? u.ch[i] : (i ? u.ch[i - 1] : u.cin), u.ch[i], i};
+}
+Layer dec(const fvm_unet &u, int i, int j) {
+  return Layer{2 * u.levels + 2 * (u.levels - 2 - i) + j, 3, j ? u.ch[i] : u.ch[i + 1] + u.ch[i], u.ch[i], i};
+}
+Layer last(const fvm_unet &u) { return Layer{4 * u.levels - 2, 1, u.ch[0], u.cout, 0}; }
+
+int unet_check(fvm_ctx *ctx, const fvm_unet *u) {
+  if (!ctx || !u || u->levels < 1 || u->levels > NN_LEVELS) return FVM_ERR_ARG;
+  const int m = (1 << (u->levels - 1)) - 1;
+  if (u->B < 1 || u->H < 1 || u->W < 1 || (u->H & m) || (u->W & m))
+    return fvm_set_err(ctx, FVM_ERR_ARG, "unet: H and W must divide by 2^(levels-1)");
+  for (int i = 0; i < u->levels; i++)
+    if (u->ch[i] < 16 || u->ch[i] % 16) return fvm_set_err(ctx, FVM_ERR_ARG, "unet: channels must be multiples of 16");
+  if (u->cin < 16 || u->cin % 16 || u->cout < 16 || u->cout % 16)
+    return fvm_set_err(ctx, FVM_ERR_ARG, "unet: channels must be multiples of 16");
+  return FVM_OK;
+}
+Input plain(const uint16_t *X, int C) { return Input{X, nullptr, C, 0}; }
+
+int fwd(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const Input &in, uint16_t *Y, float *Yf) {
+  ConvArgs a{in, u.wb[l.at], u.b[l.at], nullptr, Y, Yf, u.B, u.H >> l.lvl, u.W >> l.lvl, l.ci, l.co, Yf ? 0 : 1,
+             Yf ? u.cout_real : l.co};
+  return conv_run(ctx, a, l.K, false);
+}
+// data gradient of layer l, through the ReLU of the activations it took (mask, or null)
+int dgrad(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const uint16_t *dY, const uint16_t *mask, uint16_t *dX) {
+  ConvArgs a{plain(dY, l.co), u.wb[l.at], nullptr, mask, dX, nullptr, u.B, u.H >> l.lvl, u.W >> l.lvl, l.co, l.ci, 0, l.ci};
+  return conv_run(ctx, a, l.K, true);
+}
+int wgrad(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const Input &in, const uint16_t *dY) {
+  return wgrad_run(ctx, in, dY, u.B, u.H >> l.lvl, u.W >> l.lvl, l.ci, l.co, l.K, u.work, u.gw[l.at], u.gb[l.at]);
+}
+}  // namespace
+
+extern "C" int fvm_nn_unet_forward(fvm_ctx *ctx, const fvm_unet *up, const uint16_t *X) {
+  FVM_TRY(unet_check(ctx, up));
+  const fvm_unet &u = *up;
+  const int L = u.levels;
+  FVM_PHASE(ctx, FVM_PHASE_OTHER);
+  // the caller may refill X before the backward pass
+  const int64_t npix = (int64_t)u.B * u.H * u.W, n8 = npix * u.cin / 8;
+  if (!X) return FVM_ERR_ARG;
+  if (((uintptr_t)X & 15) == 0) k_copy8<<<nblk(n8), 256, 0, ctx->stream>>>(n8, X, u.x[0]);
+  else k_copy_channels<<<nblk(npix * u.cin), 256, 0, ctx->stream>>>(X, npix, u.cin, u.cin, 0, u.x[0], u.cin, 0);
+  for (int i = 0; i < L; i++) {
+    FVM_TRY(fwd(ctx, u, enc(u, i, 0), plain(u.x[i], enc(u, i, 0).ci), u.h[i], nullptr));
+    FVM_TRY(fwd(ctx, u, enc(u, i, 1), plain(u.h[i], u.ch[i]), u.e[i], nullptr));
+    if (i < L - 1) {
+      const int h = u.H >> i, w = u.W >> i;
+      k_pool8<<<nblk((int64_t)u.B * (h / 2) * (w / 2) * u.ch[i] / 8), 256, 0, ctx->stream>>>(u.e[i], u.B, h, w, u.ch[i],
+                                                                                         u.x[i + 1]);
+    }
+  }
+  const uint16_t *below = u.e[L - 1];
+  for (int i = L - 2; i >= 0; i--) {
+    FVM_TRY(fwd(ctx, u, dec(u, i, 0), Input{below, u.e[i], u.ch[i + 1], 1}, u.dh[i], nullptr));
+    FVM_TRY(fwd(ctx, u, dec(u, i, 1), plain(u.dh[i], u.ch[i]), u.d[i], nullptr));
+    below = u.d[i];
+  }
+  FVM_TRY(fwd(ctx, u, last(u), plain(below, u.ch[0]), nullptr, u.out));
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
+// every gw, gb from dout
+extern "C" int fvm_nn_unet_backward(fvm_ctx *ctx, const fvm_unet *up) {
+  FVM_TRY(unet_check(ctx, up));
+  const fvm_unet &u = *up;
+  const int L = u.levels;
+  FVM_PHASE(ctx, FVM_PHASE_OTHER);
+  // top: the output layer, through the ReLU of the activations below it
+  const uint16_t *act = L > 1 ? u.d[0] : u.e[0];
+  uint16_t *g = L > 1 ? u.gd[0] : u.g2[0];
+  FVM_TRY(wgrad(ctx, u, last(u), plain(act, u.ch[0]), u.dout));
+  FVM_TRY(dgrad(ctx, u, last(u), u.dout, act, g));
+  for (int i = 0; i < L - 1; i++) {
+    const int h = u.H >> (i + 1), w = u.W >> (i + 1), cc = u.ch[i + 1] + u.ch[i];
+    const uint16_t *below = i + 1 < L - 1 ? u.d[i + 1] : u.e[i + 1];
+    FVM_TRY(wgrad(ctx, u, dec(u, i, 1), plain(u.dh[i], u.ch[i]), u.gd[i]));
+    FVM_TRY(dgrad(ctx, u, dec(u, i, 1), u.gd[i], u.dh[i], u.gdh[i]));
+    FVM_TRY(wgrad(ctx, u, dec(u, i, 0), Input{below, u.e[i], u.ch[i + 1], 1}, u.gdh[i]));
+    FVM_TRY(dgrad(ctx, u, dec(u, i, 0), u.gdh[i], nullptr, u.dcat[i]));
+    k_up_bwd8<<<nblk((int64_t)u.B * h * w * u.ch[i + 1] / 8), 256, 0, ctx->stream>>>(
+        u.dcat[i], u.B, h, w, u.ch[i + 1], cc, below, i + 1 < L - 1 ? u.gd[i + 1] : u.g2[i + 1]);
+  }
+  for (int i = L - 1; i >= 0; i--) {
+    const int h = u.H >> i, w = u.W >> i;
+    if (i < L - 1)
+      k_skip_bwd8<<<nblk((int64_t)u.B * h * w * u.ch[i] / 8), 256, 0, ctx->stream>>>(
+          u.dcat[i], u.ch[i + 1] + u.ch[i], u.ch[i + 1], u.dx[i + 1], u.B, h, w, u.ch[i], u.e[i], u.g2[i]);
+    FVM_TRY(wgrad(ctx, u, enc(u, i, 1), plain(u.h[i], u.ch[i]), u.g2[i]));
+    FVM_TRY(dgrad(ctx, u, enc(u, i, 1), u.g2[i], u.h[i], u.g1[i]));
+    FVM_TRY(wgrad(ctx, u, enc(u, i, 0), plain(u.x[i], enc(u, i, 0).ci), u.g1[i]));
+    if (i > 0) FVM_TRY(dgrad(ctx, u, enc(u, i, 0), u.g1[i], nullptr, u.dx[i]));
+  }
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
+// Adam on `nt` tensors (n[k] elements; wb[k] may be null), as fvm_nn_adam on each
+extern "C" int fvm_nn_adam_all(fvm_ctx *ctx, int32_t nt, const int64_t *n, float *const *w, const float *const *g,
+                               float *const *m, float *const *v, uint16_t *const *wb, const float *wd, float lr, float b1,
+                               float b2, float eps, int32_t step) {
+  if (!ctx || nt < 0 || !n || !w || !g || !m || !v || !wb || !wd || step < 1) return FVM_ERR_ARG;
+  const float c1 = 1.f - powf(b1, (float)step), c2 = 1.f - powf(b2, (float)step);
+  FVM_PHASE(ctx, FVM_PHASE_OTHER);
+  for (int k0 = 0; k0 < nt; k0 += ADAM_MAX) {
+    AdamAll A;
+    A.n = nt - k0 < ADAM_MAX ? nt - k0 : ADAM_MAX;
+    int64_t blocks = 0;
+    for (int k = 0; k < A.n; k++) {
+      const int q = k0 + k;
+      if (!w[q] || !g[q] || !m[q] || !v[q] || n[q] < 0) return FVM_ERR_ARG;
+      A.t[k] = AdamArgs{w[q], g[q], m[q], v[q], wb[q], n[q], wd[q]};
+      A.first[k] = (int)blocks;
+      blocks += nblk(n[q]);
+      if (blocks > INT32_MAX) return FVM_ERR_ARG;
+    }
+    A.first[A.n] = (int)blocks;
+    if (blocks) k_adam_all<<<(unsigned)blocks, 256, 0, ctx->stream>>>(A, AdamRates{lr, b1, b2, eps, c1, c2});
+  }
   FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;
 }

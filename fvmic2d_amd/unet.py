@@ -37,7 +37,19 @@ _SIGS = {
     "fvm_nn_mse": [P, P, P, P, I64, I32, I32, F, P, P, P],
     "fvm_nn_adam": [P, I64, P, P, P, P, P, F, F, F, F, I32, F],
     "fvm_nn_f32_to_bf16": [P, I64, P, P],
+    "fvm_nn_unet_forward": [P, P, P],
+    "fvm_nn_unet_backward": [P, P],
+    "fvm_nn_adam_all": [P, I32, P, P, P, P, P, P, P, F, F, F, F, I32],
 }
+LEVELS = 8
+
+
+class fvm_unet(C.Structure):
+    """A network on one batch shape, for the whole-pass calls (csrc/unet.hip)."""
+    _fields_ = ([(n, I32) for n in ("levels", "B", "H", "W", "cin", "cout", "cout_real")] + [("ch", I32 * LEVELS)] +
+                [(n, P * (4 * LEVELS)) for n in ("wb", "b", "gw", "gb")] +
+                [(n, P * LEVELS) for n in ("x", "h", "e", "dh", "d")] + [("out", P)] +
+                [(n, P * LEVELS) for n in ("dx", "g1", "g2", "gdh", "gd", "dcat")] + [("dout", P), ("work", P)])
 
 
 def bind():
@@ -161,33 +173,44 @@ class UNet:
         for i in range(self.L):
             h, w = H >> i, W >> i
             cin = self.cin if i == 0 else self.ch[i - 1]
-            self.A["x%d" % i] = Buf(ctx, (B, h, w, cin), bf)
-            self.A["h%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["e%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["de%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["g1_%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["g2_%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["dx%d" % i] = Buf(ctx, (B, h, w, cin), bf)
+            for n, c in (("x", cin), ("h", self.ch[i]), ("e", self.ch[i]), ("g1_", self.ch[i]), ("g2_", self.ch[i]),
+                         ("dx", cin)):
+                self.A["%s%d" % (n, i)] = Buf(ctx, (B, h, w, c), bf)
         for i in range(self.L - 1):
             h, w = H >> i, W >> i
-            cc = self.ch[i + 1] + self.ch[i]
-            self.A["cat%d" % i] = Buf(ctx, (B, h, w, cc), bf)
-            self.A["dcat%d" % i] = Buf(ctx, (B, h, w, cc), bf)
-            self.A["dh%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["d%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["dd%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
-            self.A["gz%d" % i] = Buf(ctx, (B, h, w, self.ch[i]), bf)
+            for n, c in (("dh", self.ch[i]), ("d", self.ch[i]), ("gdh", self.ch[i]), ("gd", self.ch[i]),
+                         ("dcat", self.ch[i + 1] + self.ch[i])):
+                self.A["%s%d" % (n, i)] = Buf(ctx, (B, h, w, c), bf)
         self.A["out"] = Buf(ctx, (B, H, W, self.cout), np.float32)
         self.A["dout"] = Buf(ctx, (B, H, W, self.cout), bf)
-        self.A["ddec_top"] = Buf(ctx, (B, H, W, self.ch[0]), bf)
-        wmax = max(K * K * ci * co for _, K, ci, co, _ in self.layers)
-        self.A["wflip"] = Buf(ctx, (wmax,), bf)
         ws = max(self.lib.fvm_nn_wgrad_workspace(B, H >> self._lvl(n), W >> self._lvl(n), ci, co, K)
                  for n, K, ci, co, _ in self.layers)
         self.A["work"] = Buf(ctx, (ws // 4 + 1,), np.float32)
         npix = B * H * W
         self.A["lossw"] = Buf(ctx, ((npix * self.cout + 255) // 256 + 1,), np.float32)
         self.A["loss"] = Buf(ctx, (1,), np.float32)
+        self._describe(B, H, W)
+
+    def _describe(self, B, H, W):
+        u = fvm_unet(self.L, B, H, W, self.cin, self.cout, self.cout_real)
+        for i, c in enumerate(self.ch):
+            u.ch[i] = c
+        for i in range(self.L):
+            for n in ("x", "h", "e", "dx"):
+                getattr(u, n)[i] = self.A["%s%d" % (n, i)].ptr
+            u.g1[i], u.g2[i] = self.A["g1_%d" % i].ptr, self.A["g2_%d" % i].ptr
+        for i in range(self.L - 1):
+            for n in ("dh", "d", "gdh", "gd", "dcat"):
+                getattr(u, n)[i] = self.A["%s%d" % (n, i)].ptr
+        u.out, u.dout, u.work = self.A["out"].ptr, self.A["dout"].ptr, self.A["work"].ptr
+        self.desc = u
+
+    def _point(self, *pairs):
+        """The parameters' current buffers into the description."""
+        for k, (name, *_) in enumerate(self.layers):
+            e = self.p[name]
+            for field, key in pairs:
+                getattr(self.desc, field)[k] = e[key].ptr
 
     def _lvl(self, name):
         return 0 if name == "out" else int(name[1])
@@ -197,38 +220,14 @@ class UNet:
         if rc != 0:
             self.ctx._check(rc)
 
-    def _conv(self, name, X, Y, B, H, W, Yf=None):
-        e = self.p[name]
-        self._call("fvm_nn_conv_fwd", P(X.ptr), P(e["wb"].ptr), P(e["b"].ptr), B, H, W, e["ci"], e["co"], e["K"],
-                   1 if e["relu"] else 0, self.cout_real if name == "out" else e["co"],
-                   P(Y.ptr) if Y is not None else None, P(Yf.ptr) if Yf is not None else None)
-
     # ---- forward ----
     def forward(self, X):
         """X: Buf (B, H, W, cin) bf16 -> self.A['out'] (fp32, B H W cout)."""
         B, H, W, _ = X.shape
         self._alloc(B, H, W)
-        A = self.A
-        self._call("fvm_nn_copy_channels", P(X.ptr), I64(B * H * W), self.cin, self.cin, 0, P(A["x0"].ptr),
-                   self.cin, 0)
-        for i in range(self.L):
-            h, w = H >> i, W >> i
-            self._conv("e%d_1" % i, A["x%d" % i], A["h%d" % i], B, h, w)
-            self._conv("e%d_2" % i, A["h%d" % i], A["e%d" % i], B, h, w)
-            if i < self.L - 1:
-                self._call("fvm_nn_pool_fwd", P(A["e%d" % i].ptr), B, h, w, self.ch[i], P(A["x%d" % (i + 1)].ptr))
-        d = A["e%d" % (self.L - 1)]
-        for i in range(self.L - 2, -1, -1):
-            h, w = H >> i, W >> i
-            cc = self.ch[i + 1] + self.ch[i]
-            self._call("fvm_nn_up_fwd", P(d.ptr), B, h // 2, w // 2, self.ch[i + 1], P(A["cat%d" % i].ptr), cc, 0)
-            self._call("fvm_nn_copy_channels", P(A["e%d" % i].ptr), I64(B * h * w), self.ch[i], self.ch[i], 0,
-                       P(A["cat%d" % i].ptr), cc, self.ch[i + 1])
-            self._conv("d%d_1" % i, A["cat%d" % i], A["dh%d" % i], B, h, w)
-            self._conv("d%d_2" % i, A["dh%d" % i], A["d%d" % i], B, h, w)
-            d = A["d%d" % i]
-        self._conv("out", d, None, B, H, W, Yf=A["out"])
-        return A["out"]
+        self._point(("wb", "wb"), ("b", "b"))
+        self._call("fvm_nn_unet_forward", C.byref(self.desc), P(X.ptr))
+        return self.A["out"]
 
     # ---- loss ----
     def loss(self, T, mask=None):
@@ -242,65 +241,19 @@ class UNet:
         return float(self.A["loss"].get()[0])
 
     # ---- backward ----
-    def _wgrad(self, name, X, dY, B, H, W):
-        e = self.p[name]
-        self._call("fvm_nn_conv_wgrad", P(X.ptr), P(dY.ptr), B, H, W, e["ci"], e["co"], e["K"],
-                   P(self.A["work"].ptr), P(e["gw"].ptr), P(e["gb"].ptr))
-
-    def _dgrad(self, name, dY, dX, B, H, W):
-        e = self.p[name]
-        self._call("fvm_nn_conv_dgrad", P(dY.ptr), P(e["wb"].ptr), P(self.A["wflip"].ptr), B, H, W, e["ci"],
-                   e["co"], e["K"], P(dX.ptr))
-
-    def _relu_bwd(self, y, dy, dz):
-        self._call("fvm_nn_relu_bwd", I64(int(np.prod(y.shape))), P(y.ptr), P(dy.ptr), P(dz.ptr))
-
     def backward(self):
-        B, H, W = self.shape
-        A, L, ch = self.A, self.L, self.ch
-        d0 = A["d0"] if L > 1 else A["e0"]
-        self._wgrad("out", d0, A["dout"], B, H, W)
-        dd = A["ddec_top"]
-        self._dgrad("out", A["dout"], dd, B, H, W)
-        for i in range(0, L - 1):
-            h, w = H >> i, W >> i
-            cc = ch[i + 1] + ch[i]
-            self._relu_bwd(A["d%d" % i], dd, A["gz%d" % i])
-            self._wgrad("d%d_2" % i, A["dh%d" % i], A["gz%d" % i], B, h, w)
-            self._dgrad("d%d_2" % i, A["gz%d" % i], A["dd%d" % i], B, h, w)
-            self._relu_bwd(A["dh%d" % i], A["dd%d" % i], A["gz%d" % i])
-            self._wgrad("d%d_1" % i, A["cat%d" % i], A["gz%d" % i], B, h, w)
-            self._dgrad("d%d_1" % i, A["gz%d" % i], A["dcat%d" % i], B, h, w)
-            # skip part -> de_i; upsampled part -> gradient of the level below
-            self._call("fvm_nn_copy_channels", P(A["dcat%d" % i].ptr), I64(B * h * w), ch[i], cc, ch[i + 1],
-                       P(A["de%d" % i].ptr), ch[i], 0)
-            target = A["de%d" % (L - 1)] if i + 1 == L - 1 else A["g1_%d" % (i + 1)]
-            self._call("fvm_nn_up_bwd", P(A["dcat%d" % i].ptr), B, h // 2, w // 2, ch[i + 1], cc, 0, P(target.ptr))
-            dd = target
-        # encoder, bottom up: de_{L-1} holds the bottleneck gradient
-        dnext = None
-        for i in range(L - 1, -1, -1):
-            h, w = H >> i, W >> i
-            de = A["de%d" % i]
-            if i < L - 1:
-                self._call("fvm_nn_add_channels", P(dnext.ptr), I64(B * h * w), ch[i], ch[i], 0, P(de.ptr))
-            self._relu_bwd(A["e%d" % i], de, A["g1_%d" % i])
-            self._wgrad("e%d_2" % i, A["h%d" % i], A["g1_%d" % i], B, h, w)
-            self._dgrad("e%d_2" % i, A["g1_%d" % i], A["g2_%d" % i], B, h, w)
-            self._relu_bwd(A["h%d" % i], A["g2_%d" % i], A["g1_%d" % i])
-            self._wgrad("e%d_1" % i, A["x%d" % i], A["g1_%d" % i], B, h, w)
-            if i > 0:
-                self._dgrad("e%d_1" % i, A["g1_%d" % i], A["dx%d" % i], B, h, w)
-                self._call("fvm_nn_pool_bwd", P(A["dx%d" % i].ptr), B, h * 2, w * 2, ch[i - 1],
-                           P(A["g2_%d" % (i - 1)].ptr))
-                dnext = A["g2_%d" % (i - 1)]
+        """Every parameter's gradient (gw, gb) from A['dout'], which loss() left."""
+        self._point(("wb", "wb"), ("gw", "gw"), ("gb", "gb"))
+        self._call("fvm_nn_unet_backward", C.byref(self.desc))
 
     # ---- optimizer ----
     def adam(self, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, wd=0.0):
         self.adam_step += 1
-        for e in self.p.values():
-            n = int(np.prod(e["w"].shape))
-            self._call("fvm_nn_adam", I64(n), P(e["w"].ptr), P(e["gw"].ptr), P(e["mw"].ptr), P(e["vw"].ptr),
-                       P(e["wb"].ptr), F(lr), F(b1), F(b2), F(eps), self.adam_step, F(wd))
-            self._call("fvm_nn_adam", I64(e["co"]), P(e["b"].ptr), P(e["gb"].ptr), P(e["mb"].ptr), P(e["vb"].ptr),
-                       None, F(lr), F(b1), F(b2), F(eps), self.adam_step, F(0.0))
+        e = self.p.values()
+        t = [(x["w"], x["gw"], x["mw"], x["vw"], x["wb"].ptr) for x in e] + \
+            [(x["b"], x["gb"], x["mb"], x["vb"], None) for x in e]
+        n = len(t)
+        sizes = (I64 * n)(*(int(np.prod(x[0].shape)) for x in t))
+        tables = [(P * n)(*(x[k].ptr for x in t)) for k in range(4)] + [(P * n)(*(x[4] for x in t))]
+        decay = (F * n)(*([wd] * len(self.layers) + [0.0] * len(self.layers)))
+        self._call("fvm_nn_adam_all", n, sizes, *tables, decay, F(lr), F(b1), F(b2), F(eps), self.adam_step)

@@ -8,7 +8,7 @@ import pytest
 
 from oracle.unet_ref import bf16
 from fvmic2d_amd.lib import Context
-from fvmic2d_amd.unet import Buf, bind, from_bf16_bits, to_bf16_bits
+from fvmic2d_amd.unet import Buf, UNet, bind, from_bf16_bits, to_bf16_bits
 
 pytestmark = pytest.mark.gpu
 
@@ -127,3 +127,99 @@ def test_data_gradient(shape):
         ref += y.astype(np.float64) @ w
         mag += np.abs(y) @ np.abs(w)
     _check_bf16(from_bf16_bits(dX.get()), ref, K * K * co * 2.0 ** -23 * mag)
+
+
+
+def _layerwise(net, X, dout):
+    """forward and backward through the layer entry points, one call per layer."""
+    ctx, lib, L, ch = net.ctx, net.lib, net.L, net.ch
+    B, H, W, _ = X.shape
+    keep = []
+
+    def buf(h, w, c):
+        keep.append(Buf(ctx, (B, h, w, c), np.uint16))
+        return keep[-1]
+
+    def call(fn, *a):
+        assert getattr(lib, fn)(ctx.h, *a) == 0, fn
+
+    def size(i):
+        return H >> i, W >> i
+
+    def conv(name, x, i):
+        e = net.p[name]
+        y = buf(*size(i), e["co"])
+        call("fvm_nn_conv_fwd", x.ptr, e["wb"].ptr, e["b"].ptr, B, *size(i), e["ci"], e["co"], 3, 1, e["co"], y.ptr, None)
+        return y
+
+    def grad(name, x, dy, i, need=True):
+        e = net.p[name]
+        call("fvm_nn_conv_wgrad", x.ptr, dy.ptr, B, *size(i), e["ci"], e["co"], e["K"], net.A["work"].ptr, e["gw"].ptr,
+             e["gb"].ptr)
+        if need:
+            dx, scratch = buf(*size(i), e["ci"]), Buf(ctx, e["wb"].shape, np.uint16)
+            call("fvm_nn_conv_dgrad", dy.ptr, e["wb"].ptr, scratch.ptr, B, *size(i), e["ci"], e["co"], e["K"], dx.ptr)
+            return dx
+
+    def relu(y, dy):
+        dz = buf(*y.shape[1:])
+        call("fvm_nn_relu_bwd", int(np.prod(y.shape)), y.ptr, dy.ptr, dz.ptr)
+        return dz
+    x, h, e, cat, dh, d = {}, {}, {}, {}, {}, {}
+    x[0] = X
+    for i in range(L):
+        h[i] = conv("e%d_1" % i, x[i], i)
+        e[i] = conv("e%d_2" % i, h[i], i)
+        if i < L - 1:
+            x[i + 1] = buf(*size(i + 1), ch[i])
+            call("fvm_nn_pool_fwd", e[i].ptr, B, *size(i), ch[i], x[i + 1].ptr)
+    d[L - 1] = e[L - 1]
+    for i in range(L - 2, -1, -1):
+        cc = ch[i + 1] + ch[i]
+        cat[i] = buf(*size(i), cc)
+        call("fvm_nn_up_fwd", d[i + 1].ptr, B, *size(i + 1), ch[i + 1], cat[i].ptr, cc, 0)
+        call("fvm_nn_copy_channels", e[i].ptr, B * (H >> i) * (W >> i), ch[i], ch[i], 0, cat[i].ptr, cc, ch[i + 1])
+        dh[i] = conv("d%d_1" % i, cat[i], i)
+        d[i] = conv("d%d_2" % i, dh[i], i)
+    o = net.p["out"]
+    out = Buf(ctx, (B, H, W, net.cout), np.float32)
+    call("fvm_nn_conv_fwd", d[0].ptr, o["wb"].ptr, o["b"].ptr, B, H, W, o["ci"], o["co"], 1, 0, net.cout_real, None, out.ptr)
+    g = grad("out", d[0], dout, 0)
+    skip = {}
+    for i in range(L - 1):
+        g = grad("d%d_2" % i, dh[i], relu(d[i], g), i)
+        dcat = grad("d%d_1" % i, cat[i], relu(dh[i], g), i)
+        cc, skip[i], g = ch[i + 1] + ch[i], buf(*size(i), ch[i]), buf(*size(i + 1), ch[i + 1])
+        call("fvm_nn_copy_channels", dcat.ptr, B * (H >> i) * (W >> i), ch[i], cc, ch[i + 1], skip[i].ptr, ch[i], 0)
+        call("fvm_nn_up_bwd", dcat.ptr, B, *size(i + 1), ch[i + 1], cc, 0, g.ptr)
+    skip[L - 1] = g
+    for i in range(L - 1, -1, -1):
+        if i < L - 1:
+            call("fvm_nn_add_channels", g.ptr, B * (H >> i) * (W >> i), ch[i], ch[i], 0, skip[i].ptr)
+        g = grad("e%d_2" % i, h[i], relu(e[i], skip[i]), i)
+        dx = grad("e%d_1" % i, x[i], relu(h[i], g), i, i > 0)
+        if i > 0:
+            g = buf(*size(i - 1), ch[i - 1])
+            call("fvm_nn_pool_bwd", dx.ptr, B, *size(i - 1), ch[i - 1], g.ptr)
+    return out.get()
+
+
+@pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40)])
+def test_whole_passes_equal_the_layers(L, base, B, H, W):
+    """The one-call passes, which fuse the copies, the concatenation and the ReLU
+    passes into the kernels beside them, are bitwise the layer-by-layer ones."""
+    print("CASE unet passes", L, base, B, H, W, flush=True)
+    net = UNet(Context(), levels=L, base=base, seed=3)
+    r = np.random.default_rng(5)
+    X = np.zeros((B, H, W, net.cin), np.float32)
+    X[..., :5] = r.standard_normal((B, H, W, 5))
+    T = r.standard_normal((B, H, W, 3)).astype(np.float32)
+    dX, dT = _dev(net.ctx, X, np.uint16), _dev(net.ctx, T, np.float32)
+    out = net.forward(dX).get()
+    dX.zero()       # the caller may reuse its input before the backward pass
+    net.loss(dT)
+    net.backward()
+    grads = net.grads_numpy()
+    assert np.array_equal(out, _layerwise(net, _dev(net.ctx, X, np.uint16), net.A["dout"]))
+    for name, (gw, gb) in net.grads_numpy().items():
+        assert np.array_equal(grads[name][0], gw) and np.array_equal(grads[name][1], gb), name
