@@ -67,14 +67,7 @@ struct fvm_ctx {
 int fvm_set_err(fvm_ctx *ctx, int code, const char *fmt, ...);
 int fvm_ws(fvm_ctx *ctx, fvm_buf &b, size_t bytes);  // ensure workspace capacity
 
-// Preconditioner of a 5-point system on NX x NY nodes (mg.hip): y = M b stands for
-// the system with every row divided by its diagonal d.  scale: the couplings are
-// not divided by d yet.  *out is null where no preconditioner is offered.  It
-// belongs to the context and lasts until the next build.
-struct fvm_precond;
-int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const double *e, const double *w, const double *s,
-                      const double *n, bool scale, fvm_precond **out);
-int fvm_precond_apply(fvm_ctx *ctx, const fvm_precond *m, const double *b, double *y);
+struct fvm_precond;  // the nodal solves' preconditioner (bicgstab.h)
 void fvm_precond_free(fvm_precond *m);
 
 #define FVM_HIP(ctx, call)                                                               \

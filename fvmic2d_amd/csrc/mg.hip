@@ -10,20 +10,21 @@
 //   correction, cells aggregated in pairs along each axis (along one axis only
 //   while its couplings are much the stronger), the coarse couplings rediscretised
 //   from the aggregated ones (divided by the grown distance), restriction by sums,
-//   prolongation bilinear.  6 iterations at 257x257 (solve 31.7 -> 1.10 ms).
+//   prolongation bilinear.  6 iterations at 257x257 (solve 31.7 -> 0.85 ms).
 // * where every row is dominated by its diagonal (an energy equation with a
 //   moderate time step) the same polynomial at degree FV_POLY on the finest
 //   level alone, over the interval the row sums give: 5 iterations instead of 40
-//   at 801x401 (assembly and solve 1.67 -> 0.47 ms).
+//   at 801x401 (assembly and solve 1.67 -> 0.39 ms).
 //
 // What bounds them is latency, so a kernel does as much as its tile allows: a
 // tile and a halo as wide as the number of sweeps are read once, all sweeps run in
-// LDS (the halo is swept redundantly: 2.3 times the tile's points), and everything
-// below FV_COARSE_MAX points is one workgroup's kernel.
+// LDS (the halo is swept redundantly: 2.3 times the tile's points), everything
+// below FV_COARSE_MAX points is one workgroup's kernel, and around the one-level
+// polynomial the whole iteration is three kernels.
 #include <new>
 #include <vector>
 
-#include "fvm_internal.h"
+#include "bicgstab.h"
 
 namespace {
 
@@ -31,10 +32,12 @@ constexpr int FV_NU = 4;        // sweeps on each side of the coarse correction
 constexpr int FV_POLY = 8;      // degree of the one-level preconditioner
 constexpr int FV_T = 16;        // tile of the level kernels
 constexpr int FV_R = FV_T + 2 * FV_NU;
-constexpr int FV_PT = 32;       // tile of the one-level kernel
-constexpr int FV_PR = FV_PT + 2 * (FV_POLY - 1);
-constexpr int FV_COARSE_MAX = 4400;
-constexpr int FV_CT = 1024;     // threads of the coarse kernel
+constexpr int FV_PT = 32;       // tile of the one-level kernels
+constexpr int FV_PR = FV_PT + 2 * FV_POLY;
+// points of the finest level that the one-workgroup kernel takes: 33 x 33 and the
+// levels below cost 22 us, 65 x 65 44 us against 9 for two more level kernels
+constexpr int FV_COARSE_MAX = 1100;
+constexpr int FV_CT = 512;      // threads of the coarse kernel
 constexpr int FV_CLEVELS = 16;
 constexpr int FV_LAST = 12;     // sweeps on the last level
 
@@ -42,14 +45,16 @@ struct Coefs {
   const double *e, *w, *s, *n;
 };
 
-// Chebyshev steps d = c1 d + c2 r, x += d for the spectrum [a, b]
+// Chebyshev steps d = c1 d + c2 r, x += d for the spectrum [a, b].  A row without
+// couplings starts at its solution x = b with d = 0: its residual is 0 and the
+// steps leave it there without a branch.
 struct Cheb {
   double c1[16], c2[16];
 };
 
 struct Pt {
   double e, w, s, n;
-  __device__ __forceinline__ bool live() const { return e != 0.0 || w != 0.0 || s != 0.0 || n != 0.0; }
+  __device__ __forceinline__ bool live() const { return (fabs(e) + fabs(w)) + (fabs(s) + fabs(n)) != 0.0; }
 };
 __device__ __forceinline__ Pt load_pt(const Coefs &c, bool in, int64_t i) {
   Pt p = {0.0, 0.0, 0.0, 0.0};
@@ -57,58 +62,179 @@ __device__ __forceinline__ Pt load_pt(const Coefs &c, bool in, int64_t i) {
   return p;
 }
 
-// ---- one level: x = p(A) b ----------------------------------------------------------
-// 1024 threads sweep a 46x46 region for a 32x32 tile.
-__global__ void __launch_bounds__(1024) k_poly(int NX, int NY, Coefs c, Cheb ch, const double *__restrict__ b,
-                                               double *__restrict__ x) {
-  constexpr int RW = FV_PR + 2, NP = FV_PR * FV_PR, PTS = (NP + 1023) / 1024;
-  __shared__ double sh[2][RW * RW];
-  for (int k = threadIdx.x; k < 2 * RW * RW; k += 1024) (&sh[0][0])[k] = 0.0;
-  const int x0 = blockIdx.x * FV_PT - (FV_POLY - 1), y0 = blockIdx.y * FV_PT - (FV_POLY - 1);
+// ---- one level: the polynomial p(A), with the iteration around it --------------------
+// 1024 threads sweep a 48x48 region for a 32x32 tile: FV_POLY - 1 sweeps and the
+// product with A need a halo of FV_POLY.
+struct Region {
+  static constexpr int RW = FV_PR + 2, NP = FV_PR * FV_PR, PTS = (NP + 1023) / 1024;
   Pt p[PTS];
-  double bb[PTS], d[PTS], xv[PTS];
-  int at[PTS];
-  bool live[PTS];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < PTS; k++) {
+  int i[PTS];   // node, or -1 outside the grid
+  int at[PTS];  // place in LDS, or -1
+
+  __device__ __forceinline__ bool own(int k) const {  // of the tile
     const int q = threadIdx.x + 1024 * k, ry = q / FV_PR, rx = q - ry * FV_PR;
-    const int ix = x0 + rx, iy = y0 + ry;
-    const bool in = q < NP && ix >= 0 && ix < NX && iy >= 0 && iy < NY;
-    const int64_t i = (int64_t)iy * NX + ix;
-    p[k] = load_pt(c, in, i);
-    bb[k] = in ? b[i] : 0.0;
-    live[k] = p[k].live();
-    d[k] = live[k] ? bb[k] * ch.c2[0] : 0.0;
-    xv[k] = live[k] ? d[k] : bb[k];
-    at[k] = q < NP ? (ry + 1) * RW + rx + 1 : -1;
-    if (at[k] >= 0) sh[0][at[k]] = xv[k];
+    return i[k] >= 0 && rx >= FV_POLY && rx < FV_POLY + FV_PT && ry >= FV_POLY && ry < FV_POLY + FV_PT;
   }
-  __syncthreads();
-#pragma unroll 1
-  for (int t = 1; t < FV_POLY; t++) {
-    const double *xs = sh[(t - 1) & 1];
-    double *xn = sh[t & 1];
+
+  __device__ __forceinline__ void place(int NX, int NY, const Coefs &c) {
 #pragma unroll
     for (int k = 0; k < PTS; k++) {
-      if (at[k] < 0) continue;
-      const int a = at[k];
-      const double r = bb[k] - (xv[k] + p[k].e * xs[a + 1] + p[k].w * xs[a - 1] + p[k].s * xs[a + RW] + p[k].n * xs[a - RW]);
-      if (live[k]) {
-        d[k] = ch.c1[t] * d[k] + ch.c2[t] * r;
-        xv[k] += d[k];
-      }
-      xn[a] = xv[k];
+      const int q = threadIdx.x + 1024 * k, ry = q / FV_PR, rx = q - ry * FV_PR;
+      const int ix = (int)blockIdx.x * FV_PT - FV_POLY + rx, iy = (int)blockIdx.y * FV_PT - FV_POLY + ry;
+      const bool in = q < NP && ix >= 0 && ix < NX && iy >= 0 && iy < NY;
+      i[k] = in ? iy * NX + ix : -1;
+      at[k] = q < NP ? (ry + 1) * RW + rx + 1 : -1;
+      p[k] = load_pt(c, in, i[k]);
+    }
+  }
+  // x = p(A) b, then ax = A x of the tile's points; sh zeroed before
+  __device__ __forceinline__ void poly(const Cheb &ch, double (*sh)[RW * RW], const double *b, double *x, double *ax) {
+    double d[PTS];
+#pragma unroll
+    for (int k = 0; k < PTS; k++) {
+      const bool live = p[k].live();
+      d[k] = live ? b[k] * ch.c2[0] : 0.0;
+      x[k] = live ? d[k] : b[k];
+      if (at[k] >= 0) sh[0][at[k]] = x[k];
     }
     __syncthreads();
-  }
+#pragma unroll 1
+    for (int t = 1; t < FV_POLY; t++) {
+      const double *xs = sh[(t - 1) & 1];
+      double *xn = sh[t & 1];
 #pragma unroll
-  for (int k = 0; k < PTS; k++) {
-    const int q = threadIdx.x + 1024 * k, ry = q / FV_PR, rx = q - ry * FV_PR;
-    const int ix = x0 + rx, iy = y0 + ry;
-    if (q < NP && rx >= FV_POLY - 1 && rx < FV_PT + FV_POLY - 1 && ry >= FV_POLY - 1 && ry < FV_PT + FV_POLY - 1 && ix < NX && iy < NY)
-      x[(int64_t)iy * NX + ix] = xv[k];
+      for (int k = 0; k < PTS; k++) {
+        if (at[k] < 0) continue;
+        const int a = at[k];
+        const double r = b[k] - (x[k] + p[k].e * xs[a + 1] + p[k].w * xs[a - 1] + p[k].s * xs[a + RW] + p[k].n * xs[a - RW]);
+        d[k] = ch.c1[t] * d[k] + ch.c2[t] * r;
+        x[k] += d[k];
+        xn[a] = x[k];
+      }
+      __syncthreads();
+    }
+    const double *xs = sh[(FV_POLY - 1) & 1];
+#pragma unroll
+    for (int k = 0; k < PTS; k++) {
+      const int a = at[k];
+      ax[k] = own(k) ? x[k] + p[k].e * xs[a + 1] + p[k].w * xs[a - 1] + p[k].s * xs[a + RW] + p[k].n * xs[a - RW] : 0.0;
+    }
   }
+};
+
+// sum over the 1024 threads of a block, the same bits in every thread
+__device__ __forceinline__ double total_1024(double v) {
+  __shared__ double sh[16];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double t = 0.0;
+#pragma unroll
+  for (int k = 0; k < 16; k++) t += sh[k];
+  return t;
+}
+__device__ __forceinline__ double parts_1024(const double *__restrict__ part, int n) {
+  double s = 0.0;
+  for (int k = threadIdx.x; k < n; k += 1024) s += part[k];
+  return total_1024(s);
+}
+
+// p = r + beta (p - omega v), y = p(A) p, v = A y; partials of (rhat, v).  p and v
+// are read in the halo too, so the new ones go to other arrays.
+// (8 waves per SIMD: two blocks a CU, so that 801 x 401's 338 run at once)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_one_p(int NX, int NY, Coefs c, Cheb ch, FvmBcgOne O) {
+  __shared__ double sh[2][Region::RW * Region::RW];
+  const double rho = parts_1024(O.prho, O.n_r), rr = parts_1024(O.prr, O.n_r);
+  const bool lead = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
+  const double bb = O.first ? rr : O.sc[FVM_S_BB];
+  if (fvm_bcg_done(rr, bb, O.rtol)) {
+    if (lead) O.sc[FVM_S_DONE] = 1.0, O.sc[FVM_S_RR] = rr, O.sc[FVM_S_BB] = bb;
+    return;
+  }
+  for (int k = threadIdx.x; k < 2 * Region::RW * Region::RW; k += 1024) (&sh[0][0])[k] = 0.0;
+  const double omega = O.sc[FVM_S_OMEGA], beta = fvm_bcg_beta(O.first, rho, O.sc);
+  Region R;
+  R.place(NX, NY, c);
+  double b[Region::PTS], y[Region::PTS], v[Region::PTS];
+#pragma unroll
+  for (int k = 0; k < Region::PTS; k++) {
+    const int i = R.i[k];
+    b[k] = i >= 0 ? O.r[i] + beta * (O.p[i] - omega * O.v[i]) : 0.0;
+  }
+  __syncthreads();
+  R.poly(ch, sh, b, y, v);
+  double d = 0.0;
+#pragma unroll
+  for (int k = 0; k < Region::PTS; k++)
+    if (R.own(k)) {
+      const int i = R.i[k];
+      O.p_new[i] = b[k];
+      O.y[i] = y[k];
+      O.v_new[i] = v[k];
+      d += O.rh[i] * v[k];
+    }
+  const double t = total_1024(d);
+  if (threadIdx.x == 0) O.prv[blockIdx.y * gridDim.x + blockIdx.x] = t;
+  if (lead) {
+    O.sc[FVM_S_RHO] = rho, O.sc[FVM_S_BB] = bb, O.sc[FVM_S_RR] = rr, O.sc[FVM_S_DONE] = 0.0;
+    O.sc[FVM_S_ITS] = O.first ? 1.0 : O.sc[FVM_S_ITS] + 1.0;
+  }
+}
+
+// alpha = rho / (rhat, v), x += alpha y, s = r - alpha v, z = p(A) s, t = A z;
+// partials of (t, s) and (t, t)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_one_s(int NX, int NY, Coefs c, Cheb ch, FvmBcgOne O) {
+  __shared__ double sh[2][Region::RW * Region::RW];
+  if (O.sc[FVM_S_DONE] != 0.0) return;
+  const double rv = parts_1024(O.prv, gridDim.x * gridDim.y), alpha = rv != 0.0 ? O.sc[FVM_S_RHO] / rv : 0.0;
+  for (int k = threadIdx.x; k < 2 * Region::RW * Region::RW; k += 1024) (&sh[0][0])[k] = 0.0;
+  Region R;
+  R.place(NX, NY, c);
+  double b[Region::PTS], z[Region::PTS], t[Region::PTS];
+#pragma unroll
+  for (int k = 0; k < Region::PTS; k++) {
+    const int i = R.i[k];
+    b[k] = i >= 0 ? O.r[i] - alpha * O.v_new[i] : 0.0;
+  }
+  __syncthreads();
+  R.poly(ch, sh, b, z, t);
+  double ts = 0.0, tt = 0.0;
+#pragma unroll
+  for (int k = 0; k < Region::PTS; k++)
+    if (R.own(k)) {
+      const int i = R.i[k];
+      O.x[i] += alpha * O.y[i];
+      O.s[i] = b[k];
+      O.z[i] = z[k];
+      O.t[i] = t[k];
+      ts += t[k] * b[k];
+      tt += t[k] * t[k];
+    }
+  const double a = total_1024(ts), e = total_1024(tt);
+  if (threadIdx.x == 0) {
+    O.pts[blockIdx.y * gridDim.x + blockIdx.x] = a;
+    O.ptt[blockIdx.y * gridDim.x + blockIdx.x] = e;
+  }
+  if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) O.sc[FVM_S_ALPHA] = alpha;
+}
+
+// omega = (t, s) / (t, t), x += omega z, r = s - omega t; partials of (rhat, r), (r, r)
+__global__ void __launch_bounds__(1024) k_one_x(int64_t n, int n_t, FvmBcgOne O) {
+  if (O.sc[FVM_S_DONE] != 0.0) return;
+  const double ts = parts_1024(O.pts, n_t), tt = parts_1024(O.ptt, n_t), omega = tt != 0.0 ? ts / tt : 0.0;
+  double a = 0.0, b = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 1024) {
+    O.x[i] += omega * O.z[i];
+    const double r = O.s[i] - omega * O.t[i];
+    O.r[i] = r;
+    a += O.rh[i] * r;
+    b += r * r;
+  }
+  const double ta = total_1024(a), tb = total_1024(b);
+  if (threadIdx.x == 0) O.prho[blockIdx.x] = ta, O.prr[blockIdx.x] = tb;
+  if (blockIdx.x == 0 && threadIdx.x == 0) O.sc[FVM_S_OMEGA] = omega, O.sc[FVM_S_RHO_OLD] = O.sc[FVM_S_RHO];
 }
 
 // ---- multigrid ------------------------------------------------------------------------
@@ -132,7 +258,8 @@ __device__ __forceinline__ double row_residual(const Pt &p, double b, const doub
 
 // x = FV_NU sweeps from 0, then the residual summed over the aggregates
 __global__ void __launch_bounds__(FV_R *FV_R) k_down(Lv L, Cheb ch, const double *__restrict__ b, double *__restrict__ x,
-                                                     double *__restrict__ bc) {
+                                                     double *__restrict__ bc, const double *__restrict__ sc) {
+  if (sc[FVM_S_DONE] != 0.0) return;
   constexpr int RW = FV_R + 2;
   __shared__ double sh[2][RW * RW];
   const int t = threadIdx.x, ry = t / FV_R, rx = t - ry * FV_R;
@@ -153,14 +280,12 @@ __global__ void __launch_bounds__(FV_R *FV_R) k_down(Lv L, Cheb ch, const double
 #pragma unroll
   for (int s = 1; s < FV_NU; s++) {
     const double r = row_residual(p, bb, sh[(s - 1) & 1], a, RW);
-    if (live) {
-      d = ch.c1[s] * d + ch.c2[s] * r;
-      xv += d;
-    }
+    d = ch.c1[s] * d + ch.c2[s] * r;
+    xv += d;
     sh[s & 1][a] = xv;
     __syncthreads();
   }
-  const double r = live ? row_residual(p, bb, sh[(FV_NU - 1) & 1], a, RW) : 0.0;
+  const double r = row_residual(p, bb, sh[(FV_NU - 1) & 1], a, RW);
   const bool own = in && rx >= FV_NU && rx < FV_NU + FV_T && ry >= FV_NU && ry < FV_NU + FV_T;
   if (own) x[i] = xv;
   sh[FV_NU & 1][a] = own ? r : 0.0;
@@ -204,7 +329,9 @@ __device__ __forceinline__ double prolong(const Lv &L, const Pt &p, int ix, int 
 
 // out = FV_NU sweeps from x + P ec
 __global__ void __launch_bounds__(FV_R *FV_R) k_up(Lv L, Cheb ch, const double *__restrict__ b, const double *__restrict__ x,
-                                                   const double *__restrict__ ec, double *__restrict__ out) {
+                                                   const double *__restrict__ ec, double *__restrict__ out,
+                                                   const double *__restrict__ sc) {
+  if (sc[FVM_S_DONE] != 0.0) return;
   constexpr int RW = FV_R + 2;
   __shared__ double sh[2][RW * RW];
   const int t = threadIdx.x, ry = t / FV_R, rx = t - ry * FV_R;
@@ -224,113 +351,131 @@ __global__ void __launch_bounds__(FV_R *FV_R) k_up(Lv L, Cheb ch, const double *
 #pragma unroll
   for (int s = 0; s < FV_NU; s++) {
     const double r = row_residual(p, bb, sh[s & 1], a, RW);
-    if (live) {
-      d = ch.c1[s] * d + ch.c2[s] * r;
-      xv += d;
-    }
+    d = ch.c1[s] * d + ch.c2[s] * r;
+    xv += d;
     sh[(s + 1) & 1][a] = xv;
     __syncthreads();
   }
   if (in && rx >= FV_NU && rx < FV_NU + FV_T && ry >= FV_NU && ry < FV_NU + FV_T) out[i] = xv;
 }
 
-// Every level of at most FV_COARSE_MAX points in one workgroup: x and b of each
-// level lie in LDS between zeros wide enough for the stencil's reach (a missing
-// neighbour's coefficient is 0), a thread's rows in registers during a smoothing.
+// The levels of at most FV_COARSE_MAX points in one workgroup: their rows, right-hand
+// sides and two copies of x (a sweep reads one and writes the other) lie in LDS,
+// between zeros wide enough for the stencil's reach (a missing neighbour's
+// coefficient is 0).
 struct CoarseArgs {
   int n;
   Lv lv[FV_CLEVELS];
   int off[FV_CLEVELS];  // of point 0 in the LDS arrays
   int total;            // doubles per LDS array
 };
-constexpr int FV_LDS = 6400;  // doubles per array (x, b)
+constexpr int FV_LDS = 2400;  // doubles per array (e, w, s, n, b, x, x, 1/diagonal)
 
-template <int PTS>
-__device__ __forceinline__ void smooth(const Lv &L, const Cheb &ch, int steps, bool zero, double *x, const double *b) {
-  const int np = L.NX * L.NY;
+struct CoarseLv {
+  int NX, np, off;
+};
+// STEPS sweeps on level v from x in lds[6], or from 0 (ZERO); the sweeps alternate
+// between lds[5] and lds[6] and end in lds[6] (from 0, the first only fills lds[5])
+template <int STEPS, bool ZERO>
+__device__ __forceinline__ void coarse_sweep(const CoarseLv &v, const Cheb &ch, double (*lds)[FV_LDS]) {
+  static_assert(STEPS % 2 == 0, "coarse_sweep ends in lds[6]");
+  constexpr int PTS = (FV_COARSE_MAX + FV_CT - 1) / FV_CT;
   Pt p[PTS];
-  double d[PTS], xv[PTS];
+  double d[PTS], xv[PTS], b[PTS];
 #pragma unroll
   for (int k = 0; k < PTS; k++) {
-    const int q = threadIdx.x + FV_CT * k;
-    p[k] = load_pt(L.c, q < np, q);
+    const int q = threadIdx.x + FV_CT * k, a = v.off + q;
     d[k] = 0.0;
-    xv[k] = q < np && !zero ? x[q] : 0.0;
-    if (zero && q < np) {
-      d[k] = p[k].live() ? b[q] * ch.c2[0] : 0.0;
-      xv[k] = p[k].live() ? d[k] : b[q];
-      x[q] = xv[k];
+    if (q < v.np) {
+      p[k] = Pt{lds[0][a], lds[1][a], lds[2][a], lds[3][a]};
+      b[k] = lds[4][a];
+      if (ZERO) {
+        const bool live = p[k].live();
+        d[k] = live ? b[k] * ch.c2[0] : 0.0;
+        xv[k] = live ? d[k] : b[k];
+        lds[5][a] = xv[k];
+      } else {
+        xv[k] = lds[6][a];
+      }
     }
   }
   __syncthreads();
-  for (int s = zero ? 1 : 0; s < steps; s++) {
+#pragma unroll
+  for (int s = ZERO ? 1 : 0; s < STEPS; s++) {
+    const double *xs = lds[s & 1 ? 5 : 6];
+    double *xn = lds[s & 1 ? 6 : 5];
 #pragma unroll
     for (int k = 0; k < PTS; k++) {
-      const int q = threadIdx.x + FV_CT * k;
-      if (q < np && p[k].live()) {
-        d[k] = ch.c1[s] * d[k] + ch.c2[s] * row_residual(p[k], b[q], x, q, L.NX);
+      const int q = threadIdx.x + FV_CT * k, a = v.off + q;
+      if (q < v.np) {
+        d[k] = ch.c1[s] * d[k] + ch.c2[s] * row_residual(p[k], b[k], xs, a, v.NX);
         xv[k] += d[k];
+        xn[a] = xv[k];
       }
     }
     __syncthreads();
-#pragma unroll
-    for (int k = 0; k < PTS; k++) {
-      const int q = threadIdx.x + FV_CT * k;
-      if (q < np) x[q] = xv[k];
-    }
-    __syncthreads();
   }
 }
-__device__ __forceinline__ void smooth_any(const Lv &L, const Cheb &ch, int steps, bool zero, double *x, const double *b) {
-  const int np = L.NX * L.NY;
-  if (np > 2 * FV_CT) smooth<(FV_COARSE_MAX + FV_CT - 1) / FV_CT>(L, ch, steps, zero, x, b);
-  else if (np > FV_CT) smooth<2>(L, ch, steps, zero, x, b);
-  else smooth<1>(L, ch, steps, zero, x, b);
-}
 
-__global__ void __launch_bounds__(FV_CT) k_coarse(CoarseArgs A, Cheb ch, Cheb last, int last_steps,
-                                                  const double *__restrict__ bin, double *__restrict__ xout) {
-  __shared__ double X[FV_LDS], B[FV_LDS];
-  for (int k = threadIdx.x; k < A.total; k += FV_CT) X[k] = 0.0, B[k] = 0.0;
-  __syncthreads();
-  const int np0 = A.lv[0].NX * A.lv[0].NY;
-  for (int q = threadIdx.x; q < np0; q += FV_CT) B[A.off[0] + q] = bin[q];
+__global__ void __launch_bounds__(FV_CT) k_coarse(CoarseArgs A, Cheb ch, Cheb last,
+                                                  const double *__restrict__ bin, double *__restrict__ xout,
+                                                  const double *__restrict__ sc) {
+  if (sc[FVM_S_DONE] != 0.0) return;
+  __shared__ double lds[8][FV_LDS];
+  // every level's rows, all loads of a thread in flight together
+  for (int k = threadIdx.x; k < A.total; k += FV_CT) {
+    int l = 0;
+    while (l + 1 < A.n && k >= A.off[l + 1] - (A.lv[l + 1].NX + 1)) l++;
+    const Lv &L = A.lv[l];
+    const int q = k - A.off[l];
+    const bool in = q >= 0 && q < L.NX * L.NY;
+    const Pt p = load_pt(L.c, in, q);
+    lds[0][k] = p.e, lds[1][k] = p.w, lds[2][k] = p.s, lds[3][k] = p.n;
+    lds[4][k] = in && l == 0 ? bin[q] : 0.0;
+    lds[5][k] = lds[6][k] = 0.0;
+    lds[7][k] = in && l ? A.lv[l - 1].idc[q] : 0.0;
+  }
   __syncthreads();
 #pragma unroll 1
   for (int l = 0; l + 1 < A.n; l++) {
     const Lv &L = A.lv[l];
-    double *x = X + A.off[l], *b = B + A.off[l], *bc = B + A.off[l + 1];
-    smooth_any(L, ch, FV_NU, true, x, b);
+    const int o = A.off[l], oc = A.off[l + 1];
+    coarse_sweep<FV_NU, true>(CoarseLv{L.NX, L.NX * L.NY, o}, ch, lds);
     for (int q = threadIdx.x; q < L.NXc * L.NYc; q += FV_CT) {
       const int J = q / L.NXc, I = q - J * L.NXc;
       const int i0 = L.fx == 2 ? (I ? 2 * I - 1 : 0) : I, j0 = L.fy == 2 ? (J ? 2 * J - 1 : 0) : J;
       const int ni = agg_count(I, L.fx, L.NX), nj = agg_count(J, L.fy, L.NY);
       double v = 0.0;
-      for (int j = j0; j < j0 + nj; j++)
-        for (int i = i0; i < i0 + ni; i++) {
-          const int f = j * L.NX + i;
-          const Pt p = load_pt(L.c, true, f);
-          if (p.live()) v += row_residual(p, b[f], x, f, L.NX);
+#pragma unroll
+      for (int j = 0; j < 2; j++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+          if (i >= ni || j >= nj) continue;
+          const int a = o + (j0 + j) * L.NX + i0 + i;
+          const Pt p = {lds[0][a], lds[1][a], lds[2][a], lds[3][a]};
+          v += row_residual(p, lds[4][a], lds[6], a, L.NX);
         }
-      bc[q] = v * L.idc[q];
+      lds[4][oc + q] = v * lds[7][oc + q];
     }
     __syncthreads();
   }
-  smooth_any(A.lv[A.n - 1], last, last_steps, true, X + A.off[A.n - 1], B + A.off[A.n - 1]);
+  {
+    const Lv &L = A.lv[A.n - 1];
+    coarse_sweep<FV_LAST, true>(CoarseLv{L.NX, L.NX * L.NY, A.off[A.n - 1]}, last, lds);
+  }
 #pragma unroll 1
   for (int l = A.n - 2; l >= 0; l--) {
     const Lv &L = A.lv[l];
-    double *x = X + A.off[l];
-    const double *ec = X + A.off[l + 1];
-    for (int f = threadIdx.x; f < L.NX * L.NY; f += FV_CT) {
-      const Pt p = load_pt(L.c, true, f);
-      const int iy = f / L.NX, ix = f - iy * L.NX;
-      if (p.live()) x[f] += prolong(L, p, ix, iy, [&](int I, int J) { return ec[J * L.NXc + I]; });
+    const int o = A.off[l], oc = A.off[l + 1];
+    for (int q = threadIdx.x; q < L.NX * L.NY; q += FV_CT) {
+      const int a = o + q, iy = q / L.NX, ix = q - iy * L.NX;
+      const Pt p = {lds[0][a], lds[1][a], lds[2][a], lds[3][a]};
+      if (p.live()) lds[6][a] += prolong(L, p, ix, iy, [&](int I, int J) { return lds[6][oc + J * L.NXc + I]; });
     }
     __syncthreads();
-    smooth_any(L, ch, FV_NU, false, x, B + A.off[l]);
+    coarse_sweep<FV_NU, false>(CoarseLv{L.NX, L.NX * L.NY, o}, ch, lds);
   }
-  for (int q = threadIdx.x; q < np0; q += FV_CT) xout[q] = X[A.off[0] + q];
+  for (int q = threadIdx.x; q < A.lv[0].NX * A.lv[0].NY; q += FV_CT) xout[q] = lds[6][A.off[0] + q];
 }
 
 // The next level's rows.  A coupling between aggregates is the sum of the fine
@@ -345,23 +490,34 @@ __global__ void __launch_bounds__(256) k_coarsen(Lv L, double *__restrict__ ce, 
   const int J = (int)(q / L.NXc), I = (int)(q - (int64_t)J * L.NXc);
   const int i0 = L.fx == 2 ? (I ? 2 * I - 1 : 0) : I, j0 = L.fy == 2 ? (J ? 2 * J - 1 : 0) : J;
   const int ni = agg_count(I, L.fx, L.NX), nj = agg_count(J, L.fy, L.NY);
+  // the aggregate's rows and their neighbours', all loads in flight together
+  Pt blk[4][4];
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int ix = i0 + i - 1, iy = j0 + j - 1;
+      blk[j][i] = load_pt(L.c, ix >= 0 && ix < L.NX && iy >= 0 && iy < L.NY, (int64_t)iy * L.NX + ix);
+    }
   double off[4] = {0.0, 0.0, 0.0, 0.0}, rho = 0.0, delta = 0.0;
   int nlive = 0;
-  for (int j = j0; j < j0 + nj; j++)
-    for (int i = i0; i < i0 + ni; i++) {
-      const Pt p = load_pt(L.c, true, (int64_t)j * L.NX + i);
-      if (!p.live()) continue;
+#pragma unroll
+  for (int j = 0; j < 2; j++)
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      const Pt &p = blk[j + 1][i + 1];
+      if (i >= ni || j >= nj || !p.live()) continue;
       nlive++;
       rho += 1.0 + p.e + p.w + p.s + p.n;
       const double co[4] = {p.e, p.w, p.s, p.n};
 #pragma unroll
       for (int k = 0; k < 4; k++) {
-        const int jx = i + (k == 0) - (k == 1), jy = j + (k == 2) - (k == 3);
+        const int di = (k == 0) - (k == 1), dj = (k == 2) - (k == 3);
+        const int jx = i0 + i + di, jy = j0 + j + dj;
         if (co[k] == 0.0 || jx < 0 || jx >= L.NX || jy < 0 || jy >= L.NY) continue;
         const bool alongx = k < 2;
         const int f = alongx ? L.fx : L.fy, mine = alongx ? ni : nj;
-        const Pt o = load_pt(L.c, true, (int64_t)jy * L.NX + jx);
-        if (!o.live()) {
+        if (!blk[j + 1 + dj][i + 1 + di].live()) {
           delta -= co[k] * (f == 2 ? 2.0 / (mine + 1) : 1.0);
         } else if (agg(jx, L.fx) != I || agg(jy, L.fy) != J) {
           const int his = alongx ? agg_count(agg(jx, L.fx), L.fx, L.NX) : agg_count(agg(jy, L.fy), L.fy, L.NY);
@@ -513,7 +669,7 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
     m->x.push_back(x);
     m->y.push_back(y);
   };
-  m->one_level = m->lo >= DOMINANT;
+  m->one_level = !scale && m->lo >= DOMINANT && nn <= INT32_MAX;  // its kernels take a unit diagonal
   if (m->one_level) {
     push(NX, NY, c, nullptr, nullptr, nullptr);
     m->poly = cheb(m->lo, 2.0 - m->lo, FV_POLY);
@@ -565,26 +721,35 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   return FVM_OK;  // no level fits: no preconditioner
 }
 
-int fvm_precond_apply(fvm_ctx *ctx, const fvm_precond *m, const double *b, double *x) {
+bool fvm_precond_one_level(const fvm_precond *m) { return m->one_level; }
+
+// one iteration with the one-level preconditioner: 3 kernels (O.n_r partials of
+// (rhat, r) and (r, r) come in, FVM_ONE_BLOCKS go out)
+int fvm_precond_one_iteration(fvm_ctx *ctx, const fvm_precond *m, const FvmBcgOne &O) {
   const Lv &F = m->lv[0];
-  if (m->one_level) {
-    k_poly<<<dim3(fvm_blocks(F.NX, FV_PT), fvm_blocks(F.NY, FV_PT)), 1024, 0, ctx->stream>>>(F.NX, F.NY, F.c, m->poly, b, x);
-    FVM_LAUNCH_CHECK(ctx);
-    return FVM_OK;
-  }
+  const dim3 grid(fvm_blocks(F.NX, FV_PT), fvm_blocks(F.NY, FV_PT));
+  k_one_p<<<grid, 1024, 0, ctx->stream>>>(F.NX, F.NY, F.c, m->poly, O);
+  k_one_s<<<grid, 1024, 0, ctx->stream>>>(F.NX, F.NY, F.c, m->poly, O);
+  k_one_x<<<FVM_ONE_BLOCKS, 1024, 0, ctx->stream>>>((int64_t)F.NX * F.NY, (int)(grid.x * grid.y), O);
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
+// sc: the iteration's scalars (a finished iteration's kernels return at once)
+int fvm_precond_apply(fvm_ctx *ctx, const fvm_precond *m, const double *b, double *x, const double *sc) {
   const int fc = m->first_coarse;
   auto rhs = [&](int l) { return l ? m->b[l] : b; };
   auto res = [&](int l) { return l ? m->y[l] : x; };
   for (int l = 0; l < fc; l++) {
     const Lv &L = m->lv[l];
     k_down<<<dim3(fvm_blocks(L.NXc, FV_T / L.fx), fvm_blocks(L.NYc, FV_T / L.fy)), FV_R * FV_R, 0, ctx->stream>>>(
-        L, m->smooth, rhs(l), m->x[l], m->b[l + 1]);
+        L, m->smooth, rhs(l), m->x[l], m->b[l + 1], sc);
   }
-  k_coarse<<<1, FV_CT, 0, ctx->stream>>>(m->coarse, m->smooth, m->last, FV_LAST, rhs(fc), res(fc));
+  k_coarse<<<1, FV_CT, 0, ctx->stream>>>(m->coarse, m->smooth, m->last, rhs(fc), res(fc), sc);
   for (int l = fc - 1; l >= 0; l--) {
     const Lv &L = m->lv[l];
     k_up<<<dim3(fvm_blocks(L.NX, FV_T), fvm_blocks(L.NY, FV_T)), FV_R * FV_R, 0, ctx->stream>>>(
-        L, m->smooth, rhs(l), m->x[l], res(l + 1), res(l));
+        L, m->smooth, rhs(l), m->x[l], res(l + 1), res(l), sc);
   }
   FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;

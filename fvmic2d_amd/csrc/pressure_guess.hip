@@ -10,7 +10,9 @@
 // that does not converge, the solve starts again with Jacobi alone.  Dot products reduce in a fixed order (per-block trees,
 // then the same ordered sum in every block of the next kernel), so the
 // iteration is bitwise reproducible.
-#include "fvm_internal.h"
+#include <utility>
+
+#include "bicgstab.h"
 
 namespace {
 
@@ -106,14 +108,13 @@ __global__ void __launch_bounds__(256) k_pg_apply(PGrid g, const double *__restr
 // reproducible.  The stencil coefficients are tabulated once.
 #define BCG_BS 256
 
-enum { S_RHO = 0, S_RHO_OLD, S_ALPHA, S_OMEGA, S_RR };
-
 struct Coef {
   const double *d, *r, *l, *dn, *up;
 };
 struct BcgVecs {
   double *b, *dinv, *x, *r, *rh, *p, *v, *s, *t, *y, *z;
-  double *q;                                 // what the preconditioner is applied to
+  double *q;                                 // what the preconditioner is applied to, or the other p
+  double *v2;                                // the other v
   double *cd, *cr, *cl, *cdn, *cup;          // stencil coefficients
   double *prv, *pts, *ptt, *prho, *prr;      // per-block partial sums
   double *sc;                                // scalars (S_*)
@@ -175,9 +176,11 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_setup(PGrid g, const double *__r
     V.prr[blockIdx.x] = tot;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    V.sc[S_RHO_OLD] = 1.0;
-    V.sc[S_ALPHA] = 1.0;
-    V.sc[S_OMEGA] = 1.0;
+    V.sc[FVM_S_RHO_OLD] = 1.0;
+    V.sc[FVM_S_ALPHA] = 1.0;
+    V.sc[FVM_S_OMEGA] = 1.0;
+    V.sc[FVM_S_ITS] = 0.0;
+    V.sc[FVM_S_DONE] = 0.0;
   }
 }
 
@@ -204,31 +207,39 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_setup_sys(int64_t n, const doubl
     V.prr[blockIdx.x] = tot;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    V.sc[S_RHO_OLD] = 1.0;
-    V.sc[S_ALPHA] = 1.0;
-    V.sc[S_OMEGA] = 1.0;
+    V.sc[FVM_S_RHO_OLD] = 1.0;
+    V.sc[FVM_S_ALPHA] = 1.0;
+    V.sc[FVM_S_OMEGA] = 1.0;
+    V.sc[FVM_S_ITS] = 0.0;
+    V.sc[FVM_S_DONE] = 0.0;
   }
 }
 
 // rho = (rhat, r); beta; p = r + beta (p - omega v); y = Dinv p
-__global__ void __launch_bounds__(BCG_BS) k_bcg_p(int64_t n, int nblk, int first, BcgVecs V) {
-  const double rho = partial_total(V.prho, nblk);
-  const double omega = V.sc[S_OMEGA];
-  // after an exact solve (r = 0) rho_old and omega are 0: restart with
-  // beta = 0 instead of forming 0/0, so x stays the solution
-  const double rho_old = V.sc[S_RHO_OLD];
-  const double beta = (first || rho_old == 0.0 || omega == 0.0) ? 0.0 : (rho / rho_old) * (V.sc[S_ALPHA] / omega);
+__global__ void __launch_bounds__(BCG_BS) k_bcg_p(int64_t n, int nblk, int first, double rtol, BcgVecs V) {
+  const double rho = partial_total(V.prho, nblk), rr = partial_total(V.prr, nblk);
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  const double bb = first ? rr : V.sc[FVM_S_BB];
+  if (fvm_bcg_done(rr, bb, rtol)) {
+    if (lead) V.sc[FVM_S_DONE] = 1.0, V.sc[FVM_S_RR] = rr, V.sc[FVM_S_BB] = bb;
+    return;
+  }
+  const double omega = V.sc[FVM_S_OMEGA], beta = fvm_bcg_beta(first, rho, V.sc);
   const int64_t i = (int64_t)blockIdx.x * BCG_BS + threadIdx.x;
   if (i < n) {
     const double pi = V.r[i] + beta * (V.p[i] - omega * V.v[i]);
     V.p[i] = pi;
     V.y[i] = V.dinv[i] * pi;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) V.sc[S_RHO] = rho;
+  if (lead) {
+    V.sc[FVM_S_RHO] = rho, V.sc[FVM_S_BB] = bb, V.sc[FVM_S_RR] = rr, V.sc[FVM_S_DONE] = 0.0;
+    V.sc[FVM_S_ITS] = first ? 1.0 : V.sc[FVM_S_ITS] + 1.0;
+  }
 }
 
 // v = A y; partials of (rhat, v)
 __global__ void __launch_bounds__(BCG_BS) k_bcg_v(PGrid g, Coef c, BcgVecs V) {
+  if (V.sc[FVM_S_DONE] != 0.0) return;
   const int64_t n = (int64_t)g.NX * g.NY;
   const int64_t i = (int64_t)blockIdx.x * BCG_BS + threadIdx.x;
   double d = 0.0;
@@ -243,8 +254,9 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_v(PGrid g, Coef c, BcgVecs V) {
 
 // alpha = rho / (rhat, v); x += alpha y; s = r - alpha v; z = Dinv s
 __global__ void __launch_bounds__(BCG_BS) k_bcg_s(int64_t n, int nblk, BcgVecs V) {
+  if (V.sc[FVM_S_DONE] != 0.0) return;
   const double rv = partial_total(V.prv, nblk);
-  const double alpha = rv != 0.0 ? V.sc[S_RHO] / rv : 0.0;
+  const double alpha = rv != 0.0 ? V.sc[FVM_S_RHO] / rv : 0.0;
   const int64_t i = (int64_t)blockIdx.x * BCG_BS + threadIdx.x;
   if (i < n) {
     V.x[i] = V.x[i] + alpha * V.y[i];
@@ -252,11 +264,12 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_s(int64_t n, int nblk, BcgVecs V
     V.s[i] = si;
     V.z[i] = V.dinv[i] * si;
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) V.sc[S_ALPHA] = alpha;
+  if (blockIdx.x == 0 && threadIdx.x == 0) V.sc[FVM_S_ALPHA] = alpha;
 }
 
 // t = A z; partials of (t, s) and (t, t)
 __global__ void __launch_bounds__(BCG_BS) k_bcg_t(PGrid g, Coef c, BcgVecs V) {
+  if (V.sc[FVM_S_DONE] != 0.0) return;
   const int64_t n = (int64_t)g.NX * g.NY;
   const int64_t i = (int64_t)blockIdx.x * BCG_BS + threadIdx.x;
   double ts = 0.0, tt = 0.0;
@@ -276,6 +289,7 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_t(PGrid g, Coef c, BcgVecs V) {
 
 // omega = (t, s) / (t, t); x += omega z; r = s - omega t; partials of (rhat, r), (r, r)
 __global__ void __launch_bounds__(BCG_BS) k_bcg_x(int64_t n, int nblk, BcgVecs V) {
+  if (V.sc[FVM_S_DONE] != 0.0) return;
   const double ts = partial_total(V.pts, nblk);
   const double tt = partial_total(V.ptt, nblk);
   const double omega = tt != 0.0 ? ts / tt : 0.0;
@@ -295,14 +309,16 @@ __global__ void __launch_bounds__(BCG_BS) k_bcg_x(int64_t n, int nblk, BcgVecs V
     V.prr[blockIdx.x] = b;
   }
   if (blockIdx.x == 0 && threadIdx.x == 0) {
-    V.sc[S_OMEGA] = omega;
-    V.sc[S_RHO_OLD] = V.sc[S_RHO];
+    V.sc[FVM_S_OMEGA] = omega;
+    V.sc[FVM_S_RHO_OLD] = V.sc[FVM_S_RHO];
   }
 }
 
+// (r, r) of the last iteration, unless one has found it small enough already
 __global__ void __launch_bounds__(BCG_BS) k_bcg_norm(int nblk, BcgVecs V) {
+  if (V.sc[FVM_S_DONE] != 0.0) return;
   const double rr = partial_total(V.prr, nblk);
-  if (threadIdx.x == 0) V.sc[S_RR] = rr;
+  if (threadIdx.x == 0) V.sc[FVM_S_RR] = rr;
 }
 
 __global__ void __launch_bounds__(256) k_store_p(int64_t n, const double *__restrict__ p, double *__restrict__ S,
@@ -334,79 +350,79 @@ extern "C" int fvm_pressure_guess_apply(fvm_ctx *ctx, const fvm_grid *g, const d
   return FVM_OK;
 }
 
-// workspace: 12 vectors, 5 coefficient arrays, 5 partial arrays, scalars
+// workspace: 13 vectors, 5 coefficient arrays, 5 partial arrays, scalars
 static int bcg_vecs(fvm_ctx *ctx, int64_t n, BcgVecs *V, int *nblk_out) {
   const int64_t np = (n + 63) / 64 * 64;
   const int nblk = (int)((n + BCG_BS - 1) / BCG_BS);
-  const int64_t npart = ((int64_t)nblk + 63) / 64 * 64;
-  FVM_TRY(fvm_ws(ctx, ctx->scratch, (17 * np + 5 * npart + 64) * sizeof(double)));
+  const int64_t npart = ((int64_t)(nblk > FVM_ONE_BLOCKS ? nblk : FVM_ONE_BLOCKS) + 63) / 64 * 64;
+  FVM_TRY(fvm_ws(ctx, ctx->scratch, (18 * np + 5 * npart + 64) * sizeof(double)));
   double *w = (double *)ctx->scratch.ptr;
   double **vecs[] = {&V->b, &V->dinv, &V->x, &V->r, &V->rh, &V->p, &V->v, &V->s, &V->t, &V->y, &V->z,
-                     &V->cd, &V->cr, &V->cl, &V->cdn, &V->cup, &V->q};
-  for (int k = 0; k < 17; k++) *vecs[k] = w + (int64_t)k * np;
-  double *pw = w + 17 * np;
+                     &V->cd, &V->cr, &V->cl, &V->cdn, &V->cup, &V->q, &V->v2};
+  for (int k = 0; k < 18; k++) *vecs[k] = w + (int64_t)k * np;
+  double *pw = w + 18 * np;
   V->prv = pw, V->pts = pw + npart, V->ptt = pw + 2 * npart, V->prho = pw + 3 * npart, V->prr = pw + 4 * npart;
   V->sc = pw + 5 * npart;
   *nblk_out = nblk;
   return FVM_OK;
 }
 
-// BiCGStab from the state that `start` sets up (x = 0).  With a preconditioner
-// the host reads ||r|| after every iteration (5 to 30 are needed); without one,
-// or where that has not converged after PRECOND_MAXIT iterations, Jacobi's
-// (hundreds) are checked every eight.  it_out: of the run that gave x.
+// BiCGStab from the state that `start` sets up (x = 0).  The kernels decide
+// convergence themselves; the host enqueues a few iterations (5 to 30 are needed
+// with a preconditioner, hundreds without) between two looks, each of which costs
+// about 25 us of an idle GPU.  Without a preconditioner, or where that has not
+// converged after PRECOND_MAXIT iterations, Jacobi takes its place.  it_out: of the
+// run that gave x.
 #define PRECOND_MAXIT 60
 template <class Start>
 static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs &V, int64_t n, int nblk,
                     const fvm_precond *m, double rtol, int32_t maxit, int32_t *it_out, double *rel_out, Start start) {
   const unsigned nb = (unsigned)nblk;
   double *host = (double *)ctx->pinned.ptr;
-  auto rnorm = [&](double *out) -> int {
-    k_bcg_norm<<<1, BCG_BS, 0, ctx->stream>>>(nblk, V);
-    FVM_LAUNCH_CHECK(ctx);
-    FVM_HIP(ctx, hipMemcpyAsync(host, V.sc + S_RR, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *out = sqrt(*host);
-    return FVM_OK;
-  };
-  auto run = [&](const fvm_precond *pre, int32_t most, int every) -> int {
+  auto run = [&](const fvm_precond *pre, int32_t most, int ahead) -> int {
     FVM_TRY(start());
-    double bnorm = 0.0;
-    FVM_TRY(rnorm(&bnorm));
-    *it_out = 0;
-    *rel_out = 0.0;
-    if (!(bnorm > 0.0)) return FVM_OK;
+    const bool one = pre && fvm_precond_one_level(pre);
     BcgVecs Vp = V, Vs = V;  // where the scaled p and s go
     if (pre) Vp.y = V.q, Vs.z = V.q;
-    double rel = 1.0;
+    double *pv[2] = {V.p, V.q}, *vv[2] = {V.v, V.v2};  // the one-level iteration's
+    int n_r = nblk;          // partials of (r, r)
     int it = 0;
     for (;;) {
-      if (it && (it % every == 0 || it == most)) {
-        double rn = 0.0;
-        FVM_TRY(rnorm(&rn));
-        rel = rn / bnorm;
+      for (int k = 0; k < ahead && it < most; k++, it++) {
+        const int first = it == 0 ? 1 : 0;
+        if (one) {
+          FvmBcgOne O{V.x, V.r, V.s, V.t, V.y, V.z, pv[1], vv[1], V.rh, pv[0], vv[0],
+                      V.prv, V.pts, V.ptt, V.prho, V.prr, V.sc, n_r, first, rtol};
+          FVM_TRY(fvm_precond_one_iteration(ctx, pre, O));
+          n_r = FVM_ONE_BLOCKS;
+          std::swap(pv[0], pv[1]);
+          std::swap(vv[0], vv[1]);
+          continue;
+        }
+        k_bcg_p<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, first, rtol, Vp);
+        if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.y, V.sc));
+        k_bcg_v<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
+        k_bcg_s<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, Vs);
+        if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.z, V.sc));
+        k_bcg_t<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
+        k_bcg_x<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, V);
       }
-      if (it % every == 0 || it == most)
-        if (!(rel > rtol) || it == most) break;  // also stops on NaN
-      k_bcg_p<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, it == 0 ? 1 : 0, Vp);
-      if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.y));
-      k_bcg_v<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
-      k_bcg_s<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, Vs);
-      if (pre) FVM_TRY(fvm_precond_apply(ctx, pre, V.q, V.z));
-      k_bcg_t<<<nb, BCG_BS, 0, ctx->stream>>>(pg, c, V);
-      k_bcg_x<<<nb, BCG_BS, 0, ctx->stream>>>(n, nblk, V);
+      k_bcg_norm<<<1, BCG_BS, 0, ctx->stream>>>(n_r, V);
       FVM_LAUNCH_CHECK(ctx);
-      it++;
+      FVM_HIP(ctx, hipMemcpyAsync(host, V.sc, 8 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+      FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+      const double bnorm = sqrt(host[FVM_S_BB]);
+      *it_out = (int32_t)host[FVM_S_ITS];
+      *rel_out = bnorm > 0.0 ? sqrt(host[FVM_S_RR]) / bnorm : 0.0;
+      if (!(*rel_out > rtol) || it >= most) return FVM_OK;  // also stops on NaN
+      ahead = pre ? 2 : ahead;
     }
-    *it_out = it;
-    *rel_out = rel;
-    return FVM_OK;
   };
   if (m) {
-    FVM_TRY(run(m, maxit < PRECOND_MAXIT ? maxit : PRECOND_MAXIT, 1));
+    FVM_TRY(run(m, maxit < PRECOND_MAXIT ? maxit : PRECOND_MAXIT, 4));
     if (*rel_out <= rtol) return FVM_OK;
   }
-  return run(nullptr, maxit, 8);
+  return run(nullptr, maxit, 16);
 }
 
 extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const double *rho, double gy, double gx,
