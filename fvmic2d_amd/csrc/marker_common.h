@@ -131,9 +131,19 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     const bool vcol = PER || vyX >= 0;
     const int vyc = PER && vyX + 1 >= NX ? vyX + 1 - NX : vyX + 1;  // column of vyX + 1
     const int vyl = (PER && vyc == 0) ? NX - 1 : -1;                // offset of column vyX
-    const double *q0 = vy + (int64_t)vyY * NX + vyc, *q1 = q0 + NX;
-    const double vyur = q0[0], vylr = q1[0];
-    const double vy0 = (vcol ? q0 + vyl : q0)[0], vy1 = (vcol ? q1 + vyl : q1)[0];
+    double vyur, vylr, vy0, vy1;
+    if (PER) {
+      const double *q0 = vy + (int64_t)vyY * NX + vyc, *q1 = q0 + NX;
+      vyur = q0[0], vylr = q1[0];
+      vy0 = q0[vyl], vy1 = q1[vyl];
+    } else {
+      // both columns of a row in one load: vyX and vyX + 1, or 0 and 1 at the
+      // ghost column (where the left value is selected away)
+      const double *q0 = vy + (int64_t)vyY * NX + (vcol ? vyX : 0);
+      const fvm_pair a = load_pair(q0), b = load_pair(q0 + NX);
+      vyur = vcol ? a.b : a.a, vylr = vcol ? b.b : b.a;
+      vy0 = a.a, vy1 = b.a;
+    }
     double vyul, vyll;
     if (!PER && vyX == -1 && bv.mechBCLeft.type[1] == 0) {
       vyul = 2.0 * bv.mechBCLeft.value[1] - vyur;
@@ -251,6 +261,7 @@ __device__ __forceinline__ void rotate_eii_marker(int64_t m, int ncx, int NY,
 }
 
 // ---- A7: subgridTemperatureChanges pass 2 (subgridTemperatureChanges.c:89-103) ---
+template <bool PER>
 __device__ __forceinline__ void subgrid_t2_marker(int64_t m, const DGrid &g,
     const double *__restrict__ MX,
     const double *__restrict__ MY,
@@ -263,15 +274,13 @@ __device__ __forceinline__ void subgrid_t2_marker(int64_t m, const DGrid &g,
     double dt) {
   const int cellX = cX[m], cellY = cY[m];
   if (!cell_ok(cellX, cellY, g.ncx(), g.NY)) return;
-  const int NX = g.NX, NY = g.NY, P = g.per;
   const double dx = g.x[cellX + 1] - g.x[cellX];
   const double dy = g.y[cellY + 1] - g.y[cellY];
   const double mdx = (MX[m] - g.x[cellX]) / dx;
   const double mdy = (MY[m] - g.y[cellY]) / dy;
-  const double dtm = (gat(dT, NX, NY, P, cellY, cellX) * (1.0 - mdy) * (1.0 - mdx) +
-                      gat(dT, NX, NY, P, cellY + 1, cellX) * mdy * (1.0 - mdx) +
-                      gat(dT, NX, NY, P, cellY, cellX + 1) * (1.0 - mdy) * mdx +
-                      gat(dT, NX, NY, P, cellY + 1, cellX + 1) * mdy * mdx) +
+  const Corners q = cell_corners<PER>(dT, g.NX, cellY, cellX);
+  const double dtm = (q.f00 * (1.0 - mdy) * (1.0 - mdx) + q.f10 * mdy * (1.0 - mdx) + q.f01 * (1.0 - mdy) * mdx +
+                      q.f11 * mdy * mdx) +
                      dTsub[m];
   MT[m] = MT[m] + dtm;
   MTdot[m] = dtm / dt;

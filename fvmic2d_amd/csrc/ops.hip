@@ -11,6 +11,19 @@
 
 int fvm_fill(fvm_ctx *ctx, double *a, int64_t n, double v);  // project.hip
 
+// One thread per marker, the kernel built for each way of gathering (fvm_bil_mode).
+#define BIL_LAUNCH(g, kernel, n, args)                                                \
+  switch (fvm_bil_mode(g)) {                                                          \
+    case BIL_PLAIN:                                                                   \
+      kernel<BIL_PLAIN><<<fvm_blocks(n, 256), 256, 0, ctx->stream>>> args;            \
+      break;                                                                          \
+    case BIL_WRAP:                                                                    \
+      kernel<BIL_WRAP><<<fvm_blocks(n, 256), 256, 0, ctx->stream>>> args;             \
+      break;                                                                          \
+    default:                                                                          \
+      kernel<BIL_ANY><<<fvm_blocks(n, 256), 256, 0, ctx->stream>>> args;              \
+  }
+
 // ---- A6: advectMarkersRK (markers.c:1865-2250), body in marker_common.h ----------
 // With LDS the grid coordinates x, y, xc, yc (2 NX + 2 NY + 2 doubles) are staged
 // in LDS once per block, and each block walks `tiles` tiles of 256 markers so
@@ -114,6 +127,7 @@ extern "C" int fvm_advect_markers_rk(fvm_ctx *ctx, fvm_markers *mk, const NodalA
 }
 
 // ---- A7: subgridTemperatureChanges (subgridTemperatureChanges.c:5-124) -------
+template <bool PER>
 __global__ void __launch_bounds__(256) k_subgrid_t2(DGrid g, int32_t n, const double *__restrict__ MX,
                                                     const double *__restrict__ MY, double *__restrict__ MT,
                                                     double *__restrict__ MTdot, const int32_t *__restrict__ cX,
@@ -121,7 +135,7 @@ __global__ void __launch_bounds__(256) k_subgrid_t2(DGrid g, int32_t n, const do
                                                     const double *__restrict__ dTsub, double dt) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= n) return;
-  subgrid_t2_marker(m, g, MX, MY, MT, MTdot, cX, cY, dT, dTsub, dt);
+  subgrid_t2_marker<PER>(m, g, MX, MY, MT, MTdot, cX, cY, dT, dTsub, dt);
 }
 
 // Pass 1 and the dTsub projection of subgridTemperatureChanges; leaves dTsub
@@ -174,8 +188,8 @@ extern "C" int fvm_subgrid_temperature_changes(fvm_ctx *ctx, const double *thisT
   const int32_t n = mk->nMark;
   if (n > 0) {
     FVM_PHASE(ctx, FVM_PHASE_SUBGRID_T2);
-    k_subgrid_t2<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(dgrid(g), n, mk->X, mk->Y, mk->T, mk->Tdot, mk->cellX,
-                                                               mk->cellY, deltaT, dTsub, dt);
+    (g->xperiodic ? k_subgrid_t2<true> : k_subgrid_t2<false>)<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(
+        dgrid(g), n, mk->X, mk->Y, mk->T, mk->Tdot, mk->cellX, mk->cellY, deltaT, dTsub, dt);
     FVM_LAUNCH_CHECK(ctx);
   }
   return FVM_OK;
@@ -196,6 +210,7 @@ int fvm_advect_with_subgrid_t2(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays 
 }
 
 // ---- A8: subgridStressChanges (subgridStressChanges.c:5-318) ------------------
+template <int MODE>
 __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const double *__restrict__ MX,
                                                     const double *__restrict__ MY, const double *__restrict__ eta,
                                                     const double *__restrict__ mu, double *__restrict__ sxx,
@@ -216,7 +231,7 @@ __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const do
   }
   // no xperiodic branch in subgridStressChanges.c: the clamps keep both
   // gathers inside [0, NX-1] on a periodic grid too
-  const int NX = g.NX, NY = g.NY, P = g.per;
+  const int NX = g.NX, NY = g.NY;
   const double X = MX[m], Y = MY[m];
   const double sdm = eta[m] / mu[m];
   double sdif = -dsubgrid * dt / sdm;
@@ -230,11 +245,7 @@ __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const do
   if (cellY > NY - 2) cellY = NY - 2;
   double mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
   double mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  double sxym = 0.0;
-  sxym += (1.0 - mdx) * (1.0 - mdy) * gat(soxy, NX, NY, P, cellY, cellX);
-  sxym += (1.0 - mdx) * mdy * gat(soxy, NX, NY, P, cellY + 1, cellX);
-  sxym += mdx * (1.0 - mdy) * gat(soxy, NX, NY, P, cellY, cellX + 1);
-  sxym += mdx * mdy * gat(soxy, NX, NY, P, cellY + 1, cellX + 1);
+  const double sxym = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(soxy);
   double sxy0 = sxy[m];
   double dsxym = sxym - sxy0;
   dsxym *= sdif;
@@ -251,12 +262,13 @@ __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const do
   else if (cellX > NX - 2) cellX = NX - 2;
   mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
   mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
-  const double sxxm = bil_acc(soxx, NX, NY, P, cellY, cellX, mdx, mdy);
+  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
+  const double sxxm = at(soxx);
   const double sxx0 = sxx[m];
   double dsxxm = sxxm - sxx0;
   dsxxm *= sdif;
   sxx[m] = sxx0 + dsxxm;
-  const double syym = bil_acc(soyy, NX, NY, P, cellY, cellX, mdx, mdy);
+  const double syym = at(soyy);
   const double syy0 = syy[m];
   double dsyym = syym - syy0;
   dsyym *= sdif;
@@ -278,9 +290,9 @@ extern "C" int fvm_subgrid_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const
   if (n > 0) {
     {
       FVM_PHASE(ctx, FVM_PHASE_SUBGRID_S1);
-      k_subgrid_s1<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(dgrid(g), n, mk->X, mk->Y, mk->eta, mk->mu, mk->sxx,
-                                                                 mk->syy, mk->sxy, mk->cellX, mk->cellY, nf->soxx,
-                                                                 nf->soyy, nf->soxy, dt, dsubgrid, dxy, dxx, dyy);
+      BIL_LAUNCH(g, k_subgrid_s1, n,
+                 (dgrid(g), n, mk->X, mk->Y, mk->eta, mk->mu, mk->sxx, mk->syy, mk->sxy, mk->cellX, mk->cellY,
+                  nf->soxx, nf->soyy, nf->soxy, dt, dsubgrid, dxy, dxx, dyy));
       FVM_LAUNCH_CHECK(ctx);
     }
   }
@@ -307,6 +319,7 @@ extern "C" int fvm_subgrid_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const
 }
 
 // ---- A9: updateMarkerStress (updateMarkerStress.c:5-163) ----------------------
+template <int MODE>
 __global__ void __launch_bounds__(256) k_update_stress(DGrid g, int32_t n, const double *__restrict__ MX,
                                                        const double *__restrict__ MY, double *__restrict__ sxx,
                                                        double *__restrict__ syy, double *__restrict__ sxy,
@@ -330,8 +343,9 @@ __global__ void __launch_bounds__(256) k_update_stress(DGrid g, int32_t n, const
   else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
   double mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
   double mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
-  const double mdsxx = bil_acc(dsxx, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mdsyy = bil_acc(dsyy, NX, NY, P, cellY, cellX, mdx, mdy);
+  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
+  const double mdsxx = at(dsxx);
+  const double mdsyy = at(dsyy);
   sxx[m] = sxx[m] + mdsxx;
   syy[m] = syy[m] + mdsyy;
   cellX = c0x;
@@ -342,7 +356,7 @@ __global__ void __launch_bounds__(256) k_update_stress(DGrid g, int32_t n, const
   else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
   mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
   mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  const double mdsxy = bil_acc(dsxy, NX, NY, P, cellY, cellX, mdx, mdy);
+  const double mdsxy = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(dsxy);
   sxy[m] = sxy[m] + mdsxy;
 }
 
@@ -354,9 +368,9 @@ extern "C" int fvm_update_marker_stress(fvm_ctx *ctx, const fvm_grid *g, const N
   if (mk->nMark == 0) return FVM_OK;
   {
     FVM_PHASE(ctx, FVM_PHASE_MARKER_UPDATE);
-    k_update_stress<<<fvm_blocks(mk->nMark, 256), 256, 0, ctx->stream>>>(dgrid(g), mk->nMark, mk->X, mk->Y, mk->sxx,
-                                                                           mk->syy, mk->sxy, mk->cellX, mk->cellY,
-                                                                           nf->dsxx, nf->dsyy, nf->dsxy);
+    BIL_LAUNCH(g, k_update_stress, mk->nMark,
+               (dgrid(g), mk->nMark, mk->X, mk->Y, mk->sxx, mk->syy, mk->sxy, mk->cellX, mk->cellY, nf->dsxx,
+                nf->dsyy, nf->dsxy));
     FVM_LAUNCH_CHECK(ctx);
   }
   return FVM_OK;
@@ -366,6 +380,7 @@ extern "C" int fvm_update_marker_stress(fvm_ctx *ctx, const fvm_grid *g, const N
 struct StrainIn {
   const double *dsxx, *dsyy, *dsxy, *soxx, *soyy, *soxy, *exx, *eyy, *exy, *wxy, *p;
 };
+template <int MODE>
 __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, const double *__restrict__ MX,
                                                          const double *__restrict__ MY, const double *__restrict__ eta,
                                                          const double *__restrict__ mu, double *__restrict__ Mp,
@@ -391,12 +406,13 @@ __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, con
   else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
   double mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
   double mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
-  Mp[m] = bil_acc(F.p, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mexx = bil_acc(F.exx, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double msxx = bil_acc(F.soxx, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double msyy = bil_acc(F.soyy, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mdsxx = bil_acc(F.dsxx, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mdsyy = bil_acc(F.dsyy, NX, NY, P, cellY, cellX, mdx, mdy);
+  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
+  Mp[m] = at(F.p);
+  const double mexx = at(F.exx);
+  const double msxx = at(F.soxx);
+  const double msyy = at(F.soyy);
+  const double mdsxx = at(F.dsxx);
+  const double mdsyy = at(F.dsyy);
   cellX = c0x;
   cellY = c0y;
   if (cellY < 0) cellY = 0;
@@ -405,10 +421,11 @@ __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, con
   else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
   mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
   mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  Mwxy[m] = bil_acc(F.wxy, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mexy = bil_acc(F.exy, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double msxy = bil_acc(F.soxy, NX, NY, P, cellY, cellX, mdx, mdy);
-  const double mdsxy = bil_acc(F.dsxy, NX, NY, P, cellY, cellX, mdx, mdy);
+  const Bilinear<MODE> atb(g, cellY, cellX, mdx, mdy);
+  Mwxy[m] = atb(F.wxy);
+  const double mexy = atb(F.exy);
+  const double msxy = atb(F.soxy);
+  const double mdsxy = atb(F.dsxy);
   const double em = eta[m], um = mu[m];
   const double t11 = msxx / 2.0 / em + mdsxx / 2.0 / dt / um;
   const double t22 = msyy / 2.0 / em + mdsyy / 2.0 / dt / um;
@@ -441,9 +458,9 @@ extern "C" int fvm_update_marker_strain_pressure(fvm_ctx *ctx, const fvm_grid *g
   if (mk->nMark > 0) {
     {
       FVM_PHASE(ctx, FVM_PHASE_MARKER_UPDATE);
-      k_strain_pressure<<<fvm_blocks(mk->nMark, 256), 256, 0, ctx->stream>>>(
-          dgrid(g), mk->nMark, mk->X, mk->Y, mk->eta, mk->mu, mk->p, mk->wxy, mk->exx, mk->eyy, mk->exy,
-          mk->strainRateResidual, mk->cellX, mk->cellY, F, dt, flags);
+      BIL_LAUNCH(g, k_strain_pressure, mk->nMark,
+                 (dgrid(g), mk->nMark, mk->X, mk->Y, mk->eta, mk->mu, mk->p, mk->wxy, mk->exx, mk->eyy, mk->exy,
+                  mk->strainRateResidual, mk->cellX, mk->cellY, F, dt, flags));
       FVM_LAUNCH_CHECK(ctx);
     }
   }
@@ -694,6 +711,7 @@ extern "C" int fvm_update_global_strain_rate_residual(fvm_ctx *ctx, const fvm_gr
 }
 
 // ---- A13: projectNodalFieldToMarkersS (markers.c:1670-1706) --------------------
+template <bool PER>
 __global__ void k_nodal_to_markers(DGrid g, int32_t n, const double *__restrict__ MX, const double *__restrict__ MY,
                                    const int32_t *__restrict__ cX, const int32_t *__restrict__ cY,
                                    const double *__restrict__ f, double *__restrict__ out) {
@@ -701,13 +719,10 @@ __global__ void k_nodal_to_markers(DGrid g, int32_t n, const double *__restrict_
   if (m >= n) return;
   const int cellX = cX[m], cellY = cY[m];
   if (!cell_ok(cellX, cellY, g.ncx(), g.NY)) return;
-  const int NX = g.NX, NY = g.NY, P = g.per;
   const double mdx = (MX[m] - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
   const double mdy = (MY[m] - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  out[m] = gat(f, NX, NY, P, cellY, cellX) * (1 - mdx) * (1 - mdy) +
-           gat(f, NX, NY, P, cellY + 1, cellX) * (1 - mdx) * mdy +
-           gat(f, NX, NY, P, cellY, cellX + 1) * (mdx) * (1 - mdy) +
-           gat(f, NX, NY, P, cellY + 1, cellX + 1) * mdx * mdy;
+  const Corners q = cell_corners<PER>(f, g.NX, cellY, cellX);
+  out[m] = q.f00 * (1 - mdx) * (1 - mdy) + q.f10 * (1 - mdx) * mdy + q.f01 * (mdx) * (1 - mdy) + q.f11 * mdx * mdy;
 }
 
 extern "C" int fvm_project_nodal_field_to_markers(fvm_ctx *ctx, const fvm_grid *g, const double *nodalField,
@@ -717,9 +732,9 @@ extern "C" int fvm_project_nodal_field_to_markers(fvm_ctx *ctx, const fvm_grid *
   if (mk->nMark == 0) return FVM_OK;
   {
     FVM_PHASE(ctx, FVM_PHASE_MARKER_UPDATE);
-    k_nodal_to_markers<<<fvm_blocks(mk->nMark, 256), 256, 0, ctx->stream>>>(dgrid(g), mk->nMark, mk->X, mk->Y,
-                                                                              mk->cellX, mk->cellY, nodalField,
-                                                                              markerField);
+    (g->xperiodic ? k_nodal_to_markers<true> : k_nodal_to_markers<false>)<<<fvm_blocks(mk->nMark, 256), 256, 0,
+                                                                            ctx->stream>>>(
+        dgrid(g), mk->nMark, mk->X, mk->Y, mk->cellX, mk->cellY, nodalField, markerField);
     FVM_LAUNCH_CHECK(ctx);
   }
   return FVM_OK;
