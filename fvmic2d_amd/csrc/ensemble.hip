@@ -23,7 +23,6 @@
 // location 0.86 -> 0.68 ms, advection 3.17 -> 3.04 ms on the 64-instance step).
 #define ENS_MTILES 4
 
-int fvm_fill(fvm_ctx *ctx, double *a, int64_t n, double v);
 
 struct DensTab {
   double rho[FVM_MAXMAT], alpha[FVM_MAXMAT];
@@ -310,7 +309,7 @@ __device__ __forceinline__ void ens_advect_block(const InstDev &I, int64_t lb, c
   const int64_t m = lb * (int64_t)blockDim.x + threadIdx.x;
   if (m >= I.nMark) return;
   advect_marker<false>(m, gl, I.X, I.Y, I.VX, I.VY, I.wxy, I.cellX, I.cellY, I.vx, I.vy, I.wxyn, I.bv, I.dt, I.T,
-                       I.Tdot, deltaT + I.node_off, dTsub + I.mark_off, I.dt);
+                       I.Tdot, deltaT + I.node_off, dTsub + I.mark_off, I.dt, NoTail());
   // the rotation fused behind the RK4 stages: the batched launch keeps one kernel per phase
   rotate_eii_marker(m, I.g.ncx(), I.g.NY, I.cellX, I.cellY, I.wxy, I.sxx, I.syy, I.sxy, I.exx, I.eyy, I.exy, I.Eii,
                     I.dt, I.jaumann);

@@ -553,6 +553,17 @@ struct ProfScope {
 int fvm_subgrid_t_pass1(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, const NodalArrays *nf,
                         fvm_markers *mk, const Materials *mat, double dt, double dsubgrid, double **dTsub_out,
                         double **deltaT_out);
+// Pieces of the visco-elasto-plastic step (ops.hip): enqueued, no host wait.
+int fvm_subgrid_t_into(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk,
+                       const Materials *mat, double dt, double dsubgrid, double *dTsub, double *deltaT);
+int fvm_launch_strain_pressure(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk, double dt,
+                               int32_t *flag, double dsubgrid, double *dxx, double *dyy, double *dxy);
+int fvm_enqueue_strain_rate_residual(fvm_ctx *ctx, const fvm_grid *g, const fvm_markers *mk, double *srr, double *out);
+int fvm_project_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, const fvm_markers *mk,
+                               const double *dxx, const double *dyy, const double *dxy);
+int fvm_advect_with_stress(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays *nf, const fvm_grid *g,
+                           const BoundaryValues *bv, double dt, const double *deltaT, const double *dTsub,
+                           const double *dxx, const double *dyy, const double *dxy);
 int fvm_advect_with_subgrid_t2(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays *nf, const fvm_grid *g,
                                const BoundaryValues *bv, double dt, const double *deltaT, const double *dTsub,
                                double dt_thermal);

@@ -12,7 +12,12 @@
 // not clamped (:1965-1971), node columns wrap, the left-wall ghost rule is off
 // (:2014-2023) and the new X is wrapped into [0, LX] (:2225-2231).  The grid
 // coordinates are then read at indices -1 .. NX+1 (set by makePeriodic).
-template <bool PER>
+// tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's stages are done, with
+// its old position and cell and its new spin (NoTail: nothing).
+struct NoTail {
+  __device__ __forceinline__ void operator()(int64_t, const DGrid &, double, double, int, int, double) const {}
+};
+template <bool PER, class Tail>
 __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MX,
     double *__restrict__ MY,
@@ -30,7 +35,7 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MTdot,
     const double *__restrict__ dTn,
     const double *__restrict__ dTsub,
-    double dt_thermal) {
+    double dt_thermal, const Tail &tail) {
   const int c0x = cellXa[m], c0y = cellYa[m];
   if (!cell_ok(c0x, c0y, g.ncx(), g.NY)) return;
   const int NX = g.NX, NY = g.NY;
@@ -216,12 +221,35 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
   }
   MX[m] = Xn;
   MY[m] = Y0 + dt * VY;
+  tail(m, g, X0, Y0, c0x, c0y, wm);
 }
 
 // ---- A6, second pass: the stress rotation by the marker spin and the strain
 // invariant update (markers.c:2141-2164, 2223), after advect_marker has stored the spin
 // wxy = (k1 + 2 k2 + 2 k3 + k4) / 6.  A pass of its own: the RK4 pass then holds
 // fewer live registers and hides more of its gather latency, and this one streams.
+__device__ __forceinline__ void rotate_stress(double &sxx, double &syy, double &sxy, double wm, double dt,
+                                              int jaumann) {
+  const double msxx0 = sxx, msyy0 = syy, msxy0 = sxy;
+  if (jaumann) {
+    const double wxy1 = wm * dt;
+    sxx = msxx0 + 2.0 * msxy0 * -wxy1;
+    syy = msyy0 + 2.0 * msxy0 * wxy1;
+    sxy = msxy0 + (msxx0 - msyy0) * wxy1;
+  } else {
+    const double thetaz = -wm * dt;
+    // one shared range reduction per angle (sincos); the values are those of sin and cos
+    double c, s, s2, c2;
+    sincos(thetaz, &s, &c);
+    sincos(2.0 * thetaz, &s2, &c2);
+    // pow(v, 2.0) of markers.c:2162-2163: gcc -O3 (makefile:14) folds it to v*v,
+    // which is what the reference binary executes
+    sxx = msxx0 * (c * c) + msyy0 * (s * s) - msxy0 * s2;
+    syy = msxx0 * (s * s) + msyy0 * (c * c) + msxy0 * s2;
+    sxy = 0.5 * (msxx0 - msyy0) * s2 + msxy0 * c2;
+  }
+}
+
 // ncx: basic cells along x (NX - 1, or NX on a periodic grid)
 __device__ __forceinline__ void rotate_eii_marker(int64_t m, int ncx, int NY,
     const int32_t *__restrict__ cellXa,
@@ -237,28 +265,80 @@ __device__ __forceinline__ void rotate_eii_marker(int64_t m, int ncx, int NY,
     double dt,
     int jaumann) {
   if (!cell_ok(cellXa[m], cellYa[m], ncx, NY)) return;
-  const double wm = Mwxy[m];
-  const double msxx0 = sxx[m], msyy0 = syy[m], msxy0 = sxy[m];
-  if (jaumann) {
-    const double wxy1 = wm * dt;
-    sxx[m] = msxx0 + 2.0 * msxy0 * -wxy1;
-    syy[m] = msyy0 + 2.0 * msxy0 * wxy1;
-    sxy[m] = msxy0 + (msxx0 - msyy0) * wxy1;
-  } else {
-    const double thetaz = -wm * dt;
-    // one shared range reduction per angle (sincos); the values are those of sin and cos
-    double c, s, s2, c2;
-    sincos(thetaz, &s, &c);
-    sincos(2.0 * thetaz, &s2, &c2);
-    // pow(v, 2.0) of markers.c:2162-2163: gcc -O3 (makefile:14) folds it to v*v,
-    // which is what the reference binary executes
-    sxx[m] = msxx0 * (c * c) + msyy0 * (s * s) - msxy0 * s2;
-    syy[m] = msxx0 * (s * s) + msyy0 * (c * c) + msxy0 * s2;
-    sxy[m] = 0.5 * (msxx0 - msyy0) * s2 + msxy0 * c2;
-  }
+  double s11 = sxx[m], s22 = syy[m], s12 = sxy[m];
+  rotate_stress(s11, s22, s12, Mwxy[m], dt, jaumann);
+  sxx[m] = s11;
+  syy[m] = s22;
+  sxy[m] = s12;
   const double e11 = exx[m], e22 = eyy[m], e12 = exy[m];
   Eii[m] = Eii[m] + dt * sqrt(0.5 * (e11 * e11 + e22 * e22) + e12 * e12);
 }
+
+// ---- A9: updateMarkerStress (updateMarkerStress.c:5-163): a marker's increments ----
+template <int MODE>
+__device__ __forceinline__ void stress_increment(const DGrid &g, double X, double Y, int c0x, int c0y,
+                                                 const double *__restrict__ dsxx, const double *__restrict__ dsyy,
+                                                 const double *__restrict__ dsxy, double &mdsxx, double &mdsyy,
+                                                 double &mdsxy) {
+  const int NX = g.NX, NY = g.NY, P = g.per;
+  int cellX = c0x, cellY = c0y;
+  // periodic: the centre cell may step to NX and is then clamped to NX-1
+  // (cellXMax NX, then NX-1); node column NX is column 0
+  if (cellX < (P ? NX : NX - 2) && X >= g.xc[cellX + 1]) cellX++;
+  if (cellY < NY - 1 && Y >= g.yc[cellY + 1]) cellY++;
+  if (cellY < 1) cellY = 1;
+  else if (cellY > NY - 2) cellY = NY - 2;
+  if (cellX < 1) cellX = 1;
+  else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
+  double mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
+  double mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
+  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
+  mdsxx = at(dsxx);
+  mdsyy = at(dsyy);
+  cellX = c0x;
+  cellY = c0y;
+  if (cellY < 0) cellY = 0;
+  else if (cellY > NY - 2) cellY = NY - 2;
+  if (cellX < 0) cellX = 0;
+  else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
+  mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
+  mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
+  mdsxy = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(dsxy);
+}
+
+// The stresses of a whole visco-elasto-plastic step behind a marker's advection:
+// subgridStressChanges' own change (dxx, dyy, dxy per marker; null: none),
+// updateMarkerStress's increment at the old position, the rotation by the new spin
+// and the strain invariant, so that the stresses are read and written once.
+template <int MODE>
+struct StressTail {
+  double *sxx, *syy, *sxy, *Eii;
+  const double *exx, *eyy, *exy;           // marker strain rates
+  const double *dsxx, *dsyy, *dsxy;        // nodal increments
+  const double *dxx, *dyy, *dxy;           // per-marker subgrid changes
+  double dt;
+  int jaumann;
+  __device__ __forceinline__ void operator()(int64_t m, const DGrid &g, double X, double Y, int cx, int cy,
+                                             double wm) const {
+    double s11 = sxx[m], s22 = syy[m], s12 = sxy[m];
+    if (dxx) {
+      s11 = s11 + dxx[m];
+      s22 = s22 + dyy[m];
+      s12 = s12 + dxy[m];
+    }
+    double i11, i22, i12;
+    stress_increment<MODE>(g, X, Y, cx, cy, dsxx, dsyy, dsxy, i11, i22, i12);
+    s11 = s11 + i11;
+    s22 = s22 + i22;
+    s12 = s12 + i12;
+    rotate_stress(s11, s22, s12, wm, dt, jaumann);
+    sxx[m] = s11;
+    syy[m] = s22;
+    sxy[m] = s12;
+    const double e11 = exx[m], e22 = eyy[m], e12 = exy[m];
+    Eii[m] = Eii[m] + dt * sqrt(0.5 * (e11 * e11 + e22 * e22) + e12 * e12);
+  }
+};
 
 // ---- A7: subgridTemperatureChanges pass 2 (subgridTemperatureChanges.c:89-103) ---
 template <bool PER>

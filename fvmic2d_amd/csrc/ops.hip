@@ -9,8 +9,6 @@
 #include "rheology.h"
 #include "proj_common.h"
 
-int fvm_fill(fvm_ctx *ctx, double *a, int64_t n, double v);  // project.hip
-
 // One thread per marker, the kernel built for each way of gathering (fvm_bil_mode).
 #define BIL_LAUNCH(g, kernel, n, args)                                                \
   switch (fvm_bil_mode(g)) {                                                          \
@@ -33,8 +31,8 @@ int fvm_fill(fvm_ctx *ctx, double *a, int64_t n, double v);  // project.hip
 #define ADV_TILE_BYTES 4096
 // A periodic grid (PER) reads the grid coordinates at ghost indices -1 .. NX+1,
 // so it takes the path without staging.
-template <bool LDS, bool PER>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k_advect_rk4(DGrid g, int32_t n, double *__restrict__ MX, double *__restrict__ MY,
+template <bool LDS, bool PER, class Tail>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LDS ? 5 : 4))) k_advect_rk4(DGrid g, int32_t n, double *__restrict__ MX, double *__restrict__ MY,
                                                     double *__restrict__ MVX, double *__restrict__ MVY,
                                                     double *__restrict__ Mwxy,
                                                     const int32_t *__restrict__ cellXa, const int32_t *__restrict__ cellYa,
@@ -42,7 +40,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
                                                     const double *__restrict__ wxy, BoundaryValues bv, double dt,
                                                     double *__restrict__ MT, double *__restrict__ MTdot,
                                                     const double *__restrict__ dTn, const double *__restrict__ dTsub,
-                                                    double dt_thermal, int tiles) {
+                                                    double dt_thermal, int tiles, Tail tail) {
   if (LDS) {
     extern __shared__ double sgrid[];
     for (int i = threadIdx.x; i < g.NX; i += blockDim.x) sgrid[i] = g.x[i];
@@ -61,13 +59,13 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) k
       const int64_t m = m0 + 256 * t;
       if (m < n)
         advect_marker<PER>(m, gl, MX, MY, MVX, MVY, Mwxy, cellXa, cellYa, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub,
-                      dt_thermal);
+                      dt_thermal, tail);
     }
   } else {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= n) return;
     advect_marker<PER>(m, g, MX, MY, MVX, MVY, Mwxy, cellXa, cellYa, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub,
-                  dt_thermal);
+                  dt_thermal, tail);
   }
 }
 
@@ -83,29 +81,37 @@ __global__ void __launch_bounds__(256) k_rotate_eii(int32_t n, int ncx, int NY, 
   rotate_eii_marker(m, ncx, NY, cellXa, cellYa, Mwxy, sxx, syy, sxy, exx, eyy, exy, Eii, dt, jaumann);
 }
 
-static int launch_advect(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const NodalArrays *nf,
-                         const BoundaryValues *bv, double dt, int jaumann, const double *deltaT, const double *dTsub,
-                         double dt_thermal) {
+// The RK4 pass, tail behind every marker (`wrap` is the tail of a periodic grid).
+template <class Tail, class Wrap>
+static int launch_rk4(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const NodalArrays *nf,
+                      const BoundaryValues *bv, double dt, const double *deltaT, const double *dTsub,
+                      double dt_thermal, const Tail &tail, const Wrap &wrap) {
   const int32_t n = mk->nMark;
   const size_t lds = (size_t)(2 * g->NX + 2 * g->NY + 2) * sizeof(double);
   double *T = deltaT ? mk->T : nullptr, *Tdot = deltaT ? mk->Tdot : nullptr;
   if (g->xperiodic) {
     k_advect_rk4<false, true><<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(
         dgrid(g), n, mk->X, mk->Y, mk->VX, mk->VY, mk->wxy, mk->cellX, mk->cellY, nf->vx, nf->vy, nf->wxy, *bv, dt, T,
-        Tdot, deltaT, dTsub, dt_thermal, 1);
+        Tdot, deltaT, dTsub, dt_thermal, 1, wrap);
   } else if (lds <= 32 * 1024) {
     const int tiles = std::max(2, std::min(8, (int)(lds / ADV_TILE_BYTES)));
     k_advect_rk4<true, false><<<fvm_blocks(n, 256 * tiles), 256, lds, ctx->stream>>>(
         dgrid(g), n, mk->X, mk->Y, mk->VX, mk->VY, mk->wxy, mk->cellX, mk->cellY, nf->vx, nf->vy, nf->wxy, *bv, dt, T,
-        Tdot, deltaT, dTsub, dt_thermal,
-        tiles);
+        Tdot, deltaT, dTsub, dt_thermal, tiles, tail);
   } else {
     k_advect_rk4<false, false><<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(
         dgrid(g), n, mk->X, mk->Y, mk->VX, mk->VY, mk->wxy, mk->cellX, mk->cellY, nf->vx, nf->vy, nf->wxy, *bv, dt, T,
-        Tdot, deltaT, dTsub, dt_thermal,
-        1);
+        Tdot, deltaT, dTsub, dt_thermal, 1, tail);
   }
   FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
+}
+
+static int launch_advect(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const NodalArrays *nf,
+                         const BoundaryValues *bv, double dt, int jaumann, const double *deltaT, const double *dTsub,
+                         double dt_thermal) {
+  const int32_t n = mk->nMark;
+  FVM_TRY(launch_rk4(ctx, g, mk, nf, bv, dt, deltaT, dTsub, dt_thermal, NoTail(), NoTail()));
   k_rotate_eii<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(n, fvm_ncx(g), g->NY, mk->cellX, mk->cellY, mk->wxy, mk->sxx,
                                                             mk->syy, mk->sxy, mk->exx, mk->eyy, mk->exy, mk->Eii, dt,
                                                             jaumann);
@@ -138,16 +144,10 @@ __global__ void __launch_bounds__(256) k_subgrid_t2(DGrid g, int32_t n, const do
   subgrid_t2_marker<PER>(m, g, MX, MY, MT, MTdot, cX, cY, dT, dTsub, dt);
 }
 
-// Pass 1 and the dTsub projection of subgridTemperatureChanges; leaves dTsub
-// (per marker) and deltaT (nodal) in the context scratch for pass 2.
-int fvm_subgrid_t_pass1(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, const NodalArrays *nf,
-                        fvm_markers *mk, const Materials *mat, double dt, double dsubgrid, double **dTsub_out,
-                        double **deltaT_out) {
-  const int32_t n = mk->nMark;
-  const int64_t nn = (int64_t)g->NX * g->NY;
-  FVM_TRY(fvm_ws(ctx, ctx->scratch, ((size_t)n + (size_t)nn + 64) * sizeof(double)));
-  double *dTsub = (double *)ctx->scratch.ptr;
-  double *deltaT = dTsub + ((n + 31) / 32) * 32;
+// Pass 1 and the dTsub projection of subgridTemperatureChanges: dTsub (per
+// marker) and deltaT (nodal) for pass 2.
+int fvm_subgrid_t_into(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk,
+                       const Materials *mat, double dt, double dsubgrid, double *dTsub, double *deltaT) {
   ProjGroup pg;
   memset(&pg, 0, sizeof(pg));
   pg.stagx = pg.stagy = 0;
@@ -171,10 +171,19 @@ int fvm_subgrid_t_pass1(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, co
   sb.rho0 = mat->materialRho[0];
   sb.dt = dt;
   sb.dsub = dsubgrid;
-  FVM_TRY(fvm_project_groups(ctx, g, mk, 1, &pg, &sb));
-  *dTsub_out = dTsub;
-  *deltaT_out = deltaT;
-  return FVM_OK;
+  return fvm_project_groups(ctx, g, mk, 1, &pg, &sb);
+}
+
+// The same into the context scratch.
+int fvm_subgrid_t_pass1(fvm_ctx *ctx, const double *thisT, const fvm_grid *g, const NodalArrays *nf,
+                        fvm_markers *mk, const Materials *mat, double dt, double dsubgrid, double **dTsub_out,
+                        double **deltaT_out) {
+  const int32_t n = mk->nMark;
+  const int64_t nn = (int64_t)g->NX * g->NY;
+  FVM_TRY(fvm_ws(ctx, ctx->scratch, ((size_t)n + (size_t)nn + 64) * sizeof(double)));
+  *dTsub_out = (double *)ctx->scratch.ptr;
+  *deltaT_out = *dTsub_out + ((n + 31) / 32) * 32;
+  return fvm_subgrid_t_into(ctx, thisT, g, nf, mk, mat, dt, dsubgrid, *dTsub_out, *deltaT_out);
 }
 
 extern "C" int fvm_subgrid_temperature_changes(fvm_ctx *ctx, const double *thisT, const fvm_grid *g,
@@ -209,7 +218,63 @@ int fvm_advect_with_subgrid_t2(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays 
   return FVM_OK;
 }
 
+// The end of a visco-elasto-plastic step in one pass over the markers:
+// subgridTemperatureChanges pass 2, advectMarkersRK and its StressTail.
+// dxx .. null: no subgrid stress changes.  Three nodes a side or more.
+int fvm_advect_with_stress(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays *nf, const fvm_grid *g,
+                           const BoundaryValues *bv, double dt, const double *deltaT, const double *dTsub,
+                           const double *dxx, const double *dyy, const double *dxy) {
+  const StressTail<BIL_PLAIN> tail = {mk->sxx, mk->syy, mk->sxy, mk->Eii, mk->exx, mk->eyy, mk->exy,      nf->dsxx,
+                                      nf->dsyy, nf->dsxy, dxx,    dyy,     dxy,     dt,      ctx->jaumann};
+  StressTail<BIL_WRAP> wrap;
+  static_assert(sizeof(wrap) == sizeof(tail), "one layout");
+  memcpy(&wrap, &tail, sizeof(wrap));
+  {
+    FVM_PHASE(ctx, FVM_PHASE_ADVECT);
+    FVM_TRY(launch_rk4(ctx, g, mk, nf, bv, dt, deltaT, dTsub, dt, tail, wrap));
+  }
+  fvm_markers_moved(ctx);
+  return FVM_OK;
+}
+
 // ---- A8: subgridStressChanges (subgridStressChanges.c:5-318) ------------------
+__device__ __forceinline__ double subgrid_stress_factor(double eta, double mu, double dt, double dsubgrid) {
+  const double sdm = eta / mu;
+  double sdif = -dsubgrid * dt / sdm;
+  if (sdif < -30.0) sdif = -30.0;
+  return 1.0 - exp(sdif);
+}
+// The nodal stresses at a marker.  No xperiodic branch in subgridStressChanges.c:
+// the clamps keep both gathers inside [0, NX-1] on a periodic grid too.
+template <int MODE>
+__device__ __forceinline__ void subgrid_stress_at(const DGrid &g, double X, double Y, int c0x, int c0y,
+                                                  const double *__restrict__ soxx, const double *__restrict__ soyy,
+                                                  const double *__restrict__ soxy, double &sxxm, double &syym,
+                                                  double &sxym) {
+  const int NX = g.NX, NY = g.NY;
+  int cellY = c0y, cellX = c0x;
+  if (cellX < 0) cellX = 0;
+  if (cellX > NX - 2) cellX = NX - 2;
+  if (cellY < 0) cellY = 0;
+  if (cellY > NY - 2) cellY = NY - 2;
+  double mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
+  double mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
+  sxym = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(soxy);
+  cellX = c0x;
+  cellY = c0y;
+  if (cellX < NX - 1 && X >= g.xc[cellX + 1]) cellX++;
+  if (cellY < NY - 1 && Y >= g.yc[cellY + 1]) cellY++;
+  if (cellY < 1) cellY = 1;
+  else if (cellY > NY - 2) cellY = NY - 2;
+  if (cellX < 1) cellX = 1;
+  else if (cellX > NX - 2) cellX = NX - 2;
+  mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
+  mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
+  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
+  sxxm = at(soxx);
+  syym = at(soyy);
+}
+
 template <int MODE>
 __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const double *__restrict__ MX,
                                                     const double *__restrict__ MY, const double *__restrict__ eta,
@@ -229,52 +294,42 @@ __global__ void __launch_bounds__(256) k_subgrid_s1(DGrid g, int32_t n, const do
     dyy[m] = 0.0;
     return;
   }
-  // no xperiodic branch in subgridStressChanges.c: the clamps keep both
-  // gathers inside [0, NX-1] on a periodic grid too
-  const int NX = g.NX, NY = g.NY;
-  const double X = MX[m], Y = MY[m];
-  const double sdm = eta[m] / mu[m];
-  double sdif = -dsubgrid * dt / sdm;
-  if (sdif < -30.0) sdif = -30.0;
-  sdif = 1.0 - exp(sdif);
-
-  int cellY = c0y, cellX = c0x;
-  if (cellX < 0) cellX = 0;
-  if (cellX > NX - 2) cellX = NX - 2;
-  if (cellY < 0) cellY = 0;
-  if (cellY > NY - 2) cellY = NY - 2;
-  double mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
-  double mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  const double sxym = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(soxy);
-  double sxy0 = sxy[m];
-  double dsxym = sxym - sxy0;
-  dsxym *= sdif;
+  const double sdif = subgrid_stress_factor(eta[m], mu[m], dt, dsubgrid);
+  double sxxm, syym, sxym;
+  subgrid_stress_at<MODE>(g, MX[m], MY[m], c0x, c0y, soxx, soyy, soxy, sxxm, syym, sxym);
+  const double sxy0 = sxy[m], sxx0 = sxx[m], syy0 = syy[m];
+  const double dsxym = (sxym - sxy0) * sdif, dsxxm = (sxxm - sxx0) * sdif, dsyym = (syym - syy0) * sdif;
   sxy[m] = sxy0 + dsxym;
-  dxy[m] = dsxym;
-
-  cellX = c0x;
-  cellY = c0y;
-  if (cellX < NX - 1 && X >= g.xc[cellX + 1]) cellX++;
-  if (cellY < NY - 1 && Y >= g.yc[cellY + 1]) cellY++;
-  if (cellY < 1) cellY = 1;
-  else if (cellY > NY - 2) cellY = NY - 2;
-  if (cellX < 1) cellX = 1;
-  else if (cellX > NX - 2) cellX = NX - 2;
-  mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
-  mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
-  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
-  const double sxxm = at(soxx);
-  const double sxx0 = sxx[m];
-  double dsxxm = sxxm - sxx0;
-  dsxxm *= sdif;
   sxx[m] = sxx0 + dsxxm;
-  const double syym = at(soyy);
-  const double syy0 = syy[m];
-  double dsyym = syym - syy0;
-  dsyym *= sdif;
   syy[m] = syy0 + dsyym;
+  dxy[m] = dsxym;
   dxx[m] = dsxxm;
   dyy[m] = dsyym;
+}
+
+// The nodal part of subgridStressChanges: the markers' own changes leave the
+// nodal increments.
+int fvm_project_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, const fvm_markers *mk,
+                               const double *dxx, const double *dyy, const double *dxy) {
+  // subgridStressChanges.c:134-175 (sxy, basic nodes, <=/>= 0.5 ties) and
+  // :223-233 (sxx, syy, one cell-centre node); two groups, one node pass
+  ProjGroup pg[2];
+  memset(pg, 0, sizeof(pg));
+  pg[0].stagx = pg[0].stagy = 0;
+  pg[0].method = PM_TIES;
+  pg[0].nf = 1;
+  pg[0].src[0].col = dxy;
+  pg[0].out[0] = nf->dsxy;
+  pg[0].epilogue = EPI_SUB_FROM;
+  pg[1].stagx = pg[1].stagy = 0;
+  pg[1].method = PM_CENTRE;
+  pg[1].nf = 2;
+  pg[1].src[0].col = dxx;
+  pg[1].src[1].col = dyy;
+  pg[1].out[0] = nf->dsxx;
+  pg[1].out[1] = nf->dsyy;
+  pg[1].epilogue = EPI_SUB_FROM;
+  return fvm_project_groups(ctx, g, mk, 2, pg);
 }
 
 extern "C" int fvm_subgrid_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk,
@@ -296,29 +351,10 @@ extern "C" int fvm_subgrid_stress_changes(fvm_ctx *ctx, const fvm_grid *g, const
       FVM_LAUNCH_CHECK(ctx);
     }
   }
-  // subgridStressChanges.c:134-175 (sxy, basic nodes, <=/>= 0.5 ties) and
-  // :223-233 (sxx, syy, one cell-centre node); two groups, one node pass
-  ProjGroup pg[2];
-  memset(pg, 0, sizeof(pg));
-  pg[0].stagx = pg[0].stagy = 0;
-  pg[0].method = PM_TIES;
-  pg[0].nf = 1;
-  pg[0].src[0].col = dxy;
-  pg[0].out[0] = nf->dsxy;
-  pg[0].epilogue = EPI_SUB_FROM;
-  pg[1].stagx = pg[1].stagy = 0;
-  pg[1].method = PM_CENTRE;
-  pg[1].nf = 2;
-  pg[1].src[0].col = dxx;
-  pg[1].src[1].col = dyy;
-  pg[1].out[0] = nf->dsxx;
-  pg[1].out[1] = nf->dsyy;
-  pg[1].epilogue = EPI_SUB_FROM;
-  FVM_TRY(fvm_project_groups(ctx, g, mk, 2, pg));
-  return FVM_OK;
+  return fvm_project_stress_changes(ctx, g, nf, mk, dxx, dyy, dxy);
 }
 
-// ---- A9: updateMarkerStress (updateMarkerStress.c:5-163) ----------------------
+// ---- A9: updateMarkerStress (updateMarkerStress.c:5-163), body in marker_common.h ----
 template <int MODE>
 __global__ void __launch_bounds__(256) k_update_stress(DGrid g, int32_t n, const double *__restrict__ MX,
                                                        const double *__restrict__ MY, double *__restrict__ sxx,
@@ -330,34 +366,11 @@ __global__ void __launch_bounds__(256) k_update_stress(DGrid g, int32_t n, const
   if (m >= n) return;
   const int c0x = cXa[m], c0y = cYa[m];
   if (!cell_ok(c0x, c0y, g.ncx(), g.NY)) return;
-  const int NX = g.NX, NY = g.NY, P = g.per;
-  const double X = MX[m], Y = MY[m];
-  int cellX = c0x, cellY = c0y;
-  // periodic: the centre cell may step to NX and is then clamped to NX-1
-  // (cellXMax NX, then NX-1); node column NX is column 0
-  if (cellX < (P ? NX : NX - 2) && X >= g.xc[cellX + 1]) cellX++;
-  if (cellY < NY - 1 && Y >= g.yc[cellY + 1]) cellY++;
-  if (cellY < 1) cellY = 1;
-  else if (cellY > NY - 2) cellY = NY - 2;
-  if (cellX < 1) cellX = 1;
-  else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
-  double mdx = (X - g.xc[cellX]) / (g.xc[cellX + 1] - g.xc[cellX]);
-  double mdy = (Y - g.yc[cellY]) / (g.yc[cellY + 1] - g.yc[cellY]);
-  const Bilinear<MODE> at(g, cellY, cellX, mdx, mdy);
-  const double mdsxx = at(dsxx);
-  const double mdsyy = at(dsyy);
-  sxx[m] = sxx[m] + mdsxx;
-  syy[m] = syy[m] + mdsyy;
-  cellX = c0x;
-  cellY = c0y;
-  if (cellY < 0) cellY = 0;
-  else if (cellY > NY - 2) cellY = NY - 2;
-  if (cellX < 0) cellX = 0;
-  else if (cellX > (P ? NX - 1 : NX - 2)) cellX = P ? NX - 1 : NX - 2;
-  mdx = (X - g.x[cellX]) / (g.x[cellX + 1] - g.x[cellX]);
-  mdy = (Y - g.y[cellY]) / (g.y[cellY + 1] - g.y[cellY]);
-  const double mdsxy = Bilinear<MODE>(g, cellY, cellX, mdx, mdy)(dsxy);
-  sxy[m] = sxy[m] + mdsxy;
+  double i11, i22, i12;
+  stress_increment<MODE>(g, MX[m], MY[m], c0x, c0y, dsxx, dsyy, dsxy, i11, i22, i12);
+  sxx[m] = sxx[m] + i11;
+  syy[m] = syy[m] + i22;
+  sxy[m] = sxy[m] + i12;
 }
 
 extern "C" int fvm_update_marker_stress(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk,
@@ -380,7 +393,16 @@ extern "C" int fvm_update_marker_stress(fvm_ctx *ctx, const fvm_grid *g, const N
 struct StrainIn {
   const double *dsxx, *dsyy, *dsxy, *soxx, *soyy, *soxy, *exx, *eyy, *exy, *wxy, *p;
 };
-template <int MODE>
+// subgridStressChanges' marker part in the same pass (S1): the changes alone, the
+// marker stresses stay as they are.  On a plain grid its four gathers are three of
+// this pass's own (the centre cell steps and clamps to the same index, the basic
+// cell is the marker's); a periodic grid clamps differently and gathers again.
+struct SubStress {
+  const double *sxx, *syy, *sxy;
+  double *dxx, *dyy, *dxy;
+  double dsubgrid;
+};
+template <int MODE, bool S1>
 __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, const double *__restrict__ MX,
                                                          const double *__restrict__ MY, const double *__restrict__ eta,
                                                          const double *__restrict__ mu, double *__restrict__ Mp,
@@ -388,7 +410,7 @@ __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, con
                                                          double *__restrict__ e22, double *__restrict__ e12,
                                                          double *__restrict__ srr, const int32_t *__restrict__ cXa,
                                                          const int32_t *__restrict__ cYa, StrainIn F, double dt,
-                                                         int32_t *__restrict__ flags) {
+                                                         int32_t *__restrict__ flags, SubStress S) {
   const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (m >= n) return;
   const int c0x = cXa[m], c0y = cYa[m];
@@ -439,6 +461,43 @@ __global__ void __launch_bounds__(256) k_strain_pressure(DGrid g, int32_t n, con
   srr[m] = r;
   // the flag only goes from 0 to 1: a plain store, never an atomic per marker
   if (r != r) __hip_atomic_store(&flags[0], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if (S1) {
+    const double sdif = subgrid_stress_factor(em, um, dt, S.dsubgrid);
+    double sxxm = msxx, syym = msyy, sxym = msxy;
+    if (MODE != BIL_PLAIN) subgrid_stress_at<MODE>(g, X, Y, c0x, c0y, F.soxx, F.soyy, F.soxy, sxxm, syym, sxym);
+    S.dxy[m] = (sxym - S.sxy[m]) * sdif;
+    S.dxx[m] = (sxxm - S.sxx[m]) * sdif;
+    S.dyy[m] = (syym - S.syy[m]) * sdif;
+  }
+}
+
+// The pass over all markers; S given: with the subgrid stress changes.  flag: one
+// word that a NaN residual sets (pinned host memory will do).
+int fvm_launch_strain_pressure(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf, fvm_markers *mk, double dt,
+                               int32_t *flag, const double dsubgrid, double *dxx, double *dyy, double *dxy) {
+  const StrainIn F = {nf->dsxx, nf->dsyy, nf->dsxy, nf->soxx, nf->soyy, nf->soxy,
+                      nf->edotxx, nf->edotyy, nf->edotxy, nf->wxy, nf->p};
+  const SubStress S = {mk->sxx, mk->syy, mk->sxy, dxx, dyy, dxy, dsubgrid};
+  FVM_PHASE(ctx, FVM_PHASE_MARKER_UPDATE);
+#define STRAIN_LAUNCH(MODE, S1)                                                                                     \
+  k_strain_pressure<MODE, S1><<<fvm_blocks(mk->nMark, 256), 256, 0, ctx->stream>>>(                                  \
+      dgrid(g), mk->nMark, mk->X, mk->Y, mk->eta, mk->mu, mk->p, mk->wxy, mk->exx, mk->eyy, mk->exy,                 \
+      mk->strainRateResidual, mk->cellX, mk->cellY, F, dt, flag, S)
+  switch (fvm_bil_mode(g)) {
+    case BIL_PLAIN:
+      if (dxx) STRAIN_LAUNCH(BIL_PLAIN, true);
+      else STRAIN_LAUNCH(BIL_PLAIN, false);
+      break;
+    case BIL_WRAP:
+      if (dxx) STRAIN_LAUNCH(BIL_WRAP, true);
+      else STRAIN_LAUNCH(BIL_WRAP, false);
+      break;
+    default:
+      STRAIN_LAUNCH(BIL_ANY, false);
+  }
+#undef STRAIN_LAUNCH
+  FVM_LAUNCH_CHECK(ctx);
+  return FVM_OK;
 }
 
 extern "C" int fvm_update_marker_strain_pressure(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *nf,
@@ -452,20 +511,9 @@ extern "C" int fvm_update_marker_strain_pressure(fvm_ctx *ctx, const fvm_grid *g
                 nf->edotxx, nf->edotyy, nf->edotxy, nf->wxy, nf->p};
   if (!F.dsxx || !F.dsyy || !F.dsxy || !F.soxx || !F.soyy || !F.soxy || !F.exx || !F.exy || !F.wxy || !F.p)
     return FVM_ERR_ARG;
-  FVM_TRY(fvm_ws(ctx, ctx->red, 4096));
-  int32_t *flags = (int32_t *)ctx->red.ptr + 8;
-  FVM_HIP(ctx, hipMemsetAsync(flags, 0, sizeof(int32_t), ctx->stream));
-  if (mk->nMark > 0) {
-    {
-      FVM_PHASE(ctx, FVM_PHASE_MARKER_UPDATE);
-      BIL_LAUNCH(g, k_strain_pressure, mk->nMark,
-                 (dgrid(g), mk->nMark, mk->X, mk->Y, mk->eta, mk->mu, mk->p, mk->wxy, mk->exx, mk->eyy, mk->exy,
-                  mk->strainRateResidual, mk->cellX, mk->cellY, F, dt, flags));
-      FVM_LAUNCH_CHECK(ctx);
-    }
-  }
   int32_t *h = (int32_t *)ctx->pinned.ptr;
-  FVM_HIP(ctx, hipMemcpyAsync(h, flags, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream));
+  h[0] = 0;
+  if (mk->nMark > 0) FVM_TRY(fvm_launch_strain_pressure(ctx, g, nf, mk, dt, h, 0.0, nullptr, nullptr, nullptr));
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   if (h[0]) return fvm_set_err(ctx, FVM_ERR_NAN_RESIDUAL, "NaN strain rate residual on an active marker");
   return FVM_OK;
@@ -640,31 +688,33 @@ __global__ void __launch_bounds__(RED_BS) k_block_sum(const double *__restrict__
   if (threadIdx.x == 0) out[blockIdx.x] = s[0];
 }
 
-int fvm_reduce_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out) {
+// Enqueue the sum of d[0..n), n > 0, into *out (pinned host memory will do: the
+// last block writes it there itself).
+static int enqueue_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out) {
   const int64_t nb = n < 1024 * RED_BS ? (n + RED_BS - 1) / RED_BS : 1024;
-  const int64_t per = nb > 0 ? (n + nb - 1) / nb : 0;
+  const int64_t per = (n + nb - 1) / nb;
   FVM_TRY(fvm_ws(ctx, ctx->red, 4096 + (size_t)(nb + 1) * sizeof(double)));
   double *parts = (double *)((char *)ctx->red.ptr + 4096);
-  if (nb > 0) {
-    {
-      FVM_PHASE(ctx, FVM_PHASE_OTHER);
-      k_block_sum<<<(unsigned)nb, RED_BS, 0, ctx->stream>>>(d, n, per, parts);
-      FVM_LAUNCH_CHECK(ctx);
-    }
-    {
-      FVM_PHASE(ctx, FVM_PHASE_OTHER);
-      k_block_sum<<<1, RED_BS, 0, ctx->stream>>>(parts, nb, nb, parts + nb);
-      FVM_LAUNCH_CHECK(ctx);
-    }
+  {
+    FVM_PHASE(ctx, FVM_PHASE_OTHER);
+    k_block_sum<<<(unsigned)nb, RED_BS, 0, ctx->stream>>>(d, n, per, parts);
+    FVM_LAUNCH_CHECK(ctx);
   }
+  {
+    FVM_PHASE(ctx, FVM_PHASE_OTHER);
+    k_block_sum<<<1, RED_BS, 0, ctx->stream>>>(parts, nb, nb, out);
+    FVM_LAUNCH_CHECK(ctx);
+  }
+  return FVM_OK;
+}
+
+int fvm_reduce_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out) {
+  *out = 0.0;
+  if (n <= 0) return FVM_OK;
   double *h = (double *)ctx->pinned.ptr + 8;
-  if (nb > 0) {
-    FVM_HIP(ctx, hipMemcpyAsync(h, parts + nb, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    *out = *h;
-  } else {
-    *out = 0.0;
-  }
+  FVM_TRY(enqueue_sum(ctx, d, n, h));
+  FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  *out = *h;
   return FVM_OK;
 }
 
@@ -682,13 +732,11 @@ __global__ void k_residual_area(DGrid g, double *__restrict__ srr) {
   }
 }
 
-extern "C" int fvm_update_global_strain_rate_residual(fvm_ctx *ctx, const fvm_grid *g, const fvm_markers *mk,
-                                                      double *residual) {
-  if (!ctx || !mk || !residual) return FVM_ERR_ARG;
-  FVM_TRY(fvm_grid_check(ctx, g));
+// Enqueue the residual's sum over the nodes into *out (divide by the area for the
+// residual); srr: NX * NY doubles of workspace.
+int fvm_enqueue_strain_rate_residual(fvm_ctx *ctx, const fvm_grid *g, const fvm_markers *mk, double *srr,
+                                     double *out) {
   const int64_t nn = (int64_t)g->NX * g->NY;
-  FVM_TRY(fvm_ws(ctx, ctx->scratch, ((size_t)nn + 64) * sizeof(double)));
-  double *srr = (double *)ctx->scratch.ptr;
   ProjGroup pg;
   memset(&pg, 0, sizeof(pg));
   pg.stagx = pg.stagy = -1;
@@ -703,10 +751,18 @@ extern "C" int fvm_update_global_strain_rate_residual(fvm_ctx *ctx, const fvm_gr
     k_residual_area<<<fvm_blocks(nn, 256), 256, 0, ctx->stream>>>(dgrid(g), srr);
     FVM_LAUNCH_CHECK(ctx);
   }
-  double sum = 0.0;
-  FVM_TRY(fvm_reduce_sum(ctx, srr, nn, &sum));
-  sum /= (g->LX * g->LY);
-  *residual = sum;
+  return enqueue_sum(ctx, srr, nn, out);
+}
+
+extern "C" int fvm_update_global_strain_rate_residual(fvm_ctx *ctx, const fvm_grid *g, const fvm_markers *mk,
+                                                      double *residual) {
+  if (!ctx || !mk || !residual) return FVM_ERR_ARG;
+  FVM_TRY(fvm_grid_check(ctx, g));
+  FVM_TRY(fvm_ws(ctx, ctx->scratch, ((size_t)g->NX * g->NY + 64) * sizeof(double)));
+  double *h = (double *)ctx->pinned.ptr + 8;
+  FVM_TRY(fvm_enqueue_strain_rate_residual(ctx, g, mk, (double *)ctx->scratch.ptr, h));
+  FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
+  *residual = *h / (g->LX * g->LY);
   return FVM_OK;
 }
 

@@ -457,18 +457,13 @@ extern "C" int fvm_project_markers_nodes_from_scalar(fvm_ctx *ctx, const fvm_gri
   return fvm_project_group(ctx, g, mk, pg);
 }
 
-__global__ void k_fill(double *__restrict__ a, int64_t n, double v) {
-  int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) a[i] = v;
-}
-
-int fvm_fill(fvm_ctx *ctx, double *a, int64_t n, double v) {
-  {
-    FVM_PHASE(ctx, FVM_PHASE_OTHER);
-    k_fill<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(a, n, v);
-    FVM_LAUNCH_CHECK(ctx);
-  }
-  return FVM_OK;
+__global__ void k_fill_all2(double *__restrict__ rhodot, double *__restrict__ muS, double *__restrict__ muN,
+                            int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  rhodot[i] = 0.0;
+  muS[i] = 1e99;
+  muN[i] = 1e99;
 }
 
 extern "C" int fvm_project_markers_nodes_all2(fvm_ctx *ctx, const fvm_grid *g, const fvm_markers *mk,
@@ -489,8 +484,8 @@ extern "C" int fvm_project_markers_nodes_all2(fvm_ctx *ctx, const fvm_grid *g, c
       {mk->sxy, nullptr, nf->soxy, 0, 0, ARITHMETIC_LOCAL},
   };
   FVM_TRY(fvm_project_marker_fields(ctx, g, mk, 9, list));
-  FVM_HIP(ctx, hipMemsetAsync(nf->rhodot, 0, (size_t)nn * sizeof(double), ctx->stream));  // :21
-  FVM_TRY(fvm_fill(ctx, nf->muS, nn, 1e99));                                               // :36
-  FVM_TRY(fvm_fill(ctx, nf->muN, nn, 1e99));                                               // :37
+  FVM_PHASE(ctx, FVM_PHASE_OTHER);
+  k_fill_all2<<<fvm_blocks(nn, 256), 256, 0, ctx->stream>>>(nf->rhodot, nf->muS, nf->muN, nn);  // :21, :36, :37
+  FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;
 }
