@@ -12,7 +12,28 @@
 // not clamped (:1965-1971), node columns wrap, the left-wall ghost rule is off
 // (:2014-2023) and the new X is wrapped into [0, LX] (:2225-2231).  The grid
 // coordinates are then read at indices -1 .. NX+1 (set by makePeriodic).
-// tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's stages are done, with
+// Quotients by a shared divisor.  n / d is rcp(d) refined by two Newton steps, a
+// product and a correction: eleven instructions with the operand scaling and the
+// special cases, once for each quotient.  A stage has two quotients for each of
+// its four spacings, so the refined reciprocal is formed once per spacing and a
+// quotient takes three instructions: the bits are those of the division wherever
+// that needs no scaling, and where a quotient is not finite the stage takes the
+// divisions themselves.
+struct Spacing {
+  double d, y;
+  __device__ __forceinline__ explicit Spacing(double d_) : d(d_) {
+    y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  }
+  __device__ __forceinline__ double into(double n) const {
+    const double q = n * y;
+    return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+  }
+};
+
+// c0x, c0y, X0, Y0: the marker's stored cell and position (the caller reads them,
+// a marker ahead where it can).  tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's stages are done, with
 // its old position and cell and its new spin (NoTail: nothing).
 struct NoTail {
   __device__ __forceinline__ void operator()(int64_t, const DGrid &, double, double, int, int, double) const {}
@@ -24,8 +45,6 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MVX,
     double *__restrict__ MVY,
     double *__restrict__ Mwxy,
-    const int32_t *__restrict__ cellXa,
-    const int32_t *__restrict__ cellYa,
     const double *__restrict__ vx,
     const double *__restrict__ vy,
     const double *__restrict__ wxy,
@@ -35,14 +54,12 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MTdot,
     const double *__restrict__ dTn,
     const double *__restrict__ dTsub,
-    double dt_thermal, const Tail &tail) {
-  const int c0x = cellXa[m], c0y = cellYa[m];
+    double dt_thermal, const Tail &tail, int c0x, int c0y, double X0, double Y0) {
   if (!cell_ok(c0x, c0y, g.ncx(), g.NY)) return;
   const int NX = g.NX, NY = g.NY;
   const int XCMAX = PER ? NX - 1 : NX - 2, XCMIN = PER ? -1 : 0;
   // column offset of node ix + 1 from node ix (wraps past the last column)
   auto right = [&](int ix) -> int { return (PER && ix + 1 >= NX) ? 1 - NX : 1; };
-  const double X0 = MX[m], Y0 = MY[m];
   if (MT) {
     // subgridTemperatureChanges.c:89-103 (pass 2) on the same stored cell,
     // fused here because advectMarkersRK starts from that cell too
@@ -64,80 +81,80 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
   // expression's left-to-right order as the stages complete
   double svx = 0.0, svy = 0.0, swxy = 0.0;
   // the stages stay a loop: unrolled, they held 116-126 VGPRs (four waves per
-  // SIMD); rolled, 90-94 (five), and the issue-bound stages then hide more of
-  // their gather latency (ensemble advection 3.16 ms instead of 3.31)
+  // SIMD); rolled, 96 at most (five).  At 1.44 M markers on 201 x 201 nodes the
+  // pass takes 58 us, about 24 of them its columns and 8-9 each stage, where the
+  // SIMDs issue FP64 nearly all the time; it took 72 (12 a stage) with eight whole
+  // divisions, the walk as loops and the three fields' gathers one after another.
+  const bool top0 = bv.mechBCTop.type[0] == 0, top1 = bv.mechBCTop.type[0] == 1;
+  const bool left0 = bv.mechBCLeft.type[1] == 0, left1 = bv.mechBCLeft.type[1] == 1;
+  const double top2 = 2.0 * bv.mechBCTop.value[0], left2 = 2.0 * bv.mechBCLeft.value[1];
 #pragma unroll 1
   for (int irk = 0; irk < 4; irk++) {
+    // The walk of both axes from the marker's cell.  It rarely passes more than one
+    // cell boundary, so the four coordinates around the cell are read together and
+    // decide the first step without a branch; a marker that goes further walks on.
+    // (Walked step by step, every lane that moved sent its wavefront through the
+    // loops of all four directions, each a chain of reads: more of a stage's time
+    // than its arithmetic.)  The cell is made opaque so that the coordinates are
+    // read per stage and not held over all of them: registers are what bounds the
+    // wavefronts in flight.
     int cellX = c0x, cellY = c0y;
-    if (xcur > g.x[cellX + 1]) {
-      while (xcur > g.x[cellX + 1] && cellX < XCMAX) cellX++;
-    } else if (xcur < g.x[cellX]) {
-      while (xcur < g.x[cellX] && cellX > XCMIN) cellX--;
+    asm volatile("" : "+v"(cellX), "+v"(cellY));
+    {
+      const int lx = PER ? cellX - 1 : max(cellX - 1, 0), ly = max(cellY - 1, 0);
+      const int hx = PER ? cellX + 2 : min(cellX + 2, NX - 1), hy = min(cellY + 2, NY - 1);
+      const double xm1 = g.x[lx], x0 = g.x[cellX], x1 = g.x[cellX + 1], x2 = g.x[hx];
+      const double ym1 = g.y[ly], y0 = g.y[cellY], y1 = g.y[cellY + 1], y2 = g.y[hy];
+      const bool rx = xcur > x1, ry = ycur > y1, bx = !rx && xcur < x0, by = !ry && ycur < y0;
+      const int sx = rx ? (cellX < XCMAX ? 1 : 0) : (bx && cellX > XCMIN ? -1 : 0);
+      const int sy = ry ? (cellY < NY - 2 ? 1 : 0) : (by && cellY > 0 ? -1 : 0);
+      cellX += sx;
+      cellY += sy;
+      const bool on = (sx > 0 && xcur > x2) || (sx < 0 && xcur < xm1) || (sy > 0 && ycur > y2) || (sy < 0 && ycur < ym1);
+      if (on) {
+        if (sx > 0)
+          while (xcur > g.x[cellX + 1] && cellX < XCMAX) cellX++;
+        if (sx < 0)
+          while (xcur < g.x[cellX] && cellX > XCMIN) cellX--;
+        if (sy > 0)
+          while (ycur > g.y[cellY + 1] && cellY < NY - 2) cellY++;
+        if (sy < 0)
+          while (ycur < g.y[cellY] && cellY > 0) cellY--;
+      }
     }
-    if (ycur > g.y[cellY + 1]) {
-      while (ycur > g.y[cellY + 1] && cellY < NY - 2) cellY++;
-    } else if (ycur < g.y[cellY]) {
-      while (ycur < g.y[cellY] && cellY > 0) cellY--;
-    }
-    int vxX = cellX, vxY = cellY;
-    if (vxY > -1 && ycur < g.yc[vxY + 1]) vxY--;
-    int vyX = cellX;
-    if (vyX > -1 && xcur < g.xc[vyX + 1]) vyX--;
-    int vyY = cellY;
-    if (!PER) {
-      if (vxX < 0) vxX = 0;
-      else if (vxX > NX - 2) vxX = NX - 2;
-      if (vyX < -1) vyX = -1;
-      else if (vyX > NX - 2) vyX = NX - 2;
-    }
-    if (vxY < -1) vxY = -1;
-    else if (vxY > NY - 2) vxY = NY - 2;
-    if (vyY < 0) vyY = 0;
-    else if (vyY > NY - 2) vyY = NY - 2;
+    // the half cells: cellY in [0, NY-2], cellX in [0, NX-2] (PER: [-1, NX-1]), so
+    // the reference's clamps of vxX, vxY, vyX and vyY change nothing
+    const int vxX = cellX, vyY = cellY;
+    const double xg0 = g.x[cellX], xg1 = g.x[cellX + 1], yg0 = g.y[cellY], yg1 = g.y[cellY + 1];
+    const double xc0 = g.xc[PER ? max(cellX, 0) : cellX], xc1 = g.xc[cellX + 1], xc2 = g.xc[cellX + 2];
+    const double yc0 = g.yc[cellY], yc1 = g.yc[cellY + 1], yc2 = g.yc[cellY + 2];
+    const bool up = ycur < yc1, left = (!PER || cellX > -1) && xcur < xc1;
+    const int vxY = up ? cellY - 1 : cellY, vyX = left ? cellX - 1 : cellX;
+    const double xcl = left ? xc0 : xc1, xch = left ? xc1 : xc2, ycl = up ? yc0 : yc1, ych = up ? yc1 : yc2;
 
-    double deltaxm = xcur - g.x[vxX];
-    double deltaym = ycur - g.yc[vxY + 1];
-    double dx = g.x[vxX + 1] - g.x[vxX];
-    double dy = g.yc[vxY + 2] - g.yc[vxY + 1];
-    // vxX == cellX (cellX stays in [0, NX-2], or [-1, NX-1] when PER), so this
-    // quotient is also the wxy mdx below
-    const double qx = deltaxm / dx;
-    // vx nodes: rows vxY (-1 is the ghost row, which reads 0) and vxY + 1,
-    // columns vxX and vxX + 1 (both owned: vxX is in [0, NX-2]; when PER the
-    // columns wrap).  Loads are unconditional from a valid address; the ghost
-    // row is selected away.
+    // the twelve nodes, all loads in flight before the arithmetic of any.
+    // vx nodes: rows vxY (-1 is the ghost row) and vxY + 1, columns vxX and vxX + 1
+    // (both owned: vxX is in [0, NX-2]; when PER the columns wrap).  Loads are
+    // unconditional from a valid address; a ghost value is selected away.
     const bool vrow = vxY >= 0;
     const int vxc = PER && vxX < 0 ? vxX + NX : vxX;
     const int vxr = right(vxc);
     const double *vr1 = vx + (int64_t)(vxY + 1) * NX + vxc;
     const double *vr0 = vrow ? vr1 - NX : vr1;
-    const double vxll = vr1[0], vxlr = vr1[vxr];
-    const double vx0 = vr0[0], vx1 = vr0[vxr];
-    double vxul, vxur;
-    if (vxY == -1 && bv.mechBCTop.type[0] == 0) {
-      vxul = 2.0 * bv.mechBCTop.value[0] - vxll;
-      vxur = 2.0 * bv.mechBCTop.value[0] - vxlr;
-    } else if (vxY == -1 && bv.mechBCTop.type[0] == 1) {
-      vxul = vxll;
-      vxur = vxlr;
+    double vxll, vxlr, vx0, vx1;
+    if (PER) {
+      vxll = vr1[0], vxlr = vr1[vxr], vx0 = vr0[0], vx1 = vr0[vxr];
     } else {
-      vxul = vrow ? vx0 : 0.0;
-      vxur = vrow ? vx1 : 0.0;
+      const fvm_pair lo = load_pair(vr1), hi = load_pair(vr0);
+      vxll = lo.a, vxlr = lo.b, vx0 = hi.a, vx1 = hi.b;
     }
-    const double qyv = deltaym / dy;
-    double a = vxul * (1.0 - qx) * (1.0 - qyv);
-    a += vxur * (qx) * (1.0 - qyv);
-    a += vxll * (1.0 - qx) * (qyv);
-    a += vxlr * (deltaxm * deltaym) / dx / dy;
-
-    // vy nodes: columns vyX (-1 is the ghost column, which reads 0; when PER
-    // it is column NX-1) and vyX + 1, rows vyY and vyY + 1 (both owned: vyY
-    // is in [0, NY-2])
+    // vy nodes: columns vyX (-1 is the ghost column; when PER it is column NX-1)
+    // and vyX + 1, rows vyY and vyY + 1 (both owned: vyY is in [0, NY-2])
     const bool vcol = PER || vyX >= 0;
-    const int vyc = PER && vyX + 1 >= NX ? vyX + 1 - NX : vyX + 1;  // column of vyX + 1
-    const int vyl = (PER && vyc == 0) ? NX - 1 : -1;                // offset of column vyX
     double vyur, vylr, vy0, vy1;
     if (PER) {
+      const int vyc = vyX + 1 >= NX ? vyX + 1 - NX : vyX + 1;  // column of vyX + 1
+      const int vyl = vyc == 0 ? NX - 1 : -1;                  // offset of column vyX
       const double *q0 = vy + (int64_t)vyY * NX + vyc, *q1 = q0 + NX;
       vyur = q0[0], vylr = q1[0];
       vy0 = q0[vyl], vy1 = q1[vyl];
@@ -149,42 +166,60 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
       vyur = vcol ? a.b : a.a, vylr = vcol ? b.b : b.a;
       vy0 = a.a, vy1 = b.a;
     }
-    double vyul, vyll;
-    if (!PER && vyX == -1 && bv.mechBCLeft.type[1] == 0) {
-      vyul = 2.0 * bv.mechBCLeft.value[1] - vyur;
-      vyll = 2.0 * bv.mechBCLeft.value[1] - vylr;
-    } else if (!PER && vyX == -1 && bv.mechBCLeft.type[1] == 1) {
-      vyul = vyur;
-      vyll = vylr;
-    } else {
-      vyul = vcol ? vy0 : 0.0;
-      vyll = vcol ? vy1 : 0.0;
-    }
-    deltaxm = xcur - g.xc[vyX + 1];
-    deltaym = ycur - g.y[vyY];
-    dx = g.xc[vyX + 2] - g.xc[vyX + 1];
-    dy = g.y[vyY + 1] - g.y[vyY];
-    // vyY == cellY (cellY stays in [0, NY-2]), so this quotient is also the wxy mdy below
-    const double qy = deltaym / dy;
-    const double qxv = deltaxm / dx;
-    double b = vyul * (1.0 - qxv) * (1.0 - qy);
-    b += vyur * (qxv) * (1.0 - qy);
-    b += vyll * (1.0 - qxv) * (qy);
-    b += vylr * (deltaxm * deltaym) / dx / dy;
-
-    // markers.c:2089-2090: (xcur - x[cellX]) / (x[cellX+1] - x[cellX]), the same
-    // operands as qx and qy above, hence the same values
-    const double mdx = qx;
-    const double mdy = qy;
-    // cellX in [0, NX-2] ([-1, NX-1] wrapped when PER), cellY in [0, NY-2]:
+    // wxy: cellX in [0, NX-2] ([-1, NX-1] wrapped when PER), cellY in [0, NY-2]:
     // four owned nodes
     const int wc = PER && cellX < 0 ? cellX + NX : cellX;
     const int wr = right(wc);
     const double *w0 = wxy + (int64_t)cellY * NX + wc, *w1 = w0 + NX;
-    double w = (1.0 - mdx) * (1.0 - mdy) * w0[0];
-    w += (mdx) * (1.0 - mdy) * w0[wr];
-    w += (1.0 - mdx) * (mdy) * w1[0];
-    w += (mdx) * (mdy) * w1[wr];
+    double w00, w01, w10, w11;
+    if (PER) {
+      w00 = w0[0], w01 = w0[wr], w10 = w1[0], w11 = w1[wr];
+    } else {
+      const fvm_pair a = load_pair(w0), b = load_pair(w1);
+      w00 = a.a, w01 = a.b, w10 = b.a, w11 = b.b;
+    }
+
+    // vxX == cellX and vyY == cellY, so qx and qy are also the mdx and mdy of wxy
+    // (markers.c:2089-2090: the same operands)
+    const double dxm = xcur - xg0, dym = ycur - ycl, dxv = xcur - xcl, dyv = ycur - yg0;
+    const double nxy = vxlr * (dxm * dym), nvv = vylr * (dxv * dyv);
+    double qx, qyv, qxy, qxv, qy, qvv;
+    {
+      const Spacing hx(xg1 - xg0), hyc(ych - ycl), hxc(xch - xcl), hy(yg1 - yg0);
+      qx = hx.into(dxm);
+      qyv = hyc.into(dym);
+      qxy = hyc.into(hx.into(nxy));
+      qxv = hxc.into(dxv);
+      qy = hy.into(dyv);
+      qvv = hy.into(hxc.into(nvv));
+      // false for an infinity or a NaN in any of them
+      if (!(fabs(qx + qyv + qxy + qxv + qy + qvv) < 1e300)) {
+        qx = dxm / hx.d;
+        qyv = dym / hyc.d;
+        qxy = nxy / hx.d / hyc.d;
+        qxv = dxv / hxc.d;
+        qy = dyv / hy.d;
+        qvv = nvv / hxc.d / hy.d;
+      }
+    }
+    // ghost values by the kind of the wall: 0 a given velocity, 1 free slip, else 0
+    double vxul = vrow ? vx0 : (top0 ? top2 - vxll : (top1 ? vxll : 0.0));
+    double vxur = vrow ? vx1 : (top0 ? top2 - vxlr : (top1 ? vxlr : 0.0));
+    double a = vxul * (1.0 - qx) * (1.0 - qyv);
+    a += vxur * (qx) * (1.0 - qyv);
+    a += vxll * (1.0 - qx) * (qyv);
+    a += qxy;
+    double vyul = vcol ? vy0 : (left0 ? left2 - vyur : (left1 ? vyur : 0.0));
+    double vyll = vcol ? vy1 : (left0 ? left2 - vylr : (left1 ? vylr : 0.0));
+    double b = vyul * (1.0 - qxv) * (1.0 - qy);
+    b += vyur * (qxv) * (1.0 - qy);
+    b += vyll * (1.0 - qxv) * (qy);
+    b += qvv;
+
+    double w = (1.0 - qx) * (1.0 - qy) * w00;
+    w += (qx) * (1.0 - qy) * w01;
+    w += (1.0 - qx) * (qy) * w10;
+    w += (qx) * (qy) * w11;
     if (irk == 0) {
       svx = a;
       svy = b;

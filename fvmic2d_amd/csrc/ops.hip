@@ -32,7 +32,7 @@
 // A periodic grid (PER) reads the grid coordinates at ghost indices -1 .. NX+1,
 // so it takes the path without staging.
 template <bool LDS, bool PER, class Tail>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LDS ? 5 : 4))) k_advect_rk4(DGrid g, int32_t n, double *__restrict__ MX, double *__restrict__ MY,
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k_advect_rk4(DGrid g, int32_t n, double *__restrict__ MX, double *__restrict__ MY,
                                                     double *__restrict__ MVX, double *__restrict__ MVY,
                                                     double *__restrict__ Mwxy,
                                                     const int32_t *__restrict__ cellXa, const int32_t *__restrict__ cellYa,
@@ -53,19 +53,27 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(LDS ? 
     gl.y = sgrid + g.NX;
     gl.xc = sgrid + g.NX + g.NY;
     gl.yc = sgrid + 2 * g.NX + g.NY + 1;
+    // a tile's cells and positions are read while the one before it is advected
     const int64_t m0 = (int64_t)blockIdx.x * (256 * tiles) + threadIdx.x;
+    int cx = -1, cy = -1;
+    double X0 = 0.0, Y0 = 0.0;
+    if (m0 < n) cx = cellXa[m0], cy = cellYa[m0], X0 = MX[m0], Y0 = MY[m0];
 #pragma unroll 1
     for (int t = 0; t < tiles; t++) {
-      const int64_t m = m0 + 256 * t;
+      const int64_t m = m0 + 256 * t, m1 = m + 256;
+      int cx1 = -1, cy1 = -1;
+      double X1 = 0.0, Y1 = 0.0;
+      if (t + 1 < tiles && m1 < n) cx1 = cellXa[m1], cy1 = cellYa[m1], X1 = MX[m1], Y1 = MY[m1];
       if (m < n)
-        advect_marker<PER>(m, gl, MX, MY, MVX, MVY, Mwxy, cellXa, cellYa, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub,
-                      dt_thermal, tail);
+        advect_marker<PER>(m, gl, MX, MY, MVX, MVY, Mwxy, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub, dt_thermal, tail,
+                           cx, cy, X0, Y0);
+      cx = cx1, cy = cy1, X0 = X1, Y0 = Y1;
     }
   } else {
     const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= n) return;
-    advect_marker<PER>(m, g, MX, MY, MVX, MVY, Mwxy, cellXa, cellYa, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub,
-                  dt_thermal, tail);
+    advect_marker<PER>(m, g, MX, MY, MVX, MVY, Mwxy, vx, vy, wxy, bv, dt, MT, MTdot, dTn, dTsub, dt_thermal, tail,
+                       cellXa[m], cellYa[m], MX[m], MY[m]);
   }
 }
 
