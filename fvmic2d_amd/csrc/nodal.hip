@@ -125,24 +125,14 @@ __global__ void __launch_bounds__(256) k_nodal_heat(int NX, int NY, const double
   sii[i] = s;
 }
 
-// retrieveSolutions.c:10-36: scale the pressure entries of S in place, copy the
-// three components out
-__global__ void __launch_bounds__(256) k_retrieve(int64_t nn, double *__restrict__ S, double Kcont,
-                                                  double *__restrict__ vx, double *__restrict__ vy,
-                                                  double *__restrict__ p) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= nn) return;
-  const double sp = S[3 * i + 2] * Kcont;
-  S[3 * i + 2] = sp;
-  p[i] = sp;
-  vx[i] = S[3 * i + 0];
-  vy[i] = S[3 * i + 1];
-}
-
 // retrieveSolutions.c:49-61: p_mean = sum over ix = 1..NX-1 of p[1][ix]*dx/LX,
-// added in index order by one thread (the terms are formed in parallel)
+// added in index order by one thread (the terms are formed in parallel, from the
+// solution vector itself, so that the copy below can remove the mean as it goes:
+// no second pass over p).  The chain of additions is what the pass takes; the
+// terms come from LDS eight at a time, so that no addition waits for its term.
 #define PMEAN_CHUNK 2048
-__global__ void __launch_bounds__(256) k_pmean(DGrid g, const double *__restrict__ p, double *__restrict__ out) {
+__global__ void __launch_bounds__(256) k_pmean(DGrid g, const double *__restrict__ S, double Kcont,
+                                               double *__restrict__ out) {
   __shared__ double t[PMEAN_CHUNK];
   const int NX = g.NX;
   double acc = 0.0;
@@ -151,23 +141,39 @@ __global__ void __launch_bounds__(256) k_pmean(DGrid g, const double *__restrict
     for (int k = threadIdx.x; k < cn; k += blockDim.x) {
       const int ix = c0 + k;
       const double dx = g.x[ix] - g.x[ix - 1];
-      t[k] = N2(p, 1, ix) * dx / g.LX;
+      const double p = S[3 * ((int64_t)NX + ix) + 2] * Kcont;
+      t[k] = p * dx / g.LX;
     }
     __syncthreads();
-    if (threadIdx.x == 0)
-      for (int k = 0; k < cn; k++) acc += t[k];
+    if (threadIdx.x == 0) {
+      int k = 0;
+      for (; k + 8 <= cn; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = t[k + e];
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc += v[e];
+      }
+      for (; k < cn; k++) acc += t[k];
+    }
     __syncthreads();
   }
   if (threadIdx.x == 0) *out = acc;
 }
 
-// retrieveSolutions.c:65-75: remove the mean from every node with jy > 0, ix > 0
-__global__ void __launch_bounds__(256) k_pshift(int NX, int NY, double *__restrict__ p,
-                                                const double *__restrict__ pm) {
+// retrieveSolutions.c:10-36, 65-75: scale the pressure entries of S in place, copy
+// the three components out, without the mean (`pm`, null: nothing to remove) at
+// every node with jy > 0, ix > 0
+__global__ void __launch_bounds__(256) k_retrieve(int NX, int64_t nn, double *__restrict__ S, double Kcont,
+                                                  const double *__restrict__ pm, double *__restrict__ vx,
+                                                  double *__restrict__ vy, double *__restrict__ p) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (int64_t)NX * NY) return;
-  const int ix = (int)(i % NX), jy = (int)(i / NX);
-  if (ix > 0 && jy > 0) p[i] = p[i] - *pm;
+  if (i >= nn) return;
+  const double u = S[3 * i + 0], v = S[3 * i + 1], sp = S[3 * i + 2] * Kcont;
+  S[3 * i + 2] = sp;
+  vx[i] = u;
+  vy[i] = v;
+  p[i] = pm && i >= NX && i % NX > 0 ? sp - *pm : sp;
 }
 
 // limitTimestep.c:39-107: every node offers up to three candidate steps (vx,
@@ -317,14 +323,13 @@ extern "C" int fvm_retrieve_solutions(fvm_ctx *ctx, const fvm_grid *g, const Nod
   FVM_TRY(fvm_ws(ctx, ctx->red, 4096));
   double *pm = (double *)((char *)ctx->red.ptr + 512);
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  k_retrieve<<<fvm_blocks(nn, 256), 256, 0, ctx->stream>>>(nn, S, Kcont, nf->vx, nf->vy, nf->p);
-  FVM_LAUNCH_CHECK(ctx);
   if (g->NY > 1) {
-    k_pmean<<<1, 256, 0, ctx->stream>>>(dgrid(g), nf->p, pm);
-    FVM_LAUNCH_CHECK(ctx);
-    k_pshift<<<fvm_blocks(nn, 256), 256, 0, ctx->stream>>>(g->NX, g->NY, nf->p, pm);
+    k_pmean<<<1, 256, 0, ctx->stream>>>(dgrid(g), S, Kcont, pm);
     FVM_LAUNCH_CHECK(ctx);
   }
+  k_retrieve<<<fvm_blocks(nn, 256), 256, 0, ctx->stream>>>(g->NX, nn, S, Kcont, g->NY > 1 ? pm : nullptr, nf->vx,
+                                                           nf->vy, nf->p);
+  FVM_LAUNCH_CHECK(ctx);
   if (foundnan) *foundnan = 0;  // the reference checks for NaN only when built with TEXTURE
   return FVM_OK;
 }
@@ -337,18 +342,16 @@ extern "C" int fvm_limit_displacement_timestep(fvm_ctx *ctx, const fvm_grid *g, 
   const int64_t nn = (int64_t)g->NX * g->NY;
   const int nb = (int)std::min<int64_t>(fvm_blocks(nn, 256), DT_BLOCKS);
   FVM_TRY(fvm_ws(ctx, ctx->red, 4096 + (size_t)DT_BLOCKS * sizeof(DtPart)));
-  double *dout = (double *)((char *)ctx->red.ptr + 520);
+  double *h = (double *)ctx->pinned.ptr + 24;  // written there by the last kernel itself
   DtPart *part = (DtPart *)((char *)ctx->red.ptr + 4096);
   {
     FVM_PHASE(ctx, FVM_PHASE_OTHER);
     k_dt_partial<<<nb, 256, 0, ctx->stream>>>(dgrid(g), nf->vx, nf->vy, nf->rho, nf->rhodot,
                                               opt->displacementStepLimit, part);
     FVM_LAUNCH_CHECK(ctx);
-    k_dt_final<<<1, 256, 0, ctx->stream>>>(nb, part, nf->rhodot, *displacementdt, nullptr, dout);
+    k_dt_final<<<1, 256, 0, ctx->stream>>>(nb, part, nf->rhodot, *displacementdt, nullptr, h);
     FVM_LAUNCH_CHECK(ctx);
   }
-  double *h = (double *)ctx->pinned.ptr + 24;
-  FVM_HIP(ctx, hipMemcpyAsync(h, dout, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   *displacementdt = *h;
   return FVM_OK;
