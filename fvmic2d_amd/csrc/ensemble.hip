@@ -308,12 +308,9 @@ __device__ __forceinline__ void ens_advect_block(const InstDev &I, int64_t lb, c
                                                  const double *__restrict__ deltaT, const double *__restrict__ dTsub) {
   const int64_t m = lb * (int64_t)blockDim.x + threadIdx.x;
   if (m >= I.nMark) return;
+  const RotateTail tail = {I.sxx, I.syy, I.sxy, I.Eii, I.exx, I.eyy, I.exy, I.dt, I.jaumann};
   advect_marker<false>(m, gl, I.X, I.Y, I.VX, I.VY, I.wxy, I.vx, I.vy, I.wxyn, I.bv, I.dt, I.T, I.Tdot,
-                       deltaT + I.node_off, dTsub + I.mark_off, I.dt, NoTail(), I.cellX[m], I.cellY[m], I.X[m],
-                       I.Y[m]);
-  // the rotation fused behind the RK4 stages: the batched launch keeps one kernel per phase
-  rotate_eii_marker(m, I.g.ncx(), I.g.NY, I.cellX, I.cellY, I.wxy, I.sxx, I.syy, I.sxy, I.exx, I.eyy, I.exy, I.Eii,
-                    I.dt, I.jaumann);
+                       deltaT + I.node_off, dTsub + I.mark_off, I.dt, tail, I.cellX[m], I.cellY[m], I.X[m], I.Y[m]);
 }
 
 // ---- per-phase kernels ------------------------------------------------------------------

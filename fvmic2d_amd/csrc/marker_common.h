@@ -34,10 +34,7 @@ struct Spacing {
 
 // c0x, c0y, X0, Y0: the marker's stored cell and position (the caller reads them,
 // a marker ahead where it can).  tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's stages are done, with
-// its old position and cell and its new spin (NoTail: nothing).
-struct NoTail {
-  __device__ __forceinline__ void operator()(int64_t, const DGrid &, double, double, int, int, double) const {}
-};
+// its old position and cell and its new spin.
 template <bool PER, class Tail>
 __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MX,
@@ -259,10 +256,11 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
   tail(m, g, X0, Y0, c0x, c0y, wm);
 }
 
-// ---- A6, second pass: the stress rotation by the marker spin and the strain
-// invariant update (markers.c:2141-2164, 2223), after advect_marker has stored the spin
-// wxy = (k1 + 2 k2 + 2 k3 + k4) / 6.  A pass of its own: the RK4 pass then holds
-// fewer live registers and hides more of its gather latency, and this one streams.
+// ---- A6, second part: the stress rotation by the marker spin (k1 + 2 k2 + 2 k3 +
+// k4) / 6 and the strain invariant update (markers.c:2141-2164, 2223).  Behind the
+// stages of each marker: their registers are free by then, and the columns stream
+// while other wavefronts compute (as a pass of its own it read the cells and the
+// spin again: 4 M tracers 743 us a step, so 729; 1.44 M markers 254 either way).
 __device__ __forceinline__ void rotate_stress(double &sxx, double &syy, double &sxy, double wm, double dt,
                                               int jaumann) {
   const double msxx0 = sxx, msyy0 = syy, msxy0 = sxy;
@@ -285,29 +283,22 @@ __device__ __forceinline__ void rotate_stress(double &sxx, double &syy, double &
   }
 }
 
-// ncx: basic cells along x (NX - 1, or NX on a periodic grid)
-__device__ __forceinline__ void rotate_eii_marker(int64_t m, int ncx, int NY,
-    const int32_t *__restrict__ cellXa,
-    const int32_t *__restrict__ cellYa,
-    const double *__restrict__ Mwxy,
-    double *__restrict__ sxx,
-    double *__restrict__ syy,
-    double *__restrict__ sxy,
-    const double *__restrict__ exx,
-    const double *__restrict__ eyy,
-    const double *__restrict__ exy,
-    double *__restrict__ Eii,
-    double dt,
-    int jaumann) {
-  if (!cell_ok(cellXa[m], cellYa[m], ncx, NY)) return;
-  double s11 = sxx[m], s22 = syy[m], s12 = sxy[m];
-  rotate_stress(s11, s22, s12, Mwxy[m], dt, jaumann);
-  sxx[m] = s11;
-  syy[m] = s22;
-  sxy[m] = s12;
-  const double e11 = exx[m], e22 = eyy[m], e12 = exy[m];
-  Eii[m] = Eii[m] + dt * sqrt(0.5 * (e11 * e11 + e22 * e22) + e12 * e12);
-}
+// The rotation behind a marker's advection.
+struct RotateTail {
+  double *sxx, *syy, *sxy, *Eii;
+  const double *exx, *eyy, *exy;
+  double dt;
+  int jaumann;
+  __device__ __forceinline__ void operator()(int64_t m, const DGrid &, double, double, int, int, double wm) const {
+    double s11 = sxx[m], s22 = syy[m], s12 = sxy[m];
+    rotate_stress(s11, s22, s12, wm, dt, jaumann);
+    sxx[m] = s11;
+    syy[m] = s22;
+    sxy[m] = s12;
+    const double e11 = exx[m], e22 = eyy[m], e12 = exy[m];
+    Eii[m] = Eii[m] + dt * sqrt(0.5 * (e11 * e11 + e22 * e22) + e12 * e12);
+  }
+};
 
 // ---- A9: updateMarkerStress (updateMarkerStress.c:5-163): a marker's increments ----
 template <int MODE>

@@ -27,7 +27,7 @@
 // in LDS once per block, and each block walks `tiles` tiles of 256 markers so
 // that the staging is amortised (2 for small grids, one more per ADV_TILE_BYTES
 // of staged grid beyond that, at most 8); the per-marker arithmetic is unchanged.
-// k_rotate_eii then rotates the stresses and updates Eii in a streaming pass.
+// The tail rotates the stresses and updates Eii behind each marker.
 #define ADV_TILE_BYTES 4096
 // A periodic grid (PER) reads the grid coordinates at ghost indices -1 .. NX+1,
 // so it takes the path without staging.
@@ -77,18 +77,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(5))) k
   }
 }
 
-__global__ void __launch_bounds__(256) k_rotate_eii(int32_t n, int ncx, int NY, const int32_t *__restrict__ cellXa,
-                                                    const int32_t *__restrict__ cellYa,
-                                                    const double *__restrict__ Mwxy, double *__restrict__ sxx,
-                                                    double *__restrict__ syy, double *__restrict__ sxy,
-                                                    const double *__restrict__ exx, const double *__restrict__ eyy,
-                                                    const double *__restrict__ exy, double *__restrict__ Eii,
-                                                    double dt, int jaumann) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m >= n) return;
-  rotate_eii_marker(m, ncx, NY, cellXa, cellYa, Mwxy, sxx, syy, sxy, exx, eyy, exy, Eii, dt, jaumann);
-}
-
 // The RK4 pass, tail behind every marker (`wrap` is the tail of a periodic grid).
 template <class Tail, class Wrap>
 static int launch_rk4(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const NodalArrays *nf,
@@ -118,13 +106,8 @@ static int launch_rk4(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const No
 static int launch_advect(fvm_ctx *ctx, const fvm_grid *g, fvm_markers *mk, const NodalArrays *nf,
                          const BoundaryValues *bv, double dt, int jaumann, const double *deltaT, const double *dTsub,
                          double dt_thermal) {
-  const int32_t n = mk->nMark;
-  FVM_TRY(launch_rk4(ctx, g, mk, nf, bv, dt, deltaT, dTsub, dt_thermal, NoTail(), NoTail()));
-  k_rotate_eii<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(n, fvm_ncx(g), g->NY, mk->cellX, mk->cellY, mk->wxy, mk->sxx,
-                                                            mk->syy, mk->sxy, mk->exx, mk->eyy, mk->exy, mk->Eii, dt,
-                                                            jaumann);
-  FVM_LAUNCH_CHECK(ctx);
-  return FVM_OK;
+  const RotateTail tail = {mk->sxx, mk->syy, mk->sxy, mk->Eii, mk->exx, mk->eyy, mk->exy, dt, jaumann};
+  return launch_rk4(ctx, g, mk, nf, bv, dt, deltaT, dTsub, dt_thermal, tail, tail);
 }
 
 extern "C" int fvm_advect_markers_rk(fvm_ctx *ctx, fvm_markers *mk, const NodalArrays *nf, const fvm_grid *g,
