@@ -118,16 +118,45 @@ __global__ void __launch_bounds__(256) k_pc_plan(PcParams P, const int32_t *__re
   rem[q] = r;
 }
 
-__global__ void __launch_bounds__(256) k_pc_out_flags(int32_t n, const int32_t *__restrict__ cellX,
-                                                      int32_t *__restrict__ flag) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < n) flag[m] = cellX[m] == -1 ? 1 : 0;
+// The markers without a cell in ascending order.  Each block counts its OUT_RUN
+// markers, the counts are scanned, and a block with any lists them; the flags and
+// positions of all markers are never written (4 M markers: three passes and a scan
+// over every marker, so two reads of the cells and a scan of 2000 counts).
+#define OUT_RUN 2048
+__global__ void __launch_bounds__(256) k_pc_out_count(int32_t n, const int32_t *__restrict__ cellX,
+                                                      int32_t *__restrict__ count) {
+  __shared__ int32_t s_c[4];
+  const int64_t m0 = (int64_t)blockIdx.x * OUT_RUN + threadIdx.x;
+  int32_t c = 0;
+#pragma unroll
+  for (int k = 0; k < OUT_RUN / 256; k++) {
+    const int64_t m = m0 + 256 * k;
+    c += __popcll(__ballot(m < n && cellX[m] == -1));
+  }
+  if ((threadIdx.x & 63) == 0) s_c[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) count[blockIdx.x] = s_c[0] + s_c[1] + s_c[2] + s_c[3];
 }
 
-__global__ void __launch_bounds__(256) k_pc_out_list(int32_t n, const int32_t *__restrict__ flag,
-                                                     const int32_t *__restrict__ pos, int32_t *__restrict__ isout) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (m < n && flag[m]) isout[pos[m]] = (int32_t)m;
+__global__ void __launch_bounds__(256) k_pc_out_list(int32_t n, const int32_t *__restrict__ cellX,
+                                                     const int32_t *__restrict__ first, int32_t *__restrict__ out) {
+  __shared__ int32_t s_c[4];
+  int32_t base = first[blockIdx.x];
+  if (first[blockIdx.x + 1] == base) return;  // the whole block
+  const int64_t m0 = (int64_t)blockIdx.x * OUT_RUN + threadIdx.x;
+  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  for (int k = 0; k < OUT_RUN / 256; k++) {
+    const int64_t m = m0 + 256 * k;
+    const bool is = m < n && cellX[m] == -1;
+    const unsigned long long b = __ballot(is);
+    if (lane == 0) s_c[wv] = __popcll(b);
+    __syncthreads();
+    int32_t before = 0;
+    for (int v = 0; v < wv; v++) before += s_c[v];
+    if (is) out[base + before + __popcll(b & ((1ull << lane) - 1ull))] = (int32_t)m;
+    base += s_c[0] + s_c[1] + s_c[2] + s_c[3];
+    __syncthreads();
+  }
 }
 
 // markers.c:616-663: the rem[q] members with the lowest (key, position) leave,
@@ -388,7 +417,7 @@ __device__ __forceinline__ int build_special(const PcParams &P, const YieldParam
 }
 
 __global__ void __launch_bounds__(256) k_pc_write(PcParams P, YieldParams Yp, int32_t nAdd, NewMarkers nm,
-                                                  MarkerCols mc, int32_t *__restrict__ flags) {
+                                                  MarkerCols mc, int32_t *__restrict__ bad) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= nAdd || !nm.valid[i]) return;  // no neighbour: the slot is left as it is
   const int32_t slot = nm.slot[i], root = nm.root[i];
@@ -402,7 +431,7 @@ __global__ void __launch_bounds__(256) k_pc_write(PcParams P, YieldParams Yp, in
   } else {
     const int32_t k0 = -1 - root;  // the slab / inflow marker whose fields are copied
     if (build_special(P, Yp, nm.kind[k0], nm.X[k0], nm.Y[k0], d, n))
-      __hip_atomic_store(&flags[1], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *bad = 1;  // every writer stores the same value
     n[1] = nm.cx[k0];
     n[2] = nm.cy[k0];
   }
@@ -419,8 +448,12 @@ __global__ void k_pc_zero(int32_t *__restrict__ a, int64_t n) {
   if (i < n) a[i] = 0;
 }
 
-// largest cell width and height (one block)
-__global__ void __launch_bounds__(256) k_pc_spacing(DGrid g, double *out) {
+// largest cell width and height, and the plan's totals, to the host's pinned
+// memory (one block): out[0..1] the spacings, tot the additions, removals, markers
+// without a cell and the plan's flag
+__global__ void __launch_bounds__(256) k_pc_totals(DGrid g, const int32_t *add, const int32_t *rem,
+                                                   const int32_t *outs, const int32_t *flag, double *out,
+                                                   int32_t *tot) {
   __shared__ double s_w[256], s_h[256];
   double w = 0.0, h = 0.0;
   for (int i = threadIdx.x; i < g.NX - 1; i += 256) w = fmax(w, g.x[i + 1] - g.x[i]);
@@ -438,6 +471,10 @@ __global__ void __launch_bounds__(256) k_pc_spacing(DGrid g, double *out) {
   if (threadIdx.x == 0) {
     out[0] = s_w[0];
     out[1] = s_h[0];
+    tot[0] = *add;
+    tot[1] = *rem;
+    tot[2] = outs ? *outs : 0;
+    tot[3] = *flag;
   }
 }
 
@@ -457,10 +494,10 @@ extern "C" int fvm_check_marker_density(fvm_ctx *ctx, const fvm_grid *g, fvm_mar
   // the bucket order of the current cells (the caller ran findMarkerCells)
   FVM_TRY(fvm_sort_markers(ctx, g, mk));
   const int32_t *start = (const int32_t *)ctx->start.ptr, *perm = (const int32_t *)ctx->perm.ptr;
-  // phase-1 workspace: add, rem (nq), addOff, remOff (nq + 1), out flags / positions
-  // (n, n + 1), out list (n), two scan states, spacing (2 doubles), flags
-  const int64_t nn = n > 0 ? n : 1;
-  const int64_t sq = scan_state_words(nq), sn = scan_state_words(nn);
+  // phase-1 workspace: add, rem (nq), addOff, remOff (nq + 1), out counts / positions
+  // by block, out list (n), three scan states and the flags (zeroed together)
+  const int64_t nn = n > 0 ? n : 1, nb = (nn + OUT_RUN - 1) / OUT_RUN;
+  const int64_t sq = scan_state_words(nq), sn = scan_state_words(nb);
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -468,17 +505,16 @@ extern "C" int fvm_check_marker_density(fvm_ctx *ctx, const fvm_grid *g, fvm_mar
     return o;
   };
   const size_t o_add = take(nq * 4), o_rem = take(nq * 4), o_addOff = take((nq + 1) * 4),
-               o_remOff = take((nq + 1) * 4), o_flag = take(nn * 4), o_pos = take((nn + 1) * 4),
+               o_remOff = take((nq + 1) * 4), o_cnt = take(nb * 4), o_pos = take((nb + 1) * 4),
                o_out = take(nn * 4), o_s1 = take(sq * 8), o_s2 = take(sq * 8), o_s3 = take(sn * 8),
-               o_sp = take(16), o_fl = take(16);
+               o_fl = take(16);
   FVM_TRY(fvm_ws(ctx, ctx->popc, off));
   char *base = (char *)ctx->popc.ptr;
   int32_t *add = (int32_t *)(base + o_add), *rem = (int32_t *)(base + o_rem);
   int32_t *addOff = (int32_t *)(base + o_addOff), *remOff = (int32_t *)(base + o_remOff);
-  int32_t *flag = (int32_t *)(base + o_flag), *pos = (int32_t *)(base + o_pos), *isout = (int32_t *)(base + o_out);
+  int32_t *cnt = (int32_t *)(base + o_cnt), *pos = (int32_t *)(base + o_pos), *isout = (int32_t *)(base + o_out);
   unsigned long long *s1 = (unsigned long long *)(base + o_s1), *s2 = (unsigned long long *)(base + o_s2),
                      *s3 = (unsigned long long *)(base + o_s3);
-  double *spacing = (double *)(base + o_sp);
   int32_t *flags = (int32_t *)(base + o_fl);
 
   PcParams P;
@@ -506,36 +542,28 @@ extern "C" int fvm_check_marker_density(fvm_ctx *ctx, const fvm_grid *g, fvm_mar
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
   // zero the scan states and the flags (kernels, no memset nodes)
   {
-    int32_t *zs[4] = {(int32_t *)s1, (int32_t *)s2, (int32_t *)s3, flags};
-    const int64_t zn[4] = {2 * sq, 2 * sq, 2 * sn, 4};
-    for (int k = 0; k < 4; k++) {
-      k_pc_zero<<<fvm_blocks(zn[k], 256), 256, 0, ctx->stream>>>(zs[k], zn[k]);
-      FVM_LAUNCH_CHECK(ctx);
-    }
+    const int64_t words = (int64_t)(o_fl + 16 - o_s1) / 4;
+    k_pc_zero<<<fvm_blocks(words, 256), 256, 0, ctx->stream>>>((int32_t *)s1, words);
+    FVM_LAUNCH_CHECK(ctx);
   }
-  k_pc_spacing<<<1, 256, 0, ctx->stream>>>(P.g, spacing);
-  FVM_LAUNCH_CHECK(ctx);
   k_pc_plan<<<fvm_blocks(nq, 256), 256, 0, ctx->stream>>>(P, start, perm, mk->X, mk->Y, add, rem, flags);
   FVM_LAUNCH_CHECK(ctx);
   FVM_TRY(fvm_launch_scan_onepass(ctx, add, addOff, s1, nq));
   FVM_TRY(fvm_launch_scan_onepass(ctx, rem, remOff, s2, nq));
   if (n > 0) {
-    k_pc_out_flags<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(n, mk->cellX, flag);
+    k_pc_out_count<<<(unsigned)nb, 256, 0, ctx->stream>>>(n, mk->cellX, cnt);
     FVM_LAUNCH_CHECK(ctx);
-    FVM_TRY(fvm_launch_scan_onepass(ctx, flag, pos, s3, n));
-    k_pc_out_list<<<fvm_blocks(n, 256), 256, 0, ctx->stream>>>(n, flag, pos, isout);
+    FVM_TRY(fvm_launch_scan_onepass(ctx, cnt, pos, s3, nb));
+    k_pc_out_list<<<(unsigned)nb, 256, 0, ctx->stream>>>(n, mk->cellX, pos, isout);
     FVM_LAUNCH_CHECK(ctx);
   }
   // totals to the host: additions, removals, markers without a cell, flags
   int32_t *h = (int32_t *)ctx->pinned.ptr + 64;
-  FVM_HIP(ctx, hipMemcpyAsync(h, addOff + nq, 4, hipMemcpyDeviceToHost, ctx->stream));
-  FVM_HIP(ctx, hipMemcpyAsync(h + 1, remOff + nq, 4, hipMemcpyDeviceToHost, ctx->stream));
-  if (n > 0) FVM_HIP(ctx, hipMemcpyAsync(h + 2, pos + n, 4, hipMemcpyDeviceToHost, ctx->stream));
-  FVM_HIP(ctx, hipMemcpyAsync(h + 3, flags, 4, hipMemcpyDeviceToHost, ctx->stream));
   double *hd = (double *)ctx->pinned.ptr + 40;
-  FVM_HIP(ctx, hipMemcpyAsync(hd, spacing, 16, hipMemcpyDeviceToHost, ctx->stream));
+  k_pc_totals<<<1, 256, 0, ctx->stream>>>(P.g, addOff + nq, remOff + nq, n > 0 ? pos + nb : nullptr, flags, hd, h);
+  FVM_LAUNCH_CHECK(ctx);
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  const int32_t nAdd = h[0], nRem = h[1], nOut0 = n > 0 ? h[2] : 0;
+  const int32_t nAdd = h[0], nRem = h[1], nOut0 = h[2];
   if (h[3])
     return fvm_set_err(ctx, FVM_ERR_NEGATIVE_ADD,
                        "checkMarkerDensity: an under-full quarter's target does not exceed its count");
@@ -589,14 +617,14 @@ extern "C" int fvm_check_marker_density(fvm_ctx *ctx, const fvm_grid *g, fvm_mar
     for (int k = 0; k < 23; k++) mc.d[k] = dc[k];
     for (int k = 0; k < 5; k++) mc.n[k] = ic[k];
     const YieldParams Yp = make_yield_params(mat, opt, 0.0);
-    k_pc_write<<<fvm_blocks(nAdd, 256), 256, 0, ctx->stream>>>(P, Yp, nAdd, nm, mc, flags);
+    h[4] = 0;
+    k_pc_write<<<fvm_blocks(nAdd, 256), 256, 0, ctx->stream>>>(P, Yp, nAdd, nm, mc, h + 4);
     FVM_LAUNCH_CHECK(ctx);
-    FVM_HIP(ctx, hipMemcpyAsync(h + 3, flags + 1, 4, hipMemcpyDeviceToHost, ctx->stream));
     FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
     fvm_markers_moved(ctx);
     if (nAdd > nOut) mk->nMark = n + (nAdd - nOut);
     if (nAdded) *nAdded = nAdd;
-    if (h[3]) return fvm_set_err(ctx, FVM_ERR_VISCOSITY_LAW, "viscosity law undefined for material 0");
+    if (h[4]) return fvm_set_err(ctx, FVM_ERR_VISCOSITY_LAW, "viscosity law undefined for material 0");
   } else if (after > mk->maxMark) {
     return fvm_set_err(ctx, FVM_ERR_CAPACITY, "checkMarkerDensity: %d markers to add, %d of %d slots free", nAdd,
                        mk->maxMark - (n - nOut), mk->maxMark);
