@@ -581,14 +581,16 @@ def bench_pressure_guess(a):
            "config": {"workload": "pressure_guess_box", "grid": main_row["grid"],
                       "solver": "BiCGStab preconditioned by a multigrid V-cycle, rtol 1e-10"},
            "grids": rows,
-           # one iteration streams 37 FP64 values per node through its five kernels
-           # (p: r, p, v, Dinv -> p, y; v: y, 5 coefficients, rhat -> v; s: r, v, y, x,
-           # Dinv -> x, s, z; t: z, 5 coefficients, s -> t; x: x, z, s, t, rhat -> x, r)
-           "roofline": {"bound": "hbm", "kernel": "BiCGStab iteration (5 kernels)",
-                        "achieved": 37 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
+           # one iteration touches about 80 FP64 values per node: 37 in the iteration's
+           # own vectors and coefficients, 16 on the fine level of each of its two
+           # V-cycles (residual, correction, coefficients, down and up) and a third of
+           # those again on the coarser levels; a 257 x 257 problem stays in cache, so
+           # what bounds it is the chain of launches and the coarse levels' barriers
+           "roofline": {"bound": "hbm", "kernel": "BiCGStab iteration with two V-cycles",
+                        "achieved": 80 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
                         / (main_row["gpu_ms"] * 1e-3) / 1e9,
                         "peak": 8000.0, "unit": "GB/s",
-                        "frac": 37 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
+                        "frac": 80 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
                         / (main_row["gpu_ms"] * 1e-3) / 1e9 / 8000.0, "traffic": None},
            "cpu_baseline": None if a.no_cpu else {
                "value": main_row["cpu_direct_ms"], "unit": "ms", "cores": 1, "kind": "port",

@@ -418,7 +418,7 @@ int fvm_timer_stop(fvm_ctx *ctx, float *ms);
  * problem for the cell-centre pressure with the density-gradient source,
  * assembled as in initialPressureGuess.c:59-135 (dummy rows on ix == 0 and
  * jy == 0, pressure pinned in cell (3, 3), zero-flux sides, dp/dy = rho g on
- * top and bottom), solved on the GPU (matrix-free operator, Jacobi BiCGStab,
+ * top and bottom), solved on the GPU (matrix-free operator, multigrid BiCGStab,
  * relative residual <= rtol, at most maxit iterations).  rho: device NX*NY
  * nodal density.  The pressure goes to S[3*(jy*NX+ix) + 2] (the DOF_P slot of
  * the interleaved [vx, vy, p] Stokes vector, fdcode.h:242-245; velocities are
