@@ -146,6 +146,8 @@ __device__ __forceinline__ double parts_1024(const double *__restrict__ part, in
 // (8 waves per SIMD: two blocks a CU, so that 801 x 401's 338 run at once)
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) k_one_p(int NX, int NY, Coefs c, Cheb ch, FvmBcgOne O) {
   __shared__ double sh[2][Region::RW * Region::RW];
+  // an iteration enqueued behind the last one: k_one_x has written no partials since
+  if (O.sc[FVM_S_DONE] != 0.0) return;
   const double rho = parts_1024(O.prho, O.n_r), rr = parts_1024(O.prr, O.n_r);
   const bool lead = blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0;
   const double bb = O.first ? rr : O.sc[FVM_S_BB];

@@ -1,0 +1,42 @@
+"""The nodal solves at the limits of what they take: a zero right-hand side behind
+another solve, whose leftovers lie in the workspace."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from fvmic2d_amd import workloads
+from fvmic2d_amd.lib import Context, DeviceArray, DeviceGrid
+
+pytestmark = pytest.mark.gpu
+
+
+def _dominant(NX, NY):
+    """Rows whose diagonal outweighs the couplings (their sum: 0.4)."""
+    c = np.zeros((5, NY, NX))
+    c[0] = 1.0
+    c[1, :, :-1] = c[2, :, 1:] = -0.1
+    c[3, :-1] = c[4, 1:] = -0.1
+    return c
+
+
+def _solve(ctx, NX, NY, coef, rhs, rtol=1e-12, maxit=2000):
+    """(T, iterations, relative residual) of fvm_solve_thermal_system."""
+    grid = DeviceGrid(ctx, workloads.thermal_box(NX, NY))
+    d = [DeviceArray(ctx, np.ascontiguousarray(a).ravel()) for a in (coef, rhs, np.full(NX * NY, 7.0))]
+    its, rel = C.c_int32(-1), C.c_double(-1.0)
+    ctx.call("fvm_solve_thermal_system", grid.ref, *(C.c_void_p(a.ptr) for a in d), C.c_double(rtol),
+             C.c_int32(maxit), C.byref(its), C.byref(rel))
+    return d[2].get().reshape(NY, NX), its.value, rel.value
+
+
+@pytest.mark.parametrize("NX,NY", [(12, 9), (33, 20), (100, 47)])
+def test_zero_right_hand_side(NX, NY):
+    """x = 0 without an iteration, whatever the solve before left behind."""
+    print("CASE zero right-hand side", NX, NY, flush=True)
+    ctx = Context()
+    r = np.random.default_rng(2)
+    big = 6 * NX, 6 * NY    # its right-hand side lies over the small solve's whole workspace
+    _solve(ctx, *big, _dominant(*big), 1.0 + r.random(big[::-1]))
+    x, its, rel = _solve(ctx, NX, NY, _dominant(NX, NY), np.zeros((NY, NX)))
+    assert not np.any(x) and its == 0 and rel == 0.0
