@@ -270,15 +270,18 @@ __global__ void __launch_bounds__(256 * WN) k_conv(ConvArgs a) {
   }
 }
 
-// Layers whose patch does not fit LDS with all channels (above 600 or so): the
-// fragments come from global memory, 2 x 2 tiles per wavefront.
+// The same sums with fragments straight from global memory, 2 x 2 tiles per
+// wavefront, 64 pixels x 64 channels per block.  A pixel's addresses are formed once
+// per tap.  conv_direct says which layers take it.  TR (1x1): the weights are read as
+// they lie, 16 lanes a row; 1024 -> 1024, 4096 pixels: 55 us, 66 from turned weights.
 template <int K, bool TR>
-__global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
+__global__ void __launch_bounds__(256) k_conv_direct(ConvArgs a) {
   constexpr int T = K * K;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
   const int64_t npix = (int64_t)a.B * a.H * a.Wd;
   const int64_t p0 = (int64_t)blockIdx.x * 64 + (wv & 1) * 32;
   const int c0 = blockIdx.y * 64 + (wv >> 1) * 32;
+  const int C0 = a.in.C0, C1 = a.Cin - C0;
   int64_t pp[2];
   int pb[2], ph[2], pw[2];
 #pragma unroll
@@ -290,32 +293,41 @@ __global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
     pb[r] = (int)(q / ((int64_t)a.Wd * a.H));
   }
   const bf8 zero = __builtin_bit_cast(bf8, make_uint4(0u, 0u, 0u, 0u));
+  auto weights = [&](const uint16_t *w, int k) {
+    if (!TR) return __builtin_bit_cast(bf8, *(const uint4 *)(w + k));
+    Bf8Builder e;
+    for (int i = 0; i < 8; i++) e.h[i] = w[(int64_t)(k + i) * a.Cout];
+    return e.get();
+  };
   f4 acc[2][2] = {};
 #pragma unroll 1
   for (int t = 0; t < T; t++) {
-    const int dy = t / K - K / 2, dx = t % K - K / 2;
+    const uint16_t *xa[2], *xb[2], *w[2];  // channels below C0, from C0 on; weights
+    bool in[2], out[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      const int h = ph[r] + t / K - K / 2, ww = pw[r] + t % K - K / 2;
+      in[r] = pp[r] >= 0 && h >= 0 && h < a.H && ww >= 0 && ww < a.Wd;
+      const int hi = in[r] ? h : 0, wi = in[r] ? ww : 0;
+      xa[r] = a.in.X + (((int64_t)pb[r] * (a.H >> a.in.up) + (hi >> a.in.up)) * (a.Wd >> a.in.up) + (wi >> a.in.up)) * C0;
+      xb[r] = C1 ? a.in.X2 + (((int64_t)pb[r] * a.H + hi) * a.Wd + wi) * C1 - C0 : xa[r];
+    }
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+      const int co = c0 + 16 * n + li;
+      out[n] = co < a.Cout;
+      w[n] = TR ? a.W + (int64_t)(T - 1 - t) * a.Cin * a.Cout + (out[n] ? co : 0)
+                : a.W + ((int64_t)t * a.Cout + (out[n] ? co : 0)) * a.Cin;
+    }
     for (int k0 = 0; k0 < a.Cin; k0 += 32) {
       const int k = k0 + 8 * g;
+      const bool kin = k < a.Cin;
       bf8 fx[2], fw[2];
 #pragma unroll
-      for (int r = 0; r < 2; r++) {
-        const bool ok = pp[r] >= 0 && k < a.Cin && ph[r] + dy >= 0 && ph[r] + dy < a.H && pw[r] + dx >= 0 && pw[r] + dx < a.Wd;
-        fx[r] = ok ? __builtin_bit_cast(bf8, *(const uint4 *)input_at(a.in, a.Cin, pb[r], a.H, a.Wd, ph[r] + dy, pw[r] + dx, k))
-                   : zero;
-      }
+      for (int r = 0; r < 2; r++)
+        fx[r] = in[r] && kin ? __builtin_bit_cast(bf8, *(const uint4 *)((k < C0 ? xa[r] : xb[r]) + k)) : zero;
 #pragma unroll
-      for (int n = 0; n < 2; n++) {
-        const int co = c0 + 16 * n + li;
-        fw[n] = zero;
-        if (co >= a.Cout || k >= a.Cin) continue;
-        if (!TR) {
-          fw[n] = __builtin_bit_cast(bf8, *(const uint4 *)(a.W + ((int64_t)t * a.Cout + co) * a.Cin + k));
-        } else {
-          Bf8Builder w;
-          for (int i = 0; i < 8; i++) w.h[i] = a.W[((int64_t)(T - 1 - t) * a.Cin + k + i) * a.Cout + co];
-          fw[n] = w.get();
-        }
-      }
+      for (int n = 0; n < 2; n++) fw[n] = out[n] && kin ? weights(w[n], k) : zero;
 #pragma unroll
       for (int n = 0; n < 2; n++)
 #pragma unroll
@@ -326,18 +338,57 @@ __global__ void __launch_bounds__(256) k_conv_wide(ConvArgs a) {
   for (int n = 0; n < 2; n++) {
     const int co = c0 + 16 * n + 4 * g;
     if (co >= a.Cout) continue;
+    const f4 bv = a.bias ? ld4(a.bias + co) : (f4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int r = 0; r < 2; r++) {
       if (pp[r] < 0) continue;
+      f4 v = acc[r][n] + bv;
+      h4u h;
+#pragma unroll
       for (int i = 0; i < 4; i++) {
-        float v = acc[r][n][i] + (a.bias ? a.bias[co + i] : 0.f);
-        if (a.relu) v = v > 0.f ? v : 0.f;
-        if (co + i >= a.cout_real) v = 0.f;
-        const int64_t o = pp[r] * a.Cout + co + i;
-        if (a.Y) a.Y[o] = a.mask && !(bf2f(a.mask[o]) > 0.f) ? (uint16_t)0 : f2bf(v);
-        if (a.Yf) a.Yf[o] = v;
+        if (a.relu) v[i] = v[i] > 0.f ? v[i] : 0.f;
+        if (co + i >= a.cout_real) v[i] = 0.f;
+        h[i] = f2bf(v[i]);
       }
+      const int64_t o = pp[r] * a.Cout + co;
+      if (a.mask) {
+        const h4u y = *(const h4u *)(a.mask + o);
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (!(bf2f(y[i]) > 0.f)) h[i] = 0;
+      }
+      if (a.Y) *(h4u *)(a.Y + o) = h;
+      if (a.Yf) st4(a.Yf + o, v);
     }
+  }
+}
+
+// weights of the data gradient as a forward layer's: Wd[tap][ci][co] = W[T-1-tap][co][ci].
+// 64 x 64 of a tap per block through LDS, so that both sides move 16 bytes a lane
+// (1024 -> 1024, 3x3: 9 us; element by element 45)
+__global__ void __launch_bounds__(256) k_flip_weights(const uint16_t *__restrict__ W, int T, int Cout, int Cin,
+                                                      uint16_t *__restrict__ Wd) {
+  __shared__ uint16_t sh[64][66];
+  const int t = blockIdx.z, co0 = blockIdx.y * 64, ci0 = blockIdx.x * 64;
+  const int64_t from = (int64_t)t * Cout * Cin, to = (int64_t)(T - 1 - t) * Cin * Cout;
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int q = threadIdx.x + 256 * k, r = q >> 3, c = (q & 7) * 8;  // 8 of a row
+    if (co0 + r >= Cout || ci0 + c >= Cin) continue;
+    const uint4 v = *(const uint4 *)(W + from + (int64_t)(co0 + r) * Cin + ci0 + c);
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) *(uint32_t *)&sh[r][c + 2 * i] = w[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 2; k++) {
+    const int q = threadIdx.x + 256 * k, r = q >> 3, c = (q & 7) * 8;
+    if (ci0 + r >= Cin || co0 + c >= Cout) continue;
+    uint32_t w[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) w[i] = (uint32_t)sh[c + 2 * i][r] | ((uint32_t)sh[c + 2 * i + 1][r] << 16);
+    *(uint4 *)(Wd + to + (int64_t)(ci0 + r) * Cout + co0 + c) = make_uint4(w[0], w[1], w[2], w[3]);
   }
 }
 
@@ -362,27 +413,63 @@ bool conv_try(fvm_ctx *ctx, ConvArgs a, int64_t want, size_t most_lds) {
   return true;
 }
 
+// Layers for k_conv_direct.  The LDS kernel wins wherever two of its blocks fit a CU;
+// a block with many slabs is alone on its CU, and what it then reaches is set by
+// rounds, blocks over 256 CUs (tiled: of its smallest patch, with the channels a
+// block is left with; direct: of 64 pixels x 64 channels).  Times in us, LDS / direct:
+//   3x3, 19 or 20 slabs: 16 channels a block.  640 -> 128, 3 x 50 x 50 (5 rounds / 1):
+//     106 / 86; 16384 pixels (8 / 2): 168 / 161; 640 -> 640, 2048 pixels (5 / 2): 104 /
+//     157.  More than 20 slabs do not fit.
+//   1x1, 13 slabs and more: 32 channels a block.  512 -> 1024, 2 x 20 x 20 (3 / 1): 17.9 /
+//     11.8; 2048 pixels (4 / 2): 23.6 / 19.1; 512 -> 256, 2048 pixels (1 / 1): 7.2 / 11.7.
+//   1x1, 11 or 12 slabs: 384 -> 384, 65536 pixels (24 / 24): 142 / 135; 3 x 50 x 50 (4 / 3):
+//     24.4 / 21.9; 16384 (6 / 6): 35.8 / 38.0.
+//   1x1 on large images is bound by reading its pixels, which the LDS kernel reads
+//     once for every 32 (fewer than 64 outputs) or 64 channels; it loses where their
+//     tile is padded most or filled from little LDS work.  131072 pixels: 80 -> 48
+//     17.9 / 11.4, 32 -> 64 16.0 / 11.3, 32 -> 128 28.5 / 19.9; but 64 -> 32 9.9 / 11.4.
+bool conv_direct(const ConvArgs &a, int K) {
+  const int slabs = (a.Cin + 31) / 32;
+  const int64_t npix = (int64_t)a.B * a.H * a.Wd, patches = (int64_t)a.B * ((a.Wd + 15) / 16) * ((a.H + 3) / 4);
+  auto rounds = [](int64_t blocks) { return (blocks + 255) / 256; };
+  auto tiled = [&](int co) { return rounds(patches * ((a.Cout + co - 1) / co)); };
+  const int64_t direct = rounds((npix + 63) / 64 * ((a.Cout + 63) / 64));
+  if (K == 3) return slabs > 18 && (slabs > 20 || tiled(16) >= 4 * direct);
+  if (slabs > 12) return 2 * tiled(32) >= 3 * direct + 2;
+  if (slabs > 10) return tiled(64) > direct || tiled(64) >= 16;
+  return npix >= 65536 && ((a.Cin < 64 && a.Cout >= 64) || (a.Cout > 32 && a.Cout < 64));
+}
+
 // The largest tile that still gives every CU a block and leaves LDS for two of
 // them (CU: 160 KB), then smaller tiles, then the smallest in any case.  A large
 // tile reads its operands least often (R + NT fragments for R NT matrix
 // instructions), but the deep levels have few pixels: 2048 at 16 x 16 and batch 8,
-// 1024 when one 256 x 256 state is predicted.
+// 1024 when one 256 x 256 state is predicted.  flip: room for the weights (TR).
 template <int K, bool TR>
-void conv_launch(fvm_ctx *ctx, const ConvArgs &a) {
+void conv_launch(fvm_ctx *ctx, const ConvArgs &a, uint16_t *flip) {
   constexpr size_t HALF = 80 << 10, ALL = 160 << 10;
-  if (a.Cout >= 64) {
-    if (conv_try<K, 4, 2, 2, TR>(ctx, a, 256, HALF) || conv_try<K, 2, 2, 2, TR>(ctx, a, 256, HALF) ||
-        conv_try<K, 1, 2, 2, TR>(ctx, a, 256, ALL))
+  if (!conv_direct(a, K)) {
+    if (a.Cout >= 64) {
+      if (conv_try<K, 4, 2, 2, TR>(ctx, a, 256, HALF) || conv_try<K, 2, 2, 2, TR>(ctx, a, 256, HALF) ||
+          conv_try<K, 1, 2, 2, TR>(ctx, a, 256, ALL))
+        return;
+    } else if (a.Cout >= 32) {
+      if (conv_try<K, 4, 2, 1, TR>(ctx, a, 512, HALF) || conv_try<K, 2, 2, 1, TR>(ctx, a, 512, HALF)) return;
+    } else if (conv_try<K, 4, 1, 1, TR>(ctx, a, 512, HALF)) {
       return;
-  } else if (a.Cout >= 32) {
-    if (conv_try<K, 4, 2, 1, TR>(ctx, a, 512, HALF) || conv_try<K, 2, 2, 1, TR>(ctx, a, 512, HALF)) return;
-  } else if (conv_try<K, 4, 1, 1, TR>(ctx, a, 512, HALF)) {
-    return;
+    }
+    if (a.Cout >= 32 && conv_try<K, 1, 1, 2, TR>(ctx, a, 128, ALL)) return;
+    if (conv_try<K, 1, 1, 1, TR>(ctx, a, 0, ALL)) return;
   }
-  if (a.Cout >= 32 && conv_try<K, 1, 1, 2, TR>(ctx, a, 128, ALL)) return;
-  if (conv_try<K, 1, 1, 1, TR>(ctx, a, 0, ALL)) return;
+  ConvArgs d = a;
+  if (TR && K == 3) {  // a layer with the channels exchanged
+    k_flip_weights<<<dim3((a.Cout + 63) / 64, (a.Cin + 63) / 64, K * K), 256, 0, ctx->stream>>>(a.W, K * K, a.Cin, a.Cout,
+                                                                                              flip);
+    d.W = flip;
+  }
   const int64_t npix = (int64_t)a.B * a.H * a.Wd;
-  k_conv_wide<K, TR><<<dim3((unsigned)((npix + 63) / 64), (unsigned)((a.Cout + 63) / 64)), 256, 0, ctx->stream>>>(a);
+  k_conv_direct<K, TR && K == 1>
+      <<<dim3((unsigned)((npix + 63) / 64), (unsigned)((a.Cout + 63) / 64)), 256, 0, ctx->stream>>>(d);
 }
 
 // ---- weight gradient --------------------------------------------------------------
@@ -877,11 +964,12 @@ static int conv_check(fvm_ctx *ctx, int B, int H, int W, int Cin, int Cout, int 
   return FVM_OK;
 }
 
-static int conv_run(fvm_ctx *ctx, const ConvArgs &a, int K, bool tr) {
+// flip: K*K*Cin*Cout bf16 of workspace for a data gradient (tr), or null
+static int conv_run(fvm_ctx *ctx, const ConvArgs &a, int K, bool tr, uint16_t *flip) {
   if ((int64_t)a.B * ((a.Wd + 15) / 16) * ((a.H + 3) / 4) > INT32_MAX)
     return fvm_set_err(ctx, FVM_ERR_ARG, "conv: too many pixels");
-  if (K == 3) tr ? conv_launch<3, true>(ctx, a) : conv_launch<3, false>(ctx, a);
-  else tr ? conv_launch<1, true>(ctx, a) : conv_launch<1, false>(ctx, a);
+  if (K == 3) tr ? conv_launch<3, true>(ctx, a, flip) : conv_launch<3, false>(ctx, a, flip);
+  else tr ? conv_launch<1, true>(ctx, a, flip) : conv_launch<1, false>(ctx, a, flip);
   FVM_LAUNCH_CHECK(ctx);
   return FVM_OK;
 }
@@ -893,18 +981,19 @@ extern "C" int fvm_nn_conv_fwd(fvm_ctx *ctx, const uint16_t *X, const uint16_t *
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
   ConvArgs a{Input{X, nullptr, Cin, 0}, W, bias, nullptr, Y, Yf, B, H, Wd, Cin, Cout, relu, cout_real > 0 ? cout_real : Cout};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  return conv_run(ctx, a, K, false);
+  return conv_run(ctx, a, K, false, nullptr);
 }
 
 // dX = conv(dY, flipped transposed W), the flip and the transposition made while
-// the weights are read (Wd_scratch, K*K*Cout*Cin bf16, is no longer written)
+// the weights are read from LDS, or into Wd_scratch (K*K*Cout*Cin bf16) where they
+// are read from memory
 extern "C" int fvm_nn_conv_dgrad(fvm_ctx *ctx, const uint16_t *dY, const uint16_t *W, uint16_t *Wd_scratch, int32_t B,
                                  int32_t H, int32_t Wd, int32_t Cin, int32_t Cout, int32_t K, uint16_t *dX) {
   if (!ctx || !dY || !W || !Wd_scratch || !dX) return FVM_ERR_ARG;
   FVM_TRY(conv_check(ctx, B, H, Wd, Cin, Cout, K));
   ConvArgs a{Input{dY, nullptr, Cout, 0}, W, nullptr, nullptr, dX, nullptr, B, H, Wd, Cout, Cin, 0, Cin};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);
-  return conv_run(ctx, a, K, true);
+  return conv_run(ctx, a, K, true, Wd_scratch);
 }
 
 // bytes of fp32 workspace fvm_nn_conv_wgrad needs
@@ -1090,12 +1179,13 @@ Input plain(const uint16_t *X, int C) { return Input{X, nullptr, C, 0}; }
 int fwd(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const Input &in, uint16_t *Y, float *Yf) {
   ConvArgs a{in, u.wb[l.at], u.b[l.at], nullptr, Y, Yf, u.B, u.H >> l.lvl, u.W >> l.lvl, l.ci, l.co, Yf ? 0 : 1,
              Yf ? u.cout_real : l.co};
-  return conv_run(ctx, a, l.K, false);
+  return conv_run(ctx, a, l.K, false, nullptr);
 }
-// data gradient of layer l, through the ReLU of the activations it took (mask, or null)
+// data gradient of layer l, through the ReLU of the activations it took (mask, or null);
+// the weight gradients' workspace is free between them and has room for the weights
 int dgrad(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const uint16_t *dY, const uint16_t *mask, uint16_t *dX) {
   ConvArgs a{plain(dY, l.co), u.wb[l.at], nullptr, mask, dX, nullptr, u.B, u.H >> l.lvl, u.W >> l.lvl, l.co, l.ci, 0, l.ci};
-  return conv_run(ctx, a, l.K, true);
+  return conv_run(ctx, a, l.K, true, (uint16_t *)u.work);
 }
 int wgrad(fvm_ctx *ctx, const fvm_unet &u, const Layer &l, const Input &in, const uint16_t *dY) {
   return wgrad_run(ctx, in, dY, u.B, u.H >> l.lvl, u.W >> l.lvl, l.ci, l.co, l.K, u.work, u.gw[l.at], u.gb[l.at]);

@@ -30,6 +30,11 @@ def _taps(x, K):
 SHAPES = [(1, 1, 1, 16, 16, 3), (1, 5, 16, 16, 32, 3), (2, 16, 16, 32, 16, 1), (1, 17, 33, 48, 48, 3),
           (3, 15, 9, 32, 64, 3), (1, 16, 20, 96, 32, 3), (2, 40, 35, 16, 16, 3), (1, 8, 8, 256, 128, 3),
           (5, 33, 18, 64, 16, 1)]
+# layers that take the direct kernel, and the first below them
+TILES = {
+    "3x3 many slabs": (7, 21, 19, 640, 144, 3), "3x3 direct": (2, 9, 11, 768, 48, 3),
+    "1x1 direct, many slabs": (40, 17, 19, 528, 80, 1), "1x1 direct, large image": (1, 259, 257, 32, 80, 1),
+}
 
 
 def _operands(shape, seed=0):
@@ -129,6 +134,33 @@ def test_data_gradient(shape):
     _check_bf16(from_bf16_bits(dX.get()), ref, K * K * co * 2.0 ** -23 * mag)
 
 
+@pytest.mark.parametrize("tile", TILES)
+def test_forward_of_each_tile(tile):
+    test_forward(TILES[tile], 1)
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_data_gradient_of_each_tile(tile):
+    B, H, W, ci, co, K = TILES[tile]
+    test_data_gradient((B, H, W, co, ci, K))    # the kernel's input is the layer's output
+
+
+@pytest.mark.parametrize("tile", TILES)
+def test_an_image_alone_gives_the_same_bits(tile):
+    """The order of an output's sums does not depend on the tile, so the last image
+    of a batch comes out alike by itself, where fewer pixels take a smaller one."""
+    print("CASE conv alone", tile, flush=True)
+    B, H, W, ci, co, K = TILES[tile]
+    X, Wt, _ = _operands(TILES[tile], 6)
+    ctx, lib = Context(), bind()
+    dW, b = _dev(ctx, Wt, np.uint16), _dev(ctx, np.random.default_rng(7).standard_normal(co).astype(np.float32), np.float32)
+    out = []
+    for x in (X, X[-1:]):
+        dX, Yf = _dev(ctx, x, np.uint16), Buf(ctx, (len(x), H, W, co), np.float32)
+        assert lib.fvm_nn_conv_fwd(ctx.h, dX.ptr, dW.ptr, b.ptr, len(x), H, W, ci, co, K, 0, co, None, Yf.ptr) == 0
+        out.append(Yf.get()[-1])
+    assert np.array_equal(*out)
+
 
 def _layerwise(net, X, dout):
     """forward and backward through the layer entry points, one call per layer."""
@@ -204,7 +236,8 @@ def _layerwise(net, X, dout):
     return out.get()
 
 
-@pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40)])
+# the last: 768 concatenated channels, which the direct kernel reads from both parents
+@pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40), (4, 64, 1, 8, 16)])
 def test_whole_passes_equal_the_layers(L, base, B, H, W):
     """The one-call passes, which fuse the copies, the concatenation and the ReLU
     passes into the kernels beside them, are bitwise the layer-by-layer ones."""
