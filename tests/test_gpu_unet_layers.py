@@ -1,6 +1,7 @@
 """The network's convolution kernels at the edges of their tiles (image sides and
 channel counts that leave remainders, one pixel, one and several patches per
-block), each against a plain float64 product of the same bf16 operands.
+block; every tile shape and the direct kernel), each against a plain float64 product
+of the same bf16 operands.
 Tolerances are the rounding bound of an fp32 sum of n products in any order,
 n 2^-23 sum |a b|, and half a bf16 step for bf16 results."""
 import numpy as np
@@ -30,10 +31,20 @@ def _taps(x, K):
 SHAPES = [(1, 1, 1, 16, 16, 3), (1, 5, 16, 16, 32, 3), (2, 16, 16, 32, 16, 1), (1, 17, 33, 48, 48, 3),
           (3, 15, 9, 32, 64, 3), (1, 16, 20, 96, 32, 3), (2, 40, 35, 16, 16, 3), (1, 8, 8, 256, 128, 3),
           (5, 33, 18, 64, 16, 1)]
-# layers that take the direct kernel, and the first below them
+# The shapes above are too few pixels for any but the smallest tile; these reach one
+# kernel each (tile rows, channel tiles, wavefronts side by side of the dispatch), with
+# image sides and output channels that leave remainders.
 TILES = {
-    "3x3 many slabs": (7, 21, 19, 640, 144, 3), "3x3 direct": (2, 9, 11, 768, 48, 3),
-    "1x1 direct, many slabs": (40, 17, 19, 528, 80, 1), "1x1 direct, large image": (1, 259, 257, 32, 80, 1),
+    "3x3 rows 4, 2 x 2": (33, 17, 19, 32, 80, 3), "3x3 rows 2, 2 x 2": (33, 17, 19, 64, 80, 3),
+    "3x3 rows 1, 2 x 2": (24, 9, 19, 96, 80, 3), "3x3 rows 4, 2 x 1": (64, 17, 19, 32, 48, 3),
+    "3x3 rows 2, 2 x 1": (64, 9, 19, 96, 48, 3), "3x3 rows 4, 1 x 1": (130, 17, 19, 32, 16, 3),
+    "3x3 rows 1, 1 x 2": (20, 7, 19, 64, 48, 3), "3x3 many slabs": (7, 21, 19, 640, 144, 3),
+    "3x3 direct": (2, 9, 11, 768, 48, 3),
+    "1x1 rows 4, 2 x 2": (33, 17, 19, 48, 80, 1), "1x1 rows 2, 2 x 2": (33, 9, 19, 160, 80, 1),
+    "1x1 rows 1, 2 x 2": (24, 9, 19, 224, 80, 1), "1x1 rows 4, 2 x 1": (66, 17, 19, 64, 48, 1),
+    "1x1 rows 2, 2 x 1": (66, 9, 19, 160, 48, 1), "1x1 rows 4, 1 x 1": (130, 17, 19, 16, 16, 1),
+    "1x1 rows 1, 1 x 2": (20, 7, 19, 64, 48, 1), "1x1 direct, many slabs": (40, 17, 19, 528, 80, 1),
+    "1x1 direct, large image": (1, 259, 257, 32, 80, 1),
 }
 
 
@@ -143,6 +154,11 @@ def test_forward_of_each_tile(tile):
 def test_data_gradient_of_each_tile(tile):
     B, H, W, ci, co, K = TILES[tile]
     test_data_gradient((B, H, W, co, ci, K))    # the kernel's input is the layer's output
+
+
+@pytest.mark.parametrize("tile", ["3x3 rows 1, 2 x 2", "3x3 many slabs", "1x1 rows 1, 2 x 2", "3x3 rows 4, 2 x 2"])
+def test_weight_gradient_of_wide_layers(tile):
+    test_weight_gradient(TILES[tile])
 
 
 @pytest.mark.parametrize("tile", TILES)
