@@ -20,8 +20,14 @@ __device__ __forceinline__ double fvm_bcg_beta(int first, double rho, const doub
 }
 
 // One iteration with the one-level preconditioner: the vectors (p, v read, p_new,
-// v_new written), the partial sums and the scalars.
+// v_new written), the partial sums (fvm_one_partials of them in each array) and the
+// scalars.
 #define FVM_ONE_BLOCKS 256
+#define FVM_ONE_TILE 32  // points a side of a block's tile
+static inline int64_t fvm_one_partials(int NX, int NY) {
+  const int64_t tiles = (int64_t)((NX + FVM_ONE_TILE - 1) / FVM_ONE_TILE) * ((NY + FVM_ONE_TILE - 1) / FVM_ONE_TILE);
+  return tiles > FVM_ONE_BLOCKS ? tiles : FVM_ONE_BLOCKS;
+}
 struct FvmBcgOne {
   double *x, *r, *s, *t, *y, *z, *p_new, *v_new;
   const double *rh, *p, *v;

@@ -32,7 +32,7 @@ constexpr int FV_NU = 4;        // sweeps on each side of the coarse correction
 constexpr int FV_POLY = 8;      // degree of the one-level preconditioner
 constexpr int FV_T = 16;        // tile of the level kernels
 constexpr int FV_R = FV_T + 2 * FV_NU;
-constexpr int FV_PT = 32;       // tile of the one-level kernels
+constexpr int FV_PT = FVM_ONE_TILE;  // tile of the one-level kernels
 constexpr int FV_PR = FV_PT + 2 * FV_POLY;
 // points of the finest level that the one-workgroup kernel takes: 33 x 33 and the
 // levels below cost 22 us, 65 x 65 44 us against 9 for two more level kernels

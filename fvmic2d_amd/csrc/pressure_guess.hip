@@ -350,11 +350,13 @@ extern "C" int fvm_pressure_guess_apply(fvm_ctx *ctx, const fvm_grid *g, const d
   return FVM_OK;
 }
 
-// workspace: 13 vectors, 5 coefficient arrays, 5 partial arrays, scalars
-static int bcg_vecs(fvm_ctx *ctx, int64_t n, BcgVecs *V, int *nblk_out) {
-  const int64_t np = (n + 63) / 64 * 64;
+// workspace: 13 vectors, 5 coefficient arrays, 5 partial arrays, scalars.  A partial
+// sum per block: of 256 rows, or of a tile of the one-level iteration, which are more
+// of them on a grid of a few rows or columns.
+static int bcg_vecs(fvm_ctx *ctx, int NX, int NY, BcgVecs *V, int *nblk_out) {
+  const int64_t n = (int64_t)NX * NY, np = (n + 63) / 64 * 64, one = fvm_one_partials(NX, NY);
   const int nblk = (int)((n + BCG_BS - 1) / BCG_BS);
-  const int64_t npart = ((int64_t)(nblk > FVM_ONE_BLOCKS ? nblk : FVM_ONE_BLOCKS) + 63) / 64 * 64;
+  const int64_t npart = ((nblk > one ? nblk : one) + 63) / 64 * 64;
   FVM_TRY(fvm_ws(ctx, ctx->scratch, (18 * np + 5 * npart + 64) * sizeof(double)));
   double *w = (double *)ctx->scratch.ptr;
   double **vecs[] = {&V->b, &V->dinv, &V->x, &V->r, &V->rh, &V->p, &V->v, &V->s, &V->t, &V->y, &V->z,
@@ -434,7 +436,7 @@ extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const
   const int64_t n = (int64_t)g->NX * g->NY;
   BcgVecs V;
   int nblk = 0;
-  FVM_TRY(bcg_vecs(ctx, n, &V, &nblk));
+  FVM_TRY(bcg_vecs(ctx, g->NX, g->NY, &V, &nblk));
   const Coef c = {V.cd, V.cr, V.cl, V.cdn, V.cup};
   const PGrid pg = pgrid(g);
   const unsigned nb = (unsigned)nblk;
@@ -468,7 +470,7 @@ int fvm_bicgstab_5pt(fvm_ctx *ctx, int NX, int NY, const double *d, const double
   const int64_t n = (int64_t)NX * NY;
   BcgVecs V;
   int nblk = 0;
-  FVM_TRY(bcg_vecs(ctx, n, &V, &nblk));
+  FVM_TRY(bcg_vecs(ctx, NX, NY, &V, &nblk));
   const Coef c = {d, e, w, sth, nth};
   const PGrid pg = PGrid{NX, NY, nullptr, nullptr, nullptr, nullptr};
   FVM_PHASE(ctx, FVM_PHASE_OTHER);

@@ -1,9 +1,11 @@
 """The nodal solves at the limits of what they take: a zero right-hand side behind
-another solve, whose leftovers lie in the workspace."""
+another solve, whose leftovers lie in the workspace; grids of a few rows or columns."""
 import ctypes as C
 
 import numpy as np
 import pytest
+import scipy.sparse as sp
+import scipy.sparse.linalg as sla
 
 from fvmic2d_amd import workloads
 from fvmic2d_amd.lib import Context, DeviceArray, DeviceGrid
@@ -40,3 +42,24 @@ def test_zero_right_hand_side(NX, NY):
     _solve(ctx, *big, _dominant(*big), 1.0 + r.random(big[::-1]))
     x, its, rel = _solve(ctx, NX, NY, _dominant(NX, NY), np.zeros((NY, NX)))
     assert not np.any(x) and its == 0 and rel == 0.0
+
+
+def _matrix(c):
+    NY, NX = c.shape[1:]
+    c = c.reshape(5, -1)
+    return sp.diags([c[0], c[1, :-1], c[2, 1:], c[3, :-NX], c[4, NX:]], [0, 1, -1, NX, -NX]).tocsc()
+
+
+# more tiles of 32 x 32 than blocks of 256 rows: fewer than 8 rows or columns, and more
+# tiles than the 256 there is always room for; the last ones reach past the scalars
+@pytest.mark.parametrize("NX,NY", [(9000, 3), (3, 9000), (8300, 7), (2, 40000), (40000, 2)])
+def test_thin_grids(NX, NY):
+    """Against the direct solve: couplings of 0.2 leave a condition number below 9, so
+    a relative residual of 1e-12 bounds the error in the 2-norm by 9e-12."""
+    print("CASE thin grid", NX, NY, flush=True)
+    c, b = 2.0 * _dominant(NX, NY), np.random.default_rng(4).standard_normal((NY, NX))
+    c[0] = 1.0
+    x, its, rel = _solve(Context(), NX, NY, c, b)
+    ref = sla.spsolve(_matrix(c), b.ravel())
+    assert rel <= 1e-12 and its <= 12, (its, rel)
+    assert np.linalg.norm(x.ravel() - ref) <= 9e-12 * np.linalg.norm(ref)
