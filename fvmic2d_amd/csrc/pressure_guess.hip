@@ -373,8 +373,8 @@ static int bcg_vecs(fvm_ctx *ctx, int NX, int NY, BcgVecs *V, int *nblk_out) {
 // convergence themselves; the host enqueues a few iterations (5 to 30 are needed
 // with a preconditioner, hundreds without) between two looks, each of which costs
 // about 25 us of an idle GPU.  Without a preconditioner, or where that has not
-// converged after PRECOND_MAXIT iterations, Jacobi takes its place.  it_out: of the
-// run that gave x.
+// converged after PRECOND_MAXIT iterations, Jacobi takes its place from x = 0 for
+// what is left of maxit.  it_out: the iterations of both.
 #define PRECOND_MAXIT 60
 template <class Start>
 static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs &V, int64_t n, int nblk,
@@ -420,11 +420,15 @@ static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs 
       ahead = pre ? 2 : ahead;
     }
   };
+  int32_t spent = 0;
   if (m) {
     FVM_TRY(run(m, maxit < PRECOND_MAXIT ? maxit : PRECOND_MAXIT, 4));
-    if (*rel_out <= rtol) return FVM_OK;
+    spent = *it_out;
+    if (*rel_out <= rtol || spent >= maxit) return FVM_OK;
   }
-  return run(nullptr, maxit, 16);
+  FVM_TRY(run(nullptr, maxit - spent, 16));
+  *it_out += spent;
+  return FVM_OK;
 }
 
 extern "C" int fvm_initial_pressure_guess(fvm_ctx *ctx, const fvm_grid *g, const double *rho, double gy, double gx,

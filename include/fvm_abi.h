@@ -304,7 +304,8 @@ int fvm_form_thermal_system(fvm_ctx *ctx, const fvm_grid *g, const NodalArrays *
                             const Options *opt, double dt, int32_t doSteady, double *coef, double *rhs);
 /* The "energy_" solve of that system (the reference uses a direct LU through
  * its options file): BiCGStab from T = 0 on the system with every row divided by
- * its diagonal, to rtol relative residual of that scaled system.
+ * its diagonal, to rtol relative residual of that scaled system, in at most maxit
+ * iterations (iters and maxit as in fvm_initial_pressure_guess).
  * Synchronises; FVM_ERR_NOT_CONVERGED when rtol is not met (T is written). */
 int fvm_solve_thermal_system(fvm_ctx *ctx, const fvm_grid *g, const double *coef, const double *rhs, double *T,
                              double rtol, int32_t maxit, int32_t *iters, double *relres);
@@ -419,7 +420,8 @@ int fvm_timer_stop(fvm_ctx *ctx, float *ms);
  * assembled as in initialPressureGuess.c:59-135 (dummy rows on ix == 0 and
  * jy == 0, pressure pinned in cell (3, 3), zero-flux sides, dp/dy = rho g on
  * top and bottom), solved on the GPU (matrix-free operator, multigrid BiCGStab,
- * relative residual <= rtol, at most maxit iterations).  rho: device NX*NY
+ * relative residual <= rtol, at most maxit iterations in all, counted in iters: a
+ * preconditioned run that gave way to Jacobi's is part of them).  rho: device NX*NY
  * nodal density.  The pressure goes to S[3*(jy*NX+ix) + 2] (the DOF_P slot of
  * the interleaved [vx, vy, p] Stokes vector, fdcode.h:242-245; velocities are
  * left untouched) and/or p_out (NX*NY); either may be NULL but not both.

@@ -22,13 +22,16 @@ def _dominant(NX, NY):
     return c
 
 
-def _solve(ctx, NX, NY, coef, rhs, rtol=1e-12, maxit=2000):
+NOT_CONVERGED = 11
+
+
+def _solve(ctx, NX, NY, coef, rhs, rtol=1e-12, maxit=2000, code=0):
     """(T, iterations, relative residual) of fvm_solve_thermal_system."""
     grid = DeviceGrid(ctx, workloads.thermal_box(NX, NY))
     d = [DeviceArray(ctx, np.ascontiguousarray(a).ravel()) for a in (coef, rhs, np.full(NX * NY, 7.0))]
     its, rel = C.c_int32(-1), C.c_double(-1.0)
-    ctx.call("fvm_solve_thermal_system", grid.ref, *(C.c_void_p(a.ptr) for a in d), C.c_double(rtol),
-             C.c_int32(maxit), C.byref(its), C.byref(rel))
+    assert ctx.lib.fvm_solve_thermal_system(ctx.h, grid.ref, *(C.c_void_p(a.ptr) for a in d), C.c_double(rtol),
+                                            C.c_int32(maxit), C.byref(its), C.byref(rel)) == code
     return d[2].get().reshape(NY, NX), its.value, rel.value
 
 
@@ -63,3 +66,25 @@ def test_thin_grids(NX, NY):
     ref = sla.spsolve(_matrix(c), b.ravel())
     assert rel <= 1e-12 and its <= 12, (its, rel)
     assert np.linalg.norm(x.ravel() - ref) <= 9e-12 * np.linalg.norm(ref)
+
+
+def _poisson(NX, NY):
+    c = np.zeros((5, NY, NX))
+    c[0] = 4.0
+    c[1, :, :-1] = c[2, :, 1:] = c[3, :-1] = c[4, 1:] = -1.0
+    return c
+
+
+@pytest.mark.parametrize("maxit", [1, 3, 5])
+def test_maxit_bounds_all_iterations(maxit):
+    """Where maxit ends the preconditioned iteration no other one follows: x is its x,
+    whose residual Jacobi's would be far from (its first iterations hardly lower it on
+    a Poisson problem)."""
+    print("CASE maxit", maxit, flush=True)
+    NX, NY = 60, 40
+    c, b = _poisson(NX, NY), np.ones((NY, NX))
+    x, its, rel = _solve(Context(), NX, NY, c, b, rtol=1e-15, maxit=maxit, code=NOT_CONVERGED)
+    assert its == maxit
+    b = b.ravel() / 4.0
+    true = np.linalg.norm(b - _matrix(c / 4.0) @ x.ravel()) / np.linalg.norm(b)
+    assert rel <= 0.3 ** maxit and abs(true - rel) <= 1e-12
