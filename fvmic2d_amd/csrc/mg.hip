@@ -674,7 +674,8 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   m->one_level = !scale && m->lo >= DOMINANT && nn <= INT32_MAX;  // its kernels take a unit diagonal
   if (m->one_level) {
     push(NX, NY, c, nullptr, nullptr, nullptr);
-    m->poly = cheb(m->lo, 2.0 - m->lo, FV_POLY);
+    const double lo = m->lo < 0.99 ? m->lo : 0.99;  // rows without couplings: not an empty interval
+    m->poly = cheb(lo, 2.0 - lo, FV_POLY);
     *out = m;
     return FVM_OK;
   }

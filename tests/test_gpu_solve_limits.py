@@ -1,5 +1,6 @@
 """The nodal solves at the limits of what they take: a zero right-hand side behind
-another solve, whose leftovers lie in the workspace; grids of a few rows or columns."""
+another solve, whose leftovers lie in the workspace; grids of a few rows or columns;
+few iterations; rows without couplings."""
 import ctypes as C
 
 import numpy as np
@@ -88,3 +89,16 @@ def test_maxit_bounds_all_iterations(maxit):
     b = b.ravel() / 4.0
     true = np.linalg.norm(b - _matrix(c / 4.0) @ x.ravel()) / np.linalg.norm(b)
     assert rel <= 0.3 ** maxit and abs(true - rel) <= 1e-12
+
+
+@pytest.mark.parametrize("coupling", [0.0, 1e-30, 1e-17, 1e-9])
+def test_rows_with_next_to_no_couplings(coupling):
+    """The interval of the polynomial does not close on the spectrum {1}: the first
+    iteration solves the rows (an error below the couplings, which rtol exceeds)."""
+    print("CASE couplings of", coupling, flush=True)
+    NX, NY = 40, 33
+    c, b = coupling * 10.0 * _dominant(NX, NY), np.random.default_rng(5).standard_normal((NY, NX))
+    c[0] = 2.0
+    x, its, rel = _solve(Context(), NX, NY, c, b, rtol=1e-8)
+    assert its == 1 and rel <= 1e-8
+    assert np.linalg.norm(x - b / 2.0) <= 2e-8 * np.linalg.norm(b / 2.0)
