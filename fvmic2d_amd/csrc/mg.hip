@@ -536,13 +536,32 @@ __global__ void __launch_bounds__(256) k_coarsen(Lv L, double *__restrict__ ce, 
   idc[q] = id;
 }
 
+// sums and least value over a block of 256, in thread 0
+__device__ __forceinline__ void rows_block(double &sx, double &sy, double &lo, double &skew, double (*sh)[4]) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    sx += __shfl_xor(sx, o);
+    sy += __shfl_xor(sy, o);
+    lo = fmin(lo, __shfl_xor(lo, o));
+    skew += __shfl_xor(skew, o);
+  }
+  const int w = threadIdx.x >> 6;
+  if ((threadIdx.x & 63) == 0) sh[0][w] = sx, sh[1][w] = sy, sh[2][w] = lo, sh[3][w] = skew;
+  __syncthreads();
+  sx = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+  sy = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
+  lo = fmin(fmin(sh[2][0], sh[2][1]), fmin(sh[2][2], sh[2][3]));
+  skew = (sh[3][0] + sh[3][1]) + (sh[3][2] + sh[3][3]);
+}
+
 // rows divided by their diagonal, and per block what the choice of a
-// preconditioner needs: the sums of |e| + |w| and |s| + |n|, the least row sum
-__global__ void __launch_bounds__(256) k_rows(int64_t n, const double *__restrict__ d, Coefs c, double *__restrict__ e,
-                                              double *__restrict__ w, double *__restrict__ s, double *__restrict__ nn,
-                                              double *__restrict__ part) {
+// preconditioner needs: the sums of |e| + |w| and |s| + |n|, the least row sum, the
+// pairs of couplings of opposite signs (a skew part)
+__global__ void __launch_bounds__(256) k_rows(int64_t n, int NX, const double *__restrict__ d, Coefs c,
+                                              double *__restrict__ e, double *__restrict__ w, double *__restrict__ s,
+                                              double *__restrict__ nn, double *__restrict__ part) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  double sx = 0.0, sy = 0.0, lo = 1.0;
+  double sx = 0.0, sy = 0.0, lo = 1.0, skew = 0.0;
   if (i < n) {
     const double di = d[i];
     const Pt p = {c.e[i] / di, c.w[i] / di, c.s[i] / di, c.n[i] / di};
@@ -551,43 +570,31 @@ __global__ void __launch_bounds__(256) k_rows(int64_t n, const double *__restric
     sy = fabs(p.s) + fabs(p.n);
     lo = 1.0 - sx - sy;
     if (!(lo == lo)) lo = -1.0;  // NaN rows: no bound
+    auto opposite = [&](double to, const double *back, int64_t j) {
+      return to != 0.0 && j < n && (to < 0.0) != (back[j] < 0.0 != d[j] < 0.0) && back[j] != 0.0 ? 1.0 : 0.0;
+    };
+    skew = opposite(p.e, c.w, i + 1) + opposite(p.s, c.n, i + NX);
   }
-  __shared__ double sh[3][4];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sx += __shfl_xor(sx, o);
-    sy += __shfl_xor(sy, o);
-    lo = fmin(lo, __shfl_xor(lo, o));
-  }
-  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = sx, sh[1][threadIdx.x >> 6] = sy, sh[2][threadIdx.x >> 6] = lo;
-  __syncthreads();
+  __shared__ double sh[4][4];
+  rows_block(sx, sy, lo, skew, sh);
   if (threadIdx.x == 0) {
-    part[blockIdx.x] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
-    part[gridDim.x + blockIdx.x] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
-    part[2 * gridDim.x + blockIdx.x] = fmin(fmin(sh[2][0], sh[2][1]), fmin(sh[2][2], sh[2][3]));
+    part[blockIdx.x] = sx;
+    part[gridDim.x + blockIdx.x] = sy;
+    part[2 * gridDim.x + blockIdx.x] = lo;
+    part[3 * gridDim.x + blockIdx.x] = skew;
   }
 }
 __global__ void __launch_bounds__(256) k_rows_total(int nb, const double *__restrict__ part, double *__restrict__ out) {
-  double sx = 0.0, sy = 0.0, lo = 1.0;
+  double sx = 0.0, sy = 0.0, lo = 1.0, skew = 0.0;
   for (int k = threadIdx.x; k < nb; k += 256) {
     sx += part[k];
     sy += part[nb + k];
     lo = fmin(lo, part[2 * nb + k]);
+    skew += part[3 * nb + k];
   }
-  __shared__ double sh[3][4];
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    sx += __shfl_xor(sx, o);
-    sy += __shfl_xor(sy, o);
-    lo = fmin(lo, __shfl_xor(lo, o));
-  }
-  if ((threadIdx.x & 63) == 0) sh[0][threadIdx.x >> 6] = sx, sh[1][threadIdx.x >> 6] = sy, sh[2][threadIdx.x >> 6] = lo;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    out[0] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
-    out[1] = (sh[1][0] + sh[1][1]) + (sh[1][2] + sh[1][3]);
-    out[2] = fmin(fmin(sh[2][0], sh[2][1]), fmin(sh[2][2], sh[2][3]));
-  }
+  __shared__ double sh[4][4];
+  rows_block(sx, sy, lo, skew, sh);
+  if (threadIdx.x == 0) out[0] = sx, out[1] = sy, out[2] = lo, out[3] = skew;
 }
 
 Cheb cheb(double a, double b, int steps) {
@@ -630,12 +637,16 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   // least row sum from which the finest level alone is preconditioned: degree
   // FV_POLY then contracts every component about as well as a V-cycle does
   constexpr double DOMINANT = 0.05;
+  // least row sum from which the polynomial damps all of the disc |z - 1| <= 1 - lo by
+  // 5 or more: |T8| <= 577 on the unit disc, T8(1 / 0.6) = 3280.  Rows with couplings
+  // +-0.1 (sum 0.6): 171 us, Jacobi 430; +-0.17 (0.32): 585 and 428 (300 x 200)
+  constexpr double SKEW_DOMINANT = 0.4;
   *out = nullptr;
   const int64_t nn = (int64_t)NX * NY;
   const unsigned nb = fvm_blocks(nn, 256);
   // the finest level's rows and sweeps, the levels below (at most half the
   // points each, and a column and row more)
-  const size_t words = (size_t)(5 * padded(nn) + padded(3 * (int64_t)nb) + 64) +
+  const size_t words = (size_t)(5 * padded(nn) + padded(4 * (int64_t)nb) + 64) +
                        8 * (size_t)(nn + 24 * ((int64_t)NX + NY) + 4096);
   FVM_TRY(fvm_ws(ctx, ctx->mg, words * sizeof(double)));
   double *p = (double *)ctx->mg.ptr, *end = p + words;
@@ -649,19 +660,23 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   if (!m) return fvm_set_err(ctx, FVM_ERR_NOMEM, "preconditioner");
   m->lv.clear(), m->b.clear(), m->x.clear(), m->y.clear();
   m->first_coarse = 0;
-  double *part = take(3 * (int64_t)nb), *tot = take(4);
+  double *part = take(4 * (int64_t)nb), *tot = take(4);
   double *rows[4] = {nullptr, nullptr, nullptr, nullptr};
   Coefs c = {e, w, s, n};
   if (scale)
     for (int k = 0; k < 4; k++) rows[k] = take(nn);
-  k_rows<<<nb, 256, 0, ctx->stream>>>(nn, d, c, rows[0], rows[1], rows[2], rows[3], part);
+  k_rows<<<nb, 256, 0, ctx->stream>>>(nn, NX, d, c, rows[0], rows[1], rows[2], rows[3], part);
   k_rows_total<<<1, 256, 0, ctx->stream>>>((int)nb, part, tot);
   FVM_LAUNCH_CHECK(ctx);
   double *host = (double *)ctx->pinned.ptr;
-  FVM_HIP(ctx, hipMemcpyAsync(host, tot, 3 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
+  FVM_HIP(ctx, hipMemcpyAsync(host, tot, 4 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
   FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
   double sx = host[0], sy = host[1];
   m->lo = host[2];
+  // Both kinds are made for a spectrum near the real axis.  On rows with couplings of
+  // opposite signs it is not, and they would cost more than they give (an iteration's
+  // polynomial can grow what it should damp) unless the row sums keep it small.
+  if (host[3] > 0.0 && m->lo < SKEW_DOMINANT) return FVM_OK;
   if (scale) c = Coefs{rows[0], rows[1], rows[2], rows[3]};
   auto push = [&](int nx, int ny, const Coefs &co, double *b, double *x, double *y) {
     Lv L{};

@@ -372,10 +372,15 @@ static int bcg_vecs(fvm_ctx *ctx, int NX, int NY, BcgVecs *V, int *nblk_out) {
 // BiCGStab from the state that `start` sets up (x = 0).  The kernels decide
 // convergence themselves; the host enqueues a few iterations (5 to 30 are needed
 // with a preconditioner, hundreds without) between two looks, each of which costs
-// about 25 us of an idle GPU.  Without a preconditioner, or where that has not
-// converged after PRECOND_MAXIT iterations, Jacobi takes its place from x = 0 for
-// what is left of maxit.  it_out: the iterations of both.
+// about 25 us of an idle GPU.  Without a preconditioner, or where that does not get
+// there, Jacobi takes its place from x = 0 for what is left of maxit: after
+// PRECOND_MAXIT iterations, or as soon as a look finds the residual PRECOND_LOST times
+// b.  Rows that it solves stay below (Poisson and energy equations below 1, Helmholtz
+// shifts up to 70); upwind rows of cell Peclet number 10, which it does not, pass it within
+// some ten iterations.  40 x 33 of those: 5.8 ms with all 60 tried, 2.2 now (Jacobi alone 1.7).
+// it_out: the iterations of both.
 #define PRECOND_MAXIT 60
+#define PRECOND_LOST 200.0
 template <class Start>
 static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs &V, int64_t n, int nblk,
                     const fvm_precond *m, double rtol, int32_t maxit, int32_t *it_out, double *rel_out, Start start) {
@@ -417,6 +422,7 @@ static int bcg_loop(fvm_ctx *ctx, const PGrid &pg, const Coef &c, const BcgVecs 
       *it_out = (int32_t)host[FVM_S_ITS];
       *rel_out = bnorm > 0.0 ? sqrt(host[FVM_S_RR]) / bnorm : 0.0;
       if (!(*rel_out > rtol) || it >= most) return FVM_OK;  // also stops on NaN
+      if (pre && *rel_out > PRECOND_LOST) return FVM_OK;
       ahead = pre ? 2 : ahead;
     }
   };
