@@ -22,7 +22,6 @@
 // below FV_COARSE_MAX points is one workgroup's kernel, and around the one-level
 // polynomial the whole iteration is three kernels.
 #include <new>
-#include <vector>
 
 #include "bicgstab.h"
 
@@ -39,6 +38,7 @@ constexpr int FV_PR = FV_PT + 2 * FV_POLY;
 constexpr int FV_COARSE_MAX = 1100;
 constexpr int FV_CT = 512;      // threads of the coarse kernel
 constexpr int FV_CLEVELS = 16;
+constexpr int FV_LEVELS = 64;
 constexpr int FV_LAST = 12;     // sweeps on the last level
 
 struct Coefs {
@@ -620,10 +620,11 @@ int64_t padded(int64_t n) { return (n + 31) / 32 * 32; }
 struct fvm_precond {
   double lo = 0.0;             // least row sum
   bool one_level = false;      // the polynomial on the finest level
-  std::vector<Lv> lv;          // finest first
+  int n_lv = 0;                // each halves an axis at least: 2 x 31 of them at most
+  Lv lv[FV_LEVELS];            // finest first
   // per level: right-hand side (not the finest's), the sweeps before its
   // correction, the result (not the finest's)
-  std::vector<double *> b, x, y;
+  double *b[FV_LEVELS], *x[FV_LEVELS], *y[FV_LEVELS];
   int first_coarse = 0;        // level at which the one-workgroup kernel takes over
   CoarseArgs coarse;
   Cheb smooth, last, poly;
@@ -648,7 +649,15 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   // points each, and a column and row more)
   const size_t words = (size_t)(5 * padded(nn) + padded(4 * (int64_t)nb) + 64) +
                        8 * (size_t)(nn + 24 * ((int64_t)NX + NY) + 4096);
-  FVM_TRY(fvm_ws(ctx, ctx->mg, words * sizeof(double)));
+  // without room for the levels, or with more rows than a grid has blocks for, the
+  // solve runs without them
+  if (nn > INT32_MAX || fvm_blocks(NY, FV_T) > 65535u) return FVM_OK;
+  const int rc = fvm_ws(ctx, ctx->mg, words * sizeof(double));
+  if (rc == FVM_ERR_NOMEM) {
+    (void)hipGetLastError();
+    return FVM_OK;
+  }
+  FVM_TRY(rc);
   double *p = (double *)ctx->mg.ptr, *end = p + words;
   auto take = [&](int64_t k) {
     double *r = p;
@@ -658,8 +667,7 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   if (!ctx->precond) ctx->precond = new (std::nothrow) fvm_precond();
   fvm_precond *m = ctx->precond;
   if (!m) return fvm_set_err(ctx, FVM_ERR_NOMEM, "preconditioner");
-  m->lv.clear(), m->b.clear(), m->x.clear(), m->y.clear();
-  m->first_coarse = 0;
+  m->n_lv = m->first_coarse = 0;
   double *part = take(4 * (int64_t)nb), *tot = take(4);
   double *rows[4] = {nullptr, nullptr, nullptr, nullptr};
   Coefs c = {e, w, s, n};
@@ -681,12 +689,11 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   auto push = [&](int nx, int ny, const Coefs &co, double *b, double *x, double *y) {
     Lv L{};
     L.NX = nx, L.NY = ny, L.c = co, L.fx = L.fy = 1;
-    m->lv.push_back(L);
-    m->b.push_back(b);
-    m->x.push_back(x);
-    m->y.push_back(y);
+    m->lv[m->n_lv] = L;
+    m->b[m->n_lv] = b, m->x[m->n_lv] = x, m->y[m->n_lv] = y;
+    m->n_lv++;
   };
-  m->one_level = !scale && m->lo >= DOMINANT && nn <= INT32_MAX;  // its kernels take a unit diagonal
+  m->one_level = !scale && m->lo >= DOMINANT;  // its kernels take a unit diagonal
   if (m->one_level) {
     push(NX, NY, c, nullptr, nullptr, nullptr);
     const double lo = m->lo < 0.99 ? m->lo : 0.99;  // rows without couplings: not an empty interval
@@ -698,8 +705,8 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
   m->smooth = cheb(0.1, 2.0, FV_NU);
   m->last = cheb(0.1, 2.0, FV_LAST);
   for (;;) {
-    Lv &f = m->lv.back();
-    if ((int64_t)f.NX * f.NY <= 20 || (f.NX <= 3 && f.NY <= 3)) break;
+    Lv &f = m->lv[m->n_lv - 1];
+    if (m->n_lv == FV_LEVELS || (int64_t)f.NX * f.NY <= 20 || (f.NX <= 3 && f.NY <= 3)) break;
     f.fx = f.NX > 3 ? 2 : 1, f.fy = f.NY > 3 ? 2 : 1;
     if (f.fx == 2 && f.fy == 2) {
       if (sx > SEMI * sy) f.fy = 1, sx /= 4.0;
@@ -713,12 +720,11 @@ int fvm_precond_build(fvm_ctx *ctx, int NX, int NY, const double *d, const doubl
     f.idc = id;
     k_coarsen<<<fvm_blocks(nc, 256), 256, 0, ctx->stream>>>(f, ce, cw, cs, cn, id);
     FVM_LAUNCH_CHECK(ctx);
-    const int nx = f.NXc, ny = f.NYc;  // f dies with the push
     double *b = take(nc), *x = take(nc), *y = take(nc);
-    push(nx, ny, Coefs{ce, cw, cs, cn}, b, x, y);
+    push(f.NXc, f.NYc, Coefs{ce, cw, cs, cn}, b, x, y);
   }
   // the one-workgroup kernel takes the levels that fit its LDS and threads
-  const int n_lv = (int)m->lv.size();
+  const int n_lv = m->n_lv;
   for (int l = 0; l < n_lv; l++) {
     if ((int64_t)m->lv[l].NX * m->lv[l].NY > FV_COARSE_MAX || n_lv - l > FV_CLEVELS) continue;
     CoarseArgs &A = m->coarse;

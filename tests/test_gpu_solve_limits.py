@@ -147,3 +147,18 @@ def test_rows_of_other_kinds(rows, most):
     assert rel <= 1e-12 and its <= most, (its, rel)
     b = (b / c[0]).ravel()
     assert np.linalg.norm(b - _matrix(c / c[0]) @ x.ravel()) <= 1e-10 * np.linalg.norm(b)
+
+
+def test_more_rows_than_the_levels_have_blocks_for():
+    """1048600 rows of tiles of 16: the solve runs without the levels.  Couplings of 0.9
+    and 2 x 0.03 leave a condition number of 49, so a relative residual of 1e-12 bounds
+    the error in the 2-norm by 5e-11."""
+    print("CASE 2 x 1048600", flush=True)
+    NX, NY = 2, 1048600
+    c = np.zeros((5, NY, NX))
+    c[0] = 1.0
+    c[1, :, :-1] = c[2, :, 1:] = -0.9
+    c[3, :-1] = c[4, 1:] = -0.03
+    x = np.random.default_rng(8).standard_normal((NY, NX))
+    got, _, rel = _solve(Context(), NX, NY, c, (_matrix(c) @ x.ravel()).reshape(NY, NX))
+    assert rel <= 1e-12 and np.linalg.norm(got - x) <= 5e-11 * np.linalg.norm(x)
