@@ -1134,7 +1134,7 @@ extern "C" int fvm_nn_f32_to_bf16(fvm_ctx *ctx, int64_t n, const float *x, uint1
 // One call per pass, instead of one per layer: the host's part of a pass shrinks to its
 // launches, and the layers' copies, concatenations and ReLU passes go into the
 // kernels beside them.  Tensors are NHWC bf16 unless noted, level i at H >> i, W >> i.
-#define NN_LEVELS 8
+#define NN_LEVELS 12  // the 13th, with 65536 channels at 16 on the first, fits no card
 typedef struct {
   int32_t levels, B, H, W, cin, cout, cout_real;
   int32_t ch[NN_LEVELS];

@@ -41,7 +41,7 @@ _SIGS = {
     "fvm_nn_unet_backward": [P, P],
     "fvm_nn_adam_all": [P, I32, P, P, P, P, P, P, P, F, F, F, F, I32],
 }
-LEVELS = 8
+LEVELS = 12     # of csrc/unet.hip; the weights of more fit no card
 
 
 class fvm_unet(C.Structure):
@@ -106,6 +106,8 @@ class UNet:
     """Parameters, activations and the layer sequence of the learned guess."""
 
     def __init__(self, ctx=None, levels=4, base=32, cin=5, cout=3, seed=0):
+        if not 1 <= levels <= LEVELS:
+            raise ValueError("UNet: 1 to %d levels" % LEVELS)
         self.ctx = ctx or Context()
         self.lib = bind()
         self.L, self.c = levels, base

@@ -252,8 +252,17 @@ def _layerwise(net, X, dout):
     return out.get()
 
 
-# the last: 768 concatenated channels, which the direct kernel reads from both parents
-@pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40), (4, 64, 1, 8, 16)])
+class _Same(int):
+    """As many channels on every level (levels of their own size would be gigabytes)."""
+
+    def __mul__(self, factor):
+        return int(self)
+
+
+# the fourth: 768 concatenated channels, which the direct kernel reads from both
+# parents; then deep ones, to the most levels there are
+@pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40), (4, 64, 1, 8, 16),
+                                          (9, _Same(16), 1, 256, 256), (12, _Same(16), 1, 2048, 2048)])
 def test_whole_passes_equal_the_layers(L, base, B, H, W):
     """The one-call passes, which fuse the copies, the concatenation and the ReLU
     passes into the kernels beside them, are bitwise the layer-by-layer ones."""
@@ -272,3 +281,9 @@ def test_whole_passes_equal_the_layers(L, base, B, H, W):
     assert np.array_equal(out, _layerwise(net, _dev(net.ctx, X, np.uint16), net.A["dout"]))
     for name, (gw, gb) in net.grads_numpy().items():
         assert np.array_equal(grads[name][0], gw) and np.array_equal(grads[name][1], gb), name
+
+
+def test_more_levels_than_there_are_places():
+    """Refused before anything is allocated."""
+    with pytest.raises(ValueError):
+        UNet(levels=13, base=16)
