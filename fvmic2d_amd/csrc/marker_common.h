@@ -97,6 +97,7 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     // wavefronts in flight.
     int cellX = c0x, cellY = c0y;
     asm volatile("" : "+v"(cellX), "+v"(cellY));
+    double xg0, xg1, yg0, yg1;  // the cell's corners
     {
       const int lx = PER ? cellX - 1 : max(cellX - 1, 0), ly = max(cellY - 1, 0);
       const int hx = PER ? cellX + 2 : min(cellX + 2, NX - 1), hy = min(cellY + 2, NY - 1);
@@ -118,11 +119,16 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
         if (sy < 0)
           while (ycur < g.y[cellY] && cellY > 0) cellY--;
       }
+      if (PER && !on) {  // coordinates in memory: what has been read is not read again
+        xg0 = sx > 0 ? x1 : (sx < 0 ? xm1 : x0), xg1 = sx > 0 ? x2 : (sx < 0 ? x0 : x1);
+        yg0 = sy > 0 ? y1 : (sy < 0 ? ym1 : y0), yg1 = sy > 0 ? y2 : (sy < 0 ? y0 : y1);
+      } else {
+        xg0 = g.x[cellX], xg1 = g.x[cellX + 1], yg0 = g.y[cellY], yg1 = g.y[cellY + 1];
+      }
     }
     // the half cells: cellY in [0, NY-2], cellX in [0, NX-2] (PER: [-1, NX-1]), so
     // the reference's clamps of vxX, vxY, vyX and vyY change nothing
     const int vxX = cellX, vyY = cellY;
-    const double xg0 = g.x[cellX], xg1 = g.x[cellX + 1], yg0 = g.y[cellY], yg1 = g.y[cellY + 1];
     const double xc0 = g.xc[PER ? max(cellX, 0) : cellX], xc1 = g.xc[cellX + 1], xc2 = g.xc[cellX + 2];
     const double yc0 = g.yc[cellY], yc1 = g.yc[cellY + 1], yc2 = g.yc[cellY + 2];
     const bool up = ycur < yc1, left = (!PER || cellX > -1) && xcur < xc1;
