@@ -419,7 +419,8 @@ bool conv_try(fvm_ctx *ctx, ConvArgs a, int64_t want, size_t most_lds) {
 // block is left with; direct: of 64 pixels x 64 channels).  Times in us, LDS / direct:
 //   3x3, 19 or 20 slabs: 16 channels a block.  640 -> 128, 3 x 50 x 50 (5 rounds / 1):
 //     106 / 86; 16384 pixels (8 / 2): 168 / 161; 640 -> 640, 2048 pixels (5 / 2): 104 /
-//     157.  More than 20 slabs do not fit.
+//     157.  More than 20 slabs do not fit.  A data gradient turns its weights first
+//     (640 -> 640, 2 x 20 x 20, 4 / 1: 87 / 92).
 //   1x1, 13 slabs and more: 32 channels a block.  512 -> 1024, 2 x 20 x 20 (3 / 1): 17.9 /
 //     11.8; 2048 pixels (4 / 2): 23.6 / 19.1; 512 -> 256, 2048 pixels (1 / 1): 7.2 / 11.7.
 //   1x1, 11 or 12 slabs: 384 -> 384, 65536 pixels (24 / 24): 142 / 135; 3 x 50 x 50 (4 / 3):
@@ -428,27 +429,31 @@ bool conv_try(fvm_ctx *ctx, ConvArgs a, int64_t want, size_t most_lds) {
 //     once for every 32 (fewer than 64 outputs) or 64 channels; it loses where their
 //     tile is padded most or filled from little LDS work.  131072 pixels: 80 -> 48
 //     17.9 / 11.4, 32 -> 64 16.0 / 11.3, 32 -> 128 28.5 / 19.9; but 64 -> 32 9.9 / 11.4.
-bool conv_direct(const ConvArgs &a, int K) {
+bool conv_direct(const ConvArgs &a, int K, bool tr) {
   const int slabs = (a.Cin + 31) / 32;
   const int64_t npix = (int64_t)a.B * a.H * a.Wd, patches = (int64_t)a.B * ((a.Wd + 15) / 16) * ((a.H + 3) / 4);
   auto rounds = [](int64_t blocks) { return (blocks + 255) / 256; };
   auto tiled = [&](int co) { return rounds(patches * ((a.Cout + co - 1) / co)); };
   const int64_t direct = rounds((npix + 63) / 64 * ((a.Cout + 63) / 64));
-  if (K == 3) return slabs > 18 && (slabs > 20 || tiled(16) >= 4 * direct);
+  if (K == 3) return slabs > 18 && (slabs > 20 || tiled(16) >= 4 * direct + (tr ? 1 : 0));
   if (slabs > 12) return 2 * tiled(32) >= 3 * direct + 2;
   if (slabs > 10) return tiled(64) > direct || tiled(64) >= 16;
   return npix >= 65536 && ((a.Cin < 64 && a.Cout >= 64) || (a.Cout > 32 && a.Cout < 64));
 }
 
-// The largest tile that still gives every CU a block and leaves LDS for two of
-// them (CU: 160 KB), then smaller tiles, then the smallest in any case.  A large
-// tile reads its operands least often (R + NT fragments for R NT matrix
-// instructions), but the deep levels have few pixels: 2048 at 16 x 16 and batch 8,
-// 1024 when one 256 x 256 state is predicted.  flip: room for the weights (TR).
+// The largest tile with blocks enough for the chip that leaves LDS for two of them on a
+// CU (160 KB): 256 of 512 threads (64 channels side by side), 512 of 256 threads; then
+// smaller tiles, 128 of the last but one, the smallest in any case.  A large tile reads
+// its operands least often (R + NT fragments for R NT matrix instructions), but the
+// deep levels have few pixels: 2048 at 16 x 16 and batch 8, 1024 when one 256 x 256
+// state is predicted.  Over 980 layers (16 to 384 channels, 16 x 16 to 256 x 256 pixels,
+// both directions) half these numbers of blocks cost 1 to 11 % by kind of layer, twice
+// them 2 to 13 %, a quarter or four times 0 to 13 % and 3 to 11 %.
+// flip: room for the weights (TR).
 template <int K, bool TR>
 void conv_launch(fvm_ctx *ctx, const ConvArgs &a, uint16_t *flip) {
   constexpr size_t HALF = 80 << 10, ALL = 160 << 10;
-  if (!conv_direct(a, K)) {
+  if (!conv_direct(a, K, TR)) {
     if (a.Cout >= 64) {
       if (conv_try<K, 4, 2, 2, TR>(ctx, a, 256, HALF) || conv_try<K, 2, 2, 2, TR>(ctx, a, 256, HALF) ||
           conv_try<K, 1, 2, 2, TR>(ctx, a, 256, ALL))
@@ -488,7 +493,9 @@ void conv_launch(fvm_ctx *ctx, const ConvArgs &a, uint16_t *flip) {
 // and have 64 co x 64 ci between them.  Blocks split the patches (`nchunk`) to fill
 // the chip; their fp32 partials, and those of the bias, are added in chunk order
 // by k_wgrad_reduce.  What bounds it is getting the patches in: all loads of a
-// patch are issued together, and two blocks of a CU overlap.
+// patch are issued together, and two blocks of a CU overlap.  Two blocks leave 256
+// registers a lane, of which the sums of 64 x 64 channels (K = 3) take 144 and a patch on
+// its way 76: that form spills 85 (320 bytes a lane), read and written once a patch.
 // Before, every bf16 was gathered from global memory by itself and one thread
 // summed a weight's partials over all chunks: one optimiser step's 15 gradients at
 // batch 8, 128 x 128 took 3.29 ms; now 0.43.
