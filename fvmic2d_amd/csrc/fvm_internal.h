@@ -615,6 +615,3 @@ __device__ __forceinline__ int guess_grid(const double *__restrict__ x, int N, d
   }
   return done ? i : bisect_grid(x, N, X);
 }
-
-// deterministic double sum of n values on the device -> *out (host), ops.hip
-int fvm_reduce_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out);

@@ -699,16 +699,6 @@ static int enqueue_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out) {
   return FVM_OK;
 }
 
-int fvm_reduce_sum(fvm_ctx *ctx, const double *d, int64_t n, double *out) {
-  *out = 0.0;
-  if (n <= 0) return FVM_OK;
-  double *h = (double *)ctx->pinned.ptr + 8;
-  FVM_TRY(enqueue_sum(ctx, d, n, h));
-  FVM_HIP(ctx, hipStreamSynchronize(ctx->stream));
-  *out = *h;
-  return FVM_OK;
-}
-
 // ---- A12: updateGlobalStrainRateResidual (residual.c:12-51) --------------------
 __global__ void k_residual_area(DGrid g, double *__restrict__ srr) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
