@@ -5,7 +5,9 @@ equation).  The solution is compared with the direct solve of the oracle's
 system.  Tolerance: the solves stop at a relative residual of 1e-12; the
 condition numbers of these systems stay below 1e6 relative to it, and the
 solution's largest value is of the order of its norm, so 1e-6 covers the
-residual with room and 1e-8, the bar of the other solve tests, is kept."""
+residual with room and 1e-8, the bar of the other solve tests, is kept.  The bounds on
+the iterations are below what Jacobi's, which takes over where a preconditioner fails,
+needs on the same system (3 and more), so a broken preconditioner does not pass."""
 import numpy as np
 import pytest
 import scipy.sparse.linalg as sla
@@ -29,10 +31,10 @@ class Box:
 
 # smallest grid; one workgroup; its largest and the first beyond it; both axes
 # with remainders; y, then x much the stronger axis; a graded grid
-@pytest.mark.parametrize("NX,NY,LX,tanh", [(5, 5, 1.0, False), (33, 33, 1.0, False), (34, 37, 1.0, False),
-                                           (66, 65, 1.0, False), (97, 131, 1.0, True), (40, 150, 1.0, False),
-                                           (150, 40, 1.0, False), (129, 65, 2.0, True)])
-def test_pressure_guess_shapes(NX, NY, LX, tanh):
+@pytest.mark.parametrize("NX,NY,LX,tanh,most", [
+    (5, 5, 1.0, False, 7), (33, 33, 1.0, False, 10), (34, 37, 1.0, False, 10), (66, 65, 1.0, False, 10),
+    (97, 131, 1.0, True, 16), (40, 150, 1.0, False, 10), (150, 40, 1.0, False, 10), (129, 65, 2.0, True, 16)])
+def test_pressure_guess_shapes(NX, NY, LX, tanh, most):
     print("CASE pressure guess", NX, NY, LX, tanh, flush=True)
     ctx = Context()
     w = Box(NX, NY, LX, 1.0, tanh)
@@ -42,14 +44,14 @@ def test_pressure_guess_shapes(NX, NY, LX, tanh):
     ref = sla.spsolve(A.tocsc(), b)
     p = DeviceArray(ctx, np.zeros(NX * NY))
     its, rel = initial_pressure_guess(ctx, DeviceGrid(ctx, w), DeviceArray(ctx, rho), 9.81, gx=0.2, rtol=1e-12, p_out=p)
-    assert rel <= 1e-12 and its <= 60, (its, rel)
+    assert rel <= 1e-12 and its <= most, (its, rel)
     np.testing.assert_allclose(p.get(), ref, rtol=0, atol=1e-8 * np.abs(ref).max())
 
 
 # dt scales the diagonal's share: the one-level polynomial, then the V-cycle
-@pytest.mark.parametrize("NX,NY,top,dt", [(32, 32, 0, 1.0), (33, 65, 1, 1.0), (100, 47, 0, 3.0), (101, 90, 1, 1e4),
-                                          (64, 70, 0, 1e4)])
-def test_energy_shapes(NX, NY, top, dt):
+@pytest.mark.parametrize("NX,NY,top,dt,most", [(32, 32, 0, 1.0, 2), (33, 65, 1, 1.0, 4), (100, 47, 0, 3.0, 2),
+                                               (101, 90, 1, 1e4, 10), (64, 70, 0, 1e4, 10)])
+def test_energy_shapes(NX, NY, top, dt, most):
     print("CASE energy", NX, NY, top, dt, flush=True)
     w = workloads.thermal_box(NX, NY, top_type=top)
     mp = MarkerPath(w)
@@ -61,13 +63,13 @@ def test_energy_shapes(NX, NY, top, dt):
     A, b = TH.thermal_system(w.x, w.y, w.nodal, w.materials.materialRho[0], w.options, w.dt * dt, False,
                              w.nodal["heating"])
     ref = sla.spsolve(A.tocsc(), b)
-    assert rel <= 1e-12 and its <= 60, (its, rel)
+    assert rel <= 1e-12 and its <= most, (its, rel)
     assert np.abs(T.get().ravel() - ref).max() <= 1e-8 * np.abs(ref).max()
 
 
 def test_rows_the_preconditioner_cannot_bound_still_solve():
-    """Couplings twice the diagonal's: the polynomial's interval does not hold the
-    spectrum; the solve falls back on Jacobi."""
+    """Couplings twice the diagonal's, of opposite signs: no preconditioner is made for
+    them; Jacobi's iterations solve the system."""
     print("CASE energy solve of a system that is not diagonally dominant", flush=True)
     w = workloads.thermal_box(12, 9)
     mp = MarkerPath(w)
