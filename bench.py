@@ -581,16 +581,18 @@ def bench_pressure_guess(a):
            "config": {"workload": "pressure_guess_box", "grid": main_row["grid"],
                       "solver": "BiCGStab preconditioned by a multigrid V-cycle, rtol 1e-10"},
            "grids": rows,
-           # one iteration touches about 80 FP64 values per node: 37 in the iteration's
-           # own vectors and coefficients, 16 on the fine level of each of its two
-           # V-cycles (residual, correction, coefficients, down and up) and a third of
-           # those again on the coarser levels; a 257 x 257 problem stays in cache, so
-           # what bounds it is the chain of launches and the coarse levels' barriers
-           "roofline": {"bound": "hbm", "kernel": "BiCGStab iteration with two V-cycles",
-                        "achieved": 80 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
+           # one iteration touches about 73 FP64 values per node: 37 in the iteration's
+           # own vectors and coefficients, 13.5 on the fine level of each of its two
+           # V-cycles (down: right-hand side and 4 coefficients -> x, a quarter of a coarse
+           # right-hand side; up: those five, x, a quarter of a correction -> x) and a third
+           # of those again on the coarser levels.  A 257 x 257 problem stays in cache, so
+           # these bytes do not come from memory: what bounds it is the chain of
+           # launches and the coarse levels' barriers
+           "roofline": {"bound": "latency", "kernel": "BiCGStab iteration with two V-cycles",
+                        "achieved": 73 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
                         / (main_row["gpu_ms"] * 1e-3) / 1e9,
                         "peak": 8000.0, "unit": "GB/s",
-                        "frac": 80 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
+                        "frac": 73 * 8 * int(main_row["grid"].split("x")[0]) ** 2 * main_row["iterations"]
                         / (main_row["gpu_ms"] * 1e-3) / 1e9 / 8000.0, "traffic": None},
            "cpu_baseline": None if a.no_cpu else {
                "value": main_row["cpu_direct_ms"], "unit": "ms", "cores": 1, "kind": "port",
@@ -612,11 +614,11 @@ def vep_algorithmic_bytes(w):
     return {
         # findMarkerCells + density loop: read X, Y, T, Mat; write cellX, cellY, cpu, rho, rhodot
         "locate": n * (16 + 8 + 4 + 12 + 16),
-        # subgrid T pass 2: read X, Y, cellX, cellY, T, dTsub; write T, Tdot; gather deltaT
-        "subgrid_t2": n * (16 + 8 + 16 + 16) + nodes * 8,
-        # RK4: read X, Y, cellX, cellY, s(3), e(3), Eii; write X, Y, VX, VY, wxy, s(3), Eii;
-        # gather vx, vy, wxy
-        "advect": n * (80 + 72) + nodes * 24,
+        # RK4 with subgrid T pass 2 in front and the subgrid stress changes, the stress
+        # update and the rotation behind: read X, Y, cellX, cellY, T, dTsub, s(3), the
+        # changes (3), e(3), Eii; write T, Tdot, X, Y, VX, VY, wxy, s(3), Eii; gather
+        # deltaT, vx, vy, wxy and the increments of s(3)
+        "advect": n * (120 + 88) + nodes * 56,
     }
 
 

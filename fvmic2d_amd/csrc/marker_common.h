@@ -6,12 +6,6 @@
 #pragma once
 #include "fvm_internal.h"
 
-// ---- A6: advectMarkersRK (markers.c:1865-2250) --------------------------------
-// PER: x periodic (g.per == 1).  The walk may then leave [0, NX-1] by one cell
-// (XCMIN = -1, XCMAX = NX-1, markers.c:1908-1915), the staggered x indices are
-// not clamped (:1965-1971), node columns wrap, the left-wall ghost rule is off
-// (:2014-2023) and the new X is wrapped into [0, LX] (:2225-2231).  The grid
-// coordinates are then read at indices -1 .. NX+1 (set by makePeriodic).
 // Quotients by a shared divisor.  n / d is rcp(d) refined by two Newton steps, a
 // product and a correction: eleven instructions with the operand scaling and the
 // special cases, once for each quotient.  A stage has two quotients for each of
@@ -32,9 +26,15 @@ struct Spacing {
   }
 };
 
-// c0x, c0y, X0, Y0: the marker's stored cell and position (the caller reads them,
-// a marker ahead where it can).  tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's stages are done, with
-// its old position and cell and its new spin.
+// ---- A6: advectMarkersRK (markers.c:1865-2250) --------------------------------
+// PER: x periodic (g.per == 1).  The walk may then leave [0, NX-1] by one cell
+// (XCMIN = -1, XCMAX = NX-1, markers.c:1908-1915), the staggered x indices are
+// not clamped (:1965-1971), node columns wrap, the left-wall ghost rule is off
+// (:2014-2023) and the new X is wrapped into [0, LX] (:2225-2231).  The grid
+// coordinates are then read at indices -1 .. NX+1 (set by makePeriodic).
+// c0x, c0y, X0, Y0: the marker's stored cell and position (the caller reads them, a
+// marker ahead where it can).  tail(m, g, X0, Y0, cellX, cellY, wxy) runs once a marker's
+// stages are done, with its old position and cell and its new spin.
 template <bool PER, class Tail>
 __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
     double *__restrict__ MX,
@@ -78,10 +78,13 @@ __device__ __forceinline__ void advect_marker(int64_t m, const DGrid &g,
   // expression's left-to-right order as the stages complete
   double svx = 0.0, svy = 0.0, swxy = 0.0;
   // the stages stay a loop: unrolled, they held 116-126 VGPRs (four waves per
-  // SIMD); rolled, 96 at most (five).  At 1.44 M markers on 201 x 201 nodes the
-  // pass takes 58 us, about 24 of them its columns and 8-9 each stage, where the
-  // SIMDs issue FP64 nearly all the time; it took 72 (12 a stage) with eight whole
-  // divisions, the walk as loops and the three fields' gathers one after another.
+  // SIMD); rolled and held to 96 (five), the forms with the coordinates in LDS and
+  // the periodic one with the rotation spill two (a lane writes 8 bytes once: 5.8 of
+  // the 291 MB moved by the case below).  At 1.44 M markers on 201 x 201 nodes a stage
+  // takes 8-9 us and the columns about 24: 58 us without a tail, 86 with the rotation
+  // behind it, the VALU busy 76 % of that.  Without a tail it took 72 (12 a stage) with
+  // eight whole divisions, the walk as loops and the three fields' gathers one after
+  // another.
   const bool top0 = bv.mechBCTop.type[0] == 0, top1 = bv.mechBCTop.type[0] == 1;
   const bool left0 = bv.mechBCLeft.type[1] == 0, left1 = bv.mechBCLeft.type[1] == 1;
   const double top2 = 2.0 * bv.mechBCTop.value[0], left2 = 2.0 * bv.mechBCLeft.value[1];
