@@ -260,8 +260,10 @@ class _Same(int):
 
 
 # the fourth: 768 concatenated channels, which the direct kernel reads from both
-# parents; then deep ones, to the most levels there are
+# parents; then its data gradients through a ReLU, 3x3 and 1x1; then deep ones, to the
+# most levels there are
 @pytest.mark.parametrize("L,base,B,H,W", [(2, 16, 2, 6, 14), (2, 48, 1, 10, 18), (4, 16, 3, 24, 40), (4, 64, 1, 8, 16),
+                                          (5, 64, 1, 16, 32), (1, 64, 1, 256, 272),
                                           (9, _Same(16), 1, 256, 256), (12, _Same(16), 1, 2048, 2048)])
 def test_whole_passes_equal_the_layers(L, base, B, H, W):
     """The one-call passes, which fuse the copies, the concatenation and the ReLU
